@@ -58,7 +58,7 @@ def listed():
         # A scan that keeps suggestive pairs (p < 1e-4): many hits to decide, collect and sort.
         _case("suggestive", nid=3001, nsnp=12007, nchr=3, pval=1e-4, phen="t5", keep=32768),
         # A large cohort over a candidate region, safe mode.
-        _case("biobank", nid=50000, nsnp=4001, safe=True, phen="binary"),
+        _case("biobank", nid=50000, nsnp=4001, safe=True, phen="binary", pval=1e-6),
         # A new study from host memory: upload, transcode, phenotype preparation, scan.
         _case("new_study", kind="load", nid=2000, nsnp=20001, nchr=4, ymiss=0.01),
         # Sixteen independent small studies in one call.
