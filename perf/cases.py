@@ -19,8 +19,8 @@ A case is a dict of plain values:
   safe    the reference's safe mode (-9 is a value, no condition on the number of cells)
   ndata, nphen   kind "batch": datasets, and phenotypes of each
   keep    rows of the table into which the program copies a scan's hits, in their order
-Genotypes come in blocks of SNPs in linkage disequilibrium, with either allele counted; a few pairs
-of SNPs carry an effect on the phenotype.
+Genotypes come in blocks of SNPs in linkage disequilibrium, with either allele counted; three pairs of
+SNPs and one single SNP carry an effect on the phenotype.
 """
 import math
 
@@ -181,12 +181,20 @@ def _codes(case, nid, nsnp, seed):
 
 
 def _phenotypes(case, codes, seed):
-    """(nphen, nid) float32 phenotypes (NaN missing); three SNP pairs shift the trait in one cell."""
+    """(nphen, nid) float32 phenotypes (NaN missing): three SNP pairs interact in heterozygotes without main
+    effects, and one SNP has an additive effect of its own."""
     nsnp, nid = codes.shape
     rng = np.random.default_rng(seed)
     pairs = [rng.choice(nsnp, 2, replace=False) for _ in range(3)]
     rows = codes[torch.as_tensor(np.concatenate(pairs), device="cuda")].cpu().numpy()
-    effect = sum((rows[2 * i] == 1) & (rows[2 * i + 1] == 1) for i in range(3)) * (12.0 / math.sqrt(nid))
+
+    def unit(x):
+        x = x - x.mean()
+        return x / max(x.std(), 1e-3)
+
+    het = [unit(r == 1) for r in rows]
+    effect = sum(unit(het[2 * i] * het[2 * i + 1]) for i in range(3)) * (11.0 / math.sqrt(nid))
+    effect += unit(np.where(rows[0] == 3, 1, rows[0]).astype(float)) * (5.0 / math.sqrt(nid))
     ys = []
     for _ in range(case["nphen"]):
         d = case["phen"]
