@@ -12,7 +12,9 @@
 //     vbits [Kw]    uint32 phenotype-present bits
 //     marg  [nsnp]  Marg   per-SNP class counts and sums
 //     oidx, ocodes, ov     outlier individuals (at most OUT_MAX), their codes per SNP and values
-//     mp    [Kp]    MissPhen V, q, z per individual (SPARSE tiles)
+//     mp    [Kp]    MissPhen V, q, z per individual (SPARSE tiles), coarse phenotype v of the screen
+//     sw    [Kw][SW_ROW] uint32  the screen's FP6 codes of v and presence bits, per 32 individuals
+//     sm    [nsnp]  ScrMarg per-SNP counts and sums of v
 //   for SPARSE tiles (built at the first scan that has them, for the chromosome layout it was built for):
 //     moff  [nsnp+1] int64, mlist int32   per SNP, the individuals with a missing call
 //     vidx  [nsnp]  int32  virtual SNP index: each chromosome starts at a multiple of 64
@@ -34,6 +36,7 @@
 #include "kern_batch.h"
 #include "kern_mfma.h"
 #include "kern_plain.h"
+#include "kern_screen.h"
 #include "transcode.h"
 
 using namespace epi;
@@ -67,6 +70,11 @@ struct PhenDev {
     uint32_t *ocodes = nullptr; // [ceil(nout/16)][nsnp], built with the marginals
     OutVals *ov = nullptr;
     MissPhen *mp = nullptr;
+    uint32_t *sw = nullptr;     // screen
+    ScrMarg *sm = nullptr;
+    double sdelta = 0.0;        // q ~ sdelta v
+    double seps = 0.0;          // |r - mean(r)|, r = q - sdelta v (q units)
+    double svsum = 0.0;         // sum of v
     int nout = 0;
     int fbits = 0;  // q = round((y - centre) * 2^fbits)
     int zbits = 0;  // Z limbs hold round(q^2 / 2^zbits)
@@ -129,6 +137,10 @@ struct epi_ctx {
     unsigned long long *nhits = nullptr;
     long long cap = 1ll << 22;
     long long last_nhits = 0;
+    // screened scans: counters (behind nhits), candidates, regions to redo (behind the tiles)
+    uint32_t *scount = nullptr;
+    int4 *cand = nullptr;
+    uint32_t *redo = nullptr;
     // tiles; the device list of the last scan is kept and reused while the
     // dataset, block range, form and schedule stay the same
     int4 *tiles = nullptr;
@@ -235,6 +247,8 @@ void free_phen(PhenDev &p)
     dfree(p.ocodes);
     dfree(p.ov);
     dfree(p.mp);
+    dfree(p.sw);
+    dfree(p.sm);
 }
 
 void drop_sparse(Dataset &d)
@@ -363,9 +377,82 @@ struct PhenEnc {
     std::vector<uint32_t> vb;   // [Kw]
     std::vector<int32_t> oidx;  // outlier individuals
     std::vector<MissPhen> mp;   // [Kp]
+    std::vector<uint32_t> sw;   // [Kw][SW_ROW]
     OutVals ov = {};
     PhenDev p;                  // scalars only
 };
+
+// Coarse phenotype of the screen. Digits: the integers that FP6 E2M3 holds in
+// units of 1/8 (0..16, even to 30, multiples of 4 to 60, either sign).
+int fp6_nearest(double t)
+{
+    const double a = std::fabs(t);
+    const int st = a <= 16.0 ? 1 : a <= 31.0 ? 2 : 4;
+    const int v = std::min(60, st * (int)std::floor(a / st + 0.5));
+    return t < 0.0 ? -v : v;
+}
+
+uint32_t fp6_code(int d)
+{
+    const int a = std::abs(d);
+    const uint32_t c = a < 16 ? (uint32_t)a : a < 32 ? 16u + (uint32_t)(a / 2 - 8) : 24u + (uint32_t)(a / 4 - 8);
+    return c | (d < 0 ? 32u : 0u);
+}
+
+constexpr int SCR_VMAX = 32 * 60 + 60;
+
+// v = 32 D1 + D0 nearest to q / delta for every present individual, with
+// delta the smallest that keeps |v| <= SCR_VMAX and the sum of |v| below 2^24
+// (with room for the rounding), so that every sum of v in FP32 is exact.
+void encode_screen(const std::vector<int> &P, int Kw, PhenEnc &e)
+{
+    PhenDev &p = e.p;
+    double mx = 0.0, sum = 0.0;
+    for (int k : P) {
+        const double a = std::fabs((double)e.qv[k]);
+        mx = std::max(mx, a);
+        sum += a;
+    }
+    const double room = 16777216.0 - 2.0 * (double)P.size();  // each |v| exceeds |q| / delta by at most 2
+    p.sdelta = std::max(mx / SCR_VMAX, room > 1.0 ? sum / room : 0.0);
+    if (!(p.sdelta > 0.0) || room <= 1.0) p.sdelta = 0.0;  // constant phenotype or a huge cohort: not screened
+    e.sw.assign((size_t)Kw * SW_ROW, 0u);
+    if (p.sdelta == 0.0) return;
+    double rs = 0.0, rq = 0.0;
+    for (int k : P) {
+        const double t = (double)e.qv[k] / p.sdelta;
+        int hi = 0, lo = 0;
+        double best = INFINITY;
+        const int h0 = fp6_nearest(t / 32.0);
+        for (int dh : {0, -1, 1, -2, 2, -4, 4}) {
+            const int h = fp6_nearest((double)(h0 + dh)), l = fp6_nearest(t - 32.0 * h);
+            const double err = std::fabs(t - (32.0 * h + l));
+            if (err < best) {
+                best = err;
+                hi = h;
+                lo = l;
+            }
+            if (best <= 0.5) break;
+        }
+        const int v = 32 * hi + lo;
+        e.mp[k].sv = v;
+        p.svsum += v;
+        const double r = (double)e.qv[k] - p.sdelta * v;
+        rs += r;
+        rq += r * r;
+        // the element of individual k & 31: six bits from bit 6 slot of the word's 192
+        const int bit = 6 * scr_slot(k & 31);
+        uint32_t *row = e.sw.data() + (size_t)(k >> 5) * SW_ROW;
+        const int d[2] = {lo, hi};
+        for (int i = 0; i < 2; i++) {
+            const uint64_t c = (uint64_t)fp6_code(d[i]) << (bit & 31);
+            row[6 * i + (bit >> 5)] |= (uint32_t)c;
+            if (c >> 32) row[6 * i + (bit >> 5) + 1] |= (uint32_t)(c >> 32);
+        }
+        row[12] |= 1u << (k & 31);
+    }
+    p.seps = std::sqrt(std::max(0.0, rq - rs * rs / (double)P.size())) * (1.0 + 1e-6);
+}
 
 // Phenotype prep (src/EpiOpenCL.c:1364-1376 computes mY and SSY over all nid
 // and the kernel drops -9 values, :135-147; here the missing values are
@@ -487,6 +574,7 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
         y2 += (double)ycf * (double)ycf;
         e.vb[k >> 5] |= 1u << (k & 31);
     }
+    encode_screen(P, Kw, e);
     for (int t = 0; t < p.nout; t++) {
         const double u = std::ldexp((double)y[e.oidx[t]] - centre, f);
         e.ov.d[t] = u;
@@ -530,7 +618,7 @@ int ds_set_phenotypes(epi_ctx *c, Dataset &d, const float *phen, int nphen, int 
         p = e.p;
         if ((rc = dalloc(c, p.wts, e.w.size())) || (rc = dalloc(c, p.qv, (size_t)Kp)) ||
             (rc = dalloc(c, p.yc, (size_t)Kp)) || (rc = dalloc(c, p.vbits, (size_t)Kw)) ||
-            (rc = dalloc(c, p.ov, 1)) || (rc = dalloc(c, p.mp, (size_t)Kp)))
+            (rc = dalloc(c, p.ov, 1)) || (rc = dalloc(c, p.mp, (size_t)Kp)) || (rc = dalloc(c, p.sw, e.sw.size())))
             break;
         if (p.nout && (rc = dalloc(c, p.oidx, (size_t)p.nout))) break;
         hipError_t he = hipMemcpyAsync(p.wts, e.w.data(), e.w.size(), hipMemcpyHostToDevice, c->stream);
@@ -541,6 +629,8 @@ int ds_set_phenotypes(epi_ctx *c, Dataset &d, const float *phen, int nphen, int 
         if (he == hipSuccess) he = hipMemcpyAsync(p.ov, &e.ov, sizeof(OutVals), hipMemcpyHostToDevice, c->stream);
         if (he == hipSuccess)
             he = hipMemcpyAsync(p.mp, e.mp.data(), (size_t)Kp * sizeof(MissPhen), hipMemcpyHostToDevice, c->stream);
+        if (he == hipSuccess)
+            he = hipMemcpyAsync(p.sw, e.sw.data(), e.sw.size() * 4, hipMemcpyHostToDevice, c->stream);
         if (he == hipSuccess && p.nout)
             he = hipMemcpyAsync(p.oidx, e.oidx.data(), (size_t)p.nout * 4, hipMemcpyHostToDevice, c->stream);
         if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
@@ -589,10 +679,11 @@ int ds_marginals(epi_ctx *c, Dataset &d)
     if (d.ph.empty()) return fail(c, EPI_ERR_STATE, "phenotypes not set");
     for (auto &p : d.ph) {
         int rc = dalloc(c, p.marg, (size_t)d.nsnp);
+        if (!rc) rc = dalloc(c, p.sm, (size_t)d.nsnp);
         if (rc) return rc;
         hipLaunchKernelGGL(marginals_kernel, dim3((d.nsnp + 63) / 64), dim3(256), 0, c->stream,
                            (const uint32_t *)d.mbits, d.Kw, d.nsnp, (const uint32_t *)p.vbits, (const int32_t *)p.qv,
-                           (const float *)p.yc, (const int32_t *)d.cls, (const MissPhen *)p.mp, p.marg);
+                           (const float *)p.yc, (const int32_t *)d.cls, (const MissPhen *)p.mp, p.marg, p.sm);
         HIPCHK(c, hipGetLastError());
         if (p.nout) {
             if ((rc = dalloc(c, p.ocodes, (size_t)(p.nout + 15) / 16 * d.nsnp))) return rc;
@@ -909,12 +1000,16 @@ int copy_tiles(epi_ctx *c, int4 *dst, const TileLists &tl)
 int upload_tiles(epi_ctx *c, const TileLists &tl)
 {
     c->tl_valid = false;
-    size_t need = tl.count();
+    // behind the tiles, room for every region of the screen's tiles (four of 4 bytes, at most, per tile)
+    const size_t nt = tl.count(), need = nt + tl.fast.size();
+    static_assert(sizeof(int4) == 64 / SCR_A * sizeof(uint32_t), "a tile's regions take the room of a tile");
     if (need > c->tiles_cap) {
+        c->tiles_cap = 0;
         int rc = dalloc(c, c->tiles, need);
         if (rc) return rc;
         c->tiles_cap = need;
     }
+    c->redo = reinterpret_cast<uint32_t *>(c->tiles + nt);
     return copy_tiles(c, c->tiles, tl);
 }
 
@@ -970,15 +1065,94 @@ int check_params(epi_ctx *c, const epi_scan_params *p)
         }                                                                                                \
     } while (0)
 
-// Device buffers of a scan's pair kernels: the tile list, the hit records and the hit counter.
+// Device buffers of a scan's pair kernels: the tile list, the hit records and the hit counter, and
+// the screen's sink (no screen without it).
 struct ScanBufs {
     int4 *tiles;
     DevHit *hits;
     unsigned long long *nhits;
     long long cap;
+    CandSink cs;
 };
 
-ScanBufs ctx_bufs(const epi_ctx *c) { return {c->tiles, c->hits, c->nhits, c->cap}; }
+constexpr uint32_t CAND_CAP = 1u << 20;  // 16 MiB of candidates; beyond it regions are redone by the exact tiles
+
+ScanBufs ctx_bufs(const epi_ctx *c)
+{
+    return {c->tiles, c->hits, c->nhits, c->cap, {c->cand, c->scount, CAND_CAP, c->redo}};
+}
+
+// Lanes per candidate of resolve_kernel for a cohort of Kl individuals (one 32-individual word each).
+int resolve_lanes(int Kl)
+{
+    int g = 4;
+    while (g < 64 && g * 32 < Kl) g *= 2;
+    return g;
+}
+
+// Upper tail of chi-square with 2 h degrees of freedom.
+double chi2_tail(double x, int h)
+{
+    double t = 1.0, sum = 1.0;
+    for (int j = 1; j < h; j++) sum += t *= 0.5 * x / j;
+    return std::exp(-0.5 * x) * sum;
+}
+
+// The screen's cut for a phenotype and the scan's thresholds; false where the
+// exact tiles are the better path: thresholds so low, or a cohort so large for
+// the coarse phenotype's residue, that more than SCR_RATE of the pairs of
+// unrelated SNPs would be candidates.
+constexpr double SCR_RATE = 2e-3;
+// Pairs times individuals below which the screen's two further launches cost more than its
+// kernel saves (N = 1000, M = 1000: 20.5 us either way; N = 300, M = 2000: 25.9 us exact, 18.0 us screened).
+constexpr double SCR_MIN_WORK = 5e8;
+
+bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
+{
+    const HitSink hs = make_sink(nullptr, nullptr, 0, q);
+    if (p.nout || p.sdelta <= 0.0 || p.nV < 32 || !(hs.t1s > 0.0f)) return false;
+    const bool inter = q->test != 'f';
+    if (inter && !(hs.t2s > 0.0f)) return false;
+    if (!std::isfinite(hs.t1s) || (inter && !std::isfinite(hs.t2s))) return false;
+    const double N = p.nV, qV = (double)p.qV, sst = p.sqV - qV * qV / N, sig2 = sst / (N - 1.0);
+    if (!(sst > 0.0)) return false;
+    const double unit = 64.0 * p.sdelta * p.sdelta;  // q^2 units per unit of the kernels' sums of squares
+    // lower bound on SSB(v) of a pair with nfac occupied cells that passes
+    auto floor_f = [&](int nfac) {
+        const double k = (double)hs.t1s * (nfac - 1);
+        return std::sqrt(k / (N - nfac + k) * sst);
+    };
+    auto floor_i = [&](int nfac) {
+        const double k = 4.0 * (double)hs.t2s;
+        return std::sqrt(k / (N - nfac + k) * sst);
+    };
+    auto cut = [&](double root) { return std::pow(std::max(0.0, root - p.seps), 2); };
+    double rate = chi2_tail(cut(floor_f(9)) / sig2, 4);
+    if (inter) rate += chi2_tail(cut(floor_i(9)) / sig2, 2);
+    if (rate > SCR_RATE) return false;
+    memset(&C, 0, sizeof(C));
+    const double T = p.svsum / 64.0, T2N = T * T / (N / 64.0);
+    auto level0 = [&](int nfac) {
+        const double root = inter ? std::min(floor_f(nfac), floor_i(nfac)) : floor_f(nfac);
+        return (cut(root) / unit + T2N) * (1.0 - 1e-5);
+    };
+    const double thr9 = level0(9);
+    double slope = 0.0;
+    for (int k = inter && !q->safe ? 7 : 2; k < 9; k++) slope = std::max(slope, (thr9 - level0(k)) / (9 - k));
+    C.N = (float)(N / 64.0);
+    C.T = (float)T;
+    C.T2N = (float)T2N;
+    C.thr9 = (float)thr9;
+    C.slope = (float)(slope * (1.0 + 1e-5));
+    C.eps = (float)(p.seps / (8.0 * p.sdelta) * (1.0 + 1e-6));
+    C.sst = (float)(sst / unit * (1.0 - 1e-6));
+    C.nv = (float)N;
+    C.t1s = hs.t1s;
+    C.t2s = hs.t2s;
+    C.test = q->test;
+    C.safe = hs.safe;
+    return true;
+}
 
 // Launch the pair kernels of one scan over the uploaded tile lists (fast tiles first).
 template <bool DUMP>
@@ -1000,12 +1174,48 @@ int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, c
         A.hs = hs;
         A.ds = ds;
         if (ns && !d.sp_ok) return fail(c, EPI_ERR_STATE, "SPARSE tile data not built");
+        ScreenArgs G;
+        bool screen = !DUMP && nf && B.cs.cand && (double)nf * sc.fast_rows * TILE_B * A.S.Kl >= SCR_MIN_WORK &&
+                      (unsigned long long)d.Kw * d.nsnp * 8ull < (1ull << 32) - (1u << 20) &&
+                      screen_cut(d.ph[p->phen], p, G.cut);
+        if (screen) {
+            G.S = A.S;
+            G.sw = d.ph[p->phen].sw;
+            G.sm = d.ph[p->phen].sm;
+            G.cs = B.cs;
+            ResolveArgs R = {A.S, nullptr, hs, B.cs.cand, B.cs.count, B.cs.cap, resolve_lanes(A.S.Kl)};
+            const int4 *tiles = B.tiles;
+            for (int t0 = 0; t0 < nf;) {
+                const int nt = sc.fast_rows == 64 ? screen_threads<64>() : screen_threads<32>();
+                const int chunk = std::min((int)((1u << 31) / (unsigned)nt) & ~255, nf - t0);
+                G.tiles = tiles + t0;
+                G.ntiles = chunk;
+                G.tile0 = t0;
+                if (sc.fast_rows == 64)
+                    hipLaunchKernelGGL((screen_fast_kernel<64>), dim3(chunk), dim3(nt), 0, c->stream, G);
+                else
+                    hipLaunchKernelGGL((screen_fast_kernel<32>), dim3(chunk), dim3(nt), 0, c->stream, G);
+                HIPCHK(c, hipGetLastError());
+                c->last_launches++;
+                t0 += chunk;
+            }
+            hipLaunchKernelGGL((resolve_kernel<false, false>), dim3(4 * c->ncu), dim3(256), 0, c->stream, R);
+            HIPCHK(c, hipGetLastError());
+            if (sc.fast_rows == 64)
+                hipLaunchKernelGGL((redo_fast_kernel<64>), dim3(2 * c->ncu), dim3(fast_threads<32>()), 0, c->stream, A.S, hs,
+                                   tiles, (const uint32_t *)B.cs.count, (const uint32_t *)B.cs.redo);
+            else
+                hipLaunchKernelGGL((redo_fast_kernel<32>), dim3(2 * c->ncu), dim3(fast_threads<32>()), 0, c->stream, A.S, hs,
+                                   tiles, (const uint32_t *)B.cs.count, (const uint32_t *)B.cs.redo);
+            HIPCHK(c, hipGetLastError());
+            c->last_launches += 2;
+        }
         if (sc.fast_rows == 64) {
-            LAUNCH_TILES((mfma_fast_kernel<64, DUMP>), fast_threads<64>(), A, B.tiles, nf);
+            if (!screen) LAUNCH_TILES((mfma_fast_kernel<64, DUMP>), fast_threads<64>(), A, B.tiles, nf);
             LAUNCH_TILES((mfma_sparse_kernel<64, DUMP>), sparse_threads<64>(), A, B.tiles + nf, ns);
             LAUNCH_TILES((mfma_general_kernel<64, DUMP>), general_threads<64>(), A, B.tiles + nf + ns, ng);
         } else {
-            LAUNCH_TILES((mfma_fast_kernel<32, DUMP>), fast_threads<32>(), A, B.tiles, nf);
+            if (!screen) LAUNCH_TILES((mfma_fast_kernel<32, DUMP>), fast_threads<32>(), A, B.tiles, nf);
             LAUNCH_TILES((mfma_sparse_kernel<32, DUMP>), sparse_threads<32>(), A, B.tiles + nf, ns);
             LAUNCH_TILES((mfma_general_kernel<32, DUMP>), general_threads<32>(), A, B.tiles + nf + ns, ng);
         }
@@ -1349,7 +1559,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc)
             c->tl_sched = sc;
         }
     }
-    HIPCHK(c, hipMemsetAsync(c->nhits, 0, sizeof(unsigned long long), c->stream));
+    HIPCHK(c, hipMemsetAsync(c->nhits, 0, 2 * sizeof(unsigned long long), c->stream));  // and the screen's counters
     DumpSink ds;
     memset(&ds, 0, sizeof(ds));
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -1365,6 +1575,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc)
         tl = TileLists();
         done = build_tiles(c->d, be, p->form, sc, c->max_tiles, cur, tl);
         if ((rc = upload_tiles(c, tl))) return rc;
+        HIPCHK(c, hipMemsetAsync(c->scount, 0, 2 * sizeof(uint32_t), c->stream));
         pairs += tl.pairs;
     }
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
@@ -1497,10 +1708,11 @@ int epi_open(int device, epi_ctx **out)
     }
     if (c->ncu <= 0) c->ncu = 1;
     for (int f = 0; f < 2; f++) c->sched[f] = default_schedule(f);
-    if (dalloc(c, c->nhits, 1) || dalloc(c, c->hits, (size_t)c->cap)) {
+    if (dalloc(c, c->nhits, 2) || dalloc(c, c->hits, (size_t)c->cap) || dalloc(c, c->cand, (size_t)CAND_CAP)) {
         epi_close(c);
         return EPI_ERR_NOMEM;
     }
+    c->scount = reinterpret_cast<uint32_t *>(c->nhits + 1);
     if (scratch_of(c, &c->scratch)) {
         epi_close(c);
         return EPI_ERR_HIP;
@@ -1518,6 +1730,7 @@ void epi_close(epi_ctx *c)
     dfree(c->hits);
     dfree(c->nhits);
     dfree(c->tiles);
+    dfree(c->cand);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1662,7 +1875,7 @@ int epi_scan_noalloc(epi_ctx *c, const epi_scan_params *p, epi_hit64 *hits, int6
                     NOALLOC_TILES, NOALLOC_BYTES >> 20);
     unsigned char *base = static_cast<unsigned char *>(c->scratch);
     const ScanBufs B = {reinterpret_cast<int4 *>(base + 256), reinterpret_cast<DevHit *>(hits),
-                        reinterpret_cast<unsigned long long *>(base), (long long)cap};
+                        reinterpret_cast<unsigned long long *>(base), (long long)cap, {}};
     if ((rc = copy_tiles(c, B.tiles, tl))) return rc;
     c->last_tiles[0] = c->last_tiles[1] = c->last_tiles[2] = 0;
     hipLaunchKernelGGL(zero_counter, dim3(1), dim3(1), 0, c->stream, B.nhits);

@@ -79,7 +79,8 @@ struct MissPhen {                // per individual, for the SPARSE tiles' missin
     float zf;                    // z as FP32
     int32_t q;                   // fixed-point phenotype (0 where missing and for outliers)
     int32_t z;                   // round(q^2 / 2^zbits)
-    int32_t pad[3];
+    int32_t sv;                  // coarse phenotype of the screen (0 where missing)
+    int32_t pad[2];
 };
 
 struct OutVals {                 // values of the outlier individuals, in fixed-point units

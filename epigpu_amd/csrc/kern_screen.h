@@ -1,0 +1,579 @@
+// Screened pair scan (gfx950, v_mfma_f32_32x32x64_f8f6f4 on 6-bit operands).
+//
+// Almost no pair of a scan is a hit, so most pairs need no exact table: a bound
+// on their statistics settles them. The screen kernels contract the class
+// masks with a coarse phenotype v instead of the 24-bit q of kern_mfma.h, keep
+// every pair whose true statistics could pass the thresholds (candidates),
+// and resolve_kernel computes the candidates' tables exactly, as integers, and
+// decides them in FP64 with the same code as the exact tiles. The hits and
+// their values are those of the exact tiles.
+//
+// Coarse phenotype: v = 32 D1 + D0 with both digits representable in FP6 (E2M3:
+// in units of 1/8 the integers 0..16, then steps of 2 to 30 and of 4 to 60),
+// |v| <= 1980, v ~ q / delta with delta = max|q| / 1980 (or larger), r = q - delta v. The
+// rate of 6-bit MFMA operands is twice that of 8-bit ones, and one weight
+// count + two digits replace the count + three limbs: 12 instead of 16 INT8
+// equivalents of MACs, at twice the rate.
+//
+// What bounds it: the matrix cores. At N = 8000, M = 50000 without missing calls a scan's kernels take
+// 37.4 ms (exact 64 x 64 tiles: 92-97 ms): 2.4e14 operations at 6.4 POP/s, against the 7.3-7.5 POP/s that
+// a register-only loop of this MFMA with five VALU instructions beside each sustains (8.7 without any,
+// 4.8 for v_mfma_i32_32x32x32_i8).
+//
+// Bound: over a pair's complete cases let P y be the projection of a phenotype
+// onto the cell-constant vectors less the mean, so SSB(y) = |P y|^2. Then
+//     |P q| <= delta |P v| + |P r| <= delta |P v| + eps,   eps = |r - mean(r)|,
+// and likewise sqrt(SSI(q)) <= delta sqrt(SSI(v)) + eps, since SSI(y) = |A y|^2 with A
+// linear and SSI <= SSB <= |y|^2 for every y. With SST the total sum of squares,
+//     F > t1   <=>  SSB > k1 SST,  k1 = t1 d1 / (d2 + t1 d1)
+//     F2 > t2  =>   SSI > (4 t2 / d2) (SST - SSB), and since SSB >= SSI also
+//                   SSB > k2 SST,  k2 = 4 t2 / (d2 + 4 t2).
+// A pair is a candidate unless these fail with SSB, SSI replaced by their upper
+// bounds and the thresholds lowered by 2 % (the margin of the exact tiles'
+// FP32 screen, far above the rounding of the FP32 sums here: counts and
+// digit sums are exact integers below 2^24).
+#pragma once
+
+#include "kern_mfma.h"
+
+namespace epi {
+
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+constexpr int SW_ROW = 16;   // dwords per 32 individuals: D0 codes (6), D1 codes (6), phenotype present, pad
+constexpr int SCR_WIN = 512; // words (of 32 individuals) of weights in LDS at a time
+constexpr int SCR_LDS_ROWS = SCR_WIN + 2;  // the pipeline reads one step past the window
+constexpr int SCR_A = 16;    // a-SNPs per wave
+constexpr int SCR_REDO = 128;  // candidates of a wave's 16 x 64 pairs above which the exact tile redoes them
+
+// Per SNP and phenotype: counts and sums of v of classes 0 and 1 (present
+// phenotypes), divided by 64 as the kernels' accumulators are.
+struct ScrMarg {
+    float n0, n1, s0, s1;
+};
+
+// The cut of one scan (thresholds and phenotype), in units of v / 8 (sums of squares / 64).
+struct ScreenCut {
+    float N, T, T2N;      // complete cases / 64, sum of v / 64, T^2 / N
+    float thr9, slope;    // level 0: sum s^2 / n > thr9 - slope (9 - nfac)
+    float eps;            // |r - mean(r)| / (8 delta)
+    float sst;            // SST(q) / (64 delta^2)
+    float nv;             // complete cases
+    float t1s, t2s;       // lowered thresholds
+    int test, safe;
+};
+
+struct CandSink {
+    int4 *cand;               // {a, b, scan, 0}; a == b: void
+    uint32_t *count;          // [0] candidates, [1] regions to redo
+    uint32_t cap;
+    uint32_t *redo;           // tile * (waves per tile) + wave
+};
+
+struct ScreenArgs {
+    MfmaScan S;
+    const uint32_t *sw;       // [Kw][SW_ROW]
+    const ScrMarg *sm;        // [nsnp]
+    ScreenCut cut;
+    CandSink cs;
+    const int4 *tiles;
+    int ntiles;
+    int tile0;                // index of tiles[0] in the scan's list
+};
+
+// The FP6 image of 32 individuals in a lane: element s occupies bits 6s..6s+5 of
+// 192. Individual k (bit k of a bitplane word) goes to the element whose lowest
+// bit is at bit k of a dword: even k in the first 96 bits, odd k (after a
+// shift by one) in the last 96. The lowest bits of the elements at these
+// positions are three masks of the word, and element s = scr_slot(k).
+constexpr uint32_t SP0 = 0x41041041u, SP1 = 0x10410410u, SP2 = 0x04104104u;
+
+__host__ __device__ constexpr int scr_slot(int k)
+{
+    const int e = k & ~1;  // bit position in the (shifted) word
+    for (int s = 0; s < 16; s++)
+        if (6 * s % 32 == e) return s + (k & 1 ? 16 : 0);
+    return -1;
+}
+
+struct Fp6 {
+    uint32_t d[6];
+};
+
+// 0/1 elements (0 or 0.125) of a bitplane word: seven VALU instructions.
+__device__ __forceinline__ Fp6 scr_spread(uint32_t x)
+{
+    const uint32_t y = x >> 1;
+    return {{x & SP0, x & SP1, x & SP2, y & SP0, y & SP1, y & SP2}};
+}
+
+// All six bits of every element set: (T << 6) - T over each 96-bit half.
+__device__ __forceinline__ Fp6 scr_fill(const Fp6 &t)
+{
+    Fp6 m;
+#pragma unroll
+    for (int h = 0; h < 6; h += 3) {
+        const uint32_t t0 = t.d[h], t1 = t.d[h + 1], t2 = t.d[h + 2];
+        unsigned c0, c1, c2;
+        m.d[h] = __builtin_subc(t0 << 6, t0, 0u, &c0);
+        m.d[h + 1] = __builtin_subc(__builtin_amdgcn_alignbit(t1, t0, 26), t1, c0, &c1);
+        m.d[h + 2] = __builtin_subc(__builtin_amdgcn_alignbit(t2, t1, 26), t2, c1, &c2);
+    }
+    return m;
+}
+
+__device__ __forceinline__ v8i scr_op(const Fp6 &f)
+{
+    return (v8i){(int)f.d[0], (int)f.d[1], (int)f.d[2], (int)f.d[3], (int)f.d[4], (int)f.d[5], 0, 0};
+}
+
+// FP6 x FP6 MFMA, plain and with the A operand scaled by 32 (E8M0 exponent 132).
+__device__ __forceinline__ v16f scr_mfma(const v8i &a, const v8i &b, const v16f &c)
+{
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 2, 0, 0, 0, 0);
+}
+__device__ __forceinline__ v16f scr_mfma32(const v8i &a, const v8i &b, const v16f &c)
+{
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 2, 0, 0x84848484, 0, 0x7f7f7f7f);
+}
+
+// 1/n from above: the exponent of n negated and its mantissa mirrored, between
+// 1/n and 1.125/n (the linear bound 1 - f/2 >= 1/(1+f) on 0 <= f <= 1), huge for n = 0.
+__device__ __forceinline__ float rcp_above(float n) { return __uint_as_float(0x7F000000u - __float_as_uint(n)); }
+
+// Second stage of the screen, per lane: the bounds above in FP32, from the
+// nine cells' counts n and sums s (both / 64). SST is that of the pair's
+// complete cases from below, sst, and nc their count.
+__device__ __forceinline__ bool screen_bound(const float n[9], const float s[9], float nc, float sst, const ScreenCut &C)
+{
+    float nfac = 0.0f, N = 0.0f, T = 0.0f, m[9], q = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 9; c++) {
+        const bool occ = n[c] > 0.0f;
+        nfac += occ ? 1.0f : 0.0f;
+        N += n[c];
+        T += s[c];
+        m[c] = occ ? s[c] * __builtin_amdgcn_rcpf(n[c]) : 0.0f;
+        q += occ ? m[c] * s[c] : 0.0f;
+    }
+    const float d1 = nfac - 1.0f, d2 = nc - nfac;
+    if (!(d1 >= 1.0f) || !(d2 >= 1.0f)) return false;
+    if (C.test != 'f' && !C.safe && !(nfac > 6.0f)) return false;
+    const float mbar = T * __builtin_amdgcn_rcpf(N);
+    const float ssb = fmaxf(q - T * mbar, 0.0f);
+    const float rb = sqrtf(ssb) * 1.0001f + C.eps, ub = rb * rb;  // SSB(q) from above
+    const float k1 = C.t1s * d1;
+    if (ub * (d2 + k1) > k1 * sst) return true;
+    if (C.test == 'f') return false;
+    const float ssw = sst - ub;
+    if (!(ub * d2 > 4.0f * C.t2s * ssw)) return false;  // SSI <= SSB
+    float R[3], Cm[3];
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        const float nr = n[3 * r] + n[3 * r + 1] + n[3 * r + 2], nk = n[r] + n[r + 3] + n[r + 6];
+        R[r] = nr > 0.0f ? (s[3 * r] + s[3 * r + 1] + s[3 * r + 2]) * __builtin_amdgcn_rcpf(nr) : 0.0f;
+        Cm[r] = nk > 0.0f ? (s[r] + s[r + 3] + s[r + 6]) * __builtin_amdgcn_rcpf(nk) : 0.0f;
+    }
+    float ssi = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 9; c++) {
+        const float t = m[c] - R[c / 3] - Cm[c % 3] + mbar;
+        ssi += n[c] > 0.0f ? n[c] * t * t : 0.0f;
+    }
+    const float ri = sqrtf(ssi) * 1.0001f + C.eps;
+    return ri * ri * d2 > 4.0f * C.t2s * ssw;
+}
+
+// A wave's candidates into the list, or its region into the redo list: bit k of
+// bits is the lane's pair (a(k), b(k)). Every lane calls.
+template <int NB, class Pair>
+__device__ __forceinline__ void scr_append(const CandSink &cs, uint32_t bits, uint32_t region, int scan, Pair pair)
+{
+    if (__ballot(bits != 0u) == 0ull) return;
+    uint32_t total = 0;
+#pragma unroll
+    for (int k = 0; k < NB; k++) total += __popcll(__ballot((bits >> k) & 1u));
+    const int lane = __lane_id();
+    uint32_t base = 0;
+    if (lane == 0 && total <= SCR_REDO) base = atomicAdd(cs.count, total);
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (total > SCR_REDO || base > cs.cap || total > cs.cap - base) {
+        // too many for the list: the exact tile redoes the region. Slots already reserved are voided.
+        if (total <= SCR_REDO)
+            for (uint32_t i = base + lane; i < cs.cap && i < base + total; i += 64) cs.cand[i] = make_int4(0, 0, 0, 0);
+        if (lane == 0) cs.redo[atomicAdd(cs.count + 1, 1u)] = region;
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < NB; k++) {
+        const uint64_t mask = __ballot((bits >> k) & 1u);
+        if ((bits >> k) & 1u) {
+            int a, b;
+            pair(k, a, b);
+            cs.cand[base + __popcll(mask & ((1ull << lane) - 1ull))] = make_int4(a, b, scan, 0);
+        }
+        base += __popcll(mask);
+    }
+}
+
+// ---------------------------------------------------------------- FAST ----
+// Tile TA a x 64 b without missing calls. Each wave owns 16 a x 64 b: 32 A rows
+// (a, g) for classes g in {0, 1}, row m = 2 a + g, times three weights (the
+// mask itself for the count, and the mask AND the codes of D0 and D1), against
+// four B blocks of 32 b (class h of b-SNPs 32 bg + m): 12 MFMAs per 64
+// individuals. D1 accumulates into the accumulators of D0 with the MFMA's scale 2^5, so
+// a pair takes two accumulators per cell, 128 per lane, and two waves
+// share a SIMD. Every lane reads its rows' bitplane words from global memory
+// (one dword per operand and 64 individuals, coalesced along SNPs) and expands
+// them in registers: no operand passes through LDS, and the waves run
+// without barriers. LDS holds the phenotype's codes, which all waves share.
+template <int TA>
+constexpr int screen_threads() { return 64 * TA / SCR_A; }
+
+template <int TA>
+__device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const uint32_t *sw, const ScrMarg *sm,
+                                                 const ScreenCut &C, const CandSink &cs, int a0, int a1, int b0, int b1,
+                                                 uint32_t region0, uint32_t *wl, float4 *mg)
+{
+    constexpr int NT = screen_threads<TA>();
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int aw = a0 + SCR_A * wid;                      // the wave's first a-SNP
+    const bool work = aw < a1 && (a1 < aw + SCR_A ? a1 : aw + SCR_A) - 1 > b0;
+    const int Kw = S.Kp / 32, nw = S.Kl / 32;             // nw: words the loop covers (a multiple of 4)
+
+    for (int i = tid; i < TA + 64; i += NT) {
+        int sn = i < TA ? a0 + i : b0 + i - TA;
+        sn = sn < S.nsnp ? sn : S.nsnp - 1;
+        mg[i] = *reinterpret_cast<const float4 *>(sm + sn);
+    }
+
+    v16f av[4], al[4];  // [2 bg + h]: counts, sums of v
+#pragma unroll
+    for (int j = 0; j < 4; j++) av[j] = al[j] = (v16f){};
+
+    // Bitplanes through buffer descriptors (scalar base and row offset, 32-bit lane offset): one from
+    // class 0 on for the A rows, whose lanes hold both classes, and class 1 for the B rows (the
+    // caller checks that two planes stay below 4 GiB).
+    const uint32_t row = (uint32_t)S.nsnp * 4u, plane = (uint32_t)Kw * row;  // bytes
+    const uint64_t rest = 3ull * plane;
+    auto rsrc = [&](uint32_t o) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(S.bits) + o), 0,
+                                                 (int)(rest - o < 0xFFFFFFFFull ? rest - o : 0xFFFFFFFFull), 0x00027000);
+    };
+    const __amdgpu_buffer_rsrc_t r0 = rsrc(0u), r1 = rsrc(plane);
+    uint32_t va, vb[2];
+    {
+        int a = aw + (m >> 1);
+        a = a < S.nsnp ? a : S.nsnp - 1;
+        va = (m & 1) * plane + hf * row + (uint32_t)a * 4u;
+#pragma unroll
+        for (int bg = 0; bg < 2; bg++) {
+            int b = b0 + 32 * bg + m;
+            b = b < S.nsnp ? b : S.nsnp - 1;
+            vb[bg] = hf * row + (uint32_t)b * 4u;
+        }
+    }
+    // Software pipeline: during step t (64 individuals) the A operands and the first B operand of step
+    // t + 1 are made from bits that were loaded during step t - 1, and the bits of step t + 2 are
+    // requested. The requests run up to four words past the last: those lie in the padding or in the
+    // plane that follows (the call-present plane after class 1), and are not used.
+    struct Ops {
+        v8i A, A0, A1, B0;
+    };
+    uint32_t xa[2], xb[2][4];
+    uint32_t src = 0;  // byte offset of the step's first word within a plane
+    auto load = [&](int set) {
+        xa[set] = __builtin_amdgcn_raw_buffer_load_b32(r0, va, src, 0);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            xb[set][j] = __builtin_amdgcn_raw_buffer_load_b32(j & 1 ? r1 : r0, vb[j >> 1], src, 0);
+        src += 2 * row;
+    };
+    auto prep = [&](int set, const uint32_t *wr, Ops &o) {
+        const uint4 q0 = *reinterpret_cast<const uint4 *>(wr), q1 = *reinterpret_cast<const uint4 *>(wr + 4),
+                    q2 = *reinterpret_cast<const uint4 *>(wr + 8);
+        const Fp6 t = scr_spread(xa[set] & wr[12]), f = scr_fill(t);
+        const Fp6 f0 = {{f.d[0] & q0.x, f.d[1] & q0.y, f.d[2] & q0.z, f.d[3] & q0.w, f.d[4] & q1.x, f.d[5] & q1.y}};
+        const Fp6 f1 = {{f.d[0] & q1.z, f.d[1] & q1.w, f.d[2] & q2.x, f.d[3] & q2.y, f.d[4] & q2.z, f.d[5] & q2.w}};
+        o.A = scr_op(t);
+        o.A0 = scr_op(f0);
+        o.A1 = scr_op(f1);
+        o.B0 = scr_op(scr_spread(xb[set][0]));
+    };
+    auto step = [&](int set, const Ops &o) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const v8i B = j == 0 ? o.B0 : scr_op(scr_spread(xb[set][j]));
+            al[j] = scr_mfma(o.A0, B, al[j]);
+            av[j] = scr_mfma(o.A, B, av[j]);
+            al[j] = scr_mfma32(o.A1, B, al[j]);
+        }
+    };
+    // Masks: 0x008 MFMA, 0x002 VALU, 0x100 LDS read, 0x020 global load.
+    auto fence = [&]() {
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+        for (int u = 0; u < 12; u++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Ops o0, o1;
+    if (work) {
+        load(0);
+        load(1);
+    }
+    for (int w0 = 0; w0 < nw; w0 += SCR_WIN) {
+        const int wn = nw - w0 < SCR_WIN ? nw - w0 : SCR_WIN;
+        if (w0) __syncthreads();
+        for (int i = tid; i < wn * (SW_ROW / 4); i += NT)
+            reinterpret_cast<uint4 *>(wl)[i] = reinterpret_cast<const uint4 *>(sw + (size_t)w0 * SW_ROW)[i];
+        __syncthreads();
+        if (!work) continue;
+        const uint32_t *wr = wl + hf * SW_ROW;
+        prep(0, wr, o0);
+        __builtin_amdgcn_sched_barrier(0);
+        for (int t = 0; t < wn; t += 4, wr += 4 * SW_ROW) {
+            step(0, o0);
+            prep(1, wr + 2 * SW_ROW, o1);
+            load(0);
+            fence();
+            step(1, o1);
+            // past the window's last step: a row of the next window's place, not used
+            prep(0, wr + 4 * SW_ROW, o0);
+            load(1);
+            fence();
+        }
+    }
+    if (!work) return;
+
+    // Lane: pairs a = aw + 4j + 2hf + p, b = b0 + 32 bg + m; [2bg + h][4j + 2p + g] = X[g][h].
+    uint32_t bits = 0;
+    auto cells = [&](auto k, float n[9], float s[9]) {
+        constexpr int K = decltype(k)::value, j = K / 4, p = K / 2 % 2, bg = K % 2, e = 4 * j + 2 * p;
+        const float4 ma = mg[SCR_A * wid + 4 * j + 2 * hf + p], mb = mg[TA + 32 * bg + m];
+        auto fill = [&](float c[9], const v16f &x0, const v16f &x1, float a_0, float a_1, float b_0, float b_1, float all) {
+            c[0] = x0[e];
+            c[1] = x1[e];
+            c[3] = x0[e + 1];
+            c[4] = x1[e + 1];
+            c[2] = a_0 - c[0] - c[1];
+            c[5] = a_1 - c[3] - c[4];
+            c[6] = b_0 - c[0] - c[3];
+            c[7] = b_1 - c[1] - c[4];
+            c[8] = (all - a_0 - a_1) - c[6] - c[7];
+        };
+        fill(n, av[2 * bg], av[2 * bg + 1], ma.x, ma.y, mb.x, mb.y, C.N);
+        fill(s, al[2 * bg], al[2 * bg + 1], ma.z, ma.w, mb.z, mb.w, C.T);
+    };
+    static_for<16>([&](auto k) {
+        constexpr int K = decltype(k)::value, j = K / 4, p = K / 2 % 2, bg = K % 2;
+        float n[9], s[9];
+        cells(k, n, s);
+        const int a = aw + 4 * j + 2 * hf + p, b = b0 + 32 * bg + m;
+        const bool valid = (a < a1) & (b < b1) & (a > b);
+        float u = 0.0f, nmin = n[0];
+#pragma unroll
+        for (int c = 0; c < 9; c++) {
+            u = __builtin_fmaf(s[c] * s[c], rcp_above(n[c]), u);
+            nmin = fminf(nmin, n[c]);
+        }
+        float thr = C.thr9;
+        if (__ballot(!(nmin > 0.0f)) != 0ull) {
+            float empty = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 9; c++) empty += n[c] > 0.0f ? 0.0f : 1.0f;
+            thr -= C.slope * empty;
+        }
+        bool keep = valid & !(u <= thr);
+        if (__ballot(keep) != 0ull) {
+            keep = keep && screen_bound(n, s, C.nv, C.sst, C);
+            bits |= keep ? 1u << K : 0u;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    scr_append<16>(cs, bits, region0 + wid, S.tag, [&](int k, int &a, int &b) {
+        a = aw + 4 * (k >> 2) + 2 * hf + (k >> 1 & 1);
+        b = b0 + 32 * (k & 1) + m;
+    });
+}
+
+template <int TA>
+__global__ __launch_bounds__(screen_threads<TA>(), 2) void screen_fast_kernel(const ScreenArgs A)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_LDS_ROWS * SW_ROW];
+    __shared__ float4 mg[TA + 64];
+    const int t = xcd_tile(blockIdx.x, A.ntiles);
+    const int4 T = A.tiles[t];
+    screen_fast_tile<TA>(A.S, A.sw, A.sm, A.cut, A.cs, T.x, T.y, T.z, T.w, (uint32_t)(A.tile0 + t) * (TA / SCR_A), wl, mg);
+}
+
+// Regions that the screen handed back, through the exact tile: a persistent grid
+// over the device's count of them. Region r is wave r % (TA / 16) of tile r / (TA / 16).
+template <int TA>
+__global__ __launch_bounds__(fast_threads<32>(), fast_waves_per_simd<32>()) void redo_fast_kernel(
+    const MfmaScan S, const HitSink hs0, const int4 *tiles, const uint32_t *count, const uint32_t *redo)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t lds[fast_lds<32>()];
+    const uint32_t n = count[1];
+    HitSink hs = hs0;
+    hs.tag = S.tag;
+    const DumpSink nodump = {};
+    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+        const uint32_t r = redo[i];
+        const int4 T = tiles[r / (TA / SCR_A)];
+        const int a0 = __builtin_amdgcn_readfirstlane(T.x + SCR_A * (int)(r % (TA / SCR_A)));
+        const int a1 = __builtin_amdgcn_readfirstlane(T.y < a0 + SCR_A ? T.y : a0 + SCR_A);
+        const int b0 = __builtin_amdgcn_readfirstlane(T.z), b1 = __builtin_amdgcn_readfirstlane(T.w);
+        __syncthreads();  // the previous region is done with LDS
+        mfma_fast_tile<32, false>(S, hs, nodump, a0, a1, b0, b1, lds);
+    }
+}
+
+// --------------------------------------------------------------- resolve ----
+// The candidates' exact tables, one wave (or a part of it) per candidate: its
+// lanes take the bitplane words of both SNPs in turn and sum V (the counts),
+// the three limbs of q (and the four of z for pairs with missing calls) with
+// 4 x 8-bit dot products, exactly as the tiles' MFMAs do, in INT32. The lanes'
+// sums are added up, and lane i keeps candidate i of the wave's run, so that
+// the FP64 decision runs once for all of them, on up to 64 lanes.
+struct ResolveArgs {
+    MfmaScan S;               // single scans
+    const MfmaScan *scans;    // batches: by scan id
+    HitSink hs;
+    const int4 *cand;
+    const uint32_t *count;
+    uint32_t cap;
+    int group;                // lanes per candidate
+};
+
+// GEN: pairs of tiles with missing calls (the classes 0, 1, NM of both SNPs and
+// the sum of z); otherwise classes 0 and 1 and the SNPs' marginals. G lanes
+// share a candidate (a power of two, 64 from 33 words on), so that a wave
+// takes 64 / G candidates of a small cohort at a time.
+template <bool GEN, bool BATCH>
+__global__ __launch_bounds__(256) void resolve_kernel(const ResolveArgs A)
+{
+    constexpr int NG = GEN ? 3 : 2, NX = NG * NG, NZ = GEN ? 4 : 0, NV = 4 * NX + NZ;
+    const uint32_t n = A.count[0] < A.cap ? A.count[0] : A.cap;
+    const uint32_t nwave = gridDim.x * 4u, wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, G = A.group, sub = lane / G, gl = lane % G, step = 64 / G;
+    uint32_t per = (n + nwave - 1) / nwave;
+    per = (per + step - 1) / step * step;
+    per = per < 64u ? per : 64u;
+    for (uint32_t c0 = wave * per; c0 < n; c0 += nwave * per) {
+        const int m = (int)(n - c0 < per ? n - c0 : per);
+        int keep[NV];
+#pragma unroll
+        for (int i = 0; i < NV; i++) keep[i] = 0;
+        const int4 mine = A.cand[c0 + (lane < m ? lane : 0)];
+        for (int u = 0; u < m; u += step) {
+            const int c = u + sub;
+            const int a = __shfl(mine.x, c), b = __shfl(mine.y, c);
+            const MfmaScan &S = BATCH ? A.scans[__shfl(mine.z, c)] : A.S;
+            const bool on = c < m && a != b;
+            const int Kw = S.Kp / 32, nw = on ? S.Kl / 32 : 0;
+            const size_t plane = (size_t)Kw * S.nsnp;
+            int t[NV];
+#pragma unroll
+            for (int i = 0; i < NV; i++) t[i] = 0;
+            for (int w = gl; w < nw; w += G) {
+                const size_t o = (size_t)w * S.nsnp;
+                uint32_t x[NX];
+                {
+                    uint32_t ga[NG], hb[NG];
+#pragma unroll
+                    for (int g = 0; g < NG; g++) {
+                        ga[g] = S.bits[g * plane + o + a];
+                        hb[g] = S.bits[g * plane + o + b];
+                    }
+#pragma unroll
+                    for (int g = 0; g < NG; g++)
+#pragma unroll
+                        for (int h = 0; h < NG; h++) x[g * NG + h] = ga[g] & hb[h];
+                }
+                const int8_t *wp = S.wts + 32 * w;
+#pragma unroll
+                for (int hh = 0; hh < 2; hh++) {
+                    int4 l[4], z[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        l[i] = *reinterpret_cast<const int4 *>(wp + (size_t)i * S.Kp + 16 * hh);
+                        if (GEN) z[i] = *reinterpret_cast<const int4 *>(wp + (size_t)(4 + i) * S.Kp + 16 * hh);
+                    }
+#pragma unroll
+                    for (int i = 0; i < NX; i++) {
+                        const v4i e = expand16<false>((x[i] >> (16 * hh)) & 0xFFFFu);
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+#pragma unroll
+                            for (int k = 0; k < 4; k++) {
+                                const int lw = k == 0 ? l[q].x : k == 1 ? l[q].y : k == 2 ? l[q].z : l[q].w;
+                                t[4 * i + q] = __builtin_amdgcn_sdot4(e[k], lw, t[4 * i + q], false);
+                            }
+                        }
+                        if (GEN && i == NX - 1) {
+#pragma unroll
+                            for (int q = 0; q < 4; q++)
+#pragma unroll
+                                for (int k = 0; k < 4; k++) {
+                                    const int zw = k == 0 ? z[q].x : k == 1 ? z[q].y : k == 2 ? z[q].z : z[q].w;
+                                    t[4 * NX + q] = __builtin_amdgcn_sdot4(e[k], zw, t[4 * NX + q], false);
+                                }
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NV; i++) {
+                int v = t[i];
+                for (int o = G >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o);
+                v = __shfl(v, (lane - u) * G);
+                keep[i] = lane >= u && lane < u + step ? v : keep[i];
+            }
+        }
+        const bool valid = lane < m && mine.x != mine.y;
+        bool hit = false;
+        DevHit h;
+        HitSink hs = A.hs;
+        if (valid) {
+            const MfmaScan &S = BATCH ? A.scans[mine.z] : A.S;
+            hs.tag = S.tag;
+            int xc[3][3], nc[9];
+            double xs[3][3], sd[9], sq;
+#pragma unroll
+            for (int g = 0; g < NG; g++)
+#pragma unroll
+                for (int k = 0; k < NG; k++) {
+                    const int *v = keep + 4 * (g * NG + k);
+                    xc[g][k] = v[0];
+                    xs[g][k] = (double)v[1] + 256.0 * (double)v[2] + 65536.0 * (double)v[3];
+                }
+            if (GEN) {
+                const int *z = keep + 4 * NX;
+                sq = ((double)z[0] + 256.0 * (double)z[1] + 65536.0 * (double)z[2] + 16777216.0 * (double)z[3]) * S.zunit;
+            } else {
+                const Marg &ma = S.marg[mine.x], &mb = S.marg[mine.y];
+#pragma unroll
+                for (int g = 0; g < 2; g++) {
+                    xc[g][2] = ma.n[g];
+                    xc[2][g] = mb.n[g];
+                    xs[g][2] = (double)ma.q[g];
+                    xs[2][g] = (double)mb.q[g];
+                }
+                xc[2][2] = S.nV;
+                xs[2][2] = S.qVd;
+                sq = S.sqV;
+            }
+            cells_from_x(xc, nc);
+            cells_from_x(xs, sd);
+            hit = confirm64(hs, mine.x, mine.y, nc, sd, sq, h);
+        }
+        append_hit(hs, hit, h);
+    }
+}
+
+}  // namespace epi

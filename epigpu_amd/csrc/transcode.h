@@ -7,7 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "kern_mfma.h"
+#include "kern_screen.h"
 
 namespace epi {
 
@@ -71,16 +71,18 @@ __global__ void transcode_bits(const uint32_t *words, int nid, int npack, int re
 __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, int Kw, int nsnp,
                                                         const uint32_t *vbits, const int32_t *qv,
                                                         const float *yc, const int32_t *cls, const MissPhen *mp,
-                                                        Marg *marg)
+                                                        Marg *marg, ScrMarg *smarg)
 {
     __shared__ long long sq[4][3][64];
     __shared__ double sy[4][3][64];
     __shared__ int sn[4][3][64];
     __shared__ long long sz[4][64];
+    __shared__ int sv[4][2][64];
     const int sl = threadIdx.x & 63, grp = threadIdx.x >> 6;
     const int s = blockIdx.x * 64 + sl;
     int n[3] = {0, 0, 0};
     long long q[3] = {0, 0, 0}, z = 0;
+    int v3[3] = {0, 0, 0};  // sums of the screen's coarse phenotype (their magnitude stays below 2^24)
     double y[3] = {0.0, 0.0, 0.0};
     if (s < nsnp) {
         for (int wd = grp; wd < Kw; wd += 4) {
@@ -99,6 +101,7 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
                     q[c] += qv[k];
                     y[c] += (double)yc[k];
                     z += mp[k].z;
+                    v3[c] += mp[k].sv;
                 }
             }
         }
@@ -109,6 +112,8 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
         sy[grp][c][sl] = y[c];
     }
     sz[grp][sl] = z;
+    sv[grp][0][sl] = v3[0];
+    sv[grp][1][sl] = v3[1];
     __syncthreads();
     if (grp == 0 && s < nsnp) {
         int tn[3];
@@ -139,6 +144,9 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
         mg.pad = 0;
         mg.zs = sz[0][sl] + sz[1][sl] + sz[2][sl] + sz[3][sl];
         marg[s] = mg;
+        const int t0 = sv[0][0][sl] + sv[1][0][sl] + sv[2][0][sl] + sv[3][0][sl];
+        const int t1 = sv[0][1][sl] + sv[1][1][sl] + sv[2][1][sl] + sv[3][1][sl];
+        smarg[s] = {(float)tn[0] / 64.0f, (float)tn[1] / 64.0f, (float)t0 / 64.0f, (float)t1 / 64.0f};
     }
 }
 
