@@ -65,11 +65,15 @@ __device__ __forceinline__ void cells_from_x(const T x[3][3], T c[9])
     c[8] = x[2][2] - x[0][2] - x[1][2] - x[2][0] - x[2][1] + x[0][0] + x[0][1] + x[1][0] + x[1][1];
 }
 
-// FP64 statistics. s[] and sq in any consistent phenotype units.
+// FP64 statistics. s[] and sq in any consistent phenotype units. Products
+// and sums are rounded separately, so that every kernel that inlines this returns
+// the same bits for a pair (left to the compiler, fusing them depends on the
+// surrounding code).
 template <class S>
 __device__ __forceinline__ void stats64(const int n[9], const S s[9], double sq, double &F, double &F2,
                                         int &d1, int &d2, int &nfac)
 {
+#pragma clang fp contract(off)
     int N = 0;
     double tot = 0.0;
     nfac = 0;

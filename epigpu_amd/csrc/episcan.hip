@@ -73,8 +73,9 @@ struct PhenDev {
     uint32_t *sw = nullptr;     // screen
     ScrMarg *sm = nullptr;
     double sdelta = 0.0;        // q ~ sdelta v
-    double seps = 0.0;          // |r - mean(r)|, r = q - sdelta v (q units)
+    double seps = 0.0;          // |r|, r = q - sdelta v (q units)
     double svsum = 0.0;         // sum of v
+    double zall = 0.0;          // sum of z
     int nout = 0;
     int fbits = 0;  // q = round((y - centre) * 2^fbits)
     int zbits = 0;  // Z limbs hold round(q^2 / 2^zbits)
@@ -418,7 +419,7 @@ void encode_screen(const std::vector<int> &P, int Kw, PhenEnc &e)
     if (!(p.sdelta > 0.0) || room <= 1.0) p.sdelta = 0.0;  // constant phenotype or a huge cohort: not screened
     e.sw.assign((size_t)Kw * SW_ROW, 0u);
     if (p.sdelta == 0.0) return;
-    double rs = 0.0, rq = 0.0;
+    double rq = 0.0;
     for (int k : P) {
         const double t = (double)e.qv[k] / p.sdelta;
         int hi = 0, lo = 0;
@@ -438,7 +439,6 @@ void encode_screen(const std::vector<int> &P, int Kw, PhenEnc &e)
         e.mp[k].sv = v;
         p.svsum += v;
         const double r = (double)e.qv[k] - p.sdelta * v;
-        rs += r;
         rq += r * r;
         // the element of individual k & 31: six bits from bit 6 slot of the word's 192
         const int bit = 6 * scr_slot(k & 31);
@@ -451,7 +451,7 @@ void encode_screen(const std::vector<int> &P, int Kw, PhenEnc &e)
         }
         row[12] |= 1u << (k & 31);
     }
-    p.seps = std::sqrt(std::max(0.0, rq - rs * rs / (double)P.size())) * (1.0 + 1e-6);
+    p.seps = std::sqrt(rq) * (1.0 + 1e-6);
 }
 
 // Phenotype prep (src/EpiOpenCL.c:1364-1376 computes mY and SSY over all nid
@@ -563,6 +563,7 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
         mk.v = 1;
         mk.q = (int32_t)q;
         mk.z = (int32_t)z;
+        p.zall += (double)z;
         mk.qf = (float)q;
         mk.zf = (float)z;
         qsum += q;
@@ -1000,8 +1001,9 @@ int copy_tiles(epi_ctx *c, int4 *dst, const TileLists &tl)
 int upload_tiles(epi_ctx *c, const TileLists &tl)
 {
     c->tl_valid = false;
-    // behind the tiles, room for every region of the screen's tiles (four of 4 bytes, at most, per tile)
-    const size_t nt = tl.count(), need = nt + tl.fast.size();
+    // behind the tiles, room for every region of the screen's tiles (at most four of 4 bytes per tile, eight
+    // per SPARSE tile)
+    const size_t nt = tl.count(), need = 2 * nt + tl.sp.size();
     static_assert(sizeof(int4) == 64 / SCR_A * sizeof(uint32_t), "a tile's regions take the room of a tile");
     if (need > c->tiles_cap) {
         c->tiles_cap = 0;
@@ -1151,7 +1153,65 @@ bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
     C.t2s = hs.t2s;
     C.test = q->test;
     C.safe = hs.safe;
+    // GENERAL tiles: the pair's complete cases N' <= N and their SST vary. k / (N' - nfac + k) is smallest at
+    // N' = N; the linear form of (sqrt(k SST) - eps)^2 >= k SST - 2 eps sqrt(k SST) takes the largest
+    // k SST at N' >= N / 2 (pairs with fewer skip level 0).
+    auto kap = [&](int nfac, double n) {
+        const double k1 = (double)hs.t1s * (nfac - 1), k2 = 4.0 * (double)hs.t2s;
+        const double x = k1 / (n - nfac + k1);
+        return inter ? std::min(x, k2 / (n - nfac + k2)) : x;
+    };
+    const double k9 = kap(9, N) * (1.0 - 1e-5);
+    double ks = 0.0;
+    for (int k = inter && !q->safe ? 7 : 2; k < 9; k++) ks = std::max(ks, (k9 - kap(k, N) * (1.0 - 1e-5)) / (9 - k));
+    C.zunit = (float)(std::ldexp(1.0, p.zbits) / unit * (1.0 - 1e-6));
+    C.zall = (float)(p.zall * (1.0 + 1e-6));
+    C.kap9 = (float)(k9 * (1.0 - 1e-6));
+    C.kslope = (float)(ks * (1.0 + 1e-5));
+    C.kroot = (float)(2.0 * p.seps * std::sqrt(kap(9, std::max(0.5 * N, 16.0)) * p.sqV) / unit * (1.0 + 1e-5));
     return true;
+}
+
+// Launch of one kind of tile through the screen: bound, resolve, redo. list: the kind's tiles on the device.
+struct ScreenKind {
+    const int4 *tiles;
+    int n;
+    uint32_t *count;   // candidates and regions of this kind
+    uint32_t *redo;
+};
+
+template <bool GEN, int TA, int TB>
+int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind &K)
+{
+    const int nt = GEN ? screen_gen_threads<TA, TB>() : screen_threads<TA>();
+    G.cs.count = K.count;
+    G.cs.redo = K.redo;
+    for (int t0 = 0; t0 < K.n;) {
+        const int chunk = std::min((int)((1u << 31) / (unsigned)nt) & ~255, K.n - t0);  // as LAUNCH_TILES
+        G.tiles = K.tiles + t0;
+        G.ntiles = chunk;
+        G.tile0 = t0;
+        if constexpr (GEN)
+            hipLaunchKernelGGL((screen_gen_kernel<TA, TB>), dim3(chunk), dim3(nt), 0, c->stream, G);
+        else
+            hipLaunchKernelGGL((screen_fast_kernel<TA>), dim3(chunk), dim3(nt), 0, c->stream, G);
+        HIPCHK(c, hipGetLastError());
+        c->last_launches++;
+        t0 += chunk;
+    }
+    const ResolveArgs R = {G.S, nullptr, hs, G.cs.cand, K.count, G.cs.cap, resolve_lanes(G.S.Kl)};
+    hipLaunchKernelGGL((resolve_kernel<GEN, false>), dim3(4 * c->ncu), dim3(256), 0, c->stream, R);
+    HIPCHK(c, hipGetLastError());
+    const uint32_t *cnt = K.count, *rd = K.redo;
+    if constexpr (GEN)
+        hipLaunchKernelGGL((redo_gen_kernel<TA, TB>), dim3(2 * c->ncu), dim3(general_threads<32>()), 0, c->stream, G.S, hs,
+                           K.tiles, cnt, rd);
+    else
+        hipLaunchKernelGGL((redo_fast_kernel<TA>), dim3(2 * c->ncu), dim3(fast_threads<32>()), 0, c->stream, G.S, hs,
+                           K.tiles, cnt, rd);
+    HIPCHK(c, hipGetLastError());
+    c->last_launches += 2;
+    return EPI_OK;
 }
 
 // Launch the pair kernels of one scan over the uploaded tile lists (fast tiles first).
@@ -1174,50 +1234,44 @@ int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, c
         A.hs = hs;
         A.ds = ds;
         if (ns && !d.sp_ok) return fail(c, EPI_ERR_STATE, "SPARSE tile data not built");
+        // Each kind of tile goes through the screen where its exact tiles would take long enough.
         ScreenArgs G;
-        bool screen = !DUMP && nf && B.cs.cand && (double)nf * sc.fast_rows * TILE_B * A.S.Kl >= SCR_MIN_WORK &&
-                      (unsigned long long)d.Kw * d.nsnp * 8ull < (1ull << 32) - (1u << 20) &&
-                      screen_cut(d.ph[p->phen], p, G.cut);
-        if (screen) {
+        const double per = (double)sc.fast_rows * A.S.Kl;  // rows times individuals
+        bool sf = nf * 64 * per >= SCR_MIN_WORK, ss = ns * 64 * per * 2.5 >= SCR_MIN_WORK,
+             sg = ng * 32 * per * 2.5 >= SCR_MIN_WORK && d.missum[d.nsnp] <= (long long)d.nsnp * d.nid / 8;
+        if (DUMP || !B.cs.cand || !(sf || ss || sg) || (unsigned long long)d.Kw * d.nsnp * 8ull >= (1ull << 32) - (1u << 20) ||
+            !screen_cut(d.ph[p->phen], p, G.cut))
+            sf = ss = sg = false;
+        if (sc.dense_missing == 2) ss = false;  // SPARSE tiles asked for
+        if (sf || ss || sg) {
             G.S = A.S;
             G.sw = d.ph[p->phen].sw;
             G.sm = d.ph[p->phen].sm;
             G.cs = B.cs;
-            ResolveArgs R = {A.S, nullptr, hs, B.cs.cand, B.cs.count, B.cs.cap, resolve_lanes(A.S.Kl)};
-            const int4 *tiles = B.tiles;
-            for (int t0 = 0; t0 < nf;) {
-                const int nt = sc.fast_rows == 64 ? screen_threads<64>() : screen_threads<32>();
-                const int chunk = std::min((int)((1u << 31) / (unsigned)nt) & ~255, nf - t0);
-                G.tiles = tiles + t0;
-                G.ntiles = chunk;
-                G.tile0 = t0;
-                if (sc.fast_rows == 64)
-                    hipLaunchKernelGGL((screen_fast_kernel<64>), dim3(chunk), dim3(nt), 0, c->stream, G);
-                else
-                    hipLaunchKernelGGL((screen_fast_kernel<32>), dim3(chunk), dim3(nt), 0, c->stream, G);
-                HIPCHK(c, hipGetLastError());
-                c->last_launches++;
-                t0 += chunk;
+            int rc = EPI_OK;
+            uint32_t *redo = B.cs.redo;
+            const ScreenKind kf = {B.tiles, nf, B.cs.count, redo}, ks = {B.tiles + nf, ns, B.cs.count + 2, redo + 4 * (size_t)nf},
+                             kg = {B.tiles + nf + ns, ng, B.cs.count + 4, redo + 4 * (size_t)nf + 8 * (size_t)ns};
+            if (sc.fast_rows == 64) {
+                if (sf) rc = launch_screen<false, 64, 64>(c, G, hs, kf);
+                if (ss && !rc) rc = launch_screen<true, 64, 64>(c, G, hs, ks);
+                if (sg && !rc) rc = launch_screen<true, 64, 32>(c, G, hs, kg);
+            } else {
+                if (sf) rc = launch_screen<false, 32, 64>(c, G, hs, kf);
+                if (ss && !rc) rc = launch_screen<true, 32, 64>(c, G, hs, ks);
+                if (sg && !rc) rc = launch_screen<true, 32, 32>(c, G, hs, kg);
             }
-            hipLaunchKernelGGL((resolve_kernel<false, false>), dim3(4 * c->ncu), dim3(256), 0, c->stream, R);
-            HIPCHK(c, hipGetLastError());
-            if (sc.fast_rows == 64)
-                hipLaunchKernelGGL((redo_fast_kernel<64>), dim3(2 * c->ncu), dim3(fast_threads<32>()), 0, c->stream, A.S, hs,
-                                   tiles, (const uint32_t *)B.cs.count, (const uint32_t *)B.cs.redo);
-            else
-                hipLaunchKernelGGL((redo_fast_kernel<32>), dim3(2 * c->ncu), dim3(fast_threads<32>()), 0, c->stream, A.S, hs,
-                                   tiles, (const uint32_t *)B.cs.count, (const uint32_t *)B.cs.redo);
-            HIPCHK(c, hipGetLastError());
-            c->last_launches += 2;
+            if (rc) return rc;
         }
+        const int xf = sf ? 0 : nf, xs = ss ? 0 : ns, xg = sg ? 0 : ng;  // tiles left to the exact kernels
         if (sc.fast_rows == 64) {
-            if (!screen) LAUNCH_TILES((mfma_fast_kernel<64, DUMP>), fast_threads<64>(), A, B.tiles, nf);
-            LAUNCH_TILES((mfma_sparse_kernel<64, DUMP>), sparse_threads<64>(), A, B.tiles + nf, ns);
-            LAUNCH_TILES((mfma_general_kernel<64, DUMP>), general_threads<64>(), A, B.tiles + nf + ns, ng);
+            LAUNCH_TILES((mfma_fast_kernel<64, DUMP>), fast_threads<64>(), A, B.tiles, xf);
+            LAUNCH_TILES((mfma_sparse_kernel<64, DUMP>), sparse_threads<64>(), A, B.tiles + nf, xs);
+            LAUNCH_TILES((mfma_general_kernel<64, DUMP>), general_threads<64>(), A, B.tiles + nf + ns, xg);
         } else {
-            if (!screen) LAUNCH_TILES((mfma_fast_kernel<32, DUMP>), fast_threads<32>(), A, B.tiles, nf);
-            LAUNCH_TILES((mfma_sparse_kernel<32, DUMP>), sparse_threads<32>(), A, B.tiles + nf, ns);
-            LAUNCH_TILES((mfma_general_kernel<32, DUMP>), general_threads<32>(), A, B.tiles + nf + ns, ng);
+            LAUNCH_TILES((mfma_fast_kernel<32, DUMP>), fast_threads<32>(), A, B.tiles, xf);
+            LAUNCH_TILES((mfma_sparse_kernel<32, DUMP>), sparse_threads<32>(), A, B.tiles + nf, xs);
+            LAUNCH_TILES((mfma_general_kernel<32, DUMP>), general_threads<32>(), A, B.tiles + nf + ns, xg);
         }
     } else {
         PlainArgs P;
@@ -1559,7 +1613,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc)
             c->tl_sched = sc;
         }
     }
-    HIPCHK(c, hipMemsetAsync(c->nhits, 0, 2 * sizeof(unsigned long long), c->stream));  // and the screen's counters
+    HIPCHK(c, hipMemsetAsync(c->nhits, 0, 4 * sizeof(unsigned long long), c->stream));  // and the screen's counters
     DumpSink ds;
     memset(&ds, 0, sizeof(ds));
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -1575,7 +1629,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc)
         tl = TileLists();
         done = build_tiles(c->d, be, p->form, sc, c->max_tiles, cur, tl);
         if ((rc = upload_tiles(c, tl))) return rc;
-        HIPCHK(c, hipMemsetAsync(c->scount, 0, 2 * sizeof(uint32_t), c->stream));
+        HIPCHK(c, hipMemsetAsync(c->scount, 0, 6 * sizeof(uint32_t), c->stream));
         pairs += tl.pairs;
     }
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
@@ -1708,7 +1762,7 @@ int epi_open(int device, epi_ctx **out)
     }
     if (c->ncu <= 0) c->ncu = 1;
     for (int f = 0; f < 2; f++) c->sched[f] = default_schedule(f);
-    if (dalloc(c, c->nhits, 2) || dalloc(c, c->hits, (size_t)c->cap) || dalloc(c, c->cand, (size_t)CAND_CAP)) {
+    if (dalloc(c, c->nhits, 4) || dalloc(c, c->hits, (size_t)c->cap) || dalloc(c, c->cand, (size_t)CAND_CAP)) {
         epi_close(c);
         return EPI_ERR_NOMEM;
     }

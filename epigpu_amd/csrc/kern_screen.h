@@ -44,13 +44,16 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int SW_ROW = 16;   // dwords per 32 individuals: D0 codes (6), D1 codes (6), phenotype present, pad
 constexpr int SCR_WIN = 512; // words (of 32 individuals) of weights in LDS at a time
 constexpr int SCR_LDS_ROWS = SCR_WIN + 2;  // the pipeline reads one step past the window
+constexpr int SCR_GEN_ROWS = SCR_WIN + 4;
 constexpr int SCR_A = 16;    // a-SNPs per wave
-constexpr int SCR_REDO = 128;  // candidates of a wave's 16 x 64 pairs above which the exact tile redoes them
+constexpr int SCR_REDO = 8;   // candidates per pair slot of a wave (64 pairs) above which the exact tile redoes its region
 
 // Per SNP and phenotype: counts and sums of v of classes 0 and 1 (present
-// phenotypes), divided by 64 as the kernels' accumulators are.
+// phenotypes), divided by 64 as the kernels' accumulators are, and the sum of
+// z over all calls.
 struct ScrMarg {
     float n0, n1, s0, s1;
+    float zs, pad[3];
 };
 
 // The cut of one scan (thresholds and phenotype), in units of v / 8 (sums of squares / 64).
@@ -60,6 +63,10 @@ struct ScreenCut {
     float eps;            // |r - mean(r)| / (8 delta)
     float sst;            // SST(q) / (64 delta^2)
     float nv;             // complete cases
+    // GENERAL tiles: nv and N bound the pairs' complete cases from above
+    float zunit, zall;    // sums of squares per unit of z (from below); sum of z over all individuals
+    float kap9, kslope;   // level 0: sum s^2 / n > (kap9 - kslope (9 - nfac)) SST - kroot
+    float kroot;
     float t1s, t2s;       // lowered thresholds
     int test, safe;
 };
@@ -196,11 +203,11 @@ __device__ __forceinline__ void scr_append(const CandSink &cs, uint32_t bits, ui
     for (int k = 0; k < NB; k++) total += __popcll(__ballot((bits >> k) & 1u));
     const int lane = __lane_id();
     uint32_t base = 0;
-    if (lane == 0 && total <= SCR_REDO) base = atomicAdd(cs.count, total);
+    if (lane == 0 && total <= SCR_REDO * NB) base = atomicAdd(cs.count, total);
     base = __builtin_amdgcn_readfirstlane(base);
-    if (total > SCR_REDO || base > cs.cap || total > cs.cap - base) {
+    if (total > SCR_REDO * NB || base > cs.cap || total > cs.cap - base) {
         // too many for the list: the exact tile redoes the region. Slots already reserved are voided.
-        if (total <= SCR_REDO)
+        if (total <= SCR_REDO * NB)
             for (uint32_t i = base + lane; i < cs.cap && i < base + total; i += 64) cs.cand[i] = make_int4(0, 0, 0, 0);
         if (lane == 0) cs.redo[atomicAdd(cs.count + 1, 1u)] = region;
         return;
@@ -411,6 +418,248 @@ __global__ __launch_bounds__(screen_threads<TA>(), 2) void screen_fast_kernel(co
     screen_fast_tile<TA>(A.S, A.sw, A.sm, A.cut, A.cs, T.x, T.y, T.z, T.w, (uint32_t)(A.tile0 + t) * (TA / SCR_A), wl, mg);
 }
 
+// ------------------------------------------------------------- GENERAL ----
+// Tile TA a x TB b with missing calls (TB = 32, or 64 for tiles whose SNPs miss few calls). Each
+// wave owns 16 a x 32 b and contracts the classes 0, 1, NM of both sides with the count and the two
+// digits: 27 v_mfma_f32_16x16x128_f8f6f4 per 16 x 16 pairs and 128 individuals (the exact tile: 40 INT8
+// MACs per pair and individual, here 27 at twice the rate). The 16 x 16 shape puts a pair's 18 accumulators
+// into one lane whatever the number of rows per a-SNP: row m of A is a-SNP m, one
+// block per class and weight; lane l holds column l % 16 and rows 4 (l / 16) + i. 144 accumulators.
+// SST of a pair's complete cases is at least Z_a + Z_b - Z_all (Z the sums of q^2 over an
+// SNP's calls), less the mean's part, T^2 / N with T the sum of q: |T| / sqrt N <= delta |sum v| / sqrt N + eps.
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ v4f scr_mfma16(const v8i &a, const v8i &b, const v4f &c)
+{
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 2, 0, 0, 0, 0);
+}
+__device__ __forceinline__ v4f scr_mfma16x32(const v8i &a, const v8i &b, const v4f &c)
+{
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 2, 0, 0x84848484, 0, 0x7f7f7f7f);
+}
+
+template <int TA, int TB>
+constexpr int screen_gen_threads() { return 64 * (TA / SCR_A) * (TB / 32); }
+
+template <int TA, int TB>
+__device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const uint32_t *sw, const ScrMarg *sm, const ScreenCut &C,
+                                                const CandSink &cs, int a0, int a1, int b0, int b1, uint32_t region0,
+                                                uint32_t *wl, float *mz)
+{
+    constexpr int NT = screen_gen_threads<TA, TB>(), NWA = TA / SCR_A;
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, kq = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int al = SCR_A * (wid % NWA), bl = 32 * (wid / NWA);
+    const int aw = a0 + al, bw = b0 + bl;
+    const bool work = aw < a1 && bw < b1 && (a1 < aw + SCR_A ? a1 : aw + SCR_A) - 1 > bw;
+    const int Kw = S.Kp / 32, nw = S.Kl / 32;
+
+    for (int i = tid; i < TA + TB; i += NT) {
+        int sn = i < TA ? a0 + i : b0 + i - TA;
+        sn = sn < S.nsnp ? sn : S.nsnp - 1;
+        mz[i] = sm[sn].zs;
+    }
+
+    v4f av[2][9], as[2][9];  // [b group][3 g + h]: counts, sums of v
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 9; j++) av[i][j] = as[i][j] = (v4f){};
+
+    // bitplanes through one buffer descriptor per class (scalar base and row offset, 32-bit lane offset)
+    const uint32_t row = (uint32_t)S.nsnp * 4u, plane = (uint32_t)Kw * row;  // bytes
+    auto rsrc = [&](int g) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(S.bits) + (size_t)g * plane), 0,
+                                                 (int)plane, 0x00027000);
+    };
+    const __amdgpu_buffer_rsrc_t r[3] = {rsrc(0), rsrc(1), rsrc(2)};
+    uint32_t va, vb[2];
+    {
+        const int a = aw + m < S.nsnp ? aw + m : S.nsnp - 1;
+        va = kq * row + (uint32_t)a * 4u;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int b = bw + 16 * i + m < S.nsnp ? bw + 16 * i + m : S.nsnp - 1;
+            vb[i] = kq * row + (uint32_t)b * 4u;
+        }
+    }
+    // Software pipeline over steps of 128 individuals, in three phases, one per class g of the a-SNPs, of three
+    // groups of six MFMAs (one per B operand): the low digit, the count, the high digit. A group's
+    // operand is made one or two groups before it and dies with it, so that at most four A operands are
+    // live beside the six of B; the last group of a step makes the next step's B operands
+    // in the registers of this one's.
+    struct Weights {
+        uint4 q0, q1, q2;
+        uint32_t v;
+    };
+    uint32_t xa[3], xb[6];
+    v8i B[6];
+    uint32_t src = 0;
+    const uint32_t last = (uint32_t)(nw - 4) * row;
+    auto loadB = [&]() {
+#pragma unroll
+        for (int j = 0; j < 6; j++) xb[j] = __builtin_amdgcn_raw_buffer_load_b32(r[j >> 1], vb[j & 1], src, 0);
+    };
+    auto loadA = [&](int g) { xa[g] = __builtin_amdgcn_raw_buffer_load_b32(r[g], va, src, 0); };
+    auto low = [&](const Fp6 &f, const Weights &w) {
+        return scr_op({{f.d[0] & w.q0.x, f.d[1] & w.q0.y, f.d[2] & w.q0.z, f.d[3] & w.q0.w, f.d[4] & w.q1.x,
+                        f.d[5] & w.q1.y}});
+    };
+    auto high = [&](const Fp6 &f, const Weights &w) {
+        return scr_op({{f.d[0] & w.q1.z, f.d[1] & w.q1.w, f.d[2] & w.q2.x, f.d[3] & w.q2.y, f.d[4] & w.q2.z,
+                        f.d[5] & w.q2.w}});
+    };
+    if (work) {
+        loadA(0);
+        loadB();
+    }
+    for (int w0 = 0; w0 < nw; w0 += SCR_WIN) {
+        const int wn = nw - w0 < SCR_WIN ? nw - w0 : SCR_WIN;
+        if (w0) __syncthreads();
+        for (int i = tid; i < wn * (SW_ROW / 4); i += NT)
+            reinterpret_cast<uint4 *>(wl)[i] = reinterpret_cast<const uint4 *>(sw + (size_t)w0 * SW_ROW)[i];
+        __syncthreads();
+        if (!work) continue;
+        const uint32_t *wr = wl + kq * SW_ROW;
+        Weights w;
+        auto weights = [&](int part) {
+            if (part == 0) {
+                w.v = wr[12];
+                w.q0 = *reinterpret_cast<const uint4 *>(wr);
+                w.q1.x = wr[4];
+                w.q1.y = wr[5];
+            } else {
+                w.q1.z = wr[6];
+                w.q1.w = wr[7];
+                w.q2 = *reinterpret_cast<const uint4 *>(wr + 8);
+            }
+        };
+        weights(0);
+        weights(1);
+        Fp6 t = scr_spread(xa[0] & w.v), f = scr_fill(t);
+        v8i A0 = low(f, w);
+#pragma unroll
+        for (int j = 0; j < 6; j++) B[j] = scr_op(scr_spread(xb[j]));
+        loadA(1);
+        loadA(2);
+        __builtin_amdgcn_sched_barrier(0);
+        // Masks: 0x008 MFMA, 0x002 VALU.
+        auto fence = [&](auto nv) {
+#pragma unroll
+            for (int u = 0; u < 6; u++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, decltype(nv)::value, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        using std::integral_constant;
+        for (int wi = 0; wi < wn; wi += 4) {
+            static_for<3>([&](auto gg) {
+                constexpr int g = decltype(gg)::value, gn = (g + 1) % 3;
+                if (g == 0) {  // request the next step's words
+                    src = src + 4 * row < last ? src + 4 * row : last;
+                    loadA(0);
+                    loadB();
+                }
+                if (g == 2) {
+                    wr += 4 * SW_ROW;  // past the window's last step: not used
+                    weights(0);
+                }
+#pragma unroll
+                for (int j = 0; j < 6; j++) as[j & 1][3 * g + (j >> 1)] = scr_mfma16(A0, B[j], as[j & 1][3 * g + (j >> 1)]);
+                const Fp6 tn = scr_spread(xa[gn] & w.v);
+                if (g == 2) {
+                    loadA(1);
+                    loadA(2);
+                }
+                fence(integral_constant<int, 2>{});
+#pragma unroll
+                for (int j = 0; j < 6; j++)
+                    av[j & 1][3 * g + (j >> 1)] = scr_mfma16(scr_op(t), B[j], av[j & 1][3 * g + (j >> 1)]);
+                const v8i A1 = high(f, w);
+                if (g == 2) weights(1);
+                const Fp6 fn = scr_fill(tn);
+                fence(integral_constant<int, 3>{});
+                A0 = low(fn, w);
+#pragma unroll
+                for (int j = 0; j < 6; j++) {
+                    as[j & 1][3 * g + (j >> 1)] = scr_mfma16x32(A1, B[j], as[j & 1][3 * g + (j >> 1)]);
+                    if (g == 2) {
+                        B[j] = scr_op(scr_spread(xb[j]));
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                t = tn;
+                f = fn;
+                if (g < 2) fence(integral_constant<int, 1>{});
+            });
+        }
+    }
+    if (!work) return;
+
+    // Lane: pairs a = aw + 4 kq + i, b = bw + 16 bg + m.
+    uint32_t bits = 0;
+    static_for<8>([&](auto k) {
+        constexpr int K = decltype(k)::value, i = K / 2, bg = K % 2;
+        float n[9], s[9];
+        auto cells = [&](const v4f (&x)[9], float c[9]) {
+            const float xx[3][3] = {{x[0][i], x[1][i], x[2][i]}, {x[3][i], x[4][i], x[5][i]}, {x[6][i], x[7][i], x[8][i]}};
+            c[0] = xx[0][0];
+            c[1] = xx[0][1];
+            c[3] = xx[1][0];
+            c[4] = xx[1][1];
+            c[2] = xx[0][2] - c[0] - c[1];
+            c[5] = xx[1][2] - c[3] - c[4];
+            c[6] = xx[2][0] - c[0] - c[3];
+            c[7] = xx[2][1] - c[1] - c[4];
+            c[8] = (xx[2][2] - xx[0][2] - xx[1][2]) - c[6] - c[7];
+        };
+        cells(av[bg], n);
+        cells(as[bg], s);
+        const int a = aw + 4 * kq + i, b = bw + 16 * bg + m;
+        const bool valid = (a < a1) & (b < b1) & (a > b);
+        const float nc = av[bg][8][i], tc = as[bg][8][i];
+        const float zlow = mz[al + 4 * kq + i] + mz[TA + bl + 16 * bg + m] - C.zall;
+        float u = 0.0f, nmin = n[0];
+#pragma unroll
+        for (int c = 0; c < 9; c++) {
+            u = __builtin_fmaf(s[c] * s[c], rcp_above(n[c]), u);
+            nmin = fminf(nmin, n[c]);
+        }
+        // SST from below: (x + eps)^2 <= 2 x^2 + 2 eps^2
+        const float sst0 = zlow * C.zunit - 2.0f * (tc * tc * rcp_above(nc) + C.eps * C.eps);
+        float kap = C.kap9;
+        if (__ballot(!(nmin > 0.0f)) != 0ull) {
+            float empty = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 9; c++) empty += n[c] > 0.0f ? 0.0f : 1.0f;
+            kap -= C.kslope * empty;
+        }
+        bool keep = valid & !((u <= kap * sst0 - C.kroot) & (2.0f * nc >= C.N));
+        if (__ballot(keep) != 0ull) {
+            const float rt = fabsf(tc) * __builtin_amdgcn_rsqf(nc) * 1.0001f + C.eps;
+            keep = keep && screen_bound(n, s, 64.0f * nc, zlow * C.zunit - rt * rt, C);
+            bits |= keep ? 1u << K : 0u;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    scr_append<8>(cs, bits, region0 + wid, S.tag, [&](int k, int &a, int &b) {
+        a = aw + 4 * kq + (k >> 1);
+        b = bw + 16 * (k & 1) + m;
+    });
+}
+
+template <int TA, int TB>
+__global__ __launch_bounds__((screen_gen_threads<TA, TB>()), 2) void screen_gen_kernel(const ScreenArgs A)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * SW_ROW];
+    __shared__ float mz[TA + TB];
+    const int t = xcd_tile(blockIdx.x, A.ntiles);
+    const int4 T = A.tiles[t];
+    screen_gen_tile<TA, TB>(A.S, A.sw, A.sm, A.cut, A.cs, T.x, T.y, T.z, T.w,
+                            (uint32_t)(A.tile0 + t) * (screen_gen_threads<TA, TB>() / 64), wl, mz);
+}
+
 // Regions that the screen handed back, through the exact tile: a persistent grid
 // over the device's count of them. Region r is wave r % (TA / 16) of tile r / (TA / 16).
 template <int TA>
@@ -430,6 +679,30 @@ __global__ __launch_bounds__(fast_threads<32>(), fast_waves_per_simd<32>()) void
         const int b0 = __builtin_amdgcn_readfirstlane(T.z), b1 = __builtin_amdgcn_readfirstlane(T.w);
         __syncthreads();  // the previous region is done with LDS
         mfma_fast_tile<32, false>(S, hs, nodump, a0, a1, b0, b1, lds);
+    }
+}
+
+// The same for tiles with missing calls (GENERAL and SPARSE, TA x TB), through the exact GENERAL tile.
+template <int TA, int TB>
+__global__ __launch_bounds__(general_threads<32>(), 2) void redo_gen_kernel(const MfmaScan S, const HitSink hs0,
+                                                                           const int4 *tiles, const uint32_t *count,
+                                                                           const uint32_t *redo)
+{
+    constexpr int NWA = TA / SCR_A, NW = NWA * (TB / 32);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[general_lds<32>()];
+    const uint32_t n = count[1];
+    HitSink hs = hs0;
+    hs.tag = S.tag;
+    const DumpSink nodump = {};
+    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+        const int r = (int)(redo[i] % NW);
+        const int4 T = tiles[redo[i] / NW];
+        const int a0 = __builtin_amdgcn_readfirstlane(T.x + SCR_A * (r % NWA));
+        const int b0 = __builtin_amdgcn_readfirstlane(T.z + 32 * (r / NWA));
+        const int a1 = __builtin_amdgcn_readfirstlane(T.y < a0 + SCR_A ? T.y : a0 + SCR_A);
+        const int b1 = __builtin_amdgcn_readfirstlane(T.w < b0 + 32 ? T.w : b0 + 32);
+        __syncthreads();  // the previous region is done with LDS
+        mfma_general_tile<32, false>(S, hs, nodump, a0, a1, b0, b1, lds);
     }
 }
 

@@ -146,7 +146,8 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
         marg[s] = mg;
         const int t0 = sv[0][0][sl] + sv[1][0][sl] + sv[2][0][sl] + sv[3][0][sl];
         const int t1 = sv[0][1][sl] + sv[1][1][sl] + sv[2][1][sl] + sv[3][1][sl];
-        smarg[s] = {(float)tn[0] / 64.0f, (float)tn[1] / 64.0f, (float)t0 / 64.0f, (float)t1 / 64.0f};
+        smarg[s] = {(float)tn[0] / 64.0f, (float)tn[1] / 64.0f, (float)t0 / 64.0f, (float)t1 / 64.0f,
+                    (float)mg.zs, {0.0f, 0.0f, 0.0f}};
     }
 }
 

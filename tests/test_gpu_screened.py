@@ -110,6 +110,43 @@ def test_screened_strong_snps(sch, buf, rows):
     assert both(sch, buf, words2, nid, y, [nsnp], test="f", t1=6.5, t2=10.5) > (1 << 20)
 
 
+@pytest.mark.parametrize("rows", [32, 64])
+@pytest.mark.parametrize("gmiss", [0.002, 0.02, 0.1])
+@pytest.mark.parametrize("nid,sizes", [(120, [2900, 17]), (129, [1500, 1401]), (500, [1025, 16, 15, 33]), (1025, [700, 65]),
+                                       (16384, [300]), (16640, [257, 31])])
+def test_screened_missing(sch, buf, rows, gmiss, nid, sizes):
+    """GENERAL tiles, and at the lowest rate SPARSE ones among them."""
+    seed = nid + rows
+    words = E.synth_genotypes(seed, nid, sum(sizes), 0.02, 0.5, gmiss)
+    sch.set_schedule("mfma", fast_rows=rows)
+    t1, t2 = (float(S.f_isf(1e-5, d, nid - 9)) for d in (8, 4))
+    snp = S.unpack(words[-9:-8], nid)[0].astype(float) % 3  # an additive effect (missing calls as class 0)
+    effect = 9.0 / np.sqrt(nid) * (snp - snp.mean()) / snp.std()
+    for test, safe, kind in (("i", False, "normal"), ("f", False, "casecontrol"), ("i", True, "gamma")):
+        print(f"screened rows={rows} nid={nid} sizes={sizes} gmiss={gmiss} test={test} safe={safe}", flush=True)
+        y = phenotype(kind, nid, seed) + effect.astype(np.float32)
+        y[3::17] = np.nan
+        assert both(sch, buf, words, nid, y, sizes, test=test, safe=safe, t1=t1, t2=t2) > 0
+        kinds = sch.last_tiles()
+        assert kinds["general"] + kinds["sparse"] > 0, kinds
+
+
+@pytest.mark.parametrize("rows", [32, 64])
+def test_screened_missing_strong_snps(sch, buf, rows):
+    """Regions that the exact GENERAL tile redoes, and more candidates than the list holds, as without missing calls."""
+    nid, nsnp = 600, 5200
+    words = E.synth_genotypes(15, nid, nsnp, 0.2, 0.5, 0.01)
+    codes = S.unpack(words, nid) % 3
+    rng = np.random.default_rng(16)
+    sch.set_schedule("mfma", fast_rows=rows)
+    y = (codes[1000:1004].sum(0) + 0.5 * rng.standard_normal(nid)).astype(np.float32)
+    assert both(sch, buf, words, nid, y, [nsnp], test="f", t1=6.5, t2=10.5) > 4 * nsnp * 0.9
+    words2 = words.copy()
+    words2[::16] = words[1000]
+    y = (codes[1000] + rng.standard_normal(nid)).astype(np.float32)
+    assert both(sch, buf, words2, nid, y, [nsnp], test="f", t1=6.5, t2=10.5) > (1 << 20)
+
+
 def test_not_screened(sch, buf):
     """Thresholds that most pairs pass, negative ones, few pairs and phenotypes with outliers keep the exact tiles."""
     nid, nsnp = 800, 1400
@@ -119,5 +156,8 @@ def test_not_screened(sch, buf):
     assert both(sch, buf, words, nid, y, [nsnp], screened=False, test="f", t1=1.5, t2=10.5) > 1000
     assert both(sch, buf, words, nid, y, [nsnp], screened=False, test="i", t1=6.5, t2=-1.0) > 1000
     assert both(sch, buf, words[:300], nid, y, [300], screened=False, test="f", t1=3.0, t2=10.5) > 0
+    # so do datasets with many missing calls
+    gone = E.synth_genotypes(9, nid, nsnp, 0.05, 0.5, 0.2)
+    assert both(sch, buf, gone, nid, y, [nsnp], screened=False, test="f", t1=4.0, t2=10.5) > 0
     y[5] = 1e4
     both(sch, buf, words, nid, y, [nsnp], screened=False, test="f", t1=6.5, t2=10.5)
