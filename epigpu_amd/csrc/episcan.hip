@@ -166,10 +166,14 @@ struct epi_batch {
     std::vector<std::pair<int, int>> scans;  // (dataset, phenotype)
     MfmaScan *d_mscan = nullptr;
     PlainScan *d_pscan = nullptr;
+    ScreenCut *d_cut = nullptr;
+    uint32_t *scount = nullptr;  // the screen's counters, behind nhits: two per tile kind
+    uint32_t *redo = nullptr;    // behind the work items
     int4 *d_work = nullptr;
     int *d_qpos = nullptr, *d_qbegin = nullptr, *d_qend = nullptr;  // [NKIND][NQ]: FAST, GENERAL, SPARSE items
     size_t work_cap = 0, scan_cap = 0;
     long long nkind[NKIND] = {0, 0, 0};  // work items of each tile kind (FAST first in d_work)
+    double wkind[NKIND] = {0, 0, 0};     // pairs times individuals of each tile kind
     DevHit *hits = nullptr;
     unsigned long long *nhits = nullptr;
     long long cap = 1ll << 22;
@@ -808,6 +812,8 @@ MfmaScan mfma_scan(const Dataset &d, int r, int tag)
     S.mlist = d.mlist;
     S.mp = p.mp;
     S.tstride = d.tstride;
+    S.sw = p.sw;
+    S.sm = p.sm;
     return S;
 }
 
@@ -1144,8 +1150,9 @@ bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
     C.N = (float)(N / 64.0);
     C.T = (float)T;
     C.T2N = (float)T2N;
-    C.thr9 = (float)thr9;
-    C.slope = (float)(slope * (1.0 + 1e-5));
+    slope *= 1.0 + 1e-5;
+    C.thr0 = (float)((thr9 - 9.0 * slope) - 1e-5 * std::fabs(thr9 - 9.0 * slope));
+    C.slope2 = (float)(0.5 * slope);
     C.eps = (float)(p.seps / (8.0 * p.sdelta) * (1.0 + 1e-6));
     C.sst = (float)(sst / unit * (1.0 - 1e-6));
     C.nv = (float)N;
@@ -1153,6 +1160,7 @@ bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
     C.t2s = hs.t2s;
     C.test = q->test;
     C.safe = hs.safe;
+    C.ok = 1;
     // GENERAL tiles: the pair's complete cases N' <= N and their SST vary. k / (N' - nfac + k) is smallest at
     // N' = N; the linear form of (sqrt(k SST) - eps)^2 >= k SST - 2 eps sqrt(k SST) takes the largest
     // k SST at N' >= N / 2 (pairs with fewer skip level 0).
@@ -1166,10 +1174,19 @@ bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
     for (int k = inter && !q->safe ? 7 : 2; k < 9; k++) ks = std::max(ks, (k9 - kap(k, N) * (1.0 - 1e-5)) / (9 - k));
     C.zunit = (float)(std::ldexp(1.0, p.zbits) / unit * (1.0 - 1e-6));
     C.zall = (float)(p.zall * (1.0 + 1e-6));
-    C.kap9 = (float)(k9 * (1.0 - 1e-6));
-    C.kslope = (float)(ks * (1.0 + 1e-5));
+    ks *= 1.0 + 1e-5;
+    C.kap0 = (float)((k9 - 9.0 * ks) - 1e-5 * std::fabs(k9 - 9.0 * ks));
+    C.kslope2 = (float)(0.5 * ks);
     C.kroot = (float)(2.0 * p.seps * std::sqrt(kap(9, std::max(0.5 * N, 16.0)) * p.sqV) / unit * (1.0 + 1e-5));
     return true;
+}
+
+// The screen's 32-bit offsets reach two bitplanes, and GENERAL tiles bound SST well up to an eighth of the
+// calls missing.
+bool screen_fits(const Dataset &d)
+{
+    return (unsigned long long)d.Kw * d.nsnp * 8ull < (1ull << 32) - (1u << 20) &&
+           d.missum[d.nsnp] <= (long long)d.nsnp * d.nid / 8;
 }
 
 // Launch of one kind of tile through the screen: bound, resolve, redo. list: the kind's tiles on the device.
@@ -1202,13 +1219,8 @@ int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind
     const ResolveArgs R = {G.S, nullptr, hs, G.cs.cand, K.count, G.cs.cap, resolve_lanes(G.S.Kl)};
     hipLaunchKernelGGL((resolve_kernel<GEN, false>), dim3(4 * c->ncu), dim3(256), 0, c->stream, R);
     HIPCHK(c, hipGetLastError());
-    const uint32_t *cnt = K.count, *rd = K.redo;
-    if constexpr (GEN)
-        hipLaunchKernelGGL((redo_gen_kernel<TA, TB>), dim3(2 * c->ncu), dim3(general_threads<32>()), 0, c->stream, G.S, hs,
-                           K.tiles, cnt, rd);
-    else
-        hipLaunchKernelGGL((redo_fast_kernel<TA>), dim3(2 * c->ncu), dim3(fast_threads<32>()), 0, c->stream, G.S, hs,
-                           K.tiles, cnt, rd);
+    const RedoArgs D = {G.S, nullptr, hs, K.tiles, K.count, K.redo};
+    hipLaunchKernelGGL((redo_kernel<TA, TB, GEN, false>), dim3(2 * c->ncu), dim3(256), 0, c->stream, D);
     HIPCHK(c, hipGetLastError());
     c->last_launches += 2;
     return EPI_OK;
@@ -1238,15 +1250,13 @@ int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, c
         ScreenArgs G;
         const double per = (double)sc.fast_rows * A.S.Kl;  // rows times individuals
         bool sf = nf * 64 * per >= SCR_MIN_WORK, ss = ns * 64 * per * 2.5 >= SCR_MIN_WORK,
-             sg = ng * 32 * per * 2.5 >= SCR_MIN_WORK && d.missum[d.nsnp] <= (long long)d.nsnp * d.nid / 8;
-        if (DUMP || !B.cs.cand || !(sf || ss || sg) || (unsigned long long)d.Kw * d.nsnp * 8ull >= (1ull << 32) - (1u << 20) ||
+             sg = ng * 32 * per * 2.5 >= SCR_MIN_WORK;
+        if (DUMP || !B.cs.cand || !(sf || ss || sg) || !screen_fits(d) ||
             !screen_cut(d.ph[p->phen], p, G.cut))
             sf = ss = sg = false;
         if (sc.dense_missing == 2) ss = false;  // SPARSE tiles asked for
         if (sf || ss || sg) {
             G.S = A.S;
-            G.sw = d.ph[p->phen].sw;
-            G.sm = d.ph[p->phen].sm;
             G.cs = B.cs;
             int rc = EPI_OK;
             uint32_t *redo = B.cs.redo;
@@ -1342,6 +1352,7 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
         ct[kind].resize(nd);
     }
     b->pairs = 0;
+    for (double &x : b->wkind) x = 0.0;
     // estimated cost per pair and individual, by kind
     const double unit[NKIND] = {form == EPI_FORM_MFMA ? 16.0 : 4.0, form == EPI_FORM_MFMA ? 40.0 : 10.0, 22.0};
     for (int di = 0; di < nd; di++) {
@@ -1359,6 +1370,7 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
             for (const int4 &t : v) {
                 int ext = (t.y - t.x) | ((t.w - t.z) << 8) | (kind << 16);
                 double cst = (double)(t.y - t.x) * (t.w - t.z) * d.Kp * unit[kind] + 5e4;
+                b->wkind[kind] += (double)(t.y - t.x) * (t.w - t.z) * d.Kp * sc.size();
                 for (int s : sc) {
                     wk[kind][di].push_back(make_int4(t.x, t.z, ext, s));
                     ct[kind][di].push_back(cst);
@@ -1407,10 +1419,14 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     }
     b->nwork = (long long)work.size();
     int rc;
-    if (work.size() > b->work_cap) {
-        if ((rc = dalloc(c, b->d_work, work.size()))) return rc;
-        b->work_cap = work.size();
+    // behind the items, room for every region of the screen (at most four of 4 bytes per item, eight per SPARSE item)
+    const size_t room = 2 * work.size() + (size_t)b->nkind[2];
+    if (room > b->work_cap) {
+        b->work_cap = 0;
+        if ((rc = dalloc(c, b->d_work, room))) return rc;
+        b->work_cap = room;
     }
+    b->redo = reinterpret_cast<uint32_t *>(b->d_work + work.size());
     if (!work.empty())
         HIPCHK(c, hipMemcpyAsync(b->d_work, work.data(), work.size() * sizeof(int4), hipMemcpyHostToDevice,
                                  c->stream));
@@ -1420,7 +1436,7 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     // scan descriptors
     size_t ns = b->scans.size();
     if (ns > b->scan_cap) {
-        if ((rc = dalloc(c, b->d_mscan, ns)) || (rc = dalloc(c, b->d_pscan, ns))) return rc;
+        if ((rc = dalloc(c, b->d_mscan, ns)) || (rc = dalloc(c, b->d_pscan, ns)) || (rc = dalloc(c, b->d_cut, ns))) return rc;
         b->scan_cap = ns;
     }
     std::vector<MfmaScan> ms(ns);
@@ -1479,6 +1495,60 @@ const void *batch_kernel(int form, const epi_schedule &sc, int kind)
     return kind ? (const void *)plain_batch_kernel<1, 1> : (const void *)plain_batch_kernel<1, 0>;
 }
 
+const void *screen_batch_fn(const epi_schedule &sc, int kind)
+{
+    if (sc.fast_rows == 64)
+        return kind == 2 ? (const void *)screen_batch_kernel<64, 2>
+               : kind    ? (const void *)screen_batch_kernel<64, 1>
+                         : (const void *)screen_batch_kernel<64, 0>;
+    return kind == 2 ? (const void *)screen_batch_kernel<32, 2>
+           : kind    ? (const void *)screen_batch_kernel<32, 1>
+                     : (const void *)screen_batch_kernel<32, 0>;
+}
+
+int screen_batch_threads_of(const epi_schedule &sc, int kind)
+{
+    if (sc.fast_rows == 64)
+        return kind == 2 ? screen_batch_threads<64, 2>() : kind ? screen_batch_threads<64, 1>() : screen_batch_threads<64, 0>();
+    return kind == 2 ? screen_batch_threads<32, 2>() : kind ? screen_batch_threads<32, 1>() : screen_batch_threads<32, 0>();
+}
+
+const void *redo_batch_fn(const epi_schedule &sc, int kind)
+{
+    if (sc.fast_rows == 64)
+        return kind == 2 ? (const void *)redo_kernel<64, 64, true, true>
+               : kind    ? (const void *)redo_kernel<64, 32, true, true>
+                         : (const void *)redo_kernel<64, 64, false, true>;
+    return kind == 2 ? (const void *)redo_kernel<32, 64, true, true>
+           : kind    ? (const void *)redo_kernel<32, 32, true, true>
+                     : (const void *)redo_kernel<32, 64, false, true>;
+}
+
+// Which lists of the batch go through the screen, with the scans' cuts on the device. A list does
+// where it is long enough and at least half of the scans are screened (the tiles of the others are redone
+// whole, by exact tiles).
+int batch_screen(epi_batch *b, const epi_scan_params *p, bool use[NKIND])
+{
+    epi_ctx *c = b->ctx;
+    for (int k = 0; k < NKIND; k++) use[k] = false;
+    if (p->form != EPI_FORM_MFMA || b->nwork >= (1ll << 28)) return EPI_OK;
+    std::vector<ScreenCut> cut(b->scans.size());
+    size_t ok = 0;
+    for (size_t s = 0; s < cut.size(); s++) {
+        const Dataset &d = *b->data[b->scans[s].first];
+        memset(&cut[s], 0, sizeof(ScreenCut));
+        if (screen_fits(d) && screen_cut(d.ph[b->scans[s].second], p, cut[s])) ok++;
+        else cut[s].ok = 0;
+    }
+    if (2 * ok < cut.size()) return EPI_OK;
+    use[0] = b->wkind[0] >= SCR_MIN_WORK;
+    use[1] = 2.5 * b->wkind[1] >= SCR_MIN_WORK;
+    use[2] = 2.5 * b->wkind[2] >= SCR_MIN_WORK && b->work_sched.dense_missing != 2;
+    HIPCHK(c, hipMemcpyAsync(b->d_cut, cut.data(), cut.size() * sizeof(ScreenCut), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return EPI_OK;
+}
+
 // Capture queue reset + the persistent scan kernels as one graph: one kernel
 // per tile kind that has items (GENERAL and SPARSE first under order 1), each with a grid
 // of its occupancy times the CU count, so that every workgroup is resident and
@@ -1490,15 +1560,26 @@ int capture_batch(epi_batch *b, const epi_scan_params *p)
     BatchArgs B[NKIND];
     const void *kfn[NKIND];
     int grid[NKIND] = {0, 0, 0}, nt[NKIND];
+    bool screen[NKIND];
+    int rc = batch_screen(b, p, screen);
+    if (rc) return rc;
+    int Kl = 0;
+    for (const Dataset *d : b->data) Kl = std::max(Kl, (d->nid + KC - 1) / KC * KC);
+    ScreenBatchArgs G[NKIND];
+    const int4 *work = b->d_work;
+    uint32_t *redo = b->redo;
     for (int kind = 0; kind < NKIND; kind++) {
-        nt[kind] = batch_threads_of(p->form, b->work_sched, kind);
+        nt[kind] = screen[kind] ? screen_batch_threads_of(b->work_sched, kind) : batch_threads_of(p->form, b->work_sched, kind);
+        G[kind] = {b->d_mscan, b->d_cut, work, 0, 0, {c->cand, b->scount + 2 * kind, CAND_CAP, redo}};
+        work += b->nkind[kind];
+        redo += (kind == 2 ? 8 : 4) * (size_t)b->nkind[kind];
         B[kind].mscan = b->d_mscan;
         B[kind].pscan = b->d_pscan;
         B[kind].work = b->d_work;
         B[kind].qpos = b->d_qpos + kind * NQ;
         B[kind].qend = b->d_qend + kind * NQ;
         B[kind].hs = make_sink(b->hits, b->nhits, b->cap, p);
-        kfn[kind] = batch_kernel(p->form, b->work_sched, kind);
+        kfn[kind] = screen[kind] ? screen_batch_fn(b->work_sched, kind) : batch_kernel(p->form, b->work_sched, kind);
         int per_cu = 1;
         HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn[kind], nt[kind], 0));
         grid[kind] = std::max(1, per_cu) * c->ncu;
@@ -1506,13 +1587,34 @@ int capture_batch(epi_batch *b, const epi_scan_params *p)
     static const int korder[2][NKIND] = {{0, 2, 1}, {1, 2, 0}};
     const int *ko = korder[b->work_sched.order == 1 ? 1 : 0];
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    hipLaunchKernelGGL(batch_reset, dim3(1), dim3(64), 0, c->stream, b->d_qpos, (const int *)b->d_qbegin, b->nhits);
+    hipLaunchKernelGGL(batch_reset, dim3(1), dim3(64), 0, c->stream, b->d_qpos, (const int *)b->d_qbegin, b->nhits, b->scount);
     hipError_t le = hipGetLastError();
     for (int t = 0; t < NKIND && le == hipSuccess; t++) {
         const int kind = ko[t];
         if (b->nkind[kind] == 0) continue;
-        void *args[] = {&B[kind]};
-        le = hipLaunchKernel(kfn[kind], dim3(grid[kind]), dim3(nt[kind]), args, 0, c->stream);
+        if (!screen[kind]) {
+            void *args[] = {&B[kind]};
+            le = hipLaunchKernel(kfn[kind], dim3(grid[kind]), dim3(nt[kind]), args, 0, c->stream);
+            continue;
+        }
+        // one workgroup per item, in launches of whole XCD groups within the runtime's 2^31 work-items
+        const int4 *items = G[kind].work;
+        const int n = (int)b->nkind[kind], chunk = (int)((1u << 31) / (unsigned)nt[kind]) & ~255;
+        for (int t0 = 0; t0 < n && le == hipSuccess; t0 += chunk) {
+            G[kind].work = items + t0;
+            G[kind].item0 = t0;
+            G[kind].nitems = std::min(chunk, n - t0);
+            void *args[] = {&G[kind]};
+            le = hipLaunchKernel(kfn[kind], dim3(G[kind].nitems), dim3(nt[kind]), args, 0, c->stream);
+        }
+        ResolveArgs R = {{}, b->d_mscan, B[kind].hs, c->cand, G[kind].cs.count, CAND_CAP, resolve_lanes(Kl)};
+        RedoArgs D = {{}, b->d_mscan, B[kind].hs, items, G[kind].cs.count, G[kind].cs.redo};
+        void *rargs[] = {&R}, *dargs[] = {&D};
+        if (le == hipSuccess)
+            le = hipLaunchKernel(kind ? (const void *)resolve_kernel<true, true> : (const void *)resolve_kernel<false, true>,
+                                 dim3(4 * c->ncu), dim3(256), rargs, 0, c->stream);
+        if (le == hipSuccess)
+            le = hipLaunchKernel(redo_batch_fn(b->work_sched, kind), dim3(2 * c->ncu), dim3(256), dargs, 0, c->stream);
     }
     hipError_t ce = hipStreamEndCapture(c->stream, &b->graph);
     if (le != hipSuccess) return fail(c, EPI_ERR_HIP, "launch during capture: %s", hipGetErrorString(le));
@@ -2139,10 +2241,11 @@ int epi_batch_create(epi_ctx *c, epi_batch **out)
     int rc;
     if ((rc = dalloc(c, b->d_qpos, NKIND * NQ)) || (rc = dalloc(c, b->d_qbegin, NKIND * NQ)) ||
         (rc = dalloc(c, b->d_qend, NKIND * NQ)) ||
-        (rc = dalloc(c, b->nhits, 1)) || (rc = dalloc(c, b->hits, (size_t)b->cap))) {
+        (rc = dalloc(c, b->nhits, 4)) || (rc = dalloc(c, b->hits, (size_t)b->cap))) {
         epi_batch_destroy(b);
         return rc;
     }
+    b->scount = reinterpret_cast<uint32_t *>(b->nhits + 1);
     *out = b;
     return EPI_OK;
 }
@@ -2160,6 +2263,7 @@ void epi_batch_destroy(epi_batch *b)
     }
     dfree(b->d_mscan);
     dfree(b->d_pscan);
+    dfree(b->d_cut);
     dfree(b->d_work);
     dfree(b->d_qpos);
     dfree(b->d_qbegin);

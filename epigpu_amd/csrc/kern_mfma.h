@@ -88,6 +88,8 @@ struct OutVals {                 // values of the outlier individuals, in fixed-
     float f[OUT_MAX];
 };
 
+struct ScrMarg;
+
 struct MfmaScan {                // one dataset x one phenotype
     const uint32_t *bits;        // [3][Kw][nsnp] bitplanes: class 0, class 1, call present
     const int8_t *wts;           // [NWP][Kp] for this phenotype
@@ -113,6 +115,9 @@ struct MfmaScan {                // one dataset x one phenotype
     const int32_t *mlist;        // per SNP, ascending: the individuals with a missing call
     const MissPhen *mp;          // [Kp] for this phenotype
     long long tstride;           // uint64 words per 64-SNP column of tbits (4 nid)
+    // screen:
+    const uint32_t *sw;          // [Kp / 32][SW_ROW] codes of the coarse phenotype
+    const ScrMarg *sm;           // [nsnp]
 };
 
 // Class of outlier 16w+t at a SNP from its code word w (3: no call).

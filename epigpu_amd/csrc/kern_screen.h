@@ -48,27 +48,28 @@ constexpr int SCR_GEN_ROWS = SCR_WIN + 4;
 constexpr int SCR_A = 16;    // a-SNPs per wave
 constexpr int SCR_REDO = 8;   // candidates per pair slot of a wave (64 pairs) above which the exact tile redoes its region
 
-// Per SNP and phenotype: counts and sums of v of classes 0 and 1 (present
-// phenotypes), divided by 64 as the kernels' accumulators are, and the sum of
-// z over all calls.
+// Per SNP and phenotype: counts and sums of v of classes 0, 1 and 2 (present phenotypes),
+// divided by 64 as the kernels'
+// accumulators are, and the sum of z over all calls.
 struct ScrMarg {
     float n0, n1, s0, s1;
-    float zs, pad[3];
+    float n2, s2, zs, pad;
 };
 
 // The cut of one scan (thresholds and phenotype), in units of v / 8 (sums of squares / 64).
 struct ScreenCut {
     float N, T, T2N;      // complete cases / 64, sum of v / 64, T^2 / N
-    float thr9, slope;    // level 0: sum s^2 / n > thr9 - slope (9 - nfac)
+    float thr0, slope2;   // level 0: sum s^2 / n > thr0 + 2 nfac slope2
     float eps;            // |r - mean(r)| / (8 delta)
     float sst;            // SST(q) / (64 delta^2)
     float nv;             // complete cases
     // GENERAL tiles: nv and N bound the pairs' complete cases from above
     float zunit, zall;    // sums of squares per unit of z (from below); sum of z over all individuals
-    float kap9, kslope;   // level 0: sum s^2 / n > (kap9 - kslope (9 - nfac)) SST - kroot
+    float kap0, kslope2;  // level 0: sum s^2 / n > (kap0 + 2 nfac kslope2) SST - kroot
     float kroot;
     float t1s, t2s;       // lowered thresholds
     int test, safe;
+    int ok;               // 0: the scan is not screened
 };
 
 struct CandSink {
@@ -80,8 +81,6 @@ struct CandSink {
 
 struct ScreenArgs {
     MfmaScan S;
-    const uint32_t *sw;       // [Kw][SW_ROW]
-    const ScrMarg *sm;        // [nsnp]
     ScreenCut cut;
     CandSink cs;
     const int4 *tiles;
@@ -145,6 +144,16 @@ __device__ __forceinline__ v16f scr_mfma32(const v8i &a, const v8i &b, const v16
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 2, 0, 0x84848484, 0, 0x7f7f7f7f);
 }
 
+// Twice the number of occupied cells: a count is 0 or a float whose bits exceed 2 (min and three-operand adds;
+// a minimum with 1 would be rewritten as nine compares).
+__device__ __forceinline__ float scr_nfac2(const float n[9])
+{
+    uint32_t o[9];
+#pragma unroll
+    for (int c = 0; c < 9; c++) o[c] = __float_as_uint(n[c]) < 2u ? __float_as_uint(n[c]) : 2u;
+    return (float)(int)((o[0] + o[1] + o[2]) + (o[3] + o[4] + o[5]) + (o[6] + o[7] + o[8]));
+}
+
 // 1/n from above: the exponent of n negated and its mantissa mirrored, between
 // 1/n and 1.125/n (the linear bound 1 - f/2 >= 1/(1+f) on 0 <= f <= 1), huge for n = 0.
 __device__ __forceinline__ float rcp_above(float n) { return __uint_as_float(0x7F000000u - __float_as_uint(n)); }
@@ -190,6 +199,24 @@ __device__ __forceinline__ bool screen_bound(const float n[9], const float s[9],
     }
     const float ri = sqrtf(ssi) * 1.0001f + C.eps;
     return ri * ri * d2 > 4.0f * C.t2s * ssw;
+}
+
+// n rows of weights from global memory into LDS, four loads in flight per thread.
+template <int NT>
+__device__ __forceinline__ void scr_stage(uint32_t *wl, const uint32_t *src, int n, int tid)
+{
+    const int last = n * (SW_ROW / 4) - 1;  // threads past the end move the last piece
+    const uint4 *g = reinterpret_cast<const uint4 *>(src);
+    uint4 *l = reinterpret_cast<uint4 *>(wl);
+    for (int i = tid; i <= last; i += 4 * NT) {
+        const int i1 = i + NT < last ? i + NT : last, i2 = i + 2 * NT < last ? i + 2 * NT : last,
+                  i3 = i + 3 * NT < last ? i + 3 * NT : last;
+        const uint4 v0 = g[i], v1 = g[i1], v2 = g[i2], v3 = g[i3];
+        l[i] = v0;
+        l[i1] = v1;
+        l[i2] = v2;
+        l[i3] = v3;
+    }
 }
 
 // A wave's candidates into the list, or its region into the redo list: bit k of
@@ -239,9 +266,9 @@ template <int TA>
 constexpr int screen_threads() { return 64 * TA / SCR_A; }
 
 template <int TA>
-__device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const uint32_t *sw, const ScrMarg *sm,
-                                                 const ScreenCut &C, const CandSink &cs, int a0, int a1, int b0, int b1,
-                                                 uint32_t region0, uint32_t *wl, float4 *mg)
+__device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const ScreenCut &C, const CandSink &cs, int a0,
+                                                 int a1, int b0, int b1, uint32_t region0, uint32_t *wl,
+                                                 float4 *mg, float2 *mg2)
 {
     constexpr int NT = screen_threads<TA>();
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
@@ -253,7 +280,8 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const uint32
     for (int i = tid; i < TA + 64; i += NT) {
         int sn = i < TA ? a0 + i : b0 + i - TA;
         sn = sn < S.nsnp ? sn : S.nsnp - 1;
-        mg[i] = *reinterpret_cast<const float4 *>(sm + sn);
+        mg[i] = *reinterpret_cast<const float4 *>(S.sm + sn);
+        if (i < TA) mg2[i] = *reinterpret_cast<const float2 *>(&S.sm[sn].n2);
     }
 
     v16f av[4], al[4];  // [2 bg + h]: counts, sums of v
@@ -336,8 +364,7 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const uint32
     for (int w0 = 0; w0 < nw; w0 += SCR_WIN) {
         const int wn = nw - w0 < SCR_WIN ? nw - w0 : SCR_WIN;
         if (w0) __syncthreads();
-        for (int i = tid; i < wn * (SW_ROW / 4); i += NT)
-            reinterpret_cast<uint4 *>(wl)[i] = reinterpret_cast<const uint4 *>(sw + (size_t)w0 * SW_ROW)[i];
+        scr_stage<NT>(wl, S.sw + (size_t)w0 * SW_ROW, wn, tid);
         __syncthreads();
         if (!work) continue;
         const uint32_t *wr = wl + hf * SW_ROW;
@@ -359,10 +386,14 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const uint32
 
     // Lane: pairs a = aw + 4j + 2hf + p, b = b0 + 32 bg + m; [2bg + h][4j + 2p + g] = X[g][h].
     uint32_t bits = 0;
-    auto cells = [&](auto k, float n[9], float s[9]) {
+    const float4 mb[2] = {mg[TA + m], mg[TA + 32 + m]};
+    static_for<16>([&](auto k) {
         constexpr int K = decltype(k)::value, j = K / 4, p = K / 2 % 2, bg = K % 2, e = 4 * j + 2 * p;
-        const float4 ma = mg[SCR_A * wid + 4 * j + 2 * hf + p], mb = mg[TA + 32 * bg + m];
-        auto fill = [&](float c[9], const v16f &x0, const v16f &x1, float a_0, float a_1, float b_0, float b_1, float all) {
+        const int ia = SCR_A * wid + 4 * j + 2 * hf + p;
+        const float4 ma = mg[ia];
+        const float2 ma2 = mg2[ia];
+        float n[9], s[9];
+        auto fill = [&](float c[9], const v16f &x0, const v16f &x1, float a_0, float a_1, float a_2, float b_0, float b_1) {
             c[0] = x0[e];
             c[1] = x1[e];
             c[3] = x0[e + 1];
@@ -371,32 +402,18 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const uint32
             c[5] = a_1 - c[3] - c[4];
             c[6] = b_0 - c[0] - c[3];
             c[7] = b_1 - c[1] - c[4];
-            c[8] = (all - a_0 - a_1) - c[6] - c[7];
+            c[8] = a_2 - c[6] - c[7];
         };
-        fill(n, av[2 * bg], av[2 * bg + 1], ma.x, ma.y, mb.x, mb.y, C.N);
-        fill(s, al[2 * bg], al[2 * bg + 1], ma.z, ma.w, mb.z, mb.w, C.T);
-    };
-    static_for<16>([&](auto k) {
-        constexpr int K = decltype(k)::value, j = K / 4, p = K / 2 % 2, bg = K % 2;
-        float n[9], s[9];
-        cells(k, n, s);
-        const int a = aw + 4 * j + 2 * hf + p, b = b0 + 32 * bg + m;
-        const bool valid = (a < a1) & (b < b1) & (a > b);
-        float u = 0.0f, nmin = n[0];
+        fill(n, av[2 * bg], av[2 * bg + 1], ma.x, ma.y, ma2.x, mb[bg].x, mb[bg].y);
+        fill(s, al[2 * bg], al[2 * bg + 1], ma.z, ma.w, ma2.y, mb[bg].z, mb[bg].w);
+        float u = 0.0f;
 #pragma unroll
-        for (int c = 0; c < 9; c++) {
-            u = __builtin_fmaf(s[c] * s[c], rcp_above(n[c]), u);
-            nmin = fminf(nmin, n[c]);
-        }
-        float thr = C.thr9;
-        if (__ballot(!(nmin > 0.0f)) != 0ull) {
-            float empty = 0.0f;
-#pragma unroll
-            for (int c = 0; c < 9; c++) empty += n[c] > 0.0f ? 0.0f : 1.0f;
-            thr -= C.slope * empty;
-        }
-        bool keep = valid & !(u <= thr);
+        for (int c = 0; c < 9; c++) u = __builtin_fmaf(s[c] * s[c], rcp_above(n[c]), u);
+        const float thr = __builtin_fmaf(C.slope2, scr_nfac2(n), C.thr0);
+        bool keep = !(u <= thr);
         if (__ballot(keep) != 0ull) {
+            const int a = aw + 4 * j + 2 * hf + p, b = b0 + 32 * bg + m;
+            keep = keep & (a < a1) & (b < b1) & (a > b);
             keep = keep && screen_bound(n, s, C.nv, C.sst, C);
             bits |= keep ? 1u << K : 0u;
         }
@@ -413,9 +430,11 @@ __global__ __launch_bounds__(screen_threads<TA>(), 2) void screen_fast_kernel(co
 {
     __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_LDS_ROWS * SW_ROW];
     __shared__ float4 mg[TA + 64];
+    __shared__ float2 mg2[TA];
     const int t = xcd_tile(blockIdx.x, A.ntiles);
     const int4 T = A.tiles[t];
-    screen_fast_tile<TA>(A.S, A.sw, A.sm, A.cut, A.cs, T.x, T.y, T.z, T.w, (uint32_t)(A.tile0 + t) * (TA / SCR_A), wl, mg);
+    screen_fast_tile<TA>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, (uint32_t)(A.tile0 + t) * (TA / SCR_A), wl, mg,
+                         mg2);
 }
 
 // ------------------------------------------------------------- GENERAL ----
@@ -442,9 +461,8 @@ template <int TA, int TB>
 constexpr int screen_gen_threads() { return 64 * (TA / SCR_A) * (TB / 32); }
 
 template <int TA, int TB>
-__device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const uint32_t *sw, const ScrMarg *sm, const ScreenCut &C,
-                                                const CandSink &cs, int a0, int a1, int b0, int b1, uint32_t region0,
-                                                uint32_t *wl, float *mz)
+__device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenCut &C, const CandSink &cs, int a0, int a1,
+                                                int b0, int b1, uint32_t region0, uint32_t *wl, float *mz)
 {
     constexpr int NT = screen_gen_threads<TA, TB>(), NWA = TA / SCR_A;
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, kq = lane >> 4;
@@ -457,7 +475,7 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const uint32_
     for (int i = tid; i < TA + TB; i += NT) {
         int sn = i < TA ? a0 + i : b0 + i - TA;
         sn = sn < S.nsnp ? sn : S.nsnp - 1;
-        mz[i] = sm[sn].zs;
+        mz[i] = S.sm[sn].zs;
     }
 
     v4f av[2][9], as[2][9];  // [b group][3 g + h]: counts, sums of v
@@ -516,8 +534,7 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const uint32_
     for (int w0 = 0; w0 < nw; w0 += SCR_WIN) {
         const int wn = nw - w0 < SCR_WIN ? nw - w0 : SCR_WIN;
         if (w0) __syncthreads();
-        for (int i = tid; i < wn * (SW_ROW / 4); i += NT)
-            reinterpret_cast<uint4 *>(wl)[i] = reinterpret_cast<const uint4 *>(sw + (size_t)w0 * SW_ROW)[i];
+        scr_stage<NT>(wl, S.sw + (size_t)w0 * SW_ROW, wn, tid);
         __syncthreads();
         if (!work) continue;
         const uint32_t *wr = wl + kq * SW_ROW;
@@ -616,27 +633,18 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const uint32_
         };
         cells(av[bg], n);
         cells(as[bg], s);
-        const int a = aw + 4 * kq + i, b = bw + 16 * bg + m;
-        const bool valid = (a < a1) & (b < b1) & (a > b);
         const float nc = av[bg][8][i], tc = as[bg][8][i];
         const float zlow = mz[al + 4 * kq + i] + mz[TA + bl + 16 * bg + m] - C.zall;
-        float u = 0.0f, nmin = n[0];
+        float u = 0.0f;
 #pragma unroll
-        for (int c = 0; c < 9; c++) {
-            u = __builtin_fmaf(s[c] * s[c], rcp_above(n[c]), u);
-            nmin = fminf(nmin, n[c]);
-        }
+        for (int c = 0; c < 9; c++) u = __builtin_fmaf(s[c] * s[c], rcp_above(n[c]), u);
         // SST from below: (x + eps)^2 <= 2 x^2 + 2 eps^2
         const float sst0 = zlow * C.zunit - 2.0f * (tc * tc * rcp_above(nc) + C.eps * C.eps);
-        float kap = C.kap9;
-        if (__ballot(!(nmin > 0.0f)) != 0ull) {
-            float empty = 0.0f;
-#pragma unroll
-            for (int c = 0; c < 9; c++) empty += n[c] > 0.0f ? 0.0f : 1.0f;
-            kap -= C.kslope * empty;
-        }
-        bool keep = valid & !((u <= kap * sst0 - C.kroot) & (2.0f * nc >= C.N));
+        const float kap = __builtin_fmaf(C.kslope2, scr_nfac2(n), C.kap0);
+        bool keep = !((u <= kap * sst0 - C.kroot) & (2.0f * nc >= C.N));
         if (__ballot(keep) != 0ull) {
+            const int a = aw + 4 * kq + i, b = bw + 16 * bg + m;
+            keep = keep & (a < a1) & (b < b1) & (a > b);
             const float rt = fabsf(tc) * __builtin_amdgcn_rsqf(nc) * 1.0001f + C.eps;
             keep = keep && screen_bound(n, s, 64.0f * nc, zlow * C.zunit - rt * rt, C);
             bits |= keep ? 1u << K : 0u;
@@ -656,53 +664,64 @@ __global__ __launch_bounds__((screen_gen_threads<TA, TB>()), 2) void screen_gen_
     __shared__ float mz[TA + TB];
     const int t = xcd_tile(blockIdx.x, A.ntiles);
     const int4 T = A.tiles[t];
-    screen_gen_tile<TA, TB>(A.S, A.sw, A.sm, A.cut, A.cs, T.x, T.y, T.z, T.w,
+    screen_gen_tile<TA, TB>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w,
                             (uint32_t)(A.tile0 + t) * (screen_gen_threads<TA, TB>() / 64), wl, mz);
 }
 
-// Regions that the screen handed back, through the exact tile: a persistent grid
-// over the device's count of them. Region r is wave r % (TA / 16) of tile r / (TA / 16).
-template <int TA>
-__global__ __launch_bounds__(fast_threads<32>(), fast_waves_per_simd<32>()) void redo_fast_kernel(
-    const MfmaScan S, const HitSink hs0, const int4 *tiles, const uint32_t *count, const uint32_t *redo)
-{
-    __shared__ __attribute__((aligned(16))) uint8_t lds[fast_lds<32>()];
-    const uint32_t n = count[1];
-    HitSink hs = hs0;
-    hs.tag = S.tag;
-    const DumpSink nodump = {};
-    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-        const uint32_t r = redo[i];
-        const int4 T = tiles[r / (TA / SCR_A)];
-        const int a0 = __builtin_amdgcn_readfirstlane(T.x + SCR_A * (int)(r % (TA / SCR_A)));
-        const int a1 = __builtin_amdgcn_readfirstlane(T.y < a0 + SCR_A ? T.y : a0 + SCR_A);
-        const int b0 = __builtin_amdgcn_readfirstlane(T.z), b1 = __builtin_amdgcn_readfirstlane(T.w);
-        __syncthreads();  // the previous region is done with LDS
-        mfma_fast_tile<32, false>(S, hs, nodump, a0, a1, b0, b1, lds);
-    }
-}
+// --------------------------------------------------------------- redo ----
+// Regions that the screen handed back, and tiles of scans that it does not take (SCR_WHOLE),
+// through the exact tiles of 32 rows: a persistent grid over the device's count of them. A region r of a TA x TB
+// tile t is wave r % NW (a block wave % (TA / 16), b block wave / (TA / 16)) of tile r / NW.
+constexpr uint32_t SCR_WHOLE = 1u << 31;
 
-// The same for tiles with missing calls (GENERAL and SPARSE, TA x TB), through the exact GENERAL tile.
-template <int TA, int TB>
-__global__ __launch_bounds__(general_threads<32>(), 2) void redo_gen_kernel(const MfmaScan S, const HitSink hs0,
-                                                                           const int4 *tiles, const uint32_t *count,
-                                                                           const uint32_t *redo)
+struct RedoArgs {
+    MfmaScan S;               // single scans
+    const MfmaScan *scans;    // batches: by scan id
+    HitSink hs;
+    const int4 *tiles;        // single scans {a0, a1, b0, b1}; batches {a0, b0, extents, scan}
+    const uint32_t *count;
+    const uint32_t *redo;
+};
+
+template <int TA, int TB, bool GEN, bool BATCH>
+__global__ __launch_bounds__(256, 2) void redo_kernel(const RedoArgs A)
 {
-    constexpr int NWA = TA / SCR_A, NW = NWA * (TB / 32);
-    __shared__ __attribute__((aligned(16))) uint8_t lds[general_lds<32>()];
-    const uint32_t n = count[1];
-    HitSink hs = hs0;
-    hs.tag = S.tag;
+    static_assert(fast_threads<32>() == 256 && general_threads<32>() == 256, "threads of the 32-row tiles");
+    constexpr int RB = GEN ? 32 : 64, NW = TA / SCR_A * (TB / RB);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[GEN ? general_lds<32>() : fast_lds<32>()];
+    const uint32_t n = A.count[1];
     const DumpSink nodump = {};
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-        const int r = (int)(redo[i] % NW);
-        const int4 T = tiles[redo[i] / NW];
-        const int a0 = __builtin_amdgcn_readfirstlane(T.x + SCR_A * (r % NWA));
-        const int b0 = __builtin_amdgcn_readfirstlane(T.z + 32 * (r / NWA));
-        const int a1 = __builtin_amdgcn_readfirstlane(T.y < a0 + SCR_A ? T.y : a0 + SCR_A);
-        const int b1 = __builtin_amdgcn_readfirstlane(T.w < b0 + 32 ? T.w : b0 + 32);
-        __syncthreads();  // the previous region is done with LDS
-        mfma_general_tile<32, false>(S, hs, nodump, a0, a1, b0, b1, lds);
+        const uint32_t r = __builtin_amdgcn_readfirstlane(A.redo[i]);
+        int4 T = A.tiles[(r & ~SCR_WHOLE) / NW];
+        HitSink hs = A.hs;
+        int sc = 0;
+        if (BATCH) {
+            sc = __builtin_amdgcn_readfirstlane(T.w);
+            T = make_int4(T.x, T.x + (T.z & 255), T.y, T.y + ((T.z >> 8) & 255));
+        }
+        const MfmaScan &S = BATCH ? A.scans[sc] : A.S;
+        hs.tag = S.tag;
+        // the entry's pairs, as exact tiles of at most 32 x RB
+        int a0 = __builtin_amdgcn_readfirstlane(T.x), a1 = __builtin_amdgcn_readfirstlane(T.y);
+        int b0 = __builtin_amdgcn_readfirstlane(T.z), b1 = __builtin_amdgcn_readfirstlane(T.w);
+        if (!(r & SCR_WHOLE)) {
+            const int w = (int)(r % NW);
+            a0 += SCR_A * (w % (TA / SCR_A));
+            b0 += RB * (w / (TA / SCR_A));
+            a1 = a1 < a0 + SCR_A ? a1 : a0 + SCR_A;
+            b1 = b1 < b0 + RB ? b1 : b0 + RB;
+        }
+        for (int x = a0; x < a1; x += 32)
+            for (int y = b0; y < b1; y += RB) {
+                const int x1 = a1 < x + 32 ? a1 : x + 32, y1 = b1 < y + RB ? b1 : y + RB;
+                if (x1 - 1 <= y) continue;
+                __syncthreads();  // the previous tile is done with LDS
+                if constexpr (GEN)
+                    mfma_general_tile<32, false>(S, hs, nodump, x, x1, y, y1, lds);
+                else
+                    mfma_fast_tile<32, false>(S, hs, nodump, x, x1, y, y1, lds);
+            }
     }
 }
 

@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
     __shared__ double sy[4][3][64];
     __shared__ int sn[4][3][64];
     __shared__ long long sz[4][64];
-    __shared__ int sv[4][2][64];
+    __shared__ int sv[4][3][64];
     const int sl = threadIdx.x & 63, grp = threadIdx.x >> 6;
     const int s = blockIdx.x * 64 + sl;
     int n[3] = {0, 0, 0};
@@ -114,6 +114,7 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
     sz[grp][sl] = z;
     sv[grp][0][sl] = v3[0];
     sv[grp][1][sl] = v3[1];
+    sv[grp][2][sl] = v3[2];
     __syncthreads();
     if (grp == 0 && s < nsnp) {
         int tn[3];
@@ -146,8 +147,10 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
         marg[s] = mg;
         const int t0 = sv[0][0][sl] + sv[1][0][sl] + sv[2][0][sl] + sv[3][0][sl];
         const int t1 = sv[0][1][sl] + sv[1][1][sl] + sv[2][1][sl] + sv[3][1][sl];
-        smarg[s] = {(float)tn[0] / 64.0f, (float)tn[1] / 64.0f, (float)t0 / 64.0f, (float)t1 / 64.0f,
-                    (float)mg.zs, {0.0f, 0.0f, 0.0f}};
+        const int t2 = sv[0][2][sl] + sv[1][2][sl] + sv[2][2][sl] + sv[3][2][sl];
+        const float u = 1.0f / 64.0f;
+        smarg[s] = {(float)tn[0] * u, (float)tn[1] * u, (float)t0 * u, (float)t1 * u, (float)tn[2] * u, (float)t2 * u,
+                    (float)mg.zs, 0.0f};
     }
 }
 

@@ -147,6 +147,43 @@ def test_screened_missing_strong_snps(sch, buf, rows):
     assert both(sch, buf, words2, nid, y, [nsnp], test="f", t1=6.5, t2=10.5) > (1 << 20)
 
 
+@pytest.mark.parametrize("rows", [32, 64])
+def test_screened_batch(scanner, buf, rows):
+    """A batch over FAST, SPARSE and GENERAL lists, several phenotypes per dataset, one of them with outliers (its tiles
+    are redone whole), one dataset of strong SNPs; every scan against the exact tiles, over three replays."""
+    data = [(900, [1300, 200], 0.0, 3), (1300, [900], 0.001, 2), (700, [500, 450], 0.02, 2), (17000, [150], 0.0, 1)]
+    t1, t2 = 4.5, 6.5
+    with E.Batch(scanner) as b:
+        b.set_schedule("mfma", fast_rows=rows)
+        made = []
+        for i, (nid, sizes, gmiss, nphen) in enumerate(data):
+            words = E.synth_genotypes(100 + i, nid, sum(sizes), 0.05, 0.5, gmiss)
+            y = np.stack([phenotype(k, nid, 200 + i) for k in ("normal", "gamma", "casecontrol")[:nphen]])
+            if i == 0:
+                y[1, 7] = 1e4  # an outlier
+                y[2] += 1.5 * S.unpack(words[60:64], nid).sum(0)
+            y[:, 5::13] = np.nan
+            starts = list(np.cumsum([0] + sizes[:-1]))
+            d = b.add_dataset(words, nid, starts, sizes)
+            made += [(words, nid, sizes, yy, s) for yy, s in zip(y, b.add_phenotypes(d, y))]
+        for rep in range(3):
+            b.scan(test="i", t1=t1, t2=t2)
+            for words, nid, sizes, y, s in made:
+                print(f"screened batch rows={rows} replay={rep} scan={s}", flush=True)
+                g = b.hits(s)
+                scanner.set_genotypes(words, nid)
+                scanner.set_phenotypes(y)
+                scanner.set_chromosomes(list(np.cumsum([0] + sizes[:-1])), sizes)
+                n = scanner.scan_noalloc(buf.ptr.value, CAP, test="i", t1=t1, t2=t2)
+                assert g["nhits"] == n > 0
+                h = buf.read(S.HIT64_DTYPE, n)
+                h = h[np.lexsort((h["snp2"], h["snp1"]))]
+                o = np.lexsort((g["hits"]["snp2"], g["hits"]["snp1"]))
+                for k in ("snp1", "snp2", "df1", "df2"):
+                    assert np.array_equal(h[k], g["hits"][k][o]), k
+                assert np.array_equal(h["F"], g["F64"][o]) and np.array_equal(h["F2"], g["F2_64"][o])
+
+
 def test_not_screened(sch, buf):
     """Thresholds that most pairs pass, negative ones, few pairs and phenotypes with outliers keep the exact tiles."""
     nid, nsnp = 800, 1400
