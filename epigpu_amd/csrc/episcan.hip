@@ -13,8 +13,9 @@
 //     marg  [nsnp]  Marg   per-SNP class counts and sums
 //     oidx, ocodes, ov     outlier individuals (at most OUT_MAX), their codes per SNP and values
 //     mp    [Kp]    MissPhen V, q, z per individual (SPARSE tiles), coarse phenotype v of the screen
-//     sw    [Kw][SW_ROW] uint32  the screen's FP6 codes of v and presence bits, per 32 individuals
-//     sm    [nsnp]  ScrMarg per-SNP counts and sums of v
+//     sw    [Kw][8], [Kw][16] uint32  the screen's FP6 codes of v (one and two digits) and presence bits, per
+//                   32 individuals (behind wts)
+//     sm    [nsnp]  ScrMarg per-SNP counts and sums of v (before marg, in its allocation)
 //   for SPARSE tiles (built at the first scan that has them, for the chromosome layout it was built for):
 //     moff  [nsnp+1] int64, mlist int32   per SNP, the individuals with a missing call
 //     vidx  [nsnp]  int32  virtual SNP index: each chromosome starts at a multiple of 64
@@ -60,6 +61,14 @@ constexpr long long ZMAX = 2139062143;  // largest |z| with four balanced int8 l
 constexpr double OUT_SD = 32.0;
 constexpr double BULK_SD = 64.0;
 
+// The coarse phenotype of the screen, of one or two digits: q ~ delta v + offset.
+struct ScreenEnc {
+    double delta = 0.0;   // 0: none
+    double offset = 0.0;
+    double eps = 0.0;     // |q - delta v - offset| over the present individuals
+    double vsum = 0.0;    // sum of v
+};
+
 struct PhenDev {
     int8_t *wts = nullptr;
     int32_t *qv = nullptr;
@@ -70,11 +79,9 @@ struct PhenDev {
     uint32_t *ocodes = nullptr; // [ceil(nout/16)][nsnp], built with the marginals
     OutVals *ov = nullptr;
     MissPhen *mp = nullptr;
-    uint32_t *sw = nullptr;     // screen
-    ScrMarg *sm = nullptr;
-    double sdelta = 0.0;        // q ~ sdelta v
-    double seps = 0.0;          // |r|, r = q - sdelta v (q units)
-    double svsum = 0.0;         // sum of v
+    uint32_t *sw[2] = {nullptr, nullptr};  // screen (in the allocation of wts)
+    ScrMarg *sm = nullptr;                 // screen (owns marg)
+    ScreenEnc scr[2];
     double zall = 0.0;          // sum of z
     int nout = 0;
     int fbits = 0;  // q = round((y - centre) * 2^fbits)
@@ -247,13 +254,12 @@ void free_phen(PhenDev &p)
     dfree(p.qv);
     dfree(p.yc);
     dfree(p.vbits);
-    dfree(p.marg);
+    dfree(p.sm);
+    p.marg = nullptr;
     dfree(p.oidx);
     dfree(p.ocodes);
     dfree(p.ov);
     dfree(p.mp);
-    dfree(p.sw);
-    dfree(p.sm);
 }
 
 void drop_sparse(Dataset &d)
@@ -376,26 +382,19 @@ bool split_limbs(long long x, int n, int8_t *out)
 
 // Host-side encoding of one phenotype, before anything is allocated.
 struct PhenEnc {
-    std::vector<int8_t> w;      // [NWP][Kp]
+    std::vector<int8_t> w;      // [NWP][Kp], then the screen's weights (3 Kp bytes)
     std::vector<int32_t> qv;    // [Kp]
     std::vector<float> yc;      // [Kp]
     std::vector<uint32_t> vb;   // [Kw]
     std::vector<int32_t> oidx;  // outlier individuals
     std::vector<MissPhen> mp;   // [Kp]
-    std::vector<uint32_t> sw;   // [Kw][SW_ROW]
     OutVals ov = {};
     PhenDev p;                  // scalars only
 };
 
-// Coarse phenotype of the screen. Digits: the integers that FP6 E2M3 holds in
-// units of 1/8 (0..16, even to 30, multiples of 4 to 60, either sign).
-int fp6_nearest(double t)
-{
-    const double a = std::fabs(t);
-    const int st = a <= 16.0 ? 1 : a <= 31.0 ? 2 : 4;
-    const int v = std::min(60, st * (int)std::floor(a / st + 0.5));
-    return t < 0.0 ? -v : v;
-}
+// Coarse phenotypes of the screen. A digit is an integer that FP6 E2M3 holds in
+// units of 1/8: 0..16, even to 30, multiples of 4 to 60, either sign.
+constexpr int SCR_VMAX1 = 60, SCR_VMAX2 = 32 * 60 + 60;
 
 uint32_t fp6_code(int d)
 {
@@ -404,58 +403,132 @@ uint32_t fp6_code(int d)
     return c | (d < 0 ? 32u : 0u);
 }
 
-constexpr int SCR_VMAX = 32 * 60 + 60;
+// Nearest representable v = D0 and v = 32 D1 + D0 of every integer up to the largest, with their codes.
+struct ScrTable {
+    struct Entry {
+        int16_t v;
+        uint8_t c0, c1;
+    };
+    Entry one[2 * SCR_VMAX1 + 1], two[2 * SCR_VMAX2 + 1];
+    ScrTable()
+    {
+        std::vector<int> digit;
+        for (int d = -60; d <= 60; d++)
+            if (std::abs(d) <= 16 || (std::abs(d) <= 32 && d % 2 == 0) || d % 4 == 0) digit.push_back(d);
+        auto fill = [](Entry *t, int vmax) {  // nearest set entries into the gaps
+            std::vector<Entry> full(t, t + 2 * vmax + 1);
+            for (int i = 0; i <= 2 * vmax; i++)
+                for (int o = 0;; o++) {
+                    if (i - o >= 0 && full[i - o].v != INT16_MAX) { t[i] = full[i - o]; break; }
+                    if (i + o <= 2 * vmax && full[i + o].v != INT16_MAX) { t[i] = full[i + o]; break; }
+                }
+        };
+        for (Entry &e : one) e = {INT16_MAX, 0, 0};
+        for (Entry &e : two) e = {INT16_MAX, 0, 0};
+        for (int d : digit) one[d + SCR_VMAX1] = {(int16_t)d, (uint8_t)fp6_code(d), 0};
+        for (int h : digit)
+            for (int l : digit) two[32 * h + l + SCR_VMAX2] = {(int16_t)(32 * h + l), (uint8_t)fp6_code(l), (uint8_t)fp6_code(h)};
+        fill(one, SCR_VMAX1);
+        fill(two, SCR_VMAX2);
+    }
+    const Entry &get(int nd, double t) const
+    {
+        const int m = nd == 1 ? SCR_VMAX1 : SCR_VMAX2;
+        const int i = (int)std::lrint(std::min((double)m, std::max((double)-m, t)));
+        return (nd == 1 ? one : two)[i + m];
+    }
+};
 
-// v = 32 D1 + D0 nearest to q / delta for every present individual, with
-// delta the smallest that keeps |v| <= SCR_VMAX and the sum of |v| below 2^24
-// (with room for the rounding), so that every sum of v in FP32 is exact.
-void encode_screen(const std::vector<int> &P, int Kw, PhenEnc &e)
+const ScrTable &scr_table()
 {
-    PhenDev &p = e.p;
+    static const ScrTable t;
+    return t;
+}
+
+// Sums of a fit of q on v.
+struct ScrFit {
+    double n = 0.0, q = 0.0, v = 0.0, qq = 0.0, qv = 0.0, vv = 0.0, va = 0.0;
+    void add(double x, double y)
+    {
+        n += 1.0;
+        q += x;
+        v += y;
+        qq += x * x;
+        qv += x * y;
+        vv += y * y;
+        va += std::fabs(y);
+    }
+    // squared residue of the least-squares line
+    double residue(double &slope, double &off) const
+    {
+        const double cvv = vv - v * v / n, cqv = qv - q * v / n;
+        slope = cvv > 0.0 ? cqv / cvv : 0.0;
+        off = (q - slope * v) / n;
+        return std::max(0.0, qq - q * q / n - slope * cqv);
+    }
+};
+
+// v of nd digits for the present individuals P: q / step, rounded to what the digits hold, then the line q ~ delta v
+// + offset of least squares, whose residue is what the bound pays. Two digits: the smallest step without
+// clipping. One digit: the best of a few, clipping included, on up to 1024 individuals. The sum of |v|
+// stays below 2^24, so that every sum of v in FP32 is exact.
+void encode_screen(const std::vector<int> &P, int Kp, int nd, PhenEnc &e)
+{
+    ScreenEnc &S = e.p.scr[nd - 1];
+    S = ScreenEnc();
+    const ScrTable &T = scr_table();
     double mx = 0.0, sum = 0.0;
     for (int k : P) {
         const double a = std::fabs((double)e.qv[k]);
         mx = std::max(mx, a);
         sum += a;
     }
-    const double room = 16777216.0 - 2.0 * (double)P.size();  // each |v| exceeds |q| / delta by at most 2
-    p.sdelta = std::max(mx / SCR_VMAX, room > 1.0 ? sum / room : 0.0);
-    if (!(p.sdelta > 0.0) || room <= 1.0) p.sdelta = 0.0;  // constant phenotype or a huge cohort: not screened
-    e.sw.assign((size_t)Kw * SW_ROW, 0u);
-    if (p.sdelta == 0.0) return;
-    double rq = 0.0;
-    for (int k : P) {
-        const double t = (double)e.qv[k] / p.sdelta;
-        int hi = 0, lo = 0;
-        double best = INFINITY;
-        const int h0 = fp6_nearest(t / 32.0);
-        for (int dh : {0, -1, 1, -2, 2, -4, 4}) {
-            const int h = fp6_nearest((double)(h0 + dh)), l = fp6_nearest(t - 32.0 * h);
-            const double err = std::fabs(t - (32.0 * h + l));
-            if (err < best) {
-                best = err;
-                hi = h;
-                lo = l;
+    const double room = 16777216.0 - (nd == 1 ? 4.0 : 130.0) * (double)P.size();  // |v| exceeds |q| / step by less
+    if (!(mx > 0.0) || room <= 0.0) return;
+    const double least = sum / room;
+    double step = std::max(mx / (nd == 1 ? SCR_VMAX1 : SCR_VMAX2), least), slope, off;
+    if (nd == 1) {
+        const size_t stride = (P.size() + 1023) / 1024;
+        double best = INFINITY, top = step;
+        for (double f : {1.0, 0.8, 0.65, 0.5, 0.4}) {
+            ScrFit F;
+            for (size_t i = 0; i < P.size(); i += stride) F.add(e.qv[P[i]], T.get(1, e.qv[P[i]] / (f * top)).v);
+            const double r = F.residue(slope, off);
+            if (f * top >= least && slope > 0.0 && r < best) {
+                best = r;
+                step = f * top;
             }
-            if (best <= 0.5) break;
         }
-        const int v = 32 * hi + lo;
-        e.mp[k].sv = v;
-        p.svsum += v;
-        const double r = (double)e.qv[k] - p.sdelta * v;
-        rq += r * r;
-        // the element of individual k & 31: six bits from bit 6 slot of the word's 192
-        const int bit = 6 * scr_slot(k & 31);
-        uint32_t *row = e.sw.data() + (size_t)(k >> 5) * SW_ROW;
-        const int d[2] = {lo, hi};
-        for (int i = 0; i < 2; i++) {
-            const uint64_t c = (uint64_t)fp6_code(d[i]) << (bit & 31);
-            row[6 * i + (bit >> 5)] |= (uint32_t)c;
-            if (c >> 32) row[6 * i + (bit >> 5) + 1] |= (uint32_t)(c >> 32);
-        }
-        row[12] |= 1u << (k & 31);
     }
-    p.seps = std::sqrt(rq) * (1.0 + 1e-6);
+    ScrFit F;
+    const double inv = 1.0 / step;
+    uint32_t *rows = reinterpret_cast<uint32_t *>(e.w.data() + (size_t)NWP * Kp) + (nd == 1 ? 0 : Kp / 4);
+    const int row = 8 * nd;
+    for (int k : P) {
+        const ScrTable::Entry &t = T.get(nd, e.qv[k] * inv);
+        e.mp[k].sv[nd - 1] = t.v;
+        F.add(e.qv[k], t.v);
+        // the element of individual k & 31: six bits from bit 6 slot of the word's 192
+        static const struct Slots {
+            int bit[32];
+            Slots() { for (int i = 0; i < 32; i++) bit[i] = 6 * scr_slot(i); }
+        } slots;
+        const int bit = slots.bit[k & 31];
+        uint32_t *r = rows + (size_t)(k >> 5) * row;
+        for (int i = 0; i < nd; i++) {
+            const uint64_t c = (uint64_t)(i ? t.c1 : t.c0) << (bit & 31);
+            r[6 * i + (bit >> 5)] |= (uint32_t)c;
+            if (c >> 32) r[6 * i + (bit >> 5) + 1] |= (uint32_t)(c >> 32);
+        }
+        r[6 * nd] |= 1u << (k & 31);
+    }
+    const double r2 = F.residue(slope, off);
+    if (!(slope > 0.0) || F.va >= 16777216.0) return;
+    S.delta = slope;
+    S.offset = off;
+    // (the residue is a difference of sums of N terms: their rounding is added)
+    S.eps = std::sqrt(r2 + 1e-12 * F.qq) * (1.0 + 1e-6);
+    S.vsum = F.v;
 }
 
 // Phenotype prep (src/EpiOpenCL.c:1364-1376 computes mY and SSY over all nid
@@ -538,7 +611,7 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
     int ye = 0;
     if (maxall > 0.0) std::frexp(maxall, &ye);
     const int Kw = Kp / 32;
-    e.w.assign((size_t)NWP * Kp, 0);
+    e.w.assign((size_t)(NWP + 3) * Kp, 0);
     e.qv.assign(Kp, 0);
     e.yc.assign(Kp, 0.0f);
     e.vb.assign(Kw, 0u);
@@ -579,7 +652,7 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
         y2 += (double)ycf * (double)ycf;
         e.vb[k >> 5] |= 1u << (k & 31);
     }
-    encode_screen(P, Kw, e);
+    for (int nd : {1, 2}) encode_screen(P, Kp, nd, e);
     for (int t = 0; t < p.nout; t++) {
         const double u = std::ldexp((double)y[e.oidx[t]] - centre, f);
         e.ov.d[t] = u;
@@ -623,8 +696,10 @@ int ds_set_phenotypes(epi_ctx *c, Dataset &d, const float *phen, int nphen, int 
         p = e.p;
         if ((rc = dalloc(c, p.wts, e.w.size())) || (rc = dalloc(c, p.qv, (size_t)Kp)) ||
             (rc = dalloc(c, p.yc, (size_t)Kp)) || (rc = dalloc(c, p.vbits, (size_t)Kw)) ||
-            (rc = dalloc(c, p.ov, 1)) || (rc = dalloc(c, p.mp, (size_t)Kp)) || (rc = dalloc(c, p.sw, e.sw.size())))
+            (rc = dalloc(c, p.ov, 1)) || (rc = dalloc(c, p.mp, (size_t)Kp)))
             break;
+        p.sw[0] = reinterpret_cast<uint32_t *>(p.wts + (size_t)NWP * Kp);
+        p.sw[1] = p.sw[0] + Kp / 4;
         if (p.nout && (rc = dalloc(c, p.oidx, (size_t)p.nout))) break;
         hipError_t he = hipMemcpyAsync(p.wts, e.w.data(), e.w.size(), hipMemcpyHostToDevice, c->stream);
         if (he == hipSuccess) he = hipMemcpyAsync(p.qv, e.qv.data(), (size_t)Kp * 4, hipMemcpyHostToDevice, c->stream);
@@ -634,8 +709,6 @@ int ds_set_phenotypes(epi_ctx *c, Dataset &d, const float *phen, int nphen, int 
         if (he == hipSuccess) he = hipMemcpyAsync(p.ov, &e.ov, sizeof(OutVals), hipMemcpyHostToDevice, c->stream);
         if (he == hipSuccess)
             he = hipMemcpyAsync(p.mp, e.mp.data(), (size_t)Kp * sizeof(MissPhen), hipMemcpyHostToDevice, c->stream);
-        if (he == hipSuccess)
-            he = hipMemcpyAsync(p.sw, e.sw.data(), e.sw.size() * 4, hipMemcpyHostToDevice, c->stream);
         if (he == hipSuccess && p.nout)
             he = hipMemcpyAsync(p.oidx, e.oidx.data(), (size_t)p.nout * 4, hipMemcpyHostToDevice, c->stream);
         if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
@@ -683,9 +756,12 @@ int ds_marginals(epi_ctx *c, Dataset &d)
     if (!d.mbits) return fail(c, EPI_ERR_STATE, "genotypes not set");
     if (d.ph.empty()) return fail(c, EPI_ERR_STATE, "phenotypes not set");
     for (auto &p : d.ph) {
-        int rc = dalloc(c, p.marg, (size_t)d.nsnp);
-        if (!rc) rc = dalloc(c, p.sm, (size_t)d.nsnp);
+        // one allocation: the screen's marginals, then the others
+        const size_t per = sizeof(Marg) + sizeof(ScrMarg);
+        p.marg = nullptr;
+        int rc = dalloc(c, p.sm, (per * d.nsnp + sizeof(ScrMarg) - 1) / sizeof(ScrMarg));
         if (rc) return rc;
+        p.marg = reinterpret_cast<Marg *>(p.sm + d.nsnp);
         hipLaunchKernelGGL(marginals_kernel, dim3((d.nsnp + 63) / 64), dim3(256), 0, c->stream,
                            (const uint32_t *)d.mbits, d.Kw, d.nsnp, (const uint32_t *)p.vbits, (const int32_t *)p.qv,
                            (const float *)p.yc, (const int32_t *)d.cls, (const MissPhen *)p.mp, p.marg, p.sm);
@@ -812,7 +888,9 @@ MfmaScan mfma_scan(const Dataset &d, int r, int tag)
     S.mlist = d.mlist;
     S.mp = p.mp;
     S.tstride = d.tstride;
-    S.sw = p.sw;
+    S.rbits = d.bits;
+    S.sw[0] = p.sw[0];
+    S.sw[1] = p.sw[1];
     S.sm = p.sm;
     return S;
 }
@@ -1108,9 +1186,12 @@ double chi2_tail(double x, int h)
 
 // The screen's cut for a phenotype and the scan's thresholds; false where the
 // exact tiles are the better path: thresholds so low, or a cohort so large for
-// the coarse phenotype's residue, that more than SCR_RATE of the pairs of
-// unrelated SNPs would be candidates.
-constexpr double SCR_RATE = 2e-3;
+// the coarse phenotype's residue, that more than SCR_RATE2 of the pairs of
+// unrelated SNPs would be candidates. One digit (two thirds of the MFMAs) where SCR_RATE1 holds with it: its
+// larger residue sends more pairs to the second stage and to the resolve kernel (M = 20000, normal phenotype, no
+// missing calls: N = 1500, test i, rate 8e-5: 1.35 ms against 1.57 ms with two digits; N = 3000, test f, 4e-4:
+// 2.34 against 2.52, but with 1 % missing calls 5.38 against 5.37; N = 3000, test i, 7e-4: 3.02 against 2.64).
+constexpr double SCR_RATE1 = 2.5e-4, SCR_RATE2 = 2e-3;
 // Pairs times individuals below which the screen's two further launches cost more than its
 // kernel saves (N = 1000, M = 1000: 20.5 us either way; N = 300, M = 2000: 25.9 us exact, 18.0 us screened).
 constexpr double SCR_MIN_WORK = 5e8;
@@ -1118,66 +1199,69 @@ constexpr double SCR_MIN_WORK = 5e8;
 bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
 {
     const HitSink hs = make_sink(nullptr, nullptr, 0, q);
-    if (p.nout || p.sdelta <= 0.0 || p.nV < 32 || !(hs.t1s > 0.0f)) return false;
+    if (p.nout || p.nV < 32 || !(hs.t1s > 0.0f)) return false;
     const bool inter = q->test != 'f';
     if (inter && !(hs.t2s > 0.0f)) return false;
     if (!std::isfinite(hs.t1s) || (inter && !std::isfinite(hs.t2s))) return false;
     const double N = p.nV, qV = (double)p.qV, sst = p.sqV - qV * qV / N, sig2 = sst / (N - 1.0);
     if (!(sst > 0.0)) return false;
-    const double unit = 64.0 * p.sdelta * p.sdelta;  // q^2 units per unit of the kernels' sums of squares
-    // lower bound on SSB(v) of a pair with nfac occupied cells that passes
-    auto floor_f = [&](int nfac) {
+    // F > t1 is SSB > k1 SST, and F2 > t2 takes SSB >= SSI > k2 SST; n complete cases
+    auto k1 = [&](int nfac, double n) {
         const double k = (double)hs.t1s * (nfac - 1);
-        return std::sqrt(k / (N - nfac + k) * sst);
+        return k / (n - nfac + k);
     };
-    auto floor_i = [&](int nfac) {
+    auto k2 = [&](int nfac, double n) {
         const double k = 4.0 * (double)hs.t2s;
-        return std::sqrt(k / (N - nfac + k) * sst);
+        return k / (n - nfac + k);
     };
-    auto cut = [&](double root) { return std::pow(std::max(0.0, root - p.seps), 2); };
-    double rate = chi2_tail(cut(floor_f(9)) / sig2, 4);
-    if (inter) rate += chi2_tail(cut(floor_i(9)) / sig2, 2);
-    if (rate > SCR_RATE) return false;
+    auto kap = [&](int nfac, double n) { return inter ? std::min(k1(nfac, n), k2(nfac, n)) : k1(nfac, n); };
+    int nd = 0;
+    for (int i = 1; i <= 2 && !nd; i++) {
+        const ScreenEnc &E = p.scr[i - 1];
+        if (!(E.delta > 0.0)) continue;
+        auto tail = [&](double k, int h) { return chi2_tail(std::pow(std::max(0.0, std::sqrt(k * sst) - E.eps), 2) / sig2, h); };
+        double rate = tail(k1(9, N), 4);
+        if (inter) rate += tail(k2(9, N), 2);
+        if (rate <= (i == 1 ? SCR_RATE1 : SCR_RATE2)) nd = i;
+    }
+    if (!nd) return false;
+    const ScreenEnc &E = p.scr[nd - 1];
+    const double unit = 64.0 * E.delta * E.delta;  // q^2 units per unit of the kernels' sums of squares
     memset(&C, 0, sizeof(C));
-    const double T = p.svsum / 64.0, T2N = T * T / (N / 64.0);
+    const double T = E.vsum / 64.0, T2N = T * T / (N / 64.0);
+    // level 0 of FAST tiles: a lower bound on sum s^2 / n = SSB(v) + T^2 / N, linear in the occupied cells
     auto level0 = [&](int nfac) {
-        const double root = inter ? std::min(floor_f(nfac), floor_i(nfac)) : floor_f(nfac);
-        return (cut(root) / unit + T2N) * (1.0 - 1e-5);
+        return (std::pow(std::max(0.0, std::sqrt(kap(nfac, N) * sst) - E.eps), 2) / unit + T2N) * (1.0 - 1e-5);
     };
+    const int least = inter && !q->safe ? 7 : 2;  // occupied cells of a hit
     const double thr9 = level0(9);
     double slope = 0.0;
-    for (int k = inter && !q->safe ? 7 : 2; k < 9; k++) slope = std::max(slope, (thr9 - level0(k)) / (9 - k));
-    C.N = (float)(N / 64.0);
-    C.T = (float)T;
-    C.T2N = (float)T2N;
+    for (int k = least; k < 9; k++) slope = std::max(slope, (thr9 - level0(k)) / (9 - k));
     slope *= 1.0 + 1e-5;
     C.thr0 = (float)((thr9 - 9.0 * slope) - 1e-5 * std::fabs(thr9 - 9.0 * slope));
     C.slope2 = (float)(0.5 * slope);
-    C.eps = (float)(p.seps / (8.0 * p.sdelta) * (1.0 + 1e-6));
+    C.eps = (float)(E.eps / (8.0 * E.delta) * (1.0 + 1e-6));
     C.sst = (float)(sst / unit * (1.0 - 1e-6));
     C.nv = (float)N;
+    C.N = (float)(N / 64.0);
     C.t1s = hs.t1s;
     C.t2s = hs.t2s;
     C.test = q->test;
     C.safe = hs.safe;
-    C.ok = 1;
+    C.nd = nd;
     // GENERAL tiles: the pair's complete cases N' <= N and their SST vary. k / (N' - nfac + k) is smallest at
     // N' = N; the linear form of (sqrt(k SST) - eps)^2 >= k SST - 2 eps sqrt(k SST) takes the largest
     // k SST at N' >= N / 2 (pairs with fewer skip level 0).
-    auto kap = [&](int nfac, double n) {
-        const double k1 = (double)hs.t1s * (nfac - 1), k2 = 4.0 * (double)hs.t2s;
-        const double x = k1 / (n - nfac + k1);
-        return inter ? std::min(x, k2 / (n - nfac + k2)) : x;
-    };
     const double k9 = kap(9, N) * (1.0 - 1e-5);
     double ks = 0.0;
-    for (int k = inter && !q->safe ? 7 : 2; k < 9; k++) ks = std::max(ks, (k9 - kap(k, N) * (1.0 - 1e-5)) / (9 - k));
-    C.zunit = (float)(std::ldexp(1.0, p.zbits) / unit * (1.0 - 1e-6));
-    C.zall = (float)(p.zall * (1.0 + 1e-6));
+    for (int k = least; k < 9; k++) ks = std::max(ks, (k9 - kap(k, N) * (1.0 - 1e-5)) / (9 - k));
     ks *= 1.0 + 1e-5;
     C.kap0 = (float)((k9 - 9.0 * ks) - 1e-5 * std::fabs(k9 - 9.0 * ks));
     C.kslope2 = (float)(0.5 * ks);
-    C.kroot = (float)(2.0 * p.seps * std::sqrt(kap(9, std::max(0.5 * N, 16.0)) * p.sqV) / unit * (1.0 + 1e-5));
+    C.kroot = (float)(2.0 * E.eps * std::sqrt(kap(9, std::max(0.5 * N, 16.0)) * p.sqV) / unit * (1.0 + 1e-5));
+    C.zunit = (float)(std::ldexp(1.0, p.zbits) / unit * (1.0 - 1e-6));
+    C.zall = (float)(p.zall * (1.0 + 1e-6));
+    C.c0 = (float)(E.offset / E.delta);
     return true;
 }
 
@@ -1208,10 +1292,13 @@ int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind
         G.tiles = K.tiles + t0;
         G.ntiles = chunk;
         G.tile0 = t0;
-        if constexpr (GEN)
-            hipLaunchKernelGGL((screen_gen_kernel<TA, TB>), dim3(chunk), dim3(nt), 0, c->stream, G);
-        else
-            hipLaunchKernelGGL((screen_fast_kernel<TA>), dim3(chunk), dim3(nt), 0, c->stream, G);
+        if constexpr (GEN) {
+            if (G.cut.nd == 1) hipLaunchKernelGGL((screen_gen_kernel<TA, TB, 1>), dim3(chunk), dim3(nt), 0, c->stream, G);
+            else hipLaunchKernelGGL((screen_gen_kernel<TA, TB, 2>), dim3(chunk), dim3(nt), 0, c->stream, G);
+        } else {
+            if (G.cut.nd == 1) hipLaunchKernelGGL((screen_fast_kernel<TA, 1>), dim3(chunk), dim3(nt), 0, c->stream, G);
+            else hipLaunchKernelGGL((screen_fast_kernel<TA, 2>), dim3(chunk), dim3(nt), 0, c->stream, G);
+        }
         HIPCHK(c, hipGetLastError());
         c->last_launches++;
         t0 += chunk;
@@ -1537,8 +1624,7 @@ int batch_screen(epi_batch *b, const epi_scan_params *p, bool use[NKIND])
     for (size_t s = 0; s < cut.size(); s++) {
         const Dataset &d = *b->data[b->scans[s].first];
         memset(&cut[s], 0, sizeof(ScreenCut));
-        if (screen_fits(d) && screen_cut(d.ph[b->scans[s].second], p, cut[s])) ok++;
-        else cut[s].ok = 0;
+        if (screen_fits(d) && screen_cut(d.ph[b->scans[s].second], p, cut[s])) ok++;  // cut.nd stays 0 otherwise
     }
     if (2 * ok < cut.size()) return EPI_OK;
     use[0] = b->wkind[0] >= SCR_MIN_WORK;

@@ -130,7 +130,7 @@ template <int TA, int KIND>
 __global__ __launch_bounds__((screen_batch_threads<TA, KIND>()), 2) void screen_batch_kernel(const ScreenBatchArgs B)
 {
     constexpr int TB = KIND == 1 ? 32 : 64, NW = screen_batch_threads<TA, KIND>() / 64;
-    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * SW_ROW];
+    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * sw_row<2>()];
     __shared__ float4 mg[TA + TB];
     __shared__ float2 mg2[TA];
     const int it = xcd_tile(blockIdx.x, B.nitems);
@@ -143,14 +143,21 @@ __global__ __launch_bounds__((screen_batch_threads<TA, KIND>()), 2) void screen_
     const MfmaScan S = B.mscan[sc];
     const ScreenCut C = B.cut[sc];
     const uint32_t region0 = (uint32_t)(B.item0 + it) * NW;
-    if (!C.ok) {
+    if (!C.nd) {
         if (threadIdx.x == 0) B.cs.redo[atomicAdd(B.cs.count + 1, 1u)] = SCR_WHOLE | region0;
         return;
     }
-    if constexpr (KIND == 0)
-        screen_fast_tile<TA>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg, mg2);
-    else
-        screen_gen_tile<TA, TB>(S, C, B.cs, a0, a1, b0, b1, region0, wl, reinterpret_cast<float *>(mg));
+    if constexpr (KIND == 0) {
+        if (C.nd == 1)
+            screen_fast_tile<TA, 1>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg, mg2);
+        else
+            screen_fast_tile<TA, 2>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg, mg2);
+    } else {
+        if (C.nd == 1)
+            screen_gen_tile<TA, TB, 1>(S, C, B.cs, a0, a1, b0, b1, region0, wl, reinterpret_cast<float *>(mg));
+        else
+            screen_gen_tile<TA, TB, 2>(S, C, B.cs, a0, a1, b0, b1, region0, wl, reinterpret_cast<float *>(mg));
+    }
 }
 
 // PA: FAST tiles are 16 PA x 64 (PA = 2 or 1); GENERAL tiles are 16 x 64.

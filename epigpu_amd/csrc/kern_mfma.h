@@ -79,8 +79,8 @@ struct MissPhen {                // per individual, for the SPARSE tiles' missin
     float zf;                    // z as FP32
     int32_t q;                   // fixed-point phenotype (0 where missing and for outliers)
     int32_t z;                   // round(q^2 / 2^zbits)
-    int32_t sv;                  // coarse phenotype of the screen (0 where missing)
-    int32_t pad[2];
+    int32_t sv[2];               // coarse phenotype of the screen, one and two digits (0 where missing)
+    int32_t pad;
 };
 
 struct OutVals {                 // values of the outlier individuals, in fixed-point units
@@ -116,7 +116,8 @@ struct MfmaScan {                // one dataset x one phenotype
     const MissPhen *mp;          // [Kp] for this phenotype
     long long tstride;           // uint64 words per 64-SNP column of tbits (4 nid)
     // screen:
-    const uint32_t *sw;          // [Kp / 32][SW_ROW] codes of the coarse phenotype
+    const uint32_t *rbits;       // [3][Kw][nsnp] bitplanes: the two rarest classes of the SNP, call present
+    const uint32_t *sw[2];       // [Kp / 32][sw_row] codes of the coarse phenotype, one and two digits
     const ScrMarg *sm;           // [nsnp]
 };
 

@@ -8,17 +8,22 @@
 // decides them in FP64 with the same code as the exact tiles. The hits and
 // their values are those of the exact tiles.
 //
-// Coarse phenotype: v = 32 D1 + D0 with both digits representable in FP6 (E2M3:
+// Coarse phenotype: v = D0, or v = 32 D1 + D0, with digits representable in FP6 (E2M3:
 // in units of 1/8 the integers 0..16, then steps of 2 to 30 and of 4 to 60),
-// |v| <= 1980, v ~ q / delta with delta = max|q| / 1980 (or larger), r = q - delta v. The
-// rate of 6-bit MFMA operands is twice that of 8-bit ones, and one weight
-// count + two digits replace the count + three limbs: 12 instead of 16 INT8
-// equivalents of MACs, at twice the rate.
+// |v| <= 60 or 1980; q ~ delta v + offset by least squares, and r is the rest. The
+// rate of 6-bit MFMA operands is twice that of 8-bit ones, and a
+// count and one or two digits replace the count and three limbs: 8 or 12 instead of 16 MACs
+// per pair and individual without missing calls, at twice the rate.
 //
-// What bounds it: the matrix cores. At N = 8000, M = 50000 without missing calls a scan's kernels take
-// 37.4 ms (exact 64 x 64 tiles: 92-97 ms): 2.4e14 operations at 6.4 POP/s, against the 7.3-7.5 POP/s that
-// a register-only loop of this MFMA with five VALU instructions beside each sustains (8.7 without any,
-// 4.8 for v_mfma_i32_32x32x32_i8).
+// The class masks are those of an SNP's two rarest classes (rbits), and of the commonest where it is needed: the
+// statistics do not depend on the classes' names, and the sparser the masks, the less power the
+// MFMAs draw. A register-only loop runs 8.8 POP/s at 33 % ones, 9.1 at 22 %, 9.9 at 10 % (the clock falls to
+// about 1.8 GHz in the scans).
+//
+// What bounds it: the matrix cores and their power. At N = 8000, M = 50000 without missing calls a scan's
+// kernels take 35 ms (exact 64 x 64 tiles: 92-97 ms): 2.4e14 operations at 6.9 POP/s, against the 8.0 POP/s that
+// a register-only loop of this MFMA with five VALU instructions beside each sustains (9.1 without any,
+// 4.8 for v_mfma_i32_32x32x32_i8); the matrix cores are busy 84 % of the cycles, at 1.8 GHz.
 //
 // Bound: over a pair's complete cases let P y be the projection of a phenotype
 // onto the cell-constant vectors less the mean, so SSB(y) = |P y|^2. Then
@@ -41,24 +46,25 @@ namespace epi {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-constexpr int SW_ROW = 16;   // dwords per 32 individuals: D0 codes (6), D1 codes (6), phenotype present, pad
+// Dwords per 32 individuals of the weights of ND digits: codes of D0 (6), of D1 (6), phenotype present, pad.
+template <int ND>
+constexpr int sw_row() { return 8 * ND; }
 constexpr int SCR_WIN = 512; // words (of 32 individuals) of weights in LDS at a time
 constexpr int SCR_LDS_ROWS = SCR_WIN + 2;  // the pipeline reads one step past the window
 constexpr int SCR_GEN_ROWS = SCR_WIN + 4;
 constexpr int SCR_A = 16;    // a-SNPs per wave
 constexpr int SCR_REDO = 8;   // candidates per pair slot of a wave (64 pairs) above which the exact tile redoes its region
 
-// Per SNP and phenotype: counts and sums of v of classes 0, 1 and 2 (present phenotypes),
-// divided by 64 as the kernels'
-// accumulators are, and the sum of z over all calls.
+// Per SNP and phenotype: counts and sums of v (one and two digits) of the two rarest classes and
+// the commonest one (present phenotypes), divided by 64 as the kernels' accumulators are, and the sum of z over all calls.
 struct ScrMarg {
-    float n0, n1, s0, s1;
-    float n2, s2, zs, pad;
+    float n[3], zs;
+    float s[2][4];
 };
 
 // The cut of one scan (thresholds and phenotype), in units of v / 8 (sums of squares / 64).
 struct ScreenCut {
-    float N, T, T2N;      // complete cases / 64, sum of v / 64, T^2 / N
+    float N;              // complete cases / 64
     float thr0, slope2;   // level 0: sum s^2 / n > thr0 + 2 nfac slope2
     float eps;            // |r - mean(r)| / (8 delta)
     float sst;            // SST(q) / (64 delta^2)
@@ -66,10 +72,10 @@ struct ScreenCut {
     // GENERAL tiles: nv and N bound the pairs' complete cases from above
     float zunit, zall;    // sums of squares per unit of z (from below); sum of z over all individuals
     float kap0, kslope2;  // level 0: sum s^2 / n > (kap0 + 2 nfac kslope2) SST - kroot
-    float kroot;
+    float kroot, c0;      // c0: q ~ delta (v + c0), scaled as v is
     float t1s, t2s;       // lowered thresholds
     int test, safe;
-    int ok;               // 0: the scan is not screened
+    int nd;               // digits of v; 0: the scan is not screened
 };
 
 struct CandSink {
@@ -202,10 +208,10 @@ __device__ __forceinline__ bool screen_bound(const float n[9], const float s[9],
 }
 
 // n rows of weights from global memory into LDS, four loads in flight per thread.
-template <int NT>
+template <int NT, int ROW>
 __device__ __forceinline__ void scr_stage(uint32_t *wl, const uint32_t *src, int n, int tid)
 {
-    const int last = n * (SW_ROW / 4) - 1;  // threads past the end move the last piece
+    const int last = n * (ROW / 4) - 1;  // threads past the end move the last piece
     const uint4 *g = reinterpret_cast<const uint4 *>(src);
     uint4 *l = reinterpret_cast<uint4 *>(wl);
     for (int i = tid; i <= last; i += 4 * NT) {
@@ -265,12 +271,13 @@ __device__ __forceinline__ void scr_append(const CandSink &cs, uint32_t bits, ui
 template <int TA>
 constexpr int screen_threads() { return 64 * TA / SCR_A; }
 
-template <int TA>
+template <int TA, int ND>
 __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const ScreenCut &C, const CandSink &cs, int a0,
                                                  int a1, int b0, int b1, uint32_t region0, uint32_t *wl,
                                                  float4 *mg, float2 *mg2)
 {
-    constexpr int NT = screen_threads<TA>();
+    constexpr int NT = screen_threads<TA>(), ROW = sw_row<ND>();
+    const uint32_t *sw = S.sw[ND - 1];
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int aw = a0 + SCR_A * wid;                      // the wave's first a-SNP
@@ -280,8 +287,9 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const Screen
     for (int i = tid; i < TA + 64; i += NT) {
         int sn = i < TA ? a0 + i : b0 + i - TA;
         sn = sn < S.nsnp ? sn : S.nsnp - 1;
-        mg[i] = *reinterpret_cast<const float4 *>(S.sm + sn);
-        if (i < TA) mg2[i] = *reinterpret_cast<const float2 *>(&S.sm[sn].n2);
+        const ScrMarg &q = S.sm[sn];
+        mg[i] = make_float4(q.n[0], q.n[1], q.s[ND - 1][0], q.s[ND - 1][1]);
+        if (i < TA) mg2[i] = make_float2(q.n[2], q.s[ND - 1][2]);
     }
 
     v16f av[4], al[4];  // [2 bg + h]: counts, sums of v
@@ -294,7 +302,7 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const Screen
     const uint32_t row = (uint32_t)S.nsnp * 4u, plane = (uint32_t)Kw * row;  // bytes
     const uint64_t rest = 3ull * plane;
     auto rsrc = [&](uint32_t o) {
-        return __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(S.bits) + o), 0,
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(S.rbits) + o), 0,
                                                  (int)(rest - o < 0xFFFFFFFFull ? rest - o : 0xFFFFFFFFull), 0x00027000);
     };
     const __amdgpu_buffer_rsrc_t r0 = rsrc(0u), r1 = rsrc(plane);
@@ -327,14 +335,16 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const Screen
         src += 2 * row;
     };
     auto prep = [&](int set, const uint32_t *wr, Ops &o) {
-        const uint4 q0 = *reinterpret_cast<const uint4 *>(wr), q1 = *reinterpret_cast<const uint4 *>(wr + 4),
-                    q2 = *reinterpret_cast<const uint4 *>(wr + 8);
-        const Fp6 t = scr_spread(xa[set] & wr[12]), f = scr_fill(t);
+        const uint4 q0 = *reinterpret_cast<const uint4 *>(wr), q1 = *reinterpret_cast<const uint4 *>(wr + 4);
+        const Fp6 t = scr_spread(xa[set] & (ND == 1 ? q1.z : wr[12])), f = scr_fill(t);
         const Fp6 f0 = {{f.d[0] & q0.x, f.d[1] & q0.y, f.d[2] & q0.z, f.d[3] & q0.w, f.d[4] & q1.x, f.d[5] & q1.y}};
-        const Fp6 f1 = {{f.d[0] & q1.z, f.d[1] & q1.w, f.d[2] & q2.x, f.d[3] & q2.y, f.d[4] & q2.z, f.d[5] & q2.w}};
         o.A = scr_op(t);
         o.A0 = scr_op(f0);
-        o.A1 = scr_op(f1);
+        if constexpr (ND == 2) {
+            const uint4 q2 = *reinterpret_cast<const uint4 *>(wr + 8);
+            const Fp6 f1 = {{f.d[0] & q1.z, f.d[1] & q1.w, f.d[2] & q2.x, f.d[3] & q2.y, f.d[4] & q2.z, f.d[5] & q2.w}};
+            o.A1 = scr_op(f1);
+        }
         o.B0 = scr_op(scr_spread(xb[set][0]));
     };
     auto step = [&](int set, const Ops &o) {
@@ -343,16 +353,16 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const Screen
             const v8i B = j == 0 ? o.B0 : scr_op(scr_spread(xb[set][j]));
             al[j] = scr_mfma(o.A0, B, al[j]);
             av[j] = scr_mfma(o.A, B, av[j]);
-            al[j] = scr_mfma32(o.A1, B, al[j]);
+            if constexpr (ND == 2) al[j] = scr_mfma32(o.A1, B, al[j]);
         }
     };
     // Masks: 0x008 MFMA, 0x002 VALU, 0x100 LDS read, 0x020 global load.
     auto fence = [&]() {
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * ND, 0);
 #pragma unroll
-        for (int u = 0; u < 12; u++) {
+        for (int u = 0; u < 4 + 4 * ND; u++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, ND == 1 ? 8 : 6, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -364,20 +374,20 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const Screen
     for (int w0 = 0; w0 < nw; w0 += SCR_WIN) {
         const int wn = nw - w0 < SCR_WIN ? nw - w0 : SCR_WIN;
         if (w0) __syncthreads();
-        scr_stage<NT>(wl, S.sw + (size_t)w0 * SW_ROW, wn, tid);
+        scr_stage<NT, ROW>(wl, sw + (size_t)w0 * ROW, wn, tid);
         __syncthreads();
         if (!work) continue;
-        const uint32_t *wr = wl + hf * SW_ROW;
+        const uint32_t *wr = wl + hf * ROW;
         prep(0, wr, o0);
         __builtin_amdgcn_sched_barrier(0);
-        for (int t = 0; t < wn; t += 4, wr += 4 * SW_ROW) {
+        for (int t = 0; t < wn; t += 4, wr += 4 * ROW) {
             step(0, o0);
-            prep(1, wr + 2 * SW_ROW, o1);
+            prep(1, wr + 2 * ROW, o1);
             load(0);
             fence();
             step(1, o1);
             // past the window's last step: a row of the next window's place, not used
-            prep(0, wr + 4 * SW_ROW, o0);
+            prep(0, wr + 4 * ROW, o0);
             load(1);
             fence();
         }
@@ -425,21 +435,21 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const Screen
     });
 }
 
-template <int TA>
+template <int TA, int ND>
 __global__ __launch_bounds__(screen_threads<TA>(), 2) void screen_fast_kernel(const ScreenArgs A)
 {
-    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_LDS_ROWS * SW_ROW];
+    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_LDS_ROWS * sw_row<ND>()];
     __shared__ float4 mg[TA + 64];
     __shared__ float2 mg2[TA];
     const int t = xcd_tile(blockIdx.x, A.ntiles);
     const int4 T = A.tiles[t];
-    screen_fast_tile<TA>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, (uint32_t)(A.tile0 + t) * (TA / SCR_A), wl, mg,
+    screen_fast_tile<TA, ND>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, (uint32_t)(A.tile0 + t) * (TA / SCR_A), wl, mg,
                          mg2);
 }
 
 // ------------------------------------------------------------- GENERAL ----
 // Tile TA a x TB b with missing calls (TB = 32, or 64 for tiles whose SNPs miss few calls). Each
-// wave owns 16 a x 32 b and contracts the classes 0, 1, NM of both sides with the count and the two
+// wave owns 16 a x 32 b and contracts the three classes of both sides with the count and the two
 // digits: 27 v_mfma_f32_16x16x128_f8f6f4 per 16 x 16 pairs and 128 individuals (the exact tile: 40 INT8
 // MACs per pair and individual, here 27 at twice the rate). The 16 x 16 shape puts a pair's 18 accumulators
 // into one lane whatever the number of rows per a-SNP: row m of A is a-SNP m, one
@@ -460,11 +470,12 @@ __device__ __forceinline__ v4f scr_mfma16x32(const v8i &a, const v8i &b, const v
 template <int TA, int TB>
 constexpr int screen_gen_threads() { return 64 * (TA / SCR_A) * (TB / 32); }
 
-template <int TA, int TB>
+template <int TA, int TB, int ND>
 __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenCut &C, const CandSink &cs, int a0, int a1,
                                                 int b0, int b1, uint32_t region0, uint32_t *wl, float *mz)
 {
-    constexpr int NT = screen_gen_threads<TA, TB>(), NWA = TA / SCR_A;
+    constexpr int NT = screen_gen_threads<TA, TB>(), NWA = TA / SCR_A, ROW = sw_row<ND>();
+    const uint32_t *sw = S.sw[ND - 1];
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, kq = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int al = SCR_A * (wid % NWA), bl = 32 * (wid / NWA);
@@ -487,7 +498,7 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
     // bitplanes through one buffer descriptor per class (scalar base and row offset, 32-bit lane offset)
     const uint32_t row = (uint32_t)S.nsnp * 4u, plane = (uint32_t)Kw * row;  // bytes
     auto rsrc = [&](int g) {
-        return __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(S.bits) + (size_t)g * plane), 0,
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(reinterpret_cast<const char *>(S.rbits) + (size_t)g * plane), 0,
                                                  (int)plane, 0x00027000);
     };
     const __amdgpu_buffer_rsrc_t r[3] = {rsrc(0), rsrc(1), rsrc(2)};
@@ -519,6 +530,8 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
         for (int j = 0; j < 6; j++) xb[j] = __builtin_amdgcn_raw_buffer_load_b32(r[j >> 1], vb[j & 1], src, 0);
     };
     auto loadA = [&](int g) { xa[g] = __builtin_amdgcn_raw_buffer_load_b32(r[g], va, src, 0); };
+    // the word of B operand j = 2 h + b group; class 2 is the rest of the called individuals
+    auto word = [&](int j) { return j < 4 ? xb[j] : xb[j] & ~xb[j - 4] & ~xb[j - 2]; };
     auto low = [&](const Fp6 &f, const Weights &w) {
         return scr_op({{f.d[0] & w.q0.x, f.d[1] & w.q0.y, f.d[2] & w.q0.z, f.d[3] & w.q0.w, f.d[4] & w.q1.x,
                         f.d[5] & w.q1.y}});
@@ -534,18 +547,18 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
     for (int w0 = 0; w0 < nw; w0 += SCR_WIN) {
         const int wn = nw - w0 < SCR_WIN ? nw - w0 : SCR_WIN;
         if (w0) __syncthreads();
-        scr_stage<NT>(wl, S.sw + (size_t)w0 * SW_ROW, wn, tid);
+        scr_stage<NT, ROW>(wl, sw + (size_t)w0 * ROW, wn, tid);
         __syncthreads();
         if (!work) continue;
-        const uint32_t *wr = wl + kq * SW_ROW;
+        const uint32_t *wr = wl + kq * ROW;
         Weights w;
         auto weights = [&](int part) {
             if (part == 0) {
-                w.v = wr[12];
+                w.v = wr[6 * ND];
                 w.q0 = *reinterpret_cast<const uint4 *>(wr);
                 w.q1.x = wr[4];
                 w.q1.y = wr[5];
-            } else {
+            } else if (ND == 2) {
                 w.q1.z = wr[6];
                 w.q1.w = wr[7];
                 w.q2 = *reinterpret_cast<const uint4 *>(wr + 8);
@@ -556,7 +569,7 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
         Fp6 t = scr_spread(xa[0] & w.v), f = scr_fill(t);
         v8i A0 = low(f, w);
 #pragma unroll
-        for (int j = 0; j < 6; j++) B[j] = scr_op(scr_spread(xb[j]));
+        for (int j = 0; j < 6; j++) B[j] = scr_op(scr_spread(word(j)));
         loadA(1);
         loadA(2);
         __builtin_amdgcn_sched_barrier(0);
@@ -571,44 +584,55 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
         };
         using std::integral_constant;
         for (int wi = 0; wi < wn; wi += 4) {
+            uint32_t a01 = 0;
             static_for<3>([&](auto gg) {
                 constexpr int g = decltype(gg)::value, gn = (g + 1) % 3;
                 if (g == 0) {  // request the next step's words
+                    a01 = xa[0] | xa[1];
                     src = src + 4 * row < last ? src + 4 * row : last;
                     loadA(0);
                     loadB();
                 }
                 if (g == 2) {
-                    wr += 4 * SW_ROW;  // past the window's last step: not used
+                    wr += 4 * ROW;  // past the window's last step: not used
                     weights(0);
                 }
 #pragma unroll
                 for (int j = 0; j < 6; j++) as[j & 1][3 * g + (j >> 1)] = scr_mfma16(A0, B[j], as[j & 1][3 * g + (j >> 1)]);
-                const Fp6 tn = scr_spread(xa[gn] & w.v);
+                const Fp6 tn = scr_spread(gn == 2 ? xa[2] & ~a01 & w.v : xa[gn] & w.v);
                 if (g == 2) {
                     loadA(1);
                     loadA(2);
                 }
                 fence(integral_constant<int, 2>{});
-#pragma unroll
-                for (int j = 0; j < 6; j++)
-                    av[j & 1][3 * g + (j >> 1)] = scr_mfma16(scr_op(t), B[j], av[j & 1][3 * g + (j >> 1)]);
-                const v8i A1 = high(f, w);
-                if (g == 2) weights(1);
-                const Fp6 fn = scr_fill(tn);
-                fence(integral_constant<int, 3>{});
-                A0 = low(fn, w);
+                if constexpr (ND == 1) A0 = low(scr_fill(tn), w);
 #pragma unroll
                 for (int j = 0; j < 6; j++) {
-                    as[j & 1][3 * g + (j >> 1)] = scr_mfma16x32(A1, B[j], as[j & 1][3 * g + (j >> 1)]);
-                    if (g == 2) {
-                        B[j] = scr_op(scr_spread(xb[j]));
+                    av[j & 1][3 * g + (j >> 1)] = scr_mfma16(scr_op(t), B[j], av[j & 1][3 * g + (j >> 1)]);
+                    if (ND == 1 && g == 2) {
+                        B[j] = scr_op(scr_spread(word(j)));
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
+                if (ND == 1 && g < 2) fence(integral_constant<int, 3>{});
+                if constexpr (ND == 2) {
+                    const v8i A1 = high(f, w);
+                    if (g == 2) weights(1);
+                    const Fp6 fn = scr_fill(tn);
+                    fence(integral_constant<int, 3>{});
+                    A0 = low(fn, w);
+#pragma unroll
+                    for (int j = 0; j < 6; j++) {
+                        as[j & 1][3 * g + (j >> 1)] = scr_mfma16x32(A1, B[j], as[j & 1][3 * g + (j >> 1)]);
+                        if (g == 2) {
+                            B[j] = scr_op(scr_spread(word(j)));
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+                    f = fn;
+                    if (g < 2) fence(integral_constant<int, 1>{});
+                }
                 t = tn;
-                f = fn;
-                if (g < 2) fence(integral_constant<int, 1>{});
             });
         }
     }
@@ -618,22 +642,15 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
     uint32_t bits = 0;
     static_for<8>([&](auto k) {
         constexpr int K = decltype(k)::value, i = K / 2, bg = K % 2;
-        float n[9], s[9];
-        auto cells = [&](const v4f (&x)[9], float c[9]) {
-            const float xx[3][3] = {{x[0][i], x[1][i], x[2][i]}, {x[3][i], x[4][i], x[5][i]}, {x[6][i], x[7][i], x[8][i]}};
-            c[0] = xx[0][0];
-            c[1] = xx[0][1];
-            c[3] = xx[1][0];
-            c[4] = xx[1][1];
-            c[2] = xx[0][2] - c[0] - c[1];
-            c[5] = xx[1][2] - c[3] - c[4];
-            c[6] = xx[2][0] - c[0] - c[3];
-            c[7] = xx[2][1] - c[1] - c[4];
-            c[8] = (xx[2][2] - xx[0][2] - xx[1][2]) - c[6] - c[7];
-        };
-        cells(av[bg], n);
-        cells(as[bg], s);
-        const float nc = av[bg][8][i], tc = as[bg][8][i];
+        float n[9], s[9], nc = 0.0f, tc = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 9; c++) {
+            n[c] = av[bg][c][i];
+            s[c] = as[bg][c][i];
+            nc += n[c];
+            tc += s[c];
+        }
+        tc = __builtin_fmaf(C.c0, nc, tc);
         const float zlow = mz[al + 4 * kq + i] + mz[TA + bl + 16 * bg + m] - C.zall;
         float u = 0.0f;
 #pragma unroll
@@ -657,14 +674,14 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
     });
 }
 
-template <int TA, int TB>
+template <int TA, int TB, int ND>
 __global__ __launch_bounds__((screen_gen_threads<TA, TB>()), 2) void screen_gen_kernel(const ScreenArgs A)
 {
-    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * SW_ROW];
+    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * sw_row<ND>()];
     __shared__ float mz[TA + TB];
     const int t = xcd_tile(blockIdx.x, A.ntiles);
     const int4 T = A.tiles[t];
-    screen_gen_tile<TA, TB>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w,
+    screen_gen_tile<TA, TB, ND>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w,
                             (uint32_t)(A.tile0 + t) * (screen_gen_threads<TA, TB>() / 64), wl, mz);
 }
 

@@ -77,12 +77,12 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
     __shared__ double sy[4][3][64];
     __shared__ int sn[4][3][64];
     __shared__ long long sz[4][64];
-    __shared__ int sv[4][3][64];
+    __shared__ int sv[4][2][3][64];
     const int sl = threadIdx.x & 63, grp = threadIdx.x >> 6;
     const int s = blockIdx.x * 64 + sl;
     int n[3] = {0, 0, 0};
     long long q[3] = {0, 0, 0}, z = 0;
-    int v3[3] = {0, 0, 0};  // sums of the screen's coarse phenotype (their magnitude stays below 2^24)
+    int v3[2][3] = {};  // sums of the screen's coarse phenotype (their magnitude stays below 2^24)
     double y[3] = {0.0, 0.0, 0.0};
     if (s < nsnp) {
         for (int wd = grp; wd < Kw; wd += 4) {
@@ -101,7 +101,8 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
                     q[c] += qv[k];
                     y[c] += (double)yc[k];
                     z += mp[k].z;
-                    v3[c] += mp[k].sv;
+                    v3[0][c] += mp[k].sv[0];
+                    v3[1][c] += mp[k].sv[1];
                 }
             }
         }
@@ -112,9 +113,10 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
         sy[grp][c][sl] = y[c];
     }
     sz[grp][sl] = z;
-    sv[grp][0][sl] = v3[0];
-    sv[grp][1][sl] = v3[1];
-    sv[grp][2][sl] = v3[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) sv[grp][i][c][sl] = v3[i][c];
     __syncthreads();
     if (grp == 0 && s < nsnp) {
         int tn[3];
@@ -145,12 +147,17 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
         mg.pad = 0;
         mg.zs = sz[0][sl] + sz[1][sl] + sz[2][sl] + sz[3][sl];
         marg[s] = mg;
-        const int t0 = sv[0][0][sl] + sv[1][0][sl] + sv[2][0][sl] + sv[3][0][sl];
-        const int t1 = sv[0][1][sl] + sv[1][1][sl] + sv[2][1][sl] + sv[3][1][sl];
-        const int t2 = sv[0][2][sl] + sv[1][2][sl] + sv[2][2][sl] + sv[3][2][sl];
         const float u = 1.0f / 64.0f;
-        smarg[s] = {(float)tn[0] * u, (float)tn[1] * u, (float)t0 * u, (float)t1 * u, (float)tn[2] * u, (float)t2 * u,
-                    (float)mg.zs, 0.0f};
+        ScrMarg sm;
+        for (int p = 0; p < 3; p++) {
+            const int c = (cl >> (2 * p)) & 3;
+            sm.n[p] = (float)tn[c] * u;
+            for (int i = 0; i < 2; i++)
+                sm.s[i][p] = (float)(sv[0][i][c][sl] + sv[1][i][c][sl] + sv[2][i][c][sl] + sv[3][i][c][sl]) * u;
+        }
+        sm.zs = (float)mg.zs;
+        sm.s[0][3] = sm.s[1][3] = 0.0f;
+        smarg[s] = sm;
     }
 }
 
