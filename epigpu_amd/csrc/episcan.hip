@@ -5,9 +5,8 @@
 //   mbits   [3][Kw][nsnp]  uint32  bitplanes of classes 0, 1 and call present (MFMA form)
 //   bits    [3][Kw][nsnp]  uint32  bitplanes of the two rarest classes and call present (plain form)
 //   cls     [nsnp]         int32   plain-form plane -> class map
-//   per phenotype r:
+//   per phenotype r (wts, mp, yc, vbits, ov and oidx in one allocation):
 //     wts   [8][Kp] int8   V, 3 limbs of q, 4 limbs of round(q^2/2^zbits)
-//     qv    [Kp]    int32  fixed-point phenotype q (0 where missing and for outliers)
 //     yc    [Kp]    float  centred phenotype scaled by 2^-ybits to |yc| < 1 (0 where missing)
 //     vbits [Kw]    uint32 phenotype-present bits
 //     marg  [nsnp]  Marg   per-SNP class counts and sums
@@ -71,7 +70,6 @@ struct ScreenEnc {
 
 struct PhenDev {
     int8_t *wts = nullptr;
-    int32_t *qv = nullptr;
     float *yc = nullptr;
     uint32_t *vbits = nullptr;
     Marg *marg = nullptr;
@@ -100,7 +98,7 @@ struct PhenDev {
 };
 
 struct Dataset {
-    int nid = 0, nsnp = 0, npack = 0, remain = 0, npack1 = 0, Kp = 0, Kw = 0;
+    int nid = 0, nsnp = 0, npack1 = 0, Kp = 0, Kw = 0;
     int32_t *words = nullptr;
     uint32_t *mbits = nullptr;
     uint32_t *bits = nullptr;
@@ -250,16 +248,16 @@ int dalloc(epi_ctx *c, T *&p, size_t count)
 
 void free_phen(PhenDev &p)
 {
-    dfree(p.wts);
-    dfree(p.qv);
-    dfree(p.yc);
-    dfree(p.vbits);
+    dfree(p.wts);  // with the arrays behind it
+    p.sw[0] = p.sw[1] = nullptr;
+    p.mp = nullptr;
+    p.yc = nullptr;
+    p.vbits = nullptr;
+    p.ov = nullptr;
+    p.oidx = nullptr;
     dfree(p.sm);
     p.marg = nullptr;
-    dfree(p.oidx);
     dfree(p.ocodes);
-    dfree(p.ov);
-    dfree(p.mp);
 }
 
 void drop_sparse(Dataset &d)
@@ -309,28 +307,23 @@ int ds_upload_genotypes(epi_ctx *c, Dataset &d, const int32_t *words, int nid, i
     drop_sparse(d);
     d.nid = nid;
     d.nsnp = nsnp;
-    d.npack = nid / 16;
-    d.remain = nid % 16;
-    d.npack1 = d.npack + (d.remain > 0);
+    d.npack1 = (nid + 15) / 16;
     d.Kp = (nid + KPAD - 1) / KPAD * KPAD;
     d.Kw = d.Kp / 32;
     size_t nwords = (size_t)nsnp * d.npack1;
     int rc;
     if ((rc = dalloc(c, d.words, nwords)) || (rc = dalloc(c, d.mbits, (size_t)3 * d.Kw * nsnp)) ||
-        (rc = dalloc(c, d.bits, (size_t)3 * d.Kw * nsnp)) || (rc = dalloc(c, d.dmiss, (size_t)nsnp)) ||
+        (rc = dalloc(c, d.bits, (size_t)3 * d.Kw * nsnp)) || (rc = dalloc(c, d.dmiss, (size_t)4 * nsnp)) ||
         (rc = dalloc(c, d.cls, (size_t)nsnp)))
         return rc;
     HIPCHK(c, hipMemcpyAsync(d.words, words, nwords * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(class_order, dim3((nsnp + 255) / 256), dim3(256), 0, c->stream, (const uint32_t *)d.words, nid,
-                       d.npack, d.remain, d.npack1, nsnp, d.cls, d.dmiss);
+    int *cnt = d.dmiss + nsnp;  // class counts of the SNPs
+    HIPCHK(c, hipMemsetAsync(cnt, 0, 3 * (size_t)nsnp * sizeof(int), c->stream));
+    hipLaunchKernelGGL(transcode_kernel, dim3((nsnp + TR_SNP - 1) / TR_SNP, (d.Kw + TR_WD - 1) / TR_WD), dim3(256), 0,
+                       c->stream, (const uint32_t *)d.words, nid, d.npack1, nsnp, d.Kw, d.mbits, cnt);
     HIPCHK(c, hipGetLastError());
-    hipLaunchKernelGGL(transcode_bits, dim3((nsnp + 255) / 256, d.Kw), dim3(256), 0, c->stream,
-                       (const uint32_t *)d.words, nid, d.npack, d.remain, d.npack1, nsnp, d.Kw, (const int32_t *)d.cls,
-                       d.bits);
-    HIPCHK(c, hipGetLastError());
-    hipLaunchKernelGGL(transcode_bits, dim3((nsnp + 255) / 256, d.Kw), dim3(256), 0, c->stream,
-                       (const uint32_t *)d.words, nid, d.npack, d.remain, d.npack1, nsnp, d.Kw, (const int32_t *)nullptr,
-                       d.mbits);
+    hipLaunchKernelGGL(order_planes_kernel, dim3((nsnp + 255) / 256, (d.Kw + 3) / 4), dim3(256), 0, c->stream,
+                       (const uint32_t *)d.mbits, (const int *)cnt, nid, nsnp, d.Kw, d.bits, d.cls, d.dmiss);
     HIPCHK(c, hipGetLastError());
     d.miss.assign(nsnp, 0);
     HIPCHK(c, hipMemcpyAsync(d.miss.data(), d.dmiss, (size_t)nsnp * sizeof(int32_t), hipMemcpyDeviceToHost,
@@ -694,23 +687,25 @@ int ds_set_phenotypes(epi_ctx *c, Dataset &d, const float *phen, int nphen, int 
         PhenEnc &e = enc[r];
         PhenDev &p = ph[r];
         p = e.p;
-        if ((rc = dalloc(c, p.wts, e.w.size())) || (rc = dalloc(c, p.qv, (size_t)Kp)) ||
-            (rc = dalloc(c, p.yc, (size_t)Kp)) || (rc = dalloc(c, p.vbits, (size_t)Kw)) ||
-            (rc = dalloc(c, p.ov, 1)) || (rc = dalloc(c, p.mp, (size_t)Kp)))
-            break;
+        // one allocation and one copy: weights (with the screen's), mp, yc, vbits (Kp is a multiple of 256), ov, oidx
+        const size_t omp = e.w.size(), oyc = omp + (size_t)Kp * sizeof(MissPhen), ovb = oyc + (size_t)Kp * 4,
+                     oov = ovb + (size_t)Kw * 4, oix = oov + sizeof(OutVals);
+        std::vector<int8_t> blob(oix + sizeof(int32_t) * OUT_MAX, 0);
+        memcpy(blob.data(), e.w.data(), e.w.size());
+        memcpy(blob.data() + omp, e.mp.data(), (size_t)Kp * sizeof(MissPhen));
+        memcpy(blob.data() + oyc, e.yc.data(), (size_t)Kp * 4);
+        memcpy(blob.data() + ovb, e.vb.data(), (size_t)Kw * 4);
+        memcpy(blob.data() + oov, &e.ov, sizeof(OutVals));
+        if (p.nout) memcpy(blob.data() + oix, e.oidx.data(), (size_t)p.nout * 4);
+        if ((rc = dalloc(c, p.wts, blob.size()))) break;
         p.sw[0] = reinterpret_cast<uint32_t *>(p.wts + (size_t)NWP * Kp);
         p.sw[1] = p.sw[0] + Kp / 4;
-        if (p.nout && (rc = dalloc(c, p.oidx, (size_t)p.nout))) break;
-        hipError_t he = hipMemcpyAsync(p.wts, e.w.data(), e.w.size(), hipMemcpyHostToDevice, c->stream);
-        if (he == hipSuccess) he = hipMemcpyAsync(p.qv, e.qv.data(), (size_t)Kp * 4, hipMemcpyHostToDevice, c->stream);
-        if (he == hipSuccess) he = hipMemcpyAsync(p.yc, e.yc.data(), (size_t)Kp * 4, hipMemcpyHostToDevice, c->stream);
-        if (he == hipSuccess)
-            he = hipMemcpyAsync(p.vbits, e.vb.data(), (size_t)Kw * 4, hipMemcpyHostToDevice, c->stream);
-        if (he == hipSuccess) he = hipMemcpyAsync(p.ov, &e.ov, sizeof(OutVals), hipMemcpyHostToDevice, c->stream);
-        if (he == hipSuccess)
-            he = hipMemcpyAsync(p.mp, e.mp.data(), (size_t)Kp * sizeof(MissPhen), hipMemcpyHostToDevice, c->stream);
-        if (he == hipSuccess && p.nout)
-            he = hipMemcpyAsync(p.oidx, e.oidx.data(), (size_t)p.nout * 4, hipMemcpyHostToDevice, c->stream);
+        p.mp = reinterpret_cast<MissPhen *>(p.wts + omp);
+        p.yc = reinterpret_cast<float *>(p.wts + oyc);
+        p.vbits = reinterpret_cast<uint32_t *>(p.wts + ovb);
+        p.ov = reinterpret_cast<OutVals *>(p.wts + oov);
+        p.oidx = reinterpret_cast<int32_t *>(p.wts + oix);
+        hipError_t he = hipMemcpyAsync(p.wts, blob.data(), blob.size(), hipMemcpyHostToDevice, c->stream);
         if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
         if (he != hipSuccess) rc = fail(c, EPI_ERR_HIP, "phenotype upload failed: %s", hipGetErrorString(he));
     }
@@ -763,8 +758,8 @@ int ds_marginals(epi_ctx *c, Dataset &d)
         if (rc) return rc;
         p.marg = reinterpret_cast<Marg *>(p.sm + d.nsnp);
         hipLaunchKernelGGL(marginals_kernel, dim3((d.nsnp + 63) / 64), dim3(256), 0, c->stream,
-                           (const uint32_t *)d.mbits, d.Kw, d.nsnp, (const uint32_t *)p.vbits, (const int32_t *)p.qv,
-                           (const float *)p.yc, (const int32_t *)d.cls, (const MissPhen *)p.mp, p.marg, p.sm);
+                           (const uint32_t *)d.mbits, d.Kw, d.nsnp, (const uint32_t *)p.vbits, (const float *)p.yc,
+                           (const int32_t *)d.cls, (const MissPhen *)p.mp, p.marg, p.sm);
         HIPCHK(c, hipGetLastError());
         if (p.nout) {
             if ((rc = dalloc(c, p.ocodes, (size_t)(p.nout + 15) / 16 * d.nsnp))) return rc;

@@ -11,66 +11,114 @@
 
 namespace epi {
 
-__device__ __forceinline__ int decode(const uint32_t *w, int npack, int remain, int nid, int k)
+// Every second bit of x, from bit 0, packed into the low 16 bits.
+__device__ __forceinline__ uint32_t even_bits(uint32_t x)
 {
-    if (k >= nid) return -1;
-    int j = k >> 4, t = k & 15;
-    int sh = j < npack ? 30 - 2 * t : 2 * (remain - 1 - t);
-    return (int)((w[j] >> sh) & 3u);
+    x &= 0x55555555u;
+    x = (x | (x >> 1)) & 0x33333333u;
+    x = (x | (x >> 2)) & 0x0F0F0F0Fu;
+    x = (x | (x >> 4)) & 0x00FF00FFu;
+    return (x | (x >> 8)) & 0xFFFFu;
 }
 
-// One thread per SNP: order the genotype classes by frequency and count the
-// missing calls. The plain form stores the two rarest classes as bitplanes 0
-// and 1 and derives the most common one; cls packs plane -> class (2 bits
-// each).
-__global__ void class_order(const uint32_t *words, int nid, int npack, int remain, int npack1, int nsnp,
-                            int32_t *cls, int32_t *miss)
+// Class bits of 16 genotypes, bit t = individual t of the packed word, of which the first `have` exist.
+__device__ __forceinline__ void class_bits(uint32_t v, int have, uint32_t &c0, uint32_t &c1, uint32_t &nm)
 {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsnp) return;
-    const uint32_t *w = words + (size_t)s * npack1;
-    int n[4] = {0, 0, 0, 0};
-    for (int k = 0; k < nid; k++) n[decode(w, npack, remain, nid, k)]++;
-    int big = 0;
-    if (n[1] > n[big]) big = 1;
-    if (n[2] > n[big]) big = 2;
-    int p0 = big == 0 ? 1 : 0;
-    int p1 = big == 2 ? 1 : 2;
-    cls[s] = p0 | (p1 << 2) | (big << 4);
-    miss[s] = n[3];
+    if (have < 16) v = have > 0 ? v << (32 - 2 * have) : 0u;  // the tail word is right-aligned
+    const uint32_t r = __brev(v);                              // individual t: high bit at 2t, low bit at 2t + 1
+    const uint32_t hi = r, lo = r >> 1, ok = (1u << have) - 1u;
+    c0 = even_bits(~(hi | lo)) & ok;
+    c1 = even_bits(lo & ~hi) & ok;
+    nm = even_bits(~(hi & lo)) & ok;
 }
 
-// One thread per (word of 32 individuals, snp): bitplanes [3][Kw][nsnp] of
-// the classes cls names for planes 0 and 1 (cls == nullptr: classes 0 and 1,
-// the MFMA form's planes) and of the call-present flag in plane 2.
-__global__ void transcode_bits(const uint32_t *words, int nid, int npack, int remain, int npack1, int nsnp,
-                               int Kw, const int32_t *cls, uint32_t *bits)
+constexpr int TR_SNP = 64, TR_WD = 16;  // SNPs and 32-individual words of a workgroup
+
+// Bitplanes [3][Kw][nsnp] of classes 0 and 1 and of the call-present flag, and the counts of the three per SNP
+// (added to cnt [3][nsnp]). A workgroup takes 64 SNPs x 16 words: the packed words come in along the individuals (128
+// bytes of one SNP per eight lanes), cross in LDS, and the bitplanes go out along the SNPs. Bounded by memory; as one
+// thread per SNP and word that decoded its 32 genotypes one by one from strided loads, the transcode and the class
+// counts took 1.08 ms at N = 2000, M = 20001; this and order_planes_kernel take 0.02 ms.
+__global__ __launch_bounds__(256) void transcode_kernel(const uint32_t *words, int nid, int npack1, int nsnp, int Kw,
+                                                        uint32_t *bits, int *cnt)
 {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    int wd = blockIdx.y;
-    if (s >= nsnp) return;
-    const uint32_t *w = words + (size_t)s * npack1;
-    const int c0 = cls ? cls[s] & 3 : 0, c1 = cls ? (cls[s] >> 2) & 3 : 1;
-    uint32_t b0 = 0, b1 = 0, bn = 0;
-    for (int t = 0; t < 32; t++) {
-        int c = decode(w, npack, remain, nid, 32 * wd + t);
-        b0 |= (uint32_t)(c == c0) << t;
-        b1 |= (uint32_t)(c == c1) << t;
-        bn |= (uint32_t)(c >= 0 && c != 3) << t;
+    __shared__ uint32_t t[TR_SNP][2 * TR_WD + 1];
+    __shared__ int c[3][TR_SNP];
+    const int s0 = blockIdx.x * TR_SNP, w0 = blockIdx.y * TR_WD, tid = threadIdx.x;
+    if (tid < TR_SNP) c[0][tid] = c[1][tid] = c[2][tid] = 0;
+    for (int i = tid; i < TR_SNP * 2 * TR_WD; i += 256) {
+        const int s = i / (2 * TR_WD), j = i % (2 * TR_WD), g = 2 * w0 + j;
+        t[s][j] = s0 + s < nsnp && g < npack1 ? words[(size_t)(s0 + s) * npack1 + g] : 0u;
     }
-    bits[((size_t)0 * Kw + wd) * nsnp + s] = b0;
-    bits[((size_t)1 * Kw + wd) * nsnp + s] = b1;
-    bits[((size_t)2 * Kw + wd) * nsnp + s] = bn;
+    __syncthreads();
+    const int sl = tid & 63, s = s0 + sl;
+    int n[3] = {0, 0, 0};
+    for (int k = tid >> 6; k < TR_WD; k += 4) {
+        const int wd = w0 + k;
+        if (s >= nsnp || wd >= Kw) break;
+        uint32_t b[3] = {0u, 0u, 0u};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            int have = nid - 32 * wd - 16 * h;
+            have = have < 0 ? 0 : have > 16 ? 16 : have;
+            uint32_t x0, x1, xn;
+            class_bits(t[sl][2 * k + h], have, x0, x1, xn);
+            b[0] |= x0 << (16 * h);
+            b[1] |= x1 << (16 * h);
+            b[2] |= xn << (16 * h);
+        }
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            bits[((size_t)p * Kw + wd) * nsnp + s] = b[p];
+            n[p] += __popc(b[p]);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+        if (n[p]) atomicAdd(&c[p][sl], n[p]);
+    __syncthreads();
+    if (tid < TR_SNP && s0 + tid < nsnp)
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+            if (c[p][tid]) atomicAdd(&cnt[(size_t)p * nsnp + s0 + tid], c[p][tid]);
+}
+
+// One thread per (four words, SNP): the bitplanes of the two rarest classes and the call-present flag from those of
+// classes 0 and 1, for the plain form and the screen; the first row of workgroups also writes cls, the plane -> class map (2 bits each:
+// the two rarest classes, then the commonest), and the missing calls.
+__global__ __launch_bounds__(256) void order_planes_kernel(const uint32_t *mbits, const int *cnt, int nid, int nsnp, int Kw,
+                                                           uint32_t *bits, int32_t *cls, int32_t *miss)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nsnp) return;
+    const int n0 = cnt[s], n1 = cnt[nsnp + s], nm = cnt[2 * (size_t)nsnp + s], n2 = nm - n0 - n1;
+    int big = 0, nb = n0;
+    if (n1 > nb) big = 1, nb = n1;
+    if (n2 > nb) big = 2;
+    const int p0 = big == 0 ? 1 : 0, p1 = big == 2 ? 1 : 2;
+    if (blockIdx.y == 0) {
+        cls[s] = p0 | (p1 << 2) | (big << 4);
+        miss[s] = nid - nm;
+    }
+    for (int wd = 4 * blockIdx.y; wd < Kw && wd < 4 * (int)blockIdx.y + 4; wd++) {
+        const size_t o = (size_t)wd * nsnp + s, plane = (size_t)Kw * nsnp;
+        const uint32_t b0 = mbits[o], b1 = mbits[plane + o], bn = mbits[2 * plane + o], b2 = bn & ~b0 & ~b1;
+        bits[o] = p0 == 0 ? b0 : b1;
+        bits[plane + o] = p1 == 1 ? b1 : b2;
+        bits[2 * plane + o] = bn;
+    }
 }
 
 // Per SNP, over individuals with a call and a present phenotype: counts and
 // phenotype sums of genotype classes 0, 1 and of all calls (NM), stored per
 // class for the MFMA form and per bitplane (cls order) for the plain form.
 // One workgroup per 64 SNPs: lane = SNP (coalesced bitplane loads), four
-// groups of threads split the words and are reduced in LDS.
+// waves split the words and are reduced in LDS. Bounded by its VALU work, 35
+// instructions per individual and 64 SNPs: 0.10 ms at N = 2000, M = 20001 (0.22 ms
+// as a loop over each lane's own set bits, with gathered loads).
 __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, int Kw, int nsnp,
-                                                        const uint32_t *vbits, const int32_t *qv,
-                                                        const float *yc, const int32_t *cls, const MissPhen *mp,
+                                                        const uint32_t *vbits, const float *yc,
+                                                        const int32_t *cls, const MissPhen *mp,
                                                         Marg *marg, ScrMarg *smarg)
 {
     __shared__ long long sq[4][3][64];
@@ -78,34 +126,38 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
     __shared__ int sn[4][3][64];
     __shared__ long long sz[4][64];
     __shared__ int sv[4][2][3][64];
-    const int sl = threadIdx.x & 63, grp = threadIdx.x >> 6;
-    const int s = blockIdx.x * 64 + sl;
+    const int sl = threadIdx.x & 63, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int s = blockIdx.x * 64 + sl, sc = s < nsnp ? s : nsnp - 1;
     int n[3] = {0, 0, 0};
     long long q[3] = {0, 0, 0}, z = 0;
-    int v3[2][3] = {};  // sums of the screen's coarse phenotype (their magnitude stays below 2^24)
+    int v3[2][3] = {};  // sums of the screen's coarse phenotypes (their magnitude stays below 2^24)
     double y[3] = {0.0, 0.0, 0.0};
-    if (s < nsnp) {
-        for (int wd = grp; wd < Kw; wd += 4) {
-            const uint32_t v = vbits[wd];
-            const uint32_t b0 = mbits[((size_t)0 * Kw + wd) * nsnp + s] & v;
-            const uint32_t b1 = mbits[((size_t)1 * Kw + wd) * nsnp + s] & v;
-            const uint32_t bn = mbits[((size_t)2 * Kw + wd) * nsnp + s] & v;
-            const uint32_t m[3] = {b0, b1, bn & ~b0 & ~b1};
+    for (int wd = grp; wd < Kw; wd += 4) {
+        const uint32_t v = vbits[wd];
+        const uint32_t b0 = mbits[((size_t)0 * Kw + wd) * nsnp + sc] & v;
+        const uint32_t b1 = mbits[((size_t)1 * Kw + wd) * nsnp + sc] & v;
+        const uint32_t bn = mbits[((size_t)2 * Kw + wd) * nsnp + sc] & v;
+        const uint32_t m[3] = {b0, b1, bn & ~b0 & ~b1};
+        int q32[3] = {0, 0, 0};  // 32 |q| < 2^28
+#pragma unroll
+        for (int c = 0; c < 3; c++) n[c] += __popc(m[c]);
+        // every individual of the word in turn: its values are the wave's (scalar loads), its bit is the lane's mask
+#pragma unroll 8
+        for (int j = 0; j < 32; j++) {
+            const MissPhen &e = mp[32 * wd + j];
+            const int eq = e.q, e0 = e.sv[0], e1 = e.sv[1], ey = __float_as_int(yc[32 * wd + j]);
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                uint32_t x = m[c];
-                n[c] += __popc(x);
-                while (x) {
-                    const int k = 32 * wd + __ffs(x) - 1;
-                    x &= x - 1;
-                    q[c] += qv[k];
-                    y[c] += (double)yc[k];
-                    z += mp[k].z;
-                    v3[0][c] += mp[k].sv[0];
-                    v3[1][c] += mp[k].sv[1];
-                }
+                const int k = (int)(m[c] << (31 - j)) >> 31;
+                q32[c] += k & eq;
+                v3[0][c] += k & e0;
+                v3[1][c] += k & e1;
+                y[c] += (double)__int_as_float(k & ey);
             }
+            z += (int)(bn << (31 - j)) >> 31 & e.z;
         }
+#pragma unroll
+        for (int c = 0; c < 3; c++) q[c] += q32[c];
     }
     for (int c = 0; c < 3; c++) {
         sn[grp][c][sl] = n[c];
