@@ -178,7 +178,6 @@ struct epi_batch {
     int *d_qpos = nullptr, *d_qbegin = nullptr, *d_qend = nullptr;  // [NKIND][NQ]: FAST, GENERAL, SPARSE items
     size_t work_cap = 0, scan_cap = 0;
     long long nkind[NKIND] = {0, 0, 0};  // work items of each tile kind (FAST first in d_work)
-    double wkind[NKIND] = {0, 0, 0};     // pairs times individuals of each tile kind
     DevHit *hits = nullptr;
     unsigned long long *nhits = nullptr;
     long long cap = 1ll << 22;
@@ -1003,6 +1002,24 @@ void emit_tile(const Dataset &d, int a0, int a1, int b0, int b1, int grows, int 
     }
 }
 
+// Pairs (a > b) of the chr x chr blocks [bb, be).
+long long block_pairs(const Dataset &d, int bb, int be)
+{
+    long long n = 0;
+    const int nchr = (int)d.chrstart.size();
+    for (int i = 0; i < nchr; i++)
+        for (int j = 0; j <= i; j++) {
+            const int blk = i * (i + 1) / 2 + j;
+            if (blk < bb || blk >= be) continue;
+            // a in [A0, A1) meets b in [B0, min(B1, a))
+            const long long A0 = d.chrstart[i], A1 = A0 + d.chrsize[i], B0 = d.chrstart[j], B1 = B0 + d.chrsize[j];
+            const long long lo = std::max(A0, B0 + 1), mid = std::min(std::max(lo, B1), std::max(lo, A1));
+            n += (mid - lo) * (lo - B0 + mid - 1 - B0) / 2;  // b up to a - 1
+            if (A1 > mid) n += (A1 - mid) * std::max(0ll, B1 - B0);
+        }
+    return n;
+}
+
 // Where a piecewise tile build resumes: the next chr x chr block (index
 // i(i+1)/2 + j) and, within it, the next super-tile row.
 struct TileCursor {
@@ -1036,11 +1053,7 @@ bool build_tiles(const Dataset &d, int blk_end, int form, const epi_schedule &sc
                 cur.sa = 0;
                 continue;
             }
-            if (cur.sa == 0)
-                for (long long a = A0; a < A1; a++) {  // pairs in this block (a > b)
-                    long long lo = B0, hi = std::min<long long>(B1, a);
-                    if (hi > lo) out.pairs += hi - lo;
-                }
+            if (cur.sa == 0) out.pairs += block_pairs(d, blk, blk + 1);
             int nta = (A1 - A0 + TA - 1) / TA, ntb = (B1 - B0 + TB - 1) / TB;
             for (int sa = cur.sa; sa < nta; sa += SA) {
                 for (int sb = 0; sb < ntb; sb += SB)
@@ -1279,20 +1292,21 @@ struct ScreenKind {
 template <bool GEN, int TA, int TB>
 int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind &K)
 {
-    const int nt = GEN ? screen_gen_threads<TA, TB>() : screen_threads<TA>();
     G.cs.count = K.count;
     G.cs.redo = K.redo;
+    G.halves = GEN ? TB / 32 : 1;
     for (int t0 = 0; t0 < K.n;) {
-        const int chunk = std::min((int)((1u << 31) / (unsigned)nt) & ~255, K.n - t0);  // as LAUNCH_TILES
+        const int chunk = std::min((int)((1u << 31) / (scr_threads<TA>() * G.halves)) & ~255, K.n - t0);  // as LAUNCH_TILES
+        const dim3 grid(chunk * G.halves), block(scr_threads<TA>());
         G.tiles = K.tiles + t0;
         G.ntiles = chunk;
         G.tile0 = t0;
         if constexpr (GEN) {
-            if (G.cut.nd == 1) hipLaunchKernelGGL((screen_gen_kernel<TA, TB, 1>), dim3(chunk), dim3(nt), 0, c->stream, G);
-            else hipLaunchKernelGGL((screen_gen_kernel<TA, TB, 2>), dim3(chunk), dim3(nt), 0, c->stream, G);
+            if (G.cut.nd == 1) hipLaunchKernelGGL((screen_gen_kernel<TA, 1>), grid, block, 0, c->stream, G);
+            else hipLaunchKernelGGL((screen_gen_kernel<TA, 2>), grid, block, 0, c->stream, G);
         } else {
-            if (G.cut.nd == 1) hipLaunchKernelGGL((screen_fast_kernel<TA, 1>), dim3(chunk), dim3(nt), 0, c->stream, G);
-            else hipLaunchKernelGGL((screen_fast_kernel<TA, 2>), dim3(chunk), dim3(nt), 0, c->stream, G);
+            if (G.cut.nd == 1) hipLaunchKernelGGL((screen_fast_kernel<TA, 1>), grid, block, 0, c->stream, G);
+            else hipLaunchKernelGGL((screen_fast_kernel<TA, 2>), grid, block, 0, c->stream, G);
         }
         HIPCHK(c, hipGetLastError());
         c->last_launches++;
@@ -1308,10 +1322,24 @@ int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind
     return EPI_OK;
 }
 
+// Tile height of a screened scan. The K loop of a small cohort's tile is short, and workgroups of two waves overlap
+// their starts and ends better (kernel time of 64 rows over 32: N = 500 to 1500 1.03 without missing calls and 1.01
+// with 1 %, N = 2000 1.02 and 0.98, N = 3000 0.99 and 0.95, N = 20000 0.99 and 0.97); the list of 64-row tiles is half as
+// long, which a first scan pays for on the host.
+int screen_rows(int nid) { return nid >= 2000 ? 64 : 32; }
+
+// Whether the scan of phenotype p.phen over `pairs` pairs goes through the screen, and its cut.
+bool screened(const Dataset &d, const epi_scan_params *p, long long pairs, ScreenCut &C)
+{
+    const double unit = d.missum[d.nsnp] ? 2.5 : 1.0;  // of the exact tiles' cost
+    return p->form == EPI_FORM_MFMA && unit * (double)pairs * d.nid >= SCR_MIN_WORK && screen_fits(d) &&
+           screen_cut(d.ph[p->phen], p, C);
+}
+
 // Launch the pair kernels of one scan over the uploaded tile lists (fast tiles first).
 template <bool DUMP>
 int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, const TileLists &tl,
-                 const DumpSink &ds, const ScanBufs &B)
+                 const DumpSink &ds, const ScanBufs &B, const ScreenCut *cut = nullptr)
 {
     const Dataset &d = c->d;
     if (tl.count() > (size_t)INT32_MAX)
@@ -1328,22 +1356,18 @@ int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, c
         A.hs = hs;
         A.ds = ds;
         if (ns && !d.sp_ok) return fail(c, EPI_ERR_STATE, "SPARSE tile data not built");
-        // Each kind of tile goes through the screen where its exact tiles would take long enough.
-        ScreenArgs G;
-        const double per = (double)sc.fast_rows * A.S.Kl;  // rows times individuals
-        bool sf = nf * 64 * per >= SCR_MIN_WORK, ss = ns * 64 * per * 2.5 >= SCR_MIN_WORK,
-             sg = ng * 32 * per * 2.5 >= SCR_MIN_WORK;
-        if (DUMP || !B.cs.cand || !(sf || ss || sg) || !screen_fits(d) ||
-            !screen_cut(d.ph[p->phen], p, G.cut))
-            sf = ss = sg = false;
-        if (sc.dense_missing == 2) ss = false;  // SPARSE tiles asked for
+        // Every kind of tile goes through the screen with a cut (SPARSE tiles that the schedule asks for do not).
+        const bool sf = cut && nf, ss = cut && ns && sc.dense_missing != 2, sg = cut && ng;
         if (sf || ss || sg) {
+            ScreenArgs G;
             G.S = A.S;
+            G.cut = *cut;
             G.cs = B.cs;
-            int rc = EPI_OK;
             uint32_t *redo = B.cs.redo;
-            const ScreenKind kf = {B.tiles, nf, B.cs.count, redo}, ks = {B.tiles + nf, ns, B.cs.count + 2, redo + 4 * (size_t)nf},
+            const ScreenKind kf = {B.tiles, nf, B.cs.count, redo},
+                             ks = {B.tiles + nf, ns, B.cs.count + 2, redo + 4 * (size_t)nf},
                              kg = {B.tiles + nf + ns, ng, B.cs.count + 4, redo + 4 * (size_t)nf + 8 * (size_t)ns};
+            int rc = EPI_OK;
             if (sc.fast_rows == 64) {
                 if (sf) rc = launch_screen<false, 64, 64>(c, G, hs, kf);
                 if (ss && !rc) rc = launch_screen<true, 64, 64>(c, G, hs, ks);
@@ -1434,7 +1458,6 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
         ct[kind].resize(nd);
     }
     b->pairs = 0;
-    for (double &x : b->wkind) x = 0.0;
     // estimated cost per pair and individual, by kind
     const double unit[NKIND] = {form == EPI_FORM_MFMA ? 16.0 : 4.0, form == EPI_FORM_MFMA ? 40.0 : 10.0, 22.0};
     for (int di = 0; di < nd; di++) {
@@ -1452,7 +1475,6 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
             for (const int4 &t : v) {
                 int ext = (t.y - t.x) | ((t.w - t.z) << 8) | (kind << 16);
                 double cst = (double)(t.y - t.x) * (t.w - t.z) * d.Kp * unit[kind] + 5e4;
-                b->wkind[kind] += (double)(t.y - t.x) * (t.w - t.z) * d.Kp * sc.size();
                 for (int s : sc) {
                     wk[kind][di].push_back(make_int4(t.x, t.z, ext, s));
                     ct[kind][di].push_back(cst);
@@ -1588,13 +1610,6 @@ const void *screen_batch_fn(const epi_schedule &sc, int kind)
                      : (const void *)screen_batch_kernel<32, 0>;
 }
 
-int screen_batch_threads_of(const epi_schedule &sc, int kind)
-{
-    if (sc.fast_rows == 64)
-        return kind == 2 ? screen_batch_threads<64, 2>() : kind ? screen_batch_threads<64, 1>() : screen_batch_threads<64, 0>();
-    return kind == 2 ? screen_batch_threads<32, 2>() : kind ? screen_batch_threads<32, 1>() : screen_batch_threads<32, 0>();
-}
-
 const void *redo_batch_fn(const epi_schedule &sc, int kind)
 {
     if (sc.fast_rows == 64)
@@ -1606,51 +1621,49 @@ const void *redo_batch_fn(const epi_schedule &sc, int kind)
                      : (const void *)redo_kernel<32, 64, false, true>;
 }
 
-// Which lists of the batch go through the screen, with the scans' cuts on the device. A list does
-// where it is long enough and at least half of the scans are screened (the tiles of the others are redone
-// whole, by exact tiles).
-int batch_screen(epi_batch *b, const epi_scan_params *p, bool use[NKIND])
+// The scans' cuts, and whether the batch goes through the screen: where it is long enough and at least half of
+// its scans are screened (the tiles of the others are redone whole, by exact tiles).
+bool batch_screen(const epi_batch *b, const epi_scan_params *p, std::vector<ScreenCut> &cut)
 {
-    epi_ctx *c = b->ctx;
-    for (int k = 0; k < NKIND; k++) use[k] = false;
-    if (p->form != EPI_FORM_MFMA || b->nwork >= (1ll << 28)) return EPI_OK;
-    std::vector<ScreenCut> cut(b->scans.size());
+    if (p->form != EPI_FORM_MFMA) return false;
+    cut.resize(b->scans.size());
     size_t ok = 0;
+    double work = 0.0;
     for (size_t s = 0; s < cut.size(); s++) {
         const Dataset &d = *b->data[b->scans[s].first];
+        const int nchr = (int)d.chrstart.size();
         memset(&cut[s], 0, sizeof(ScreenCut));
         if (screen_fits(d) && screen_cut(d.ph[b->scans[s].second], p, cut[s])) ok++;  // cut.nd stays 0 otherwise
+        work += (double)block_pairs(d, 0, nchr * (nchr + 1) / 2) * d.nid * (d.missum[d.nsnp] ? 2.5 : 1.0);
     }
-    if (2 * ok < cut.size()) return EPI_OK;
-    use[0] = b->wkind[0] >= SCR_MIN_WORK;
-    use[1] = 2.5 * b->wkind[1] >= SCR_MIN_WORK;
-    use[2] = 2.5 * b->wkind[2] >= SCR_MIN_WORK && b->work_sched.dense_missing != 2;
-    HIPCHK(c, hipMemcpyAsync(b->d_cut, cut.data(), cut.size() * sizeof(ScreenCut), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return EPI_OK;
+    return 2 * ok >= cut.size() && work >= SCR_MIN_WORK;
 }
 
 // Capture queue reset + the persistent scan kernels as one graph: one kernel
 // per tile kind that has items (GENERAL and SPARSE first under order 1), each with a grid
 // of its occupancy times the CU count, so that every workgroup is resident and
 // pulls work until its queues run dry.
-int capture_batch(epi_batch *b, const epi_scan_params *p)
+int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<ScreenCut> *cut)
 {
     epi_ctx *c = b->ctx;
     drop_graph(b);
+    if (b->nwork >= (1ll << 28)) cut = nullptr;  // regions are numbered in 31 bits
+    if (cut) {
+        HIPCHK(c, hipMemcpyAsync(b->d_cut, cut->data(), cut->size() * sizeof(ScreenCut), hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+    }
     BatchArgs B[NKIND];
     const void *kfn[NKIND];
     int grid[NKIND] = {0, 0, 0}, nt[NKIND];
     bool screen[NKIND];
-    int rc = batch_screen(b, p, screen);
-    if (rc) return rc;
     int Kl = 0;
     for (const Dataset *d : b->data) Kl = std::max(Kl, (d->nid + KC - 1) / KC * KC);
     ScreenBatchArgs G[NKIND];
     const int4 *work = b->d_work;
     uint32_t *redo = b->redo;
     for (int kind = 0; kind < NKIND; kind++) {
-        nt[kind] = screen[kind] ? screen_batch_threads_of(b->work_sched, kind) : batch_threads_of(p->form, b->work_sched, kind);
+        screen[kind] = cut && !(kind == 2 && b->work_sched.dense_missing == 2);  // SPARSE tiles that the schedule asks for
+        nt[kind] = screen[kind] ? 4 * b->work_sched.fast_rows : batch_threads_of(p->form, b->work_sched, kind);
         G[kind] = {b->d_mscan, b->d_cut, work, 0, 0, {c->cand, b->scount + 2 * kind, CAND_CAP, redo}};
         work += b->nkind[kind];
         redo += (kind == 2 ? 8 : 4) * (size_t)b->nkind[kind];
@@ -1680,13 +1693,14 @@ int capture_batch(epi_batch *b, const epi_scan_params *p)
         }
         // one workgroup per item, in launches of whole XCD groups within the runtime's 2^31 work-items
         const int4 *items = G[kind].work;
-        const int n = (int)b->nkind[kind], chunk = (int)((1u << 31) / (unsigned)nt[kind]) & ~255;
+        const int n = (int)b->nkind[kind], halves = kind == 2 ? 2 : 1;
+        const int chunk = (int)((1u << 31) / (unsigned)(nt[kind] * halves)) & ~255;
         for (int t0 = 0; t0 < n && le == hipSuccess; t0 += chunk) {
             G[kind].work = items + t0;
             G[kind].item0 = t0;
             G[kind].nitems = std::min(chunk, n - t0);
             void *args[] = {&G[kind]};
-            le = hipLaunchKernel(kfn[kind], dim3(G[kind].nitems), dim3(nt[kind]), args, 0, c->stream);
+            le = hipLaunchKernel(kfn[kind], dim3(G[kind].nitems * halves), dim3(nt[kind]), args, 0, c->stream);
         }
         ResolveArgs R = {{}, b->d_mscan, B[kind].hs, c->cand, G[kind].cs.count, CAND_CAP, resolve_lanes(Kl)};
         RedoArgs D = {{}, b->d_mscan, B[kind].hs, items, G[kind].cs.count, G[kind].cs.redo};
@@ -1718,13 +1732,18 @@ int batch_prepare(epi_batch *b, const epi_scan_params *p)
     if (p->form == EPI_FORM_MFMA)
         for (const auto &x : b->scans)
             if ((rc = check_mfma_phen(b->ctx, *b->data[x.first], x.second))) return rc;
-    const epi_schedule &sc = b->sched[p->form];
+    epi_schedule sc = b->sched[p->form];
+    std::vector<ScreenCut> cut;
+    const bool screen = batch_screen(b, p, cut);
+    int nid = 0;
+    for (const Dataset *d : b->data) nid = std::max(nid, d->nid);
+    if (screen) sc.fast_rows = screen_rows(nid);
     if (b->dirty || b->work_form != p->form || !same_schedule(b->work_sched, sc)) {
         drop_graph(b);
         if ((rc = build_batch_work(b, p->form, sc))) return rc;
     }
     if (!b->gvalid || !same_key(b->gkey, *p))
-        if ((rc = capture_batch(b, p))) return rc;
+        if ((rc = capture_batch(b, p, screen ? &cut : nullptr))) return rc;
     return EPI_OK;
 }
 
@@ -1772,12 +1791,18 @@ int batch_fetch(epi_batch *b)
 // list of up to c->max_tiles tiles is built once and kept on the device; a
 // longer one is built, uploaded and launched in pieces of about that many
 // tiles, and the timed region then also holds the uploads of the later pieces.
-int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc)
+int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
 {
     int rc;
     int nchr = (int)c->d.chrstart.size();
     int nblk = nchr * (nchr + 1) / 2;
     int bb = std::max(0, p->blk_begin), be = p->blk_end <= 0 ? nblk : std::min(nblk, p->blk_end);
+    ScreenCut cut;
+    const bool screen = screened(c->d, p, block_pairs(c->d, bb, be), cut);
+    epi_schedule sc = asked;
+    if (screen) sc.fast_rows = screen_rows(c->d.nid);
+    // a screened list takes as much room again for its regions, within the same bound
+    const size_t max_tiles = screen ? std::max<size_t>(1, c->max_tiles / 2) : c->max_tiles;
     TileLists &tl = c->tl;
     const bool cached =
         c->tl_valid && c->tl_bb == bb && c->tl_be == be && c->tl_form == p->form && same_schedule(c->tl_sched, sc);
@@ -1786,7 +1811,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc)
     bool done = cached;
     if (!cached) {
         tl = TileLists();
-        done = build_tiles(c->d, be, p->form, sc, c->max_tiles, cur, tl);
+        done = build_tiles(c->d, be, p->form, sc, max_tiles, cur, tl);
         if ((rc = upload_tiles(c, tl))) return rc;
         if (done) {
             c->tl_valid = true;
@@ -1804,13 +1829,13 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc)
     c->last_tiles[0] = c->last_tiles[1] = c->last_tiles[2] = 0;
     int launches = 0;
     for (;;) {
-        if ((rc = launch_pairs<false>(c, p, sc, tl, ds, ctx_bufs(c)))) return rc;
+        if ((rc = launch_pairs<false>(c, p, sc, tl, ds, ctx_bufs(c), screen ? &cut : nullptr))) return rc;
         launches += c->last_launches;
         if (done) break;
         // the launched kernels read the device tile list that the next piece overwrites
         HIPCHK(c, hipStreamSynchronize(c->stream));
         tl = TileLists();
-        done = build_tiles(c->d, be, p->form, sc, c->max_tiles, cur, tl);
+        done = build_tiles(c->d, be, p->form, sc, max_tiles, cur, tl);
         if ((rc = upload_tiles(c, tl))) return rc;
         HIPCHK(c, hipMemsetAsync(c->scount, 0, 6 * sizeof(uint32_t), c->stream));
         pairs += tl.pairs;

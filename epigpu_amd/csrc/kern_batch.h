@@ -120,31 +120,28 @@ __global__ __launch_bounds__((batch_threads<TA, KIND>()), (batch_waves_per_simd<
     }
 }
 
-// A list through the screen: one workgroup per item (KIND as above), in the order of the list, with the XCD mapping
-// of single scans (a persistent grid that pulls from the queues measured 5 % more at N = 4000, M = 20000). Tiles of
-// scans that the screen does not take go to the redo list whole.
+// A list through the screen: one workgroup per item (two per SPARSE item), in the order of the list, with the XCD
+// mapping of single scans (a persistent grid that pulls from the queues measured 5 % more at N = 4000, M = 20000).
+// Tiles of scans that the screen does not take go to the redo list whole.
 template <int TA, int KIND>
-constexpr int screen_batch_threads() { return KIND == 0 ? screen_threads<TA>() : screen_gen_threads<TA, KIND == 1 ? 32 : 64>(); }
-
-template <int TA, int KIND>
-__global__ __launch_bounds__((screen_batch_threads<TA, KIND>()), 2) void screen_batch_kernel(const ScreenBatchArgs B)
+__global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_batch_kernel(const ScreenBatchArgs B)
 {
-    constexpr int TB = KIND == 1 ? 32 : 64, NW = screen_batch_threads<TA, KIND>() / 64;
+    constexpr int HALVES = KIND == 2 ? 2 : 1, NW = HALVES * (TA / SCR_A);
     __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * sw_row<2>()];
-    __shared__ float4 mg[TA + TB];
+    __shared__ float4 mg[TA + 64];
     __shared__ float2 mg2[TA];
-    const int it = xcd_tile(blockIdx.x, B.nitems);
+    const int t = xcd_tile(blockIdx.x, B.nitems * HALVES), it = t / HALVES;
     const int4 w = B.work[it];
-    const int a0 = __builtin_amdgcn_readfirstlane(w.x), b0 = __builtin_amdgcn_readfirstlane(w.y);
-    const int ext = __builtin_amdgcn_readfirstlane(w.z), sc = __builtin_amdgcn_readfirstlane(w.w);
-    const int a1 = a0 + (ext & 255), b1 = b0 + ((ext >> 8) & 255);
+    const int a0 = __builtin_amdgcn_readfirstlane(w.x), ext = __builtin_amdgcn_readfirstlane(w.z);
+    const int sc = __builtin_amdgcn_readfirstlane(w.w), a1 = a0 + (ext & 255);
+    int b0 = __builtin_amdgcn_readfirstlane(w.y), b1 = b0 + ((ext >> 8) & 255);
     // by value: the descriptors' fields would otherwise be loaded again wherever a store may alias them
     // (N = 4000, M = 20000 with 1 % missing calls: 9.1 against 7.2 ms a phenotype)
     const MfmaScan S = B.mscan[sc];
     const ScreenCut C = B.cut[sc];
-    const uint32_t region0 = (uint32_t)(B.item0 + it) * NW;
+    uint32_t region0 = (uint32_t)(B.item0 + it) * NW;
     if (!C.nd) {
-        if (threadIdx.x == 0) B.cs.redo[atomicAdd(B.cs.count + 1, 1u)] = SCR_WHOLE | region0;
+        if (threadIdx.x == 0 && t % HALVES == 0) B.cs.redo[atomicAdd(B.cs.count + 1, 1u)] = SCR_WHOLE | region0;
         return;
     }
     if constexpr (KIND == 0) {
@@ -153,10 +150,11 @@ __global__ __launch_bounds__((screen_batch_threads<TA, KIND>()), 2) void screen_
         else
             screen_fast_tile<TA, 2>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg, mg2);
     } else {
+        if (!scr_half<TA>(t % HALVES, HALVES, (uint32_t)(B.item0 + it), b0, b1, region0)) return;
         if (C.nd == 1)
-            screen_gen_tile<TA, TB, 1>(S, C, B.cs, a0, a1, b0, b1, region0, wl, reinterpret_cast<float *>(mg));
+            screen_gen_tile<TA, 1>(S, C, B.cs, a0, a1, b0, b1, region0, wl, reinterpret_cast<float *>(mg));
         else
-            screen_gen_tile<TA, TB, 2>(S, C, B.cs, a0, a1, b0, b1, region0, wl, reinterpret_cast<float *>(mg));
+            screen_gen_tile<TA, 2>(S, C, B.cs, a0, a1, b0, b1, region0, wl, reinterpret_cast<float *>(mg));
     }
 }
 

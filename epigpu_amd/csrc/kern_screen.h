@@ -53,6 +53,8 @@ constexpr int SCR_WIN = 512; // words (of 32 individuals) of weights in LDS at a
 constexpr int SCR_LDS_ROWS = SCR_WIN + 2;  // the pipeline reads one step past the window
 constexpr int SCR_GEN_ROWS = SCR_WIN + 4;
 constexpr int SCR_A = 16;    // a-SNPs per wave
+template <int TA>
+constexpr int scr_threads() { return 64 * TA / SCR_A; }  // a workgroup takes a tile of TA = 32 or 64 a-SNPs
 constexpr int SCR_REDO = 8;   // candidates per pair slot of a wave (64 pairs) above which the exact tile redoes its region
 
 // Per SNP and phenotype: counts and sums of v (one and two digits) of the two rarest classes and
@@ -92,6 +94,7 @@ struct ScreenArgs {
     const int4 *tiles;
     int ntiles;
     int tile0;                // index of tiles[0] in the scan's list
+    int halves;               // GENERAL kernel: workgroups per tile (1: 32 b, 2: SPARSE tiles of 64 b)
 };
 
 // The FP6 image of 32 individuals in a lane: element s occupies bits 6s..6s+5 of
@@ -268,15 +271,12 @@ __device__ __forceinline__ void scr_append(const CandSink &cs, uint32_t bits, ui
 // (one dword per operand and 64 individuals, coalesced along SNPs) and expands
 // them in registers: no operand passes through LDS, and the waves run
 // without barriers. LDS holds the phenotype's codes, which all waves share.
-template <int TA>
-constexpr int screen_threads() { return 64 * TA / SCR_A; }
-
 template <int TA, int ND>
 __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const ScreenCut &C, const CandSink &cs, int a0,
                                                  int a1, int b0, int b1, uint32_t region0, uint32_t *wl,
                                                  float4 *mg, float2 *mg2)
 {
-    constexpr int NT = screen_threads<TA>(), ROW = sw_row<ND>();
+    constexpr int NT = scr_threads<TA>(), ROW = sw_row<ND>();
     const uint32_t *sw = S.sw[ND - 1];
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, hf = lane >> 5;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -436,7 +436,7 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const Screen
 }
 
 template <int TA, int ND>
-__global__ __launch_bounds__(screen_threads<TA>(), 2) void screen_fast_kernel(const ScreenArgs A)
+__global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_fast_kernel(const ScreenArgs A)
 {
     __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_LDS_ROWS * sw_row<ND>()];
     __shared__ float4 mg[TA + 64];
@@ -444,11 +444,11 @@ __global__ __launch_bounds__(screen_threads<TA>(), 2) void screen_fast_kernel(co
     const int t = xcd_tile(blockIdx.x, A.ntiles);
     const int4 T = A.tiles[t];
     screen_fast_tile<TA, ND>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, (uint32_t)(A.tile0 + t) * (TA / SCR_A), wl, mg,
-                         mg2);
+                             mg2);
 }
 
 // ------------------------------------------------------------- GENERAL ----
-// Tile TA a x TB b with missing calls (TB = 32, or 64 for tiles whose SNPs miss few calls). Each
+// Tile TA a x 32 b with missing calls (a SPARSE tile, whose SNPs miss few calls, is two of them). Each
 // wave owns 16 a x 32 b and contracts the three classes of both sides with the count and the two
 // digits: 27 v_mfma_f32_16x16x128_f8f6f4 per 16 x 16 pairs and 128 individuals (the exact tile: 40 INT8
 // MACs per pair and individual, here 27 at twice the rate). The 16 x 16 shape puts a pair's 18 accumulators
@@ -467,20 +467,16 @@ __device__ __forceinline__ v4f scr_mfma16x32(const v8i &a, const v8i &b, const v
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 2, 0, 0x84848484, 0, 0x7f7f7f7f);
 }
 
-template <int TA, int TB>
-constexpr int screen_gen_threads() { return 64 * (TA / SCR_A) * (TB / 32); }
-
-template <int TA, int TB, int ND>
+template <int TA, int ND>
 __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenCut &C, const CandSink &cs, int a0, int a1,
                                                 int b0, int b1, uint32_t region0, uint32_t *wl, float *mz)
 {
-    constexpr int NT = screen_gen_threads<TA, TB>(), NWA = TA / SCR_A, ROW = sw_row<ND>();
+    constexpr int TB = 32, NT = scr_threads<TA>(), ROW = sw_row<ND>();
     const uint32_t *sw = S.sw[ND - 1];
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, kq = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int al = SCR_A * (wid % NWA), bl = 32 * (wid / NWA);
-    const int aw = a0 + al, bw = b0 + bl;
-    const bool work = aw < a1 && bw < b1 && (a1 < aw + SCR_A ? a1 : aw + SCR_A) - 1 > bw;
+    const int al = SCR_A * wid, aw = a0 + al, bw = b0;
+    const bool work = aw < a1 && (a1 < aw + SCR_A ? a1 : aw + SCR_A) - 1 > bw;
     const int Kw = S.Kp / 32, nw = S.Kl / 32;
 
     for (int i = tid; i < TA + TB; i += NT) {
@@ -651,7 +647,7 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
             tc += s[c];
         }
         tc = __builtin_fmaf(C.c0, nc, tc);
-        const float zlow = mz[al + 4 * kq + i] + mz[TA + bl + 16 * bg + m] - C.zall;
+        const float zlow = mz[al + 4 * kq + i] + mz[TA + 16 * bg + m] - C.zall;
         float u = 0.0f;
 #pragma unroll
         for (int c = 0; c < 9; c++) u = __builtin_fmaf(s[c] * s[c], rcp_above(n[c]), u);
@@ -674,21 +670,33 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
     });
 }
 
-template <int TA, int TB, int ND>
-__global__ __launch_bounds__((screen_gen_threads<TA, TB>()), 2) void screen_gen_kernel(const ScreenArgs A)
+// The workgroup's half of 32 b (or the whole) of a tile: b range and first region. False: no b-SNPs.
+template <int TA>
+__device__ __forceinline__ bool scr_half(int h, int halves, uint32_t tile, int &b0, int &b1, uint32_t &region0)
+{
+    b0 += 32 * h;
+    region0 = (tile * halves + h) * (TA / SCR_A);
+    const bool any = b0 < b1;
+    b1 = b1 < b0 + 32 ? b1 : b0 + 32;
+    return any;
+}
+
+template <int TA, int ND>
+__global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_gen_kernel(const ScreenArgs A)
 {
     __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * sw_row<ND>()];
-    __shared__ float mz[TA + TB];
-    const int t = xcd_tile(blockIdx.x, A.ntiles);
-    const int4 T = A.tiles[t];
-    screen_gen_tile<TA, TB, ND>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w,
-                            (uint32_t)(A.tile0 + t) * (screen_gen_threads<TA, TB>() / 64), wl, mz);
+    __shared__ float mz[TA + 32];
+    const int t = xcd_tile(blockIdx.x, A.ntiles * A.halves);
+    int4 T = A.tiles[t / A.halves];
+    uint32_t region0;
+    if (!scr_half<TA>(t % A.halves, A.halves, (uint32_t)(A.tile0 + t / A.halves), T.z, T.w, region0)) return;
+    screen_gen_tile<TA, ND>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, region0, wl, mz);
 }
 
 // --------------------------------------------------------------- redo ----
 // Regions that the screen handed back, and tiles of scans that it does not take (SCR_WHOLE),
-// through the exact tiles of 32 rows: a persistent grid over the device's count of them. A region r of a TA x TB
-// tile t is wave r % NW (a block wave % (TA / 16), b block wave / (TA / 16)) of tile r / NW.
+// through the exact tiles of 32 rows: a persistent grid over the device's count of them. Region r of a TA x TB
+// tile is block r % NW (a block r % NWA, b block r % NW / NWA) of tile r / NW.
 constexpr uint32_t SCR_WHOLE = 1u << 31;
 
 struct RedoArgs {
@@ -704,7 +712,7 @@ template <int TA, int TB, bool GEN, bool BATCH>
 __global__ __launch_bounds__(256, 2) void redo_kernel(const RedoArgs A)
 {
     static_assert(fast_threads<32>() == 256 && general_threads<32>() == 256, "threads of the 32-row tiles");
-    constexpr int RB = GEN ? 32 : 64, NW = TA / SCR_A * (TB / RB);
+    constexpr int RB = GEN ? 32 : 64, NWA = TA / SCR_A, NW = NWA * (TB / RB);
     __shared__ __attribute__((aligned(16))) uint8_t lds[GEN ? general_lds<32>() : fast_lds<32>()];
     const uint32_t n = A.count[1];
     const DumpSink nodump = {};
@@ -724,8 +732,8 @@ __global__ __launch_bounds__(256, 2) void redo_kernel(const RedoArgs A)
         int b0 = __builtin_amdgcn_readfirstlane(T.z), b1 = __builtin_amdgcn_readfirstlane(T.w);
         if (!(r & SCR_WHOLE)) {
             const int w = (int)(r % NW);
-            a0 += SCR_A * (w % (TA / SCR_A));
-            b0 += RB * (w / (TA / SCR_A));
+            a0 += SCR_A * (w % NWA);
+            b0 += RB * (w / NWA);
             a1 = a1 < a0 + SCR_A ? a1 : a0 + SCR_A;
             b1 = b1 < b0 + RB ? b1 : b0 + RB;
         }

@@ -181,7 +181,8 @@ int epi_set_hit_capacity(epi_ctx *ctx, int64_t cap);
  * 260,000 to 520,000 SNPs, by tile shape) is built, uploaded and launched in
  * pieces of about this many tiles (whole rows of super-tiles), with the
  * same hits; its epi_last_scan_stats time then includes the later pieces'
- * uploads. No counterpart in the reference, which launches per chunk of
+ * uploads. A screened scan (below) counts a tile twice: its list takes as much
+ * room again for the regions that the exact tiles redo. No counterpart in the reference, which launches per chunk of
  * -i SNPs (src/EpiOpenCL.c:1564-1607). 1 <= max_tiles <= 2^30 - 1. */
 int epi_set_max_tiles(epi_ctx *ctx, int64_t max_tiles);
 
@@ -195,7 +196,13 @@ int epi_set_max_tiles(epi_ctx *ctx, int64_t max_tiles);
  * rates). A tile can be SPARSE when every SNP of its ranges misses at most
  * max(8, nid / 16) calls; dense_missing 0 makes it SPARSE when its SNPs
  * also miss at most 1/150 of their calls on average. The plain form's GENERAL
- * tiles are 16 x 64. */
+ * tiles are 16 x 64.
+ * MFMA scans and batches of more than a few hundred million pairs times
+ * individuals, at thresholds that few pairs pass, are screened: their tiles,
+ * whose height follows nid and not fast_rows, first bound every pair's statistics, and
+ * only the pairs that could pass are computed exactly, with the same hits and
+ * values. fast_rows and queues then have no effect, and SPARSE tiles are kept
+ * only where dense_missing is 2. */
 typedef struct epi_schedule {
     int32_t fast_rows;  /* MFMA form: 64 or 32; plain form: 32 or 16 */
     int32_t super_a;    /* tiles are issued in super-tiles of super_a x super_b */
