@@ -5,9 +5,10 @@
 //   mbits   [3][Kw][nsnp]  uint32  bitplanes of classes 0, 1 and call present (MFMA form)
 //   bits    [3][Kw][nsnp]  uint32  bitplanes of the two rarest classes and call present (plain form)
 //   cls     [nsnp]         int32   plain-form plane -> class map
-//   per phenotype r (wts, mp, yc, vbits, ov and oidx in one allocation):
+//   per phenotype r (wts, mp, yc, yw, vbits, ov and oidx in one allocation):
 //     wts   [8][Kp] int8   V, 3 limbs of q, 4 limbs of round(q^2/2^zbits)
 //     yc    [Kp]    float  centred phenotype scaled by 2^-ybits to |yc| < 1 (0 where missing)
+//     yw    [2][Kp] float  yc and its square as the plain kernel reads them
 //     vbits [Kw]    uint32 phenotype-present bits
 //     marg  [nsnp]  Marg   per-SNP class counts and sums
 //     oidx, ocodes, ov     outlier individuals (at most OUT_MAX), their codes per SNP and values
@@ -72,6 +73,7 @@ struct ScreenEnc {
 struct PhenDev {
     int8_t *wts = nullptr;
     float *yc = nullptr;
+    float *yw = nullptr;
     uint32_t *vbits = nullptr;
     Marg *marg = nullptr;
     int32_t *oidx = nullptr;    // [nout] outlier individuals
@@ -252,6 +254,7 @@ void free_phen(PhenDev &p)
     p.sw[0] = p.sw[1] = nullptr;
     p.mp = nullptr;
     p.yc = nullptr;
+    p.yw = nullptr;
     p.vbits = nullptr;
     p.ov = nullptr;
     p.oidx = nullptr;
@@ -378,6 +381,7 @@ struct PhenEnc {
     std::vector<int8_t> w;      // [NWP][Kp], then the screen's weights (3 Kp bytes)
     std::vector<int32_t> qv;    // [Kp]
     std::vector<float> yc;      // [Kp]
+    std::vector<float> yw;      // [2][Kp]
     std::vector<uint32_t> vb;   // [Kw]
     std::vector<int32_t> oidx;  // outlier individuals
     std::vector<MissPhen> mp;   // [Kp]
@@ -607,6 +611,7 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
     e.w.assign((size_t)(NWP + 3) * Kp, 0);
     e.qv.assign(Kp, 0);
     e.yc.assign(Kp, 0.0f);
+    e.yw.assign((size_t)2 * Kp, 0.0f);
     e.vb.assign(Kw, 0u);
     e.mp.assign(Kp, MissPhen{});
     long long qmax2 = 0;
@@ -641,6 +646,8 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
         const double dv = (double)y[k] - centre;
         const float ycf = (float)std::ldexp(dv, -ye);
         e.yc[k] = ycf;
+        e.yw[k] = plain_weight(ycf, k);
+        e.yw[Kp + k] = plain_weight(ycf * ycf, k);
         ys += (double)ycf;
         y2 += (double)ycf * (double)ycf;
         e.vb[k >> 5] |= 1u << (k & 31);
@@ -687,13 +694,14 @@ int ds_set_phenotypes(epi_ctx *c, Dataset &d, const float *phen, int nphen, int 
         PhenEnc &e = enc[r];
         PhenDev &p = ph[r];
         p = e.p;
-        // one allocation and one copy: weights (with the screen's), mp, yc, vbits (Kp is a multiple of 256), ov, oidx
-        const size_t omp = e.w.size(), oyc = omp + (size_t)Kp * sizeof(MissPhen), ovb = oyc + (size_t)Kp * 4,
-                     oov = ovb + (size_t)Kw * 4, oix = oov + sizeof(OutVals);
+        // one allocation and one copy: weights (with the screen's), mp, yc, yw, vbits (Kp is a multiple of 256), ov, oidx
+        const size_t omp = e.w.size(), oyc = omp + (size_t)Kp * sizeof(MissPhen), oyw = oyc + (size_t)Kp * 4,
+                     ovb = oyw + (size_t)Kp * 8, oov = ovb + (size_t)Kw * 4, oix = oov + sizeof(OutVals);
         std::vector<int8_t> blob(oix + sizeof(int32_t) * OUT_MAX, 0);
         memcpy(blob.data(), e.w.data(), e.w.size());
         memcpy(blob.data() + omp, e.mp.data(), (size_t)Kp * sizeof(MissPhen));
         memcpy(blob.data() + oyc, e.yc.data(), (size_t)Kp * 4);
+        memcpy(blob.data() + oyw, e.yw.data(), (size_t)Kp * 8);
         memcpy(blob.data() + ovb, e.vb.data(), (size_t)Kw * 4);
         memcpy(blob.data() + oov, &e.ov, sizeof(OutVals));
         if (p.nout) memcpy(blob.data() + oix, e.oidx.data(), (size_t)p.nout * 4);
@@ -702,6 +710,7 @@ int ds_set_phenotypes(epi_ctx *c, Dataset &d, const float *phen, int nphen, int 
         p.sw[1] = p.sw[0] + Kp / 4;
         p.mp = reinterpret_cast<MissPhen *>(p.wts + omp);
         p.yc = reinterpret_cast<float *>(p.wts + oyc);
+        p.yw = reinterpret_cast<float *>(p.wts + oyw);
         p.vbits = reinterpret_cast<uint32_t *>(p.wts + ovb);
         p.ov = reinterpret_cast<OutVals *>(p.wts + oov);
         p.oidx = reinterpret_cast<int32_t *>(p.wts + oix);
@@ -895,11 +904,12 @@ PlainScan plain_scan(const Dataset &d, int r, int tag)
     const PhenDev &p = d.ph[r];
     PlainScan S;
     S.bits = d.bits;
-    S.yc = p.yc;
+    S.yw = p.yw;
     S.vbits = p.vbits;
     S.marg = p.marg;
     S.nsnp = d.nsnp;
     S.Kw = d.Kw;
+    S.nw = (d.nid + 31) / 32;
     S.nV = p.nV;
     S.tag = tag;
     S.ysV = p.ysV;
@@ -1396,10 +1406,10 @@ int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, c
         P.hs = hs;
         P.ds = ds;
         if (sc.fast_rows == 32)
-            LAUNCH_TILES((plain_kernel<2, 4, true, DUMP>), 256, P, B.tiles, nf);
+            LAUNCH_TILES((plain_kernel<512, true, DUMP>), 512, P, B.tiles, nf);
         else
-            LAUNCH_TILES((plain_kernel<1, 4, true, DUMP>), 256, P, B.tiles, nf);
-        LAUNCH_TILES((plain_kernel<1, 4, false, DUMP>), 256, P, B.tiles + nf + ns, ng);
+            LAUNCH_TILES((plain_kernel<256, true, DUMP>), 256, P, B.tiles, nf);
+        LAUNCH_TILES((plain_kernel<256, false, DUMP>), 256, P, B.tiles + nf + ns, ng);
     }
     return EPI_OK;
 }
@@ -1615,7 +1625,7 @@ void drop_graph(epi_batch *b)
 // Threads per workgroup of batch_kernel(form, sc, kind).
 int batch_threads_of(int form, const epi_schedule &sc, int kind)
 {
-    if (form != EPI_FORM_MFMA) return 256;
+    if (form != EPI_FORM_MFMA) return kind ? 256 : 16 * sc.fast_rows;
     if (sc.fast_rows == 64)
         return kind == 2 ? batch_threads<64, 2>() : kind ? batch_threads<64, 1>() : batch_threads<64, 0>();
     return kind == 2 ? batch_threads<32, 2>() : kind ? batch_threads<32, 1>() : batch_threads<32, 0>();
@@ -1634,8 +1644,8 @@ const void *batch_kernel(int form, const epi_schedule &sc, int kind)
     }
     // the plain form has no SPARSE tiles
     if (sc.fast_rows == 32)
-        return kind ? (const void *)plain_batch_kernel<2, 1> : (const void *)plain_batch_kernel<2, 0>;
-    return kind ? (const void *)plain_batch_kernel<1, 1> : (const void *)plain_batch_kernel<1, 0>;
+        return kind ? (const void *)plain_batch_kernel<256, 1> : (const void *)plain_batch_kernel<512, 0>;
+    return kind ? (const void *)plain_batch_kernel<256, 1> : (const void *)plain_batch_kernel<256, 0>;
 }
 
 const void *screen_batch_fn(const epi_schedule &sc, int kind)

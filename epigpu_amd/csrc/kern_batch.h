@@ -158,10 +158,11 @@ __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_batch_kernel(cons
     }
 }
 
-// PA: FAST tiles are 16 PA x 64 (PA = 2 or 1); GENERAL tiles are 16 x 64.
-template <int PA, int GEN>
-__global__ __launch_bounds__(256) void plain_batch_kernel(const BatchArgs B)
+// NT: FAST tiles are NT/16 x 64 (NT = 512 or 256); GENERAL tiles are 16 x 64.
+template <int NT, int GEN>
+__global__ __launch_bounds__(NT, GEN ? 2 : 4) void plain_batch_kernel(const BatchArgs B)
 {
+    __shared__ PlainLds<!GEN> lds;
     __shared__ int item;
     __shared__ int4 wsh;
     const int home = blockIdx.x % NQ;
@@ -188,10 +189,10 @@ __global__ __launch_bounds__(256) void plain_batch_kernel(const BatchArgs B)
         HitSink hs = B.hs;
         hs.tag = sc;
         const int a1 = a0 + (ext & 255), b1 = b0 + ((ext >> 8) & 255);
-        if (GEN)
-            plain_tile<1, 4, false, false>(S, hs, nodump, a0, a1, b0, b1);
+        if constexpr (GEN)
+            plain_tile<256, false, false>(S, hs, nodump, a0, a1, b0, b1, lds);
         else
-            plain_tile<PA, 4, true, false>(S, hs, nodump, a0, a1, b0, b1);
+            plain_tile<NT, true, false>(S, hs, nodump, a0, a1, b0, b1, lds);
     }
 }
 

@@ -1,18 +1,32 @@
 // Plain popcount form of the pair scan (gfx950 VALU).
 //
 // Genotypes are class bitplanes (bit k of word w = individual 32w + k) laid
-// out [plane][word][snp], so one stage of a SNP tile is a set of contiguous
-// runs and loads coalesce. A 256-thread workgroup stages KW words (256
-// individuals) of its a- and b-tiles and of the phenotype in LDS; every thread
-// owns PA x PB pairs:
+// out [plane][word][snp]. A workgroup of NT threads takes a tile of NT/16 x 64
+// pairs, every thread 2 x 2 of them, and goes through the individuals a word
+// (32) at a time: it writes y_k [k in B_h] of its 64 b-SNPs to LDS (two
+// buffers, one barrier per word) and holds its a-SNPs' words in registers.
 //   counts  X[g][h] += popcount(A_g & V & B_h)      (AND + v_bcnt per word)
-//   sums    X[g][h] += y_k * [k in A_g & V] * [k in B_h]   (masked FP32 FMA)
+//   sums    X[g][h] += [k in A_g] * (y_k [k in B_h])         (masked FP32 FMA)
 // FP32 partial sums are promoted to FP64 after every word. The two bitplanes
 // of a SNP hold its two rarest genotype classes and the most common class is
 // derived (by subtraction from the NM totals), so a small cell never inherits
 // the rounding error of a large one. FAST tiles use the planes {0,1}; GENERAL
 // tiles add the NM plane and the sum of y^2 over complete cases. The per-pair
 // epilogue is shared with the MFMA form.
+//
+// What bounds it: VALU issue, at half the rate for instructions with a scalar
+// operand, shifts left, bit-field extracts, conversions and popcounts (two waves
+// of a SIMD issue FMAs, adds, ANDs and shifts right together where all operands
+// are vector registers or literals: 0.37-0.39 a cycle measured in registers,
+// 0.24 with a scalar factor). So the factor [k in A_g] of an FMA is one AND: bit
+// 16 + j of an a-word, kept in its place, is as FP32 the (denormal) number
+// 2^(j - 133), and yw holds y_k 2^(126 - j) for j = k mod 8. Both factors are
+// powers of two away from [bit] and y_k, so every partial sum is the plain one
+// times PLAIN_SCALE, with the same roundings. 2 x 2 pairs a thread leave FAST
+// tiles four waves per SIMD (128 registers); 4 x 2 with two waves took 5-10 % more.
+// N = 4000, M = 8000: 17.3 ms with every mask extracted and converted by each
+// thread, 12.6 ms; N = 1500, M = 6000: 3.8 -> 3.0 ms; N = 1500, M = 4001, 2 %
+// missing calls: 4.3 -> 3.3 ms. At that rate the FMAs alone are 0.68 of the first.
 #pragma once
 
 #include "epilogue.h"
@@ -20,15 +34,35 @@
 
 namespace epi {
 
-constexpr int KW = 8;  // words (of 32 individuals) per LDS stage
+constexpr double PLAIN_SCALE = 1.0 / 128;  // of the partial sums (2^(126 - j + 16 + j - 149))
+
+// A factor y of individual k (|y| < 1) as the kernel reads it.
+inline float plain_weight(float y, int k) { return y * (0x1p126f / (float)(1 << (k & 7))); }
+
+// Factors of N individuals of a word, the same for a whole wave, through the scalar cache.
+template <int N>
+using plain_y = float __attribute__((ext_vector_type(N), aligned(4)));
+template <int N>
+__device__ __forceinline__ plain_y<N> plain_sload(const float *p)
+{
+    return *reinterpret_cast<const __attribute__((address_space(4))) plain_y<N> *>(reinterpret_cast<uintptr_t>(p));
+}
+
+// LDS of a tile: y_k [k in B_h] (and y_k^2 [k in NM] of GENERAL tiles) of 32 individuals and 64 SNPs, twice.
+template <bool FAST>
+struct PlainLds {
+    typedef float row __attribute__((ext_vector_type(FAST ? 2 : 4)));
+    __attribute__((aligned(16))) row y[2][32][64];
+};
 
 struct PlainScan {          // one dataset x one phenotype
     const uint32_t *bits;   // [3][Kw][nsnp]
-    const float *yc;        // [Kp] centred FP32 phenotype, 0 where missing
+    const float *yw;        // [2][Kp] centred FP32 phenotype y (0 where missing) and y^2, as plain_weight
     const uint32_t *vbits;  // [Kw] phenotype-present bits
     const Marg *marg;       // [nsnp]
     int nsnp;
     int Kw;
+    int nw;                 // words that hold individuals
     int nV;
     int tag;                // written into the hits
     double ysV;             // sum of yc over present
@@ -43,19 +77,22 @@ struct PlainArgs {
     DumpSink ds;
 };
 
-template <int PA, int PB, bool FAST, bool DUMP>
+template <int NT, bool FAST, bool DUMP>
 __device__ __forceinline__ void plain_tile(const PlainScan &P, const HitSink &hs, const DumpSink &dsk, int a0, int a1,
-                                           int b0, int b1)
+                                           int b0, int b1, PlainLds<FAST> &lds)
 {
-    constexpr int NP = FAST ? 2 : 3;
-    constexpr int TA = 16 * PA, TB = 16 * PB;
-    __shared__ uint32_t sA[NP][KW][TA];
-    __shared__ uint32_t sB[NP][KW][TB];
-    __shared__ __attribute__((aligned(16))) float sy[KW * 32];
-    __shared__ uint32_t sv[KW];
-
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+    constexpr int NP = FAST ? 2 : 3, PA = 2, PB = 2, NI = 2048 / NT;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     const int nsnp = P.nsnp;
+    const size_t plane = (size_t)P.Kw * nsnp;
+    // staging: lane = b-SNP, a wave takes eight individuals of the word
+    const int sl = threadIdx.x & 63, sk = NI * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t sb = b0 + sl < nsnp ? b0 + sl : nsnp - 1;
+    uint32_t as[PA], bs[PB];
+#pragma unroll
+    for (int i = 0; i < PA; i++) as[i] = a0 + PA * ty + i < nsnp ? a0 + PA * ty + i : nsnp - 1;
+#pragma unroll
+    for (int j = 0; j < PB; j++) bs[j] = b0 + PB * tx + j < nsnp ? b0 + PB * tx + j : nsnp - 1;
 
     int cnt[PA][PB][NP][NP];
     float sf[PA][PB][NP][NP];
@@ -78,112 +115,123 @@ __device__ __forceinline__ void plain_tile(const PlainScan &P, const HitSink &hs
                 }
         }
 
-    constexpr int NA = NP * KW * TA, NB = NP * KW * TB, NTOT = NA + NB + KW * 32 + KW;
-    for (int w0 = 0; w0 < P.Kw; w0 += KW) {
-        __syncthreads();
-        for (int c = tid; c < NTOT; c += 256) {
-            if (c < NA) {
-                int s = c % TA, w = (c / TA) % KW, p = c / (TA * KW);
-                int snp = a0 + s < nsnp ? a0 + s : nsnp - 1;
-                sA[p][w][s] = P.bits[((size_t)p * P.Kw + w0 + w) * nsnp + snp];
-            } else if (c < NA + NB) {
-                int d = c - NA;
-                int s = d % TB, w = (d / TB) % KW, p = d / (TB * KW);
-                int snp = b0 + s < nsnp ? b0 + s : nsnp - 1;
-                sB[p][w][s] = P.bits[((size_t)p * P.Kw + w0 + w) * nsnp + snp];
-            } else if (c < NA + NB + KW * 32) {
-                int d = c - NA - NB;
-                sy[d] = P.yc[(size_t)w0 * 32 + d];
-            } else {
-                int d = c - NA - NB - KW * 32;
-                sv[d] = P.vbits[w0 + d];
+    uint32_t sw[NP];  // the staged b-SNP's words
+    auto load = [&](int w) {
+        const uint32_t *row = P.bits + (size_t)w * nsnp;
+#pragma unroll
+        for (int h = 0; h < NP; h++) sw[h] = (row + h * plane)[sb];
+    };
+    auto stage = [&](int w) {
+        const auto y8 = plain_sload<NI>(P.yw + 32 * w + sk);
+        plain_y<NI> q8 = {};
+        if (!FAST) q8 = plain_sload<NI>(P.yw + 32 * (P.Kw + w) + sk);
+#pragma unroll
+        for (int k = 0; k < NI; k++) {
+            typename PlainLds<FAST>::row r;
+#pragma unroll
+            for (int h = 0; h < NP; h++) {
+                const int m = __builtin_amdgcn_sbfe((int)(sw[h] >> sk), k, 1);
+                r[h] = __int_as_float(m & __float_as_int(y8[k]));
+                if (h == 2) r[NP] = __int_as_float(m & __float_as_int(q8[k]));
             }
+            lds.y[w & 1][sk + k][sl] = r;
         }
-        __syncthreads();
+    };
+    uint32_t aw[PA][NP], bw[PB][NP], v;
+    auto words = [&](int w) {
+        const uint32_t *row = P.bits + (size_t)w * nsnp;
+        v = P.vbits[w];
+#pragma unroll
+        for (int g = 0; g < NP; g++) {
+#pragma unroll
+            for (int i = 0; i < PA; i++) aw[i][g] = (row + g * plane)[as[i]];
+#pragma unroll
+            for (int j = 0; j < PB; j++) bw[j][g] = (row + g * plane)[bs[j]];
+        }
+    };
 
-        for (int w = 0; w < KW; w++) {
-            const uint32_t v = sv[w];
-            uint32_t aw[PA][NP], bw[PB][NP];
+    load(0);
+    __syncthreads();  // an earlier tile is done with LDS
+    stage(0);
+    if (P.nw > 1) load(1);
+    words(0);
+    __syncthreads();
+    for (int w = 0; w < P.nw; w++) {
+        if (w + 1 < P.nw) stage(w + 1);
+        if (w + 2 < P.nw) load(w + 2);
 #pragma unroll
-            for (int i = 0; i < PA; i++)
-#pragma unroll
-                for (int g = 0; g < NP; g++) aw[i][g] = sA[g][w][ty + 16 * i] & v;
+        for (int i = 0; i < PA; i++)
 #pragma unroll
             for (int j = 0; j < PB; j++)
 #pragma unroll
-                for (int h = 0; h < NP; h++) bw[j][h] = sB[h][w][tx + 16 * j];
+                for (int g = 0; g < NP; g++)
+#pragma unroll
+                    for (int h = 0; h < NP; h++) cnt[i][j][g][h] += __popc(aw[i][g] & v & bw[j][h]);
+        uint32_t ax[PA][NP];
+#pragma unroll
+        for (int i = 0; i < PA; i++)
+#pragma unroll
+            for (int g = 0; g < NP; g++) ax[i][g] = aw[i][g];
+        if (w + 1 < P.nw) words(w + 1);
+        // the rows of individual k + DEPTH are read while those of k are used (three ahead: no faster, one wave less)
+        constexpr int DEPTH = 1;
+        typename PlainLds<FAST>::row r[DEPTH + 1][PB];
+        auto fetch = [&](int k) {
+#pragma unroll
+            for (int j = 0; j < PB; j++) r[k % (DEPTH + 1)][j] = lds.y[w & 1][k][PB * tx + j];
+        };
+#pragma unroll
+        for (int k = 0; k < DEPTH; k++) fetch(k);
+        uint32_t ac[PA][NP];
+#pragma unroll
+        for (int k = 0; k < 32; k++) {
+            if (k % 8 == 0)
+#pragma unroll
+                for (int i = 0; i < PA; i++)
+#pragma unroll
+                    for (int g = 0; g < NP; g++) ac[i][g] = k < 24 ? ax[i][g] << (16 - k) : ax[i][g] >> 8;
+            if (k + DEPTH < 32) fetch(k + DEPTH);
+            const auto &y = r[k % (DEPTH + 1)];
 #pragma unroll
             for (int i = 0; i < PA; i++)
 #pragma unroll
-                for (int j = 0; j < PB; j++)
+                for (int g = 0; g < NP; g++) {
+                    const float m = __uint_as_float(ac[i][g] & (1u << (16 + k % 8)));
 #pragma unroll
-                    for (int g = 0; g < NP; g++)
+                    for (int j = 0; j < PB; j++) {
 #pragma unroll
-                        for (int h = 0; h < NP; h++) cnt[i][j][g][h] += __popc(aw[i][g] & bw[j][h]);
-            const float4 *y4 = reinterpret_cast<const float4 *>(sy + 32 * w);
-#pragma unroll
-            for (int k4 = 0; k4 < 8; k4++) {
-                const float4 yv = y4[k4];
-                const float yk[4] = {yv.x, yv.y, yv.z, yv.w};
-#pragma unroll
-                for (int kk = 0; kk < 4; kk++) {
-                    const int k = 4 * k4 + kk;
-                    const int ybits = __float_as_int(yk[kk]);
-                    float ya[PA][NP], bb[PB][NP];
-#pragma unroll
-                    for (int i = 0; i < PA; i++)
-#pragma unroll
-                        for (int g = 0; g < NP; g++)
-                            ya[i][g] = __int_as_float(__builtin_amdgcn_sbfe((int)aw[i][g], k, 1) & ybits);
-#pragma unroll
-                    for (int j = 0; j < PB; j++)
-#pragma unroll
-                        for (int h = 0; h < NP; h++)
-                            bb[j][h] = (float)__builtin_amdgcn_ubfe(bw[j][h], k, 1);
-#pragma unroll
-                    for (int i = 0; i < PA; i++)
-#pragma unroll
-                        for (int j = 0; j < PB; j++)
-#pragma unroll
-                            for (int g = 0; g < NP; g++)
-#pragma unroll
-                                for (int h = 0; h < NP; h++) sf[i][j][g][h] = fmaf(ya[i][g], bb[j][h], sf[i][j][g][h]);
-                    if (!FAST) {
-#pragma unroll
-                        for (int i = 0; i < PA; i++) {
-                            const float y2 = ya[i][2] * yk[kk];
-#pragma unroll
-                            for (int j = 0; j < PB; j++) qf[i][j] = fmaf(y2, bb[j][2], qf[i][j]);
-                        }
+                        for (int h = 0; h < NP; h++) sf[i][j][g][h] = fmaf(m, y[j][h], sf[i][j][g][h]);
+                        if (g == 2) qf[i][j] = fmaf(m, y[j][NP], qf[i][j]);
                     }
                 }
-            }
-            // promote the word's FP32 partial sums
-#pragma unroll
-            for (int i = 0; i < PA; i++)
-#pragma unroll
-                for (int j = 0; j < PB; j++) {
-                    qd[i][j] += (double)qf[i][j];
-                    qf[i][j] = 0.0f;
-#pragma unroll
-                    for (int g = 0; g < NP; g++)
-#pragma unroll
-                        for (int h = 0; h < NP; h++) {
-                            sd[i][j][g][h] += (double)sf[i][j][g][h];
-                            sf[i][j][g][h] = 0.0f;
-                        }
-                }
+            __builtin_amdgcn_sched_barrier(0);
         }
+        // promote the word's FP32 partial sums
+#pragma unroll
+        for (int i = 0; i < PA; i++)
+#pragma unroll
+            for (int j = 0; j < PB; j++) {
+                if (!FAST) qd[i][j] += (double)qf[i][j];
+                qf[i][j] = 0.0f;
+#pragma unroll
+                for (int g = 0; g < NP; g++)
+#pragma unroll
+                    for (int h = 0; h < NP; h++) {
+                        sd[i][j][g][h] += (double)sf[i][j][g][h];
+                        sf[i][j][g][h] = 0.0f;
+                    }
+            }
+        __syncthreads();  // the next word is staged, this one read
     }
 
 #pragma unroll
     for (int i = 0; i < PA; i++) {
-        const int a = a0 + ty + 16 * i;
-        const Marg ma = P.marg[a < nsnp ? a : nsnp - 1];
+        const int a = a0 + PA * ty + i;
+        const Marg ma = P.marg[as[i]];
 #pragma unroll
         for (int j = 0; j < PB; j++) {
-            const int b = b0 + tx + 16 * j;
-            const Marg mb = P.marg[b < nsnp ? b : nsnp - 1];
+            const int b = b0 + PB * tx + j;
+            const Marg mb = P.marg[bs[j]];
             int xc[3][3];
             double xs[3][3];
             double sq;
@@ -193,7 +241,7 @@ __device__ __forceinline__ void plain_tile(const PlainScan &P, const HitSink &hs
 #pragma unroll
                     for (int h = 0; h < 2; h++) {
                         xc[g][h] = cnt[i][j][g][h];
-                        xs[g][h] = sd[i][j][g][h];
+                        xs[g][h] = sd[i][j][g][h] / PLAIN_SCALE;
                     }
                     xc[g][2] = ma.pn[g];
                     xs[g][2] = ma.ys[g];
@@ -209,9 +257,9 @@ __device__ __forceinline__ void plain_tile(const PlainScan &P, const HitSink &hs
 #pragma unroll
                     for (int h = 0; h < 3; h++) {
                         xc[g][h] = cnt[i][j][g % NP][h % NP];
-                        xs[g][h] = sd[i][j][g % NP][h % NP];
+                        xs[g][h] = sd[i][j][g % NP][h % NP] / PLAIN_SCALE;
                     }
-                sq = qd[i][j];
+                sq = qd[i][j] / PLAIN_SCALE;
             }
             int n[9];
             double s[9];
@@ -231,13 +279,14 @@ __device__ __forceinline__ void plain_tile(const PlainScan &P, const HitSink &hs
     }
 }
 
-template <int PA, int PB, bool FAST, bool DUMP>
-__global__ __launch_bounds__(256) void plain_kernel(const PlainArgs A)
+template <int NT, bool FAST, bool DUMP>
+__global__ __launch_bounds__(NT, FAST ? 4 : 2) void plain_kernel(const PlainArgs A)
 {
+    __shared__ PlainLds<FAST> lds;
     const int4 T = A.tiles[xcd_tile(blockIdx.x, A.ntiles)];
     HitSink hs = A.hs;
     hs.tag = A.S.tag;
-    plain_tile<PA, PB, FAST, DUMP>(A.S, hs, A.ds, T.x, T.y, T.z, T.w);
+    plain_tile<NT, FAST, DUMP>(A.S, hs, A.ds, T.x, T.y, T.z, T.w, lds);
 }
 
 }  // namespace epi
