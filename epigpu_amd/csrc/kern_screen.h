@@ -767,6 +767,31 @@ struct ResolveArgs {
     int group;                // lanes per candidate
 };
 
+// Sums of t over groups of G lanes, in all of them: within 16 lanes each addition takes its other operand from another
+// lane (DPP), beyond through LDS. Step by step for all values together, so that they hide each other's latency.
+// (Values one after the other, up to six dependent rounds through LDS each: 4,000 candidates with missing calls at N = 1237
+// 46 -> 21 us; 3,000 without at N = 500 18.5 -> 15.5 us, most of that the chain of loads and the FP64 statistics.)
+template <int NV>
+__device__ __forceinline__ void resolve_sum(int (&t)[NV], int G)
+{
+    auto add = [&](auto ctrl) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) t[i] += __builtin_amdgcn_mov_dpp(t[i], decltype(ctrl)::value, 0xF, 0xF, true);
+    };
+    using std::integral_constant;
+    add(integral_constant<int, 0xB1>{});                 // lane ^ 1
+    add(integral_constant<int, 0x4E>{});                 // lane ^ 2
+    if (G >= 8) add(integral_constant<int, 0x141>{});    // the other half of 8 lanes, mirrored
+    if (G >= 16) add(integral_constant<int, 0x140>{});   // the other half of 16 lanes, mirrored
+    for (int o = 16; o < G; o *= 2) {
+        int v[NV];
+#pragma unroll
+        for (int i = 0; i < NV; i++) v[i] = __shfl_xor(t[i], o);
+#pragma unroll
+        for (int i = 0; i < NV; i++) t[i] += v[i];
+    }
+}
+
 // GEN: pairs of tiles with missing calls (the classes 0, 1, NM of both SNPs and
 // the sum of z); otherwise classes 0 and 1 and the SNPs' marginals. G lanes
 // share a candidate (a power of two, 64 from 33 words on), so that a wave
@@ -844,11 +869,10 @@ __global__ __launch_bounds__(256) void resolve_kernel(const ResolveArgs A)
                     }
                 }
             }
+            resolve_sum<NV>(t, G);
 #pragma unroll
             for (int i = 0; i < NV; i++) {
-                int v = t[i];
-                for (int o = G >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o);
-                v = __shfl(v, (lane - u) * G);
+                const int v = G < 64 ? __shfl(t[i], (lane - u) * G) : t[i];
                 keep[i] = lane >= u && lane < u + step ? v : keep[i];
             }
         }
