@@ -14,7 +14,7 @@
 //     oidx, ocodes, ov     outlier individuals (at most OUT_MAX), their codes per SNP and values
 //     mp    [Kp]    MissPhen V, q, z per individual (SPARSE tiles), coarse phenotype v of the screen
 //     sw    [Kw][8], [Kw][16] uint32  the screen's FP6 codes of v (one and two digits) and presence bits, per
-//                   32 individuals (behind wts)
+//                   32 individuals (behind wts), then [3][Kp] int8, v in base-256 digits (marginals)
 //     sm    [nsnp]  ScrMarg per-SNP counts and sums of v (before marg, in its allocation)
 //   for SPARSE tiles (built at the first scan that has them, for the chromosome layout it was built for):
 //     moff  [nsnp+1] int64, mlist int32   per SNP, the individuals with a missing call
@@ -378,7 +378,7 @@ bool split_limbs(long long x, int n, int8_t *out)
 
 // Host-side encoding of one phenotype, before anything is allocated.
 struct PhenEnc {
-    std::vector<int8_t> w;      // [NWP][Kp], then the screen's weights (3 Kp bytes)
+    std::vector<int8_t> w;      // [NWP][Kp], then the screen's weights (3 Kp bytes) and [NWC][Kp]
     std::vector<int32_t> qv;    // [Kp]
     std::vector<float> yc;      // [Kp]
     std::vector<float> yw;      // [2][Kp]
@@ -608,7 +608,7 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
     int ye = 0;
     if (maxall > 0.0) std::frexp(maxall, &ye);
     const int Kw = Kp / 32;
-    e.w.assign((size_t)(NWP + 3) * Kp, 0);
+    e.w.assign((size_t)(NWP + 3 + NWC) * Kp, 0);
     e.qv.assign(Kp, 0);
     e.yc.assign(Kp, 0.0f);
     e.yw.assign((size_t)2 * Kp, 0.0f);
@@ -653,6 +653,13 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
         e.vb[k >> 5] |= 1u << (k & 31);
     }
     for (int nd : {1, 2}) encode_screen(P, Kp, nd, e);
+    int8_t *cw = e.w.data() + (size_t)(NWP + 3) * Kp;
+    for (int k : P) {
+        const int v = e.mp[k].sv[1], lo = (int8_t)(v & 255);
+        cw[k] = (int8_t)e.mp[k].sv[0];
+        cw[Kp + k] = (int8_t)lo;
+        cw[2 * (size_t)Kp + k] = (int8_t)((v - lo) / 256);
+    }
     for (int t = 0; t < p.nout; t++) {
         const double u = std::ldexp((double)y[e.oidx[t]] - centre, f);
         e.ov.d[t] = u;
@@ -768,7 +775,8 @@ int ds_marginals(epi_ctx *c, Dataset &d)
         p.marg = reinterpret_cast<Marg *>(p.sm + d.nsnp);
         hipLaunchKernelGGL(marginals_kernel, dim3((d.nsnp + 63) / 64), dim3(256), 0, c->stream,
                            (const uint32_t *)d.mbits, d.Kw, d.nsnp, (const uint32_t *)p.vbits, (const float *)p.yc,
-                           (const int32_t *)d.cls, (const MissPhen *)p.mp, p.marg, p.sm);
+                           (const int32_t *)d.cls, (const int8_t *)p.wts,
+                           (const int8_t *)(p.wts + (size_t)(NWP + 3) * d.Kp), p.marg, p.sm);
         HIPCHK(c, hipGetLastError());
         if (p.nout) {
             if ((rc = dalloc(c, p.ocodes, (size_t)(p.nout + 15) / 16 * d.nsnp))) return rc;

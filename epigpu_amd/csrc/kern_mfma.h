@@ -58,6 +58,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 constexpr int KC = 128;          // individuals per LDS stage
 constexpr int ROWB = KC + 16;    // LDS row pitch in bytes (bank-conflict padding)
 constexpr int NWP = 8;           // weight rows: V, L0, L1, L2, Z0, Z1, Z2, Z3
+constexpr int NWC = 3;           // weight rows of the screen's coarse phenotypes: one digit; two digits, base 256
 constexpr int OUT_MAX = 32;      // outlier individuals carried exactly, per phenotype
 
 // Identity class map: plane p holds class p (the MFMA form keeps genotype order).

@@ -113,12 +113,14 @@ __global__ __launch_bounds__(256) void order_planes_kernel(const uint32_t *mbits
 // phenotype sums of genotype classes 0, 1 and of all calls (NM), stored per
 // class for the MFMA form and per bitplane (cls order) for the plain form.
 // One workgroup per 64 SNPs: lane = SNP (coalesced bitplane loads), four
-// waves split the words and are reduced in LDS. Bounded by its VALU work, 35
-// instructions per individual and 64 SNPs: 0.10 ms at N = 2000, M = 20001 (0.22 ms
-// as a loop over each lane's own set bits, with gathered loads).
+// waves split the words and are reduced in LDS. The integer sums are 4 x 8-bit dot products of byte masks with
+// the limbs of q and z and the digits of v (the wave's, scalar loads), the sum of the plain form's FP32
+// phenotype an FP64 FMA with 0 or 1 per class. Bounded by its VALU work, 20 instructions per individual
+// and 64 SNPs: 0.045 ms at N = 2000, M = 20001 (0.10 ms with each value masked and added by itself,
+// 0.22 ms as a loop over each lane's own set bits, with gathered loads).
 __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, int Kw, int nsnp,
                                                         const uint32_t *vbits, const float *yc,
-                                                        const int32_t *cls, const MissPhen *mp,
+                                                        const int32_t *cls, const int8_t *wts, const int8_t *cw,
                                                         Marg *marg, ScrMarg *smarg)
 {
     __shared__ long long sq[4][3][64];
@@ -127,10 +129,9 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
     __shared__ long long sz[4][64];
     __shared__ int sv[4][2][3][64];
     const int sl = threadIdx.x & 63, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int s = blockIdx.x * 64 + sl, sc = s < nsnp ? s : nsnp - 1;
+    const int s = blockIdx.x * 64 + sl, sc = s < nsnp ? s : nsnp - 1, Kp = 32 * Kw;
     int n[3] = {0, 0, 0};
-    long long q[3] = {0, 0, 0}, z = 0;
-    int v3[2][3] = {};  // sums of the screen's coarse phenotypes (their magnitude stays below 2^24)
+    int t[3][6] = {}, tz[4] = {};  // limbs of q, v of one digit, digits of v of two; limbs of z (below 2^28)
     double y[3] = {0.0, 0.0, 0.0};
     for (int wd = grp; wd < Kw; wd += 4) {
         const uint32_t v = vbits[wd];
@@ -138,27 +139,50 @@ __global__ __launch_bounds__(256) void marginals_kernel(const uint32_t *mbits, i
         const uint32_t b1 = mbits[((size_t)1 * Kw + wd) * nsnp + sc] & v;
         const uint32_t bn = mbits[((size_t)2 * Kw + wd) * nsnp + sc] & v;
         const uint32_t m[3] = {b0, b1, bn & ~b0 & ~b1};
-        int q32[3] = {0, 0, 0};  // 32 |q| < 2^28
 #pragma unroll
         for (int c = 0; c < 3; c++) n[c] += __popc(m[c]);
-        // every individual of the word in turn: its values are the wave's (scalar loads), its bit is the lane's mask
-#pragma unroll 8
-        for (int j = 0; j < 32; j++) {
-            const MissPhen &e = mp[32 * wd + j];
-            const int eq = e.q, e0 = e.sv[0], e1 = e.sv[1], ey = __float_as_int(yc[32 * wd + j]);
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const int k = (int)(m[c] << (31 - j)) >> 31;
-                q32[c] += k & eq;
-                v3[0][c] += k & e0;
-                v3[1][c] += k & e1;
-                y[c] += (double)__int_as_float(k & ey);
+        for (int hf = 0; hf < 2; hf++) {  // 16 individuals
+            const int8_t *wp = wts + 32 * wd + 16 * hf, *cp = cw + 32 * wd + 16 * hf;
+            v4i e[3];
+#pragma unroll
+            for (int c = 0; c < 3; c++) e[c] = expand16<false>((m[c] >> (16 * hf)) & 0xFFFFu);
+#pragma unroll
+            for (int l = 0; l < 6; l++) {
+                const v4i w = *reinterpret_cast<const v4i *>(l < 3 ? wp + (size_t)(1 + l) * Kp : cp + (size_t)(l - 3) * Kp);
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+#pragma unroll
+                    for (int c = 0; c < 3; c++) t[c][l] = __builtin_amdgcn_sdot4(e[c][k], w[k], t[c][l], false);
             }
-            z += (int)(bn << (31 - j)) >> 31 & e.z;
-        }
+            const v4i en = e[0] | e[1] | e[2];
 #pragma unroll
-        for (int c = 0; c < 3; c++) q[c] += q32[c];
+            for (int l = 0; l < 4; l++) {
+                const v4i w = *reinterpret_cast<const v4i *>(wp + (size_t)(4 + l) * Kp);
+#pragma unroll
+                for (int k = 0; k < 4; k++) tz[l] = __builtin_amdgcn_sdot4(en[k], w[k], tz[l], false);
+            }
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                const double yd = (double)yc[32 * wd + 16 * hf + j];
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    int k = __builtin_amdgcn_sbfe((int)m[c], 16 * hf + j, 1);
+                    asm("" : "+v"(k));  // kept a mask (a compare and a select otherwise)
+                    y[c] = __builtin_fma(__hiloint2double(k & 0x3FF00000, 0), yd, y[c]);
+                }
+            }
+        }
     }
+    long long q[3], z;
+    int v3[2][3];  // sums of the screen's coarse phenotypes (their magnitude stays below 2^24)
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        q[c] = (long long)t[c][0] + 256ll * t[c][1] + 65536ll * t[c][2];
+        v3[0][c] = t[c][3];
+        v3[1][c] = t[c][4] + 256 * t[c][5];
+    }
+    z = (long long)tz[0] + 256ll * tz[1] + 65536ll * tz[2] + 16777216ll * tz[3];
     for (int c = 0; c < 3; c++) {
         sn[grp][c][sl] = n[c];
         sq[grp][c][sl] = q[c];
