@@ -27,7 +27,7 @@
 //
 // Bound: over a pair's complete cases let P y be the projection of a phenotype
 // onto the cell-constant vectors less the mean, so SSB(y) = |P y|^2. Then
-//     |P q| <= delta |P v| + |P r| <= delta |P v| + eps,   eps = |r - mean(r)|,
+//     |P q| <= delta |P v| + |P r| <= delta |P v| + eps,   eps = |r|,
 // and likewise sqrt(SSI(q)) <= delta sqrt(SSI(v)) + eps, since SSI(y) = |A y|^2 with A
 // linear and SSI <= SSB <= |y|^2 for every y. With SST the total sum of squares,
 //     F > t1   <=>  SSB > k1 SST,  k1 = t1 d1 / (d2 + t1 d1)
@@ -68,7 +68,7 @@ struct ScrMarg {
 struct ScreenCut {
     float N;              // complete cases / 64
     float thr0, slope2;   // level 0: sum s^2 / n > thr0 + 2 nfac slope2
-    float eps;            // |r - mean(r)| / (8 delta)
+    float eps;            // |r| / (8 delta)
     float sst;            // SST(q) / (64 delta^2)
     float nv;             // complete cases
     // GENERAL tiles: nv and N bound the pairs' complete cases from above
