@@ -1286,6 +1286,7 @@ bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
     C.kap0 = (float)((k9 - 9.0 * ks) - 1e-5 * std::fabs(k9 - 9.0 * ks));
     C.kslope2 = (float)(0.5 * ks);
     C.kroot = (float)(2.0 * E.eps * std::sqrt(kap(9, std::max(0.5 * N, 16.0)) * p.sqV) / unit * (1.0 + 1e-5));
+    C.vs = (float)(E.vsum / 64.0);
     C.zunit = (float)(std::ldexp(1.0, p.zbits) / unit * (1.0 - 1e-6));
     C.zall = (float)(p.zall * (1.0 + 1e-6));
     C.c0 = (float)(E.offset / E.delta);
@@ -1329,8 +1330,15 @@ int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind
         G.ntiles = chunk;
         G.tile0 = t0;
         if constexpr (GEN) {
-            if (G.cut.nd == 1) hipLaunchKernelGGL((screen_gen_kernel<TA, 1>), grid, block, 0, c->stream, G);
-            else hipLaunchKernelGGL((screen_gen_kernel<TA, 2>), grid, block, 0, c->stream, G);
+            constexpr bool NC = TA == 64;
+            const bool nocall = NC && scr_nocall(G.S.Kl);
+            if (G.cut.nd == 1) {
+                if (nocall) hipLaunchKernelGGL((screen_gen_kernel<TA, 1, NC>), grid, block, 0, c->stream, G);
+                else hipLaunchKernelGGL((screen_gen_kernel<TA, 1, false>), grid, block, 0, c->stream, G);
+            } else {
+                if (nocall) hipLaunchKernelGGL((screen_gen_kernel<TA, 2, NC>), grid, block, 0, c->stream, G);
+                else hipLaunchKernelGGL((screen_gen_kernel<TA, 2, false>), grid, block, 0, c->stream, G);
+            }
         } else {
             if (G.cut.nd == 1) hipLaunchKernelGGL((screen_fast_kernel<TA, 1>), grid, block, 0, c->stream, G);
             else hipLaunchKernelGGL((screen_fast_kernel<TA, 2>), grid, block, 0, c->stream, G);
@@ -1666,12 +1674,27 @@ const void *batch_kernel(int form, const epi_schedule &sc, int kind)
     return kind ? (const void *)plain_batch_kernel<256, 1> : (const void *)plain_batch_kernel<256, 0>;
 }
 
-const void *screen_batch_fn(const epi_schedule &sc, int kind)
+// Whether a batch's tiles with missing calls contract those: one answer for the list, that of most of its work.
+bool batch_nocall(const epi_batch *b)
 {
-    if (sc.fast_rows == 64)
-        return kind == 2 ? (const void *)screen_batch_kernel<64, 2>
-               : kind    ? (const void *)screen_batch_kernel<64, 1>
-                         : (const void *)screen_batch_kernel<64, 0>;
+    double large = 0.0, all = 0.0;
+    for (const auto &x : b->scans) {
+        const Dataset &d = *b->data[x.first];
+        if (!d.missum[d.nsnp]) continue;
+        const double w = (double)d.nsnp * d.nsnp * d.nid;
+        all += w;
+        if (scr_nocall((d.nid + KC - 1) / KC * KC)) large += w;
+    }
+    return 2.0 * large > all;
+}
+
+const void *screen_batch_fn(const epi_schedule &sc, int kind, bool nocall)
+{
+    if (sc.fast_rows == 64) {
+        if (kind == 2) return nocall ? (const void *)screen_batch_kernel<64, 2, true> : (const void *)screen_batch_kernel<64, 2>;
+        if (kind) return nocall ? (const void *)screen_batch_kernel<64, 1, true> : (const void *)screen_batch_kernel<64, 1>;
+        return (const void *)screen_batch_kernel<64, 0>;
+    }
     return kind == 2 ? (const void *)screen_batch_kernel<32, 2>
            : kind    ? (const void *)screen_batch_kernel<32, 1>
                      : (const void *)screen_batch_kernel<32, 0>;
@@ -1740,7 +1763,7 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
         B[kind].qpos = b->d_qpos + kind * NQ;
         B[kind].qend = b->d_qend + kind * NQ;
         B[kind].hs = make_sink(b->hits, b->nhits, b->cap, p);
-        kfn[kind] = screen[kind] ? screen_batch_fn(b->work_sched, kind) : batch_kernel(p->form, b->work_sched, kind);
+        kfn[kind] = screen[kind] ? screen_batch_fn(b->work_sched, kind, batch_nocall(b)) : batch_kernel(p->form, b->work_sched, kind);
         int per_cu = 1;
         HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn[kind], nt[kind], 0));
         grid[kind] = std::max(1, per_cu) * c->ncu;

@@ -122,13 +122,14 @@ __global__ __launch_bounds__((batch_threads<TA, KIND>()), (batch_waves_per_simd<
 
 // A list through the screen: one workgroup per item (two per SPARSE item), in the order of the list, with the XCD
 // mapping of single scans (a persistent grid that pulls from the queues measured 5 % more at N = 4000, M = 20000).
-// Tiles of scans that the screen does not take go to the redo list whole.
-template <int TA, int KIND>
+// Tiles of scans that the screen does not take go to the redo list whole. NC (screen_gen_tile) is one for the list: both
+// variants in one kernel cost 1.5 % at N = 2504.
+template <int TA, int KIND, bool NC = false>
 __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_batch_kernel(const ScreenBatchArgs B)
 {
     constexpr int HALVES = KIND == 2 ? 2 : 1, NW = HALVES * (TA / SCR_A);
     __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * sw_row<2>()];
-    __shared__ float4 mg[TA + 64];
+    __shared__ float4 mg[KIND ? 2 * (TA + 32) : TA + 64];
     __shared__ float2 mg2[TA];
     const int t = xcd_tile(blockIdx.x, B.nitems * HALVES), it = t / HALVES;
     const int4 w = B.work[it];
@@ -152,9 +153,9 @@ __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_batch_kernel(cons
     } else {
         if (!scr_half<TA>(t % HALVES, HALVES, (uint32_t)(B.item0 + it), b0, b1, region0)) return;
         if (C.nd == 1)
-            screen_gen_tile<TA, 1>(S, C, B.cs, a0, a1, b0, b1, region0, wl, reinterpret_cast<float *>(mg));
+            screen_gen_tile<TA, 1, NC>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg);
         else
-            screen_gen_tile<TA, 2>(S, C, B.cs, a0, a1, b0, b1, region0, wl, reinterpret_cast<float *>(mg));
+            screen_gen_tile<TA, 2, NC>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg);
     }
 }
 

@@ -72,6 +72,7 @@ struct ScreenCut {
     float sst;            // SST(q) / (64 delta^2)
     float nv;             // complete cases
     // GENERAL tiles: nv and N bound the pairs' complete cases from above
+    float vs;             // sum of v over the phenotypes present / 64
     float zunit, zall;    // sums of squares per unit of z (from below); sum of z over all individuals
     float kap0, kslope2;  // level 0: sum s^2 / n > (kap0 + 2 nfac kslope2) SST - kroot
     float kroot, c0;      // c0: q ~ delta (v + c0), scaled as v is
@@ -449,11 +450,15 @@ __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_fast_kernel(const
 
 // ------------------------------------------------------------- GENERAL ----
 // Tile TA a x 32 b with missing calls (a SPARSE tile, whose SNPs miss few calls, is two of them). Each
-// wave owns 16 a x 32 b and contracts the three classes of both sides with the count and the two
+// wave owns 16 a x 32 b and contracts three masks of both sides with the count and the two
 // digits: 27 v_mfma_f32_16x16x128_f8f6f4 per 16 x 16 pairs and 128 individuals (the exact tile: 40 INT8
 // MACs per pair and individual, here 27 at twice the rate). The 16 x 16 shape puts a pair's 18 accumulators
 // into one lane whatever the number of rows per a-SNP: row m of A is a-SNP m, one
 // block per class and weight; lane l holds column l % 16 and rows 4 (l / 16) + i. 144 accumulators.
+// The masks are the two rarest classes and, with NC, the missing calls (the commonest class's cells follow from
+// those and the SNPs' own sums: 36 more instructions a pair slot), otherwise the commonest class itself. Missing calls
+// are the sparser operand, and the matrix cores' power bounds the clock: from N = 3000 the scan gains (kernel time of
+// NC over not, 1 % missing calls: N = 500 1.09, 2000 1.03, 3000 0.99, 4000 0.97, 8000 0.95, 20000 0.92).
 // SST of a pair's complete cases is at least Z_a + Z_b - Z_all (Z the sums of q^2 over an
 // SNP's calls), less the mean's part, T^2 / N with T the sum of q: |T| / sqrt N <= delta |sum v| / sqrt N + eps.
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -467,9 +472,9 @@ __device__ __forceinline__ v4f scr_mfma16x32(const v8i &a, const v8i &b, const v
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 2, 0, 0x84848484, 0, 0x7f7f7f7f);
 }
 
-template <int TA, int ND>
+template <int TA, int ND, bool NC>
 __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenCut &C, const CandSink &cs, int a0, int a1,
-                                                int b0, int b1, uint32_t region0, uint32_t *wl, float *mz)
+                                                int b0, int b1, uint32_t region0, uint32_t *wl, float4 *mg)
 {
     constexpr int TB = 32, NT = scr_threads<TA>(), ROW = sw_row<ND>();
     const uint32_t *sw = S.sw[ND - 1];
@@ -479,10 +484,20 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
     const bool work = aw < a1 && (a1 < aw + SCR_A ? a1 : aw + SCR_A) - 1 > bw;
     const int Kw = S.Kp / 32, nw = S.Kl / 32;
 
+    float *mz = reinterpret_cast<float *>(mg);  // without NC: the sums of z alone
     for (int i = tid; i < TA + TB; i += NT) {
         int sn = i < TA ? a0 + i : b0 + i - TA;
         sn = sn < S.nsnp ? sn : S.nsnp - 1;
-        mz[i] = S.sm[sn].zs;
+        const ScrMarg &q = S.sm[sn];
+        if constexpr (!NC) {
+            mz[i] = q.zs;
+            continue;
+        }
+        const float *qs = q.s[ND - 1];
+        mg[i] = make_float4(q.n[0], q.n[1], qs[0], qs[1]);
+        // a: the commonest class; b: missing calls
+        mg[TA + TB + i] = i < TA ? make_float4(q.n[2], qs[2], q.zs, 0.0f)
+                                 : make_float4(C.N - q.n[0] - q.n[1] - q.n[2], C.vs - qs[0] - qs[1] - qs[2], q.zs, 0.0f);
     }
 
     v4f av[2][9], as[2][9];  // [b group][3 g + h]: counts, sums of v
@@ -526,8 +541,8 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
         for (int j = 0; j < 6; j++) xb[j] = __builtin_amdgcn_raw_buffer_load_b32(r[j >> 1], vb[j & 1], src, 0);
     };
     auto loadA = [&](int g) { xa[g] = __builtin_amdgcn_raw_buffer_load_b32(r[g], va, src, 0); };
-    // the word of B operand j = 2 h + b group; class 2 is the rest of the called individuals
-    auto word = [&](int j) { return j < 4 ? xb[j] : xb[j] & ~xb[j - 4] & ~xb[j - 2]; };
+    // the word of B operand j = 2 h + b group; h = 2: no call, or the commonest class (the rest of the called)
+    auto word = [&](int j) { return j < 4 ? xb[j] : NC ? ~xb[j] : xb[j] & ~xb[j - 4] & ~xb[j - 2]; };
     auto low = [&](const Fp6 &f, const Weights &w) {
         return scr_op({{f.d[0] & w.q0.x, f.d[1] & w.q0.y, f.d[2] & w.q0.z, f.d[3] & w.q0.w, f.d[4] & w.q1.x,
                         f.d[5] & w.q1.y}});
@@ -595,7 +610,7 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
                 }
 #pragma unroll
                 for (int j = 0; j < 6; j++) as[j & 1][3 * g + (j >> 1)] = scr_mfma16(A0, B[j], as[j & 1][3 * g + (j >> 1)]);
-                const Fp6 tn = scr_spread(gn == 2 ? xa[2] & ~a01 & w.v : xa[gn] & w.v);
+                const Fp6 tn = scr_spread(gn < 2 ? xa[gn] & w.v : NC ? ~xa[2] & w.v : xa[2] & ~a01 & w.v);
                 if (g == 2) {
                     loadA(1);
                     loadA(2);
@@ -636,18 +651,48 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
 
     // Lane: pairs a = aw + 4 kq + i, b = bw + 16 bg + m.
     uint32_t bits = 0;
+    float4 mb[2] = {}, mb2[2] = {};
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        if (NC) mb[j] = mg[TA + 16 * j + m], mb2[j] = mg[TA + TB + TA + 16 * j + m];
+        else mb2[j].z = mz[TA + 16 * j + m];
+    }
     static_for<8>([&](auto k) {
         constexpr int K = decltype(k)::value, i = K / 2, bg = K % 2;
-        float n[9], s[9], nc = 0.0f, tc = 0.0f;
+        const int ia = al + 4 * kq + i;
+        float4 ma = {}, ma2 = {};
+        if (NC) ma = mg[ia], ma2 = mg[TA + TB + ia];
+        else ma2.z = mz[ia];
+        float n[9], s[9];
+        // the table from the sums over {0, 1, no call}^2 and the SNPs' own; returns its total
+        auto fill = [&](float c[9], const v4f (&X)[9], float a_0, float a_1, float a_2, float b_0, float b_1, float b_m) {
+            c[0] = X[0][i];
+            c[1] = X[1][i];
+            c[3] = X[3][i];
+            c[4] = X[4][i];
+            c[2] = a_0 - c[0] - c[1] - X[2][i];
+            c[5] = a_1 - c[3] - c[4] - X[5][i];
+            c[6] = b_0 - c[0] - c[3] - X[6][i];
+            c[7] = b_1 - c[1] - c[4] - X[7][i];
+            const float lost = b_m - X[8][i];  // called in a, not in b
+            c[8] = a_2 - c[6] - c[7] - (lost - X[2][i] - X[5][i]);
+            return a_0 + a_1 + a_2 - lost;
+        };
+        float nc = 0.0f, tc = 0.0f;
+        if constexpr (NC) {
+            nc = fill(n, av[bg], ma.x, ma.y, ma2.x, mb[bg].x, mb[bg].y, mb2[bg].x);
+            tc = fill(s, as[bg], ma.z, ma.w, ma2.y, mb[bg].z, mb[bg].w, mb2[bg].y);
+        } else {
 #pragma unroll
-        for (int c = 0; c < 9; c++) {
-            n[c] = av[bg][c][i];
-            s[c] = as[bg][c][i];
-            nc += n[c];
-            tc += s[c];
+            for (int c = 0; c < 9; c++) {
+                n[c] = av[bg][c][i];
+                s[c] = as[bg][c][i];
+                nc += n[c];
+                tc += s[c];
+            }
         }
         tc = __builtin_fmaf(C.c0, nc, tc);
-        const float zlow = mz[al + 4 * kq + i] + mz[TA + 16 * bg + m] - C.zall;
+        const float zlow = ma2.z + mb2[bg].z - C.zall;
         float u = 0.0f;
 #pragma unroll
         for (int c = 0; c < 9; c++) u = __builtin_fmaf(s[c] * s[c], rcp_above(n[c]), u);
@@ -670,6 +715,9 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
     });
 }
 
+// Whether a scan of Kl individuals (a multiple of 128) contracts the missing calls. Only with 64-row tiles.
+__host__ __device__ constexpr bool scr_nocall(int Kl) { return Kl >= 3000; }
+
 // The workgroup's half of 32 b (or the whole) of a tile: b range and first region. False: no b-SNPs.
 template <int TA>
 __device__ __forceinline__ bool scr_half(int h, int halves, uint32_t tile, int &b0, int &b1, uint32_t &region0)
@@ -681,16 +729,16 @@ __device__ __forceinline__ bool scr_half(int h, int halves, uint32_t tile, int &
     return any;
 }
 
-template <int TA, int ND>
+template <int TA, int ND, bool NC>
 __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_gen_kernel(const ScreenArgs A)
 {
     __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * sw_row<ND>()];
-    __shared__ float mz[TA + 32];
+    __shared__ float4 mg[2 * (TA + 32)];
     const int t = xcd_tile(blockIdx.x, A.ntiles * A.halves);
     int4 T = A.tiles[t / A.halves];
     uint32_t region0;
     if (!scr_half<TA>(t % A.halves, A.halves, (uint32_t)(A.tile0 + t / A.halves), T.z, T.w, region0)) return;
-    screen_gen_tile<TA, ND>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, region0, wl, mz);
+    screen_gen_tile<TA, ND, NC>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, region0, wl, mg);
 }
 
 // --------------------------------------------------------------- redo ----
