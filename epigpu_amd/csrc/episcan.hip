@@ -3,6 +3,7 @@
 // Device state of one dataset (a context holds one; a batch holds many):
 //   words   [nsnp][npack1] int32   genotypes as uploaded (layout A1), freed after the transcode
 //   mbits   [3][Kw][nsnp]  uint32  bitplanes of classes 0, 1 and call present (MFMA form)
+//   sbits   [3][nsnp][Kw]  uint32  the same by SNP (resolve kernel), or null
 //   bits    [3][Kw][nsnp]  uint32  bitplanes of the two rarest classes and call present (plain form)
 //   cls     [nsnp]         int32   plain-form plane -> class map
 //   per phenotype r (wts, mp, yc, yw, vbits, ov and oidx in one allocation):
@@ -104,6 +105,7 @@ struct Dataset {
     int nid = 0, nsnp = 0, npack1 = 0, Kp = 0, Kw = 0;
     int32_t *words = nullptr;
     uint32_t *mbits = nullptr;
+    uint32_t *sbits = nullptr;  // behind mbits
     uint32_t *bits = nullptr;
     int32_t *dmiss = nullptr;
     int32_t *cls = nullptr;
@@ -283,6 +285,7 @@ void free_dataset(Dataset &d)
 {
     dfree(d.words);
     dfree(d.mbits);
+    d.sbits = nullptr;
     dfree(d.bits);
     dfree(d.dmiss);
     dfree(d.cls);
@@ -304,6 +307,9 @@ int sparse_max(int nid) { return std::min(65535, std::max(8, nid / 16)); }
 // (0.5 %: 17.7 ms against 20.5 ms for the scan; 1 %: 24.7 against 20.5).
 constexpr long long SPARSE_RATE = 150;
 
+// Two bitplanes below 4 GiB, as the screen's buffer descriptors take them.
+bool planes_fit(const Dataset &d) { return (unsigned long long)d.Kw * d.nsnp * 8ull < (1ull << 32) - (1u << 20); }
+
 int ds_upload_genotypes(epi_ctx *c, Dataset &d, const int32_t *words, int nid, int nsnp)
 {
     if (!d.ph.empty() && nid != d.nid) drop_phenotypes(d);  // a new cohort: the old phenotypes no longer apply
@@ -315,7 +321,19 @@ int ds_upload_genotypes(epi_ctx *c, Dataset &d, const int32_t *words, int nid, i
     d.Kw = d.Kp / 32;
     size_t nwords = (size_t)nsnp * d.npack1;
     int rc;
-    if ((rc = dalloc(c, d.words, nwords)) || (rc = dalloc(c, d.mbits, (size_t)3 * d.Kw * nsnp)) ||
+    // Bits by SNP, where the screen can run and memory allows (scans without it take the exact tiles): the lanes of the resolve kernel, one word each,
+    // then read a SNP's words in a row (N = 3001, 67,000 hits: resolve 250 -> 156 us; N = 2000: 84 -> 42 us).
+    const size_t planes = (size_t)3 * d.Kw * nsnp;
+    dfree(d.mbits);
+    d.sbits = nullptr;
+    if (planes_fit(d) && hipMalloc((void **)&d.mbits, 2 * planes * sizeof(uint32_t)) == hipSuccess) {
+        d.sbits = d.mbits + planes;
+    } else {
+        d.mbits = nullptr;
+        (void)hipGetLastError();
+        if ((rc = dalloc(c, d.mbits, planes))) return rc;
+    }
+    if ((rc = dalloc(c, d.words, nwords)) ||
         (rc = dalloc(c, d.bits, (size_t)3 * d.Kw * nsnp)) || (rc = dalloc(c, d.dmiss, (size_t)4 * nsnp)) ||
         (rc = dalloc(c, d.cls, (size_t)nsnp)))
         return rc;
@@ -323,7 +341,8 @@ int ds_upload_genotypes(epi_ctx *c, Dataset &d, const int32_t *words, int nid, i
     int *cnt = d.dmiss + nsnp;  // class counts of the SNPs
     HIPCHK(c, hipMemsetAsync(cnt, 0, 3 * (size_t)nsnp * sizeof(int), c->stream));
     hipLaunchKernelGGL(transcode_kernel, dim3((nsnp + TR_SNP - 1) / TR_SNP, (d.Kw + TR_WD - 1) / TR_WD), dim3(256), 0,
-                       c->stream, (const uint32_t *)d.words, nid, d.npack1, nsnp, d.Kw, d.mbits, cnt);
+                       c->stream, (const uint32_t *)d.words, nid, d.npack1, nsnp, d.Kw, d.mbits, d.sbits,
+                       cnt);
     HIPCHK(c, hipGetLastError());
     hipLaunchKernelGGL(order_planes_kernel, dim3((nsnp + 255) / 256, (d.Kw + 3) / 4), dim3(256), 0, c->stream,
                        (const uint32_t *)d.mbits, (const int *)cnt, nid, nsnp, d.Kw, d.bits, d.cls, d.dmiss);
@@ -878,6 +897,7 @@ MfmaScan mfma_scan(const Dataset &d, int r, int tag)
     const PhenDev &p = d.ph[r];
     MfmaScan S;
     S.bits = d.mbits;
+    S.sbits = d.sbits;
     S.wts = p.wts;
     S.marg = p.marg;
     S.nsnp = d.nsnp;
@@ -1293,12 +1313,11 @@ bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
     return true;
 }
 
-// The screen's 32-bit offsets reach two bitplanes, and GENERAL tiles bound SST well up to an eighth of the
-// calls missing.
+// The screen's 32-bit offsets reach two bitplanes (planes_fit; the resolve kernel's copy of them exists only then), and
+// GENERAL tiles bound SST well up to an eighth of the calls missing.
 bool screen_fits(const Dataset &d)
 {
-    return (unsigned long long)d.Kw * d.nsnp * 8ull < (1ull << 32) - (1u << 20) &&
-           d.missum[d.nsnp] <= (long long)d.nsnp * d.nid / 8;
+    return d.sbits && d.missum[d.nsnp] <= (long long)d.nsnp * d.nid / 8;
 }
 
 // One kind of tile through the screen. tiles: the kind's list on the device.

@@ -866,19 +866,18 @@ __global__ __launch_bounds__(256) void resolve_kernel(const ResolveArgs A)
             const MfmaScan &S = BATCH ? A.scans[__shfl(mine.z, c)] : A.S;
             const bool on = c < m && a != b;
             const int Kw = S.Kp / 32, nw = on ? S.Kl / 32 : 0;
-            const size_t plane = (size_t)Kw * S.nsnp;
+            const size_t plane = (size_t)Kw * S.nsnp, oa = (size_t)a * Kw, ob = (size_t)b * Kw;
             int t[NV];
 #pragma unroll
             for (int i = 0; i < NV; i++) t[i] = 0;
             for (int w = gl; w < nw; w += G) {
-                const size_t o = (size_t)w * S.nsnp;
                 uint32_t x[NX];
                 {
                     uint32_t ga[NG], hb[NG];
 #pragma unroll
                     for (int g = 0; g < NG; g++) {
-                        ga[g] = S.bits[g * plane + o + a];
-                        hb[g] = S.bits[g * plane + o + b];
+                        ga[g] = S.sbits[g * plane + oa + w];
+                        hb[g] = S.sbits[g * plane + ob + w];
                     }
 #pragma unroll
                     for (int g = 0; g < NG; g++)
