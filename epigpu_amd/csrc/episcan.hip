@@ -1239,7 +1239,7 @@ double chi2_tail(double x, int h)
 // missing calls: N = 1500, test i, rate 8e-5: 1.35 ms against 1.57 ms with two digits; N = 3000, test f, 4e-4:
 // 2.34 against 2.52, but with 1 % missing calls 5.38 against 5.37; N = 3000, test i, 7e-4: 3.02 against 2.64).
 constexpr double SCR_RATE1 = 2.5e-4, SCR_RATE2 = 2e-3;
-// Pairs times individuals below which the screen's two further launches cost more than its
+// Pairs times individuals below which the screen's further launches (measured with two) cost more than its
 // kernel saves (N = 1000, M = 1000: 20.5 us either way; N = 300, M = 2000: 25.9 us exact, 18.0 us screened).
 constexpr double SCR_MIN_WORK = 5e8;
 
