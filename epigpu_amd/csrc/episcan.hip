@@ -1237,7 +1237,7 @@ double chi2_tail(double x, int h)
 // unrelated SNPs would be candidates. One digit (two thirds of the MFMAs) where SCR_RATE1 holds with it: its
 // larger residue sends more pairs to the second stage and to the resolve kernel (M = 20000, normal phenotype, no
 // missing calls: N = 1500, test i, rate 8e-5: 1.35 ms against 1.57 ms with two digits; N = 3000, test f, 4e-4:
-// 2.34 against 2.52, but with 1 % missing calls 5.38 against 5.37; N = 3000, test i, 7e-4: 3.02 against 2.64).
+// 0.87-0.96 of two digits by phenotype, but with 1 % missing calls 0.91-1.03; N = 3000, test i, 7e-4: 3.02 against 2.64).
 constexpr double SCR_RATE1 = 2.5e-4, SCR_RATE2 = 2e-3;
 // Pairs times individuals below which the screen's further launches (measured with two) cost more than its
 // kernel saves (N = 1000, M = 1000: 20.5 us either way; N = 300, M = 2000: 25.9 us exact, 18.0 us screened).
