@@ -166,6 +166,8 @@ struct epi_ctx {
     long long last_pairs = 0;
     int last_launches = 0;
     long long last_tiles[3] = {0, 0, 0};  // FAST, SPARSE, GENERAL tiles of the last scan
+    int last_digits = 0;                  // of the screen in the last scan; 0: not screened
+    long long last_cand = 0, last_redone = 0;
     epi_schedule sched[2];  // per form
     void *scratch = nullptr;  // this device's no-allocation scratch (address from hipGetSymbolAddress)
 };
@@ -202,6 +204,9 @@ struct epi_batch {
     // results
     long long last_nhits = 0;
     double last_ms = 0.0;
+    int gscreened = 0;  // scans that the captured graph screens
+    int last_screened = 0;
+    long long last_cand = 0, last_redone = 0;
     bool fetched = false;
     std::vector<DevHit> hh;
     std::vector<std::vector<int>> by_scan;
@@ -1653,6 +1658,16 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     return EPI_OK;
 }
 
+// The hit counter and, behind it, the screen's counters (candidates and regions to redo of each tile kind), as one
+// copy reads them.
+struct Counters {
+    unsigned long long nhits;
+    uint32_t screen[2 * NKIND];
+    long long candidates() const { return (long long)screen[0] + screen[2] + screen[4]; }
+    long long redone() const { return (long long)screen[1] + screen[3] + screen[5]; }
+};
+static_assert(sizeof(Counters) == 4 * sizeof(unsigned long long), "the counters of a context or a batch");
+
 bool same_key(const epi_scan_params &x, const epi_scan_params &y)
 {
     return x.test == y.test && x.form == y.form && x.t1 == y.t1 && x.t2 == y.t2 && (x.safe != 0) == (y.safe != 0);
@@ -1826,6 +1841,9 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
     HIPCHK(c, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
     b->gkey = *p;
     b->gvalid = true;
+    b->gscreened = 0;
+    if (cut)
+        for (const ScreenCut &x : *cut) b->gscreened += x.nd != 0;
     b->grid = 0;
     for (int kind = 0; kind < NKIND; kind++)
         if (b->nkind[kind]) b->grid = std::max(b->grid, grid[kind]);
@@ -1863,13 +1881,16 @@ int batch_run(epi_batch *b, double *ms_out)
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     HIPCHK(c, hipGraphLaunch(b->exec, c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-    unsigned long long nh = 0;
-    HIPCHK(c, hipMemcpyAsync(&nh, b->nhits, sizeof(nh), hipMemcpyDeviceToHost, c->stream));
+    Counters n;
+    HIPCHK(c, hipMemcpyAsync(&n, b->nhits, sizeof(n), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     float ms = 0.0f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     b->last_ms = ms;
-    b->last_nhits = (long long)nh;
+    b->last_nhits = (long long)n.nhits;
+    b->last_screened = b->gscreened;
+    b->last_cand = n.candidates();
+    b->last_redone = n.redone();
     b->fetched = false;
     if (ms_out) *ms_out = ms;
     return EPI_OK;
@@ -1936,13 +1957,10 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     long long pairs = tl.pairs;
     c->last_tiles[0] = c->last_tiles[1] = c->last_tiles[2] = 0;
+    c->last_digits = screen ? cut.nd : 0;
+    c->last_cand = c->last_redone = 0;
     int launches = 0;
-    // the hit counter and, behind it, the screen's counters
-    struct Counters {
-        unsigned long long nhits;
-        uint32_t screen[6];
-    } n;
-    static_assert(sizeof(n) == 4 * sizeof(unsigned long long), "the counters of a context");
+    Counters n;
     for (;;) {
         if ((rc = launch_pairs<false>(c, p, sc, tl, ds, ctx_bufs(c), screen ? &cut : nullptr))) return rc;
         launches += c->last_launches;
@@ -1950,7 +1968,9 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
         // the launched kernels read the device tile list that the next piece overwrites
         HIPCHK(c, hipMemcpyAsync(&n, c->nhits, sizeof(n), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        if (n.screen[1] | n.screen[3] | n.screen[5]) {
+        c->last_cand += n.candidates();
+        c->last_redone += n.redone();
+        if (n.redone()) {
             // few scans have regions to redo: launched for every kind in every scan, N = 500, M = 2000 took 102.7 us, not 100.6
             if ((rc = launch_pairs<false>(c, p, sc, tl, ds, ctx_bufs(c), &cut, n.screen))) return rc;
             launches += c->last_launches;
@@ -2374,6 +2394,15 @@ int epi_last_tiles(epi_ctx *c, int64_t *fast, int64_t *sparse, int64_t *general)
     return EPI_OK;
 }
 
+int epi_last_screen(epi_ctx *c, int32_t *digits, int64_t *candidates, int64_t *redone)
+{
+    if (!c) return EPI_ERR_ARG;
+    if (digits) *digits = c->last_digits;
+    if (candidates) *candidates = c->last_cand;
+    if (redone) *redone = c->last_redone;
+    return EPI_OK;
+}
+
 int epi_pair_dump(epi_ctx *c, const epi_scan_params *p, int32_t a0, int32_t a1, int32_t b0, int32_t b1,
                   int32_t *counts, double *sums, double *F, double *F2)
 {
@@ -2665,6 +2694,15 @@ int epi_batch_stats(epi_batch *b, double *kernel_ms, int64_t *pairs, int64_t *ti
     if (pairs) *pairs = b->pairs;
     if (tiles) *tiles = b->nwork;
     if (captures) *captures = b->captures;
+    return EPI_OK;
+}
+
+int epi_batch_last_screen(epi_batch *b, int32_t *scans, int64_t *candidates, int64_t *redone)
+{
+    if (!b) return EPI_ERR_ARG;
+    if (scans) *scans = b->last_screened;
+    if (candidates) *candidates = b->last_cand;
+    if (redone) *redone = b->last_redone;
     return EPI_OK;
 }
 

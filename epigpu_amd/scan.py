@@ -156,6 +156,8 @@ def _declare(name, L):
             "epi_set_hit_capacity": (ctypes.c_int, [vp, i64]),
             "epi_last_scan_stats": (ctypes.c_int, [vp, _p(f64), _p(i64), _p(i32)]),
             "epi_last_tiles": (ctypes.c_int, [vp, _p(i64), _p(i64), _p(i64)]),
+            "epi_last_screen": (ctypes.c_int, [vp, _p(i32), _p(i64), _p(i64)]),
+            "epi_batch_last_screen": (ctypes.c_int, [vp, _p(i32), _p(i64), _p(i64)]),
             "epi_pair_dump": (ctypes.c_int, [vp, _p(ScanParams), i32, i32, i32, i32, vp, vp, vp, vp]),
             "epi_batch_create": (ctypes.c_int, [vp, _p(vp)]),
             "epi_batch_destroy": (None, [vp]),
@@ -673,6 +675,13 @@ class Scanner:
                   "epi_last_tiles")
         return {"fast": f.value, "sparse": sp.value, "general": g.value}
 
+    def last_screen(self):
+        """What the screen did in the last scan: digits (0: not screened), candidates and redone regions."""
+        d, c, r = ctypes.c_int32(), ctypes.c_int64(), ctypes.c_int64()
+        self._chk(self.L.epi_last_screen(self.ctx, ctypes.byref(d), ctypes.byref(c), ctypes.byref(r)),
+                  "epi_last_screen")
+        return {"digits": d.value, "candidates": c.value, "redone": r.value}
+
     def scan_noalloc(self, hits_dev, cap, test="f", form="mfma", t1=6.5, t2=10.5, phen=0, blk_begin=0, blk_end=0,
                      safe=False):
         """epi_scan_noalloc: hits (HIT64_DTYPE records, unsorted) into the device buffer at address hits_dev of
@@ -768,6 +777,13 @@ class Batch:
         n, ovf = self.hit_count(-1)
         return {"kernel_ms": ms.value, "pairs": pairs.value, "tiles": tiles.value, "captures": cap.value,
                 "grid": grid.value, "nhits": n, "overflow": ovf}
+
+    def last_screen(self):
+        """What the screen did in the last scan of the batch: screened scans, candidates and redone regions."""
+        s, c, r = ctypes.c_int32(), ctypes.c_int64(), ctypes.c_int64()
+        self._chk(self.L.epi_batch_last_screen(self.b, ctypes.byref(s), ctypes.byref(c), ctypes.byref(r)),
+                  "epi_batch_last_screen")
+        return {"scans": s.value, "candidates": c.value, "redone": r.value}
 
     def schedule(self, form="mfma"):
         sc = Schedule()

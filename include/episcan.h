@@ -255,6 +255,13 @@ int epi_last_scan_stats(epi_ctx *ctx, double *kernel_ms, int64_t *pairs, int32_t
  * reference; for tests and measurement. */
 int epi_last_tiles(epi_ctx *ctx, int64_t *fast, int64_t *sparse, int64_t *general);
 
+/* What the screen (see epi_schedule) did in the last epi_scan: the digits of
+ * its coarse phenotype (1 or 2; 0: the scan was not screened), the pairs that
+ * it kept one by one and that were then computed exactly (candidates), and the
+ * regions of tiles that exact tiles redid. No counterpart in the reference; for
+ * tests and measurement. */
+int epi_last_screen(epi_ctx *ctx, int32_t *digits, int64_t *candidates, int64_t *redone);
+
 /* Debug / parity entry: every pair (a, b) with a0 <= a < a1, b0 <= b < b1 and
  * a > b, through the same kernels as epi_scan, writes its 3x3 table and FP64
  * statistics into dense arrays indexed p = (a-a0)*(b1-b0) + (b-b0):
@@ -319,6 +326,10 @@ int epi_batch_get_hits(epi_batch *batch, int32_t scan, epi_hit *hits, double *F6
  * far and the persistent grid (workgroups) of the last capture. */
 int epi_batch_stats(epi_batch *batch, double *kernel_ms, int64_t *pairs, int64_t *tiles,
                     int32_t *captures, int32_t *grid);
+
+/* As epi_last_screen, for the last epi_batch_scan: how many of its scans were
+ * screened, and the candidates and redone regions of all of them. */
+int epi_batch_last_screen(epi_batch *batch, int32_t *scans, int64_t *candidates, int64_t *redone);
 
 /* Schedule of the batch's scans of one form (defaults as epi_set_schedule,
  * 8 queues, locality order). */
