@@ -1402,6 +1402,7 @@ int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, c
     if (tl.count() > (size_t)INT32_MAX)
         return fail(c, EPI_ERR_RANGE, "a super-tile row of this scan exceeds 2^31 tiles");
     const int nf = (int)tl.fast.size(), ns = (int)tl.sp.size(), ng = (int)tl.gen.size();
+    if (tl.count() > SCR_TILES) cut = nullptr;  // one row of super-tiles beyond what the screen can number
     c->last_launches = 0;
     if (!counts) {
         c->last_tiles[0] += nf;
@@ -1771,7 +1772,7 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
 {
     epi_ctx *c = b->ctx;
     drop_graph(b);
-    if (b->nwork >= (1ll << 28)) cut = nullptr;  // regions are numbered in 31 bits
+    if (b->nwork > (long long)SCR_TILES) cut = nullptr;
     if (cut) {
         HIPCHK(c, hipMemcpyAsync(b->d_cut, cut->data(), cut->size() * sizeof(ScreenCut), hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1931,8 +1932,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
     const bool screen = screened(c->d, p, block_pairs(c->d, bb, be), cut);
     epi_schedule sc = asked;
     if (screen) sc.fast_rows = screen_rows(c->d.nid);
-    // a screened list takes as much room again for its regions, within the same bound
-    const size_t max_tiles = screen ? std::max<size_t>(1, c->max_tiles / 2) : c->max_tiles;
+    const size_t max_tiles = screen ? scr_piece(c->max_tiles) : c->max_tiles;
     TileLists &tl = c->tl;
     const bool cached =
         c->tl_valid && c->tl_bb == bb && c->tl_be == be && c->tl_form == p->form && same_schedule(c->tl_sched, sc);

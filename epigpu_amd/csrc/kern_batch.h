@@ -127,7 +127,7 @@ __global__ __launch_bounds__((batch_threads<TA, KIND>()), (batch_waves_per_simd<
 template <int TA, int KIND, bool NC = false>
 __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_batch_kernel(const ScreenBatchArgs B)
 {
-    constexpr int HALVES = KIND == 2 ? 2 : 1, NW = HALVES * (TA / SCR_A);
+    constexpr int HALVES = KIND == 2 ? 2 : 1, NW = scr_regions(TA, KIND == 1 ? 32 : 64, KIND != 0);
     __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * sw_row<2>()];
     __shared__ float4 mg[KIND ? 2 * (TA + 32) : TA + 64];
     __shared__ float2 mg2[TA];

@@ -40,6 +40,7 @@
 #pragma once
 
 #include "kern_mfma.h"
+#include "screen_rules.h"
 
 namespace epi {
 
@@ -52,7 +53,6 @@ constexpr int sw_row() { return 8 * ND; }
 constexpr int SCR_WIN = 512; // words (of 32 individuals) of weights in LDS at a time
 constexpr int SCR_LDS_ROWS = SCR_WIN + 2;  // the pipeline reads one step past the window
 constexpr int SCR_GEN_ROWS = SCR_WIN + 4;
-constexpr int SCR_A = 16;    // a-SNPs per wave
 template <int TA>
 constexpr int scr_threads() { return 64 * TA / SCR_A; }  // a workgroup takes a tile of TA = 32 or 64 a-SNPs
 constexpr int SCR_REDO = 8;   // candidates per pair slot of a wave (64 pairs) above which the exact tile redoes its region
@@ -745,8 +745,6 @@ __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_gen_kernel(const 
 // Regions that the screen handed back, and tiles of scans that it does not take (SCR_WHOLE),
 // through the exact tiles of 32 rows: a persistent grid over the device's count of them. Region r of a TA x TB
 // tile is block r % NW (a block r % NWA, b block r % NW / NWA) of tile r / NW.
-constexpr uint32_t SCR_WHOLE = 1u << 31;
-
 struct RedoArgs {
     MfmaScan S;               // single scans
     const MfmaScan *scans;    // batches: by scan id
@@ -760,7 +758,7 @@ template <int TA, int TB, bool GEN, bool BATCH>
 __global__ __launch_bounds__(256, 2) void redo_kernel(const RedoArgs A)
 {
     static_assert(fast_threads<32>() == 256 && general_threads<32>() == 256, "threads of the 32-row tiles");
-    constexpr int RB = GEN ? 32 : 64, NWA = TA / SCR_A, NW = NWA * (TB / RB);
+    constexpr int RB = GEN ? 32 : 64, NWA = TA / SCR_A, NW = scr_regions(TA, TB, GEN);
     __shared__ __attribute__((aligned(16))) uint8_t lds[GEN ? general_lds<32>() : fast_lds<32>()];
     const uint32_t n = A.count[1];
     const DumpSink nodump = {};

@@ -1,0 +1,48 @@
+"""Limits of the screened scans, on the CPU: a C++ program that includes epigpu_amd/csrc/screen_rules.h (no HIP)
+checks them at the ends of their ranges. No GPU is used."""
+import os
+import subprocess
+
+from conftest import ROOT
+
+PROGRAM = r"""
+#include "screen_rules.h"
+#include <cstdio>
+#include <initializer_list>
+using namespace epi;
+static int bad = 0;
+#define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); bad = 1; } } while (0)
+
+int main()
+{
+    // a region's number leads back to its tile and stays below the bit of whole tiles, up to the longest list
+    for (int TA : {32, 64})
+        for (int kind = 0; kind < 3; kind++) {
+            const uint64_t n = scr_regions(TA, kind == 1 ? 32 : 64, kind != 0);
+            CHECK(n >= 2 && n <= 8);
+            for (uint64_t tile : {(uint64_t)0, (uint64_t)SCR_TILES / 2, (uint64_t)SCR_TILES - 1})
+                for (uint64_t k = 0; k < n; k++) {
+                    const uint64_t r = tile * n + k;
+                    CHECK(r < SCR_WHOLE);
+                    CHECK((uint32_t)r / n == tile && (uint32_t)r % n == k);
+                }
+        }
+    // every bound that epi_set_max_tiles takes: a piece stays below the longest list with as much room to spare
+    for (uint64_t m : {(uint64_t)1, (uint64_t)2, (uint64_t)3, (uint64_t)1 << 25, (uint64_t)1 << 28, ((uint64_t)1 << 30) - 1}) {
+        CHECK(scr_piece(m) >= 1 && (scr_piece(m) <= m / 2 || m < 2));
+        CHECK(2 * (uint64_t)scr_piece(m) <= SCR_TILES);
+    }
+    CHECK(scr_piece((uint64_t)1 << 25) == (uint64_t)1 << 24);
+    return bad;
+}
+"""
+
+
+def test_limits(tmp_path):
+    src = tmp_path / "rules.cpp"
+    src.write_text(PROGRAM)
+    exe = tmp_path / "rules"
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I" + os.path.join(ROOT, "epigpu_amd", "csrc"), str(src),
+                    "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
