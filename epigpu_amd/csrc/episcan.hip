@@ -27,6 +27,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -145,11 +146,10 @@ struct epi_ctx {
     Dataset d;
     // hits
     DevHit *hits = nullptr;
-    unsigned long long *nhits = nullptr;
     long long cap = 1ll << 22;
     long long last_nhits = 0;
-    // screened scans: counters (behind nhits), candidates, regions to redo (behind the tiles)
-    uint32_t *scount = nullptr;
+    // counters of the hits and of the screen; candidates; regions to redo (behind the tiles)
+    Counters *count = nullptr;
     int4 *cand = nullptr;
     uint32_t *redo = nullptr;
     // tiles; the device list of the last scan is kept and reused while the
@@ -179,14 +179,14 @@ struct epi_batch {
     MfmaScan *d_mscan = nullptr;
     PlainScan *d_pscan = nullptr;
     ScreenCut *d_cut = nullptr;
-    uint32_t *scount = nullptr;  // the screen's counters, behind nhits: two per tile kind
     uint32_t *redo = nullptr;    // behind the work items
     int4 *d_work = nullptr;
     int *d_qpos = nullptr, *d_qbegin = nullptr, *d_qend = nullptr;  // [NKIND][NQ]: FAST, GENERAL, SPARSE items
     size_t work_cap = 0, scan_cap = 0;
     long long nkind[NKIND] = {0, 0, 0};  // work items of each tile kind (FAST first in d_work)
+    std::vector<std::pair<int, long long>> segs[NKIND];  // the datasets of a list, in its order, and their items
     DevHit *hits = nullptr;
-    unsigned long long *nhits = nullptr;
+    Counters *count = nullptr;
     long long cap = 1ll << 22;
     // work list of the last build
     epi_schedule sched[2];  // per form
@@ -1211,13 +1211,12 @@ struct ScanBufs {
     unsigned long long *nhits;
     long long cap;
     CandSink cs;
+    unsigned long long *emptied;
 };
-
-constexpr uint32_t CAND_CAP = 1u << 20;  // 16 MiB of candidates; beyond it regions are redone by the exact tiles
 
 ScanBufs ctx_bufs(const epi_ctx *c)
 {
-    return {c->tiles, c->hits, c->nhits, c->cap, {c->cand, c->scount, CAND_CAP, c->redo}};
+    return {c->tiles, c->hits, &c->count->nhits, c->cap, {c->cand, c->count->screen, CAND_CAP, c->redo}, &c->count->emptied};
 }
 
 // Lanes per candidate of resolve_kernel for a cohort of Kl individuals (one 32-individual word each).
@@ -1268,11 +1267,12 @@ bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
     };
     auto kap = [&](int nfac, double n) { return inter ? std::min(k1(nfac, n), k2(nfac, n)) : k1(nfac, n); };
     int nd = 0;
+    double rate = 0.0;
     for (int i = 1; i <= 2 && !nd; i++) {
         const ScreenEnc &E = p.scr[i - 1];
         if (!(E.delta > 0.0)) continue;
         auto tail = [&](double k, int h) { return chi2_tail(std::pow(std::max(0.0, std::sqrt(k * sst) - E.eps), 2) / sig2, h); };
-        double rate = tail(k1(9, N), 4);
+        rate = tail(k1(9, N), 4);
         if (inter) rate += tail(k2(9, N), 2);
         if (rate <= (i == 1 ? SCR_RATE1 : SCR_RATE2)) nd = i;
     }
@@ -1301,6 +1301,7 @@ bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
     C.test = q->test;
     C.safe = hs.safe;
     C.nd = nd;
+    C.rate = (float)rate;
     // GENERAL tiles: the pair's complete cases N' <= N and their SST vary. k / (N' - nfac + k) is smallest at
     // N' = N; the linear form of (sqrt(k SST) - eps)^2 >= k SST - 2 eps sqrt(k SST) takes the largest
     // k SST at N' >= N / 2 (pairs with fewer skip level 0).
@@ -1331,9 +1332,10 @@ struct ScreenKind {
     int n;
     uint32_t *count;   // candidates and regions of this kind
     uint32_t *redo;
+    unsigned long long *emptied;
 };
 
-// Launch of the bound and the resolve kernel; or, once the host has their counters, of the redo of K's regions.
+// Launches of the bound and the resolve kernel, a list of candidates at a time; or, once the host has their counters, of the redo of K's regions.
 template <bool GEN, int TA, int TB>
 int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind &K, bool redo)
 {
@@ -1347,8 +1349,10 @@ int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind
     G.cs.count = K.count;
     G.cs.redo = K.redo;
     G.halves = GEN ? TB / 32 : 1;
+    const ResolveArgs R = {G.S, nullptr, hs, G.cs.cand, K.count, G.cs.cap, resolve_lanes(G.S.Kl)};
+    const int most = scr_chunk(G.cut.rate, TA, TB, scr_threads<TA>() * G.halves);
     for (int t0 = 0; t0 < K.n;) {
-        const int chunk = std::min((int)((1u << 31) / (scr_threads<TA>() * G.halves)) & ~255, K.n - t0);  // as LAUNCH_TILES
+        const int chunk = std::min(most, K.n - t0);
         const dim3 grid(chunk * G.halves), block(scr_threads<TA>());
         G.tiles = K.tiles + t0;
         G.ntiles = chunk;
@@ -1368,13 +1372,15 @@ int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind
             else hipLaunchKernelGGL((screen_fast_kernel<TA, 2>), grid, block, 0, c->stream, G);
         }
         HIPCHK(c, hipGetLastError());
-        c->last_launches++;
+        hipLaunchKernelGGL((resolve_kernel<GEN, false>), dim3(4 * c->ncu), dim3(256), 0, c->stream, R);
+        HIPCHK(c, hipGetLastError());
+        c->last_launches += 2;
         t0 += chunk;
+        if (t0 == K.n) break;
+        hipLaunchKernelGGL(empty_list, dim3(1), dim3(1), 0, c->stream, K.count, G.cs.cap, K.emptied);
+        HIPCHK(c, hipGetLastError());
+        c->last_launches++;
     }
-    const ResolveArgs R = {G.S, nullptr, hs, G.cs.cand, K.count, G.cs.cap, resolve_lanes(G.S.Kl)};
-    hipLaunchKernelGGL((resolve_kernel<GEN, false>), dim3(4 * c->ncu), dim3(256), 0, c->stream, R);
-    HIPCHK(c, hipGetLastError());
-    c->last_launches++;
     return EPI_OK;
 }
 
@@ -1424,9 +1430,9 @@ int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, c
             G.cut = *cut;
             G.cs = B.cs;
             uint32_t *redo = B.cs.redo;
-            const ScreenKind kf = {B.tiles, nf, B.cs.count, redo},
-                             ks = {B.tiles + nf, ns, B.cs.count + 2, redo + 4 * (size_t)nf},
-                             kg = {B.tiles + nf + ns, ng, B.cs.count + 4, redo + 4 * (size_t)nf + 8 * (size_t)ns};
+            const ScreenKind kf = {B.tiles, nf, B.cs.count, redo, B.emptied},
+                             ks = {B.tiles + nf, ns, B.cs.count + 2, redo + 4 * (size_t)nf, B.emptied},
+                             kg = {B.tiles + nf + ns, ng, B.cs.count + 4, redo + 4 * (size_t)nf + 8 * (size_t)ns, B.emptied};
             const bool again = counts != nullptr;
             const bool lf = sf && (!again || counts[1]), ls = ss && (!again || counts[3]), lg = sg && (!again || counts[5]);
             int rc = EPI_OK;
@@ -1595,7 +1601,9 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     for (int kind = 0; kind < NKIND; kind++) {
         const int base = (int)work.size();
         std::vector<double> cost;
+        b->segs[kind].clear();
         for (int di : dorder) {
+            if (!wk[kind][di].empty()) b->segs[kind].push_back({di, (long long)wk[kind][di].size()});
             work.insert(work.end(), wk[kind][di].begin(), wk[kind][di].end());
             cost.insert(cost.end(), ct[kind][di].begin(), ct[kind][di].end());
         }
@@ -1659,15 +1667,14 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     return EPI_OK;
 }
 
-// The hit counter and, behind it, the screen's counters (candidates and regions to redo of each tile kind), as one
-// copy reads them.
-struct Counters {
-    unsigned long long nhits;
-    uint32_t screen[2 * NKIND];
-    long long candidates() const { return (long long)screen[0] + screen[2] + screen[4]; }
-    long long redone() const { return (long long)screen[1] + screen[3] + screen[5]; }
-};
-static_assert(sizeof(Counters) == 4 * sizeof(unsigned long long), "the counters of a context or a batch");
+long long candidates(const Counters &n)
+{
+    long long c = (long long)n.emptied;
+    for (int k = 0; k < NKIND; k++) c += std::min(n.screen[2 * k], CAND_CAP);
+    return c;
+}
+
+long long redone(const Counters &n) { return (long long)n.screen[1] + n.screen[3] + n.screen[5]; }
 
 bool same_key(const epi_scan_params &x, const epi_scan_params &y)
 {
@@ -1764,6 +1771,39 @@ bool batch_screen(const epi_batch *b, const epi_scan_params *p, std::vector<Scre
     return 2 * ok >= cut.size() && work >= SCR_MIN_WORK;
 }
 
+// Items of the next launch of a list through the screen, of `left`: as many as scr_chunk allows at the mean rate of each
+// dataset's scans (the items of a dataset follow one another, tile by tile, each for every scan). (seg, used): the
+// list's segment and the items taken from it.
+int batch_chunk(const epi_batch *b, const std::vector<ScreenCut> &cut, int kind, int threads, int left, size_t &seg, long long &used)
+{
+    const int TA = b->work_sched.fast_rows, TB = kind == 1 ? 32 : 64;
+    int n = 0;
+    double full = 0.0;  // part of a launch taken
+    while (seg < b->segs[kind].size() && n < left) {
+        const auto &s = b->segs[kind][seg];
+        double rate = 0.0;
+        int ns = 0;
+        for (size_t i = 0; i < b->scans.size(); i++)
+            if (b->scans[i].first == s.first) rate += cut[i].rate, ns++;
+        const double most = scr_chunk(rate / ns, TA, TB, threads);
+        const long long fit = (long long)((1.0 - full) * most), take = std::min(s.second - used, fit);
+        n += (int)take;
+        used += take;
+        full += (double)take / most;
+        if (used < s.second) break;
+        seg++;
+        used = 0;
+    }
+    // whole XCD groups: a few items more than a launch's share at most
+    const int up = std::min(left, (n + 255) / 256 * 256);
+    for (int more = up - n; more > 0 && seg < b->segs[kind].size();) {
+        const int take = (int)std::min<long long>(more, b->segs[kind][seg].second - used);
+        more -= take;
+        if ((used += take) == b->segs[kind][seg].second) seg++, used = 0;
+    }
+    return up;
+}
+
 // Capture queue reset + the persistent scan kernels as one graph: one kernel
 // per tile kind that has items (GENERAL and SPARSE first under order 1), each with a grid
 // of its occupancy times the CU count, so that every workgroup is resident and
@@ -1789,7 +1829,7 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
     for (int kind = 0; kind < NKIND; kind++) {
         screen[kind] = cut && !(kind == 2 && b->work_sched.dense_missing == 2);  // SPARSE tiles that the schedule asks for
         nt[kind] = screen[kind] ? 4 * b->work_sched.fast_rows : batch_threads_of(p->form, b->work_sched, kind);
-        G[kind] = {b->d_mscan, b->d_cut, work, 0, 0, {c->cand, b->scount + 2 * kind, CAND_CAP, redo}};
+        G[kind] = {b->d_mscan, b->d_cut, work, 0, 0, {c->cand, b->count->screen + 2 * kind, CAND_CAP, redo}};
         work += b->nkind[kind];
         redo += (kind == 2 ? 8 : 4) * (size_t)b->nkind[kind];
         B[kind].mscan = b->d_mscan;
@@ -1797,7 +1837,7 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
         B[kind].work = b->d_work;
         B[kind].qpos = b->d_qpos + kind * NQ;
         B[kind].qend = b->d_qend + kind * NQ;
-        B[kind].hs = make_sink(b->hits, b->nhits, b->cap, p);
+        B[kind].hs = make_sink(b->hits, &b->count->nhits, b->cap, p);
         kfn[kind] = screen[kind] ? screen_batch_fn(b->work_sched, kind, batch_nocall(b)) : batch_kernel(p->form, b->work_sched, kind);
         int per_cu = 1;
         HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn[kind], nt[kind], 0));
@@ -1806,7 +1846,7 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
     static const int korder[2][NKIND] = {{0, 2, 1}, {1, 2, 0}};
     const int *ko = korder[b->work_sched.order == 1 ? 1 : 0];
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    hipLaunchKernelGGL(batch_reset, dim3(1), dim3(64), 0, c->stream, b->d_qpos, (const int *)b->d_qbegin, b->nhits, b->scount);
+    hipLaunchKernelGGL(batch_reset, dim3(1), dim3(64), 0, c->stream, b->d_qpos, (const int *)b->d_qbegin, b->count);
     hipError_t le = hipGetLastError();
     for (int t = 0; t < NKIND && le == hipSuccess; t++) {
         const int kind = ko[t];
@@ -1816,23 +1856,28 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
             le = hipLaunchKernel(kfn[kind], dim3(grid[kind]), dim3(nt[kind]), args, 0, c->stream);
             continue;
         }
-        // one workgroup per item, in launches of whole XCD groups within the runtime's 2^31 work-items
+        // one workgroup per item, a list of candidates at a time
         const int4 *items = G[kind].work;
         const int n = (int)b->nkind[kind], halves = kind == 2 ? 2 : 1;
-        const int chunk = (int)((1u << 31) / (unsigned)(nt[kind] * halves)) & ~255;
-        for (int t0 = 0; t0 < n && le == hipSuccess; t0 += chunk) {
-            G[kind].work = items + t0;
-            G[kind].item0 = t0;
-            G[kind].nitems = std::min(chunk, n - t0);
-            void *args[] = {&G[kind]};
-            le = hipLaunchKernel(kfn[kind], dim3(G[kind].nitems * halves), dim3(nt[kind]), args, 0, c->stream);
-        }
         ResolveArgs R = {{}, b->d_mscan, B[kind].hs, c->cand, G[kind].cs.count, CAND_CAP, resolve_lanes(Kl)};
         RedoArgs D = {{}, b->d_mscan, B[kind].hs, items, G[kind].cs.count, G[kind].cs.redo};
         void *rargs[] = {&R}, *dargs[] = {&D};
-        if (le == hipSuccess)
-            le = hipLaunchKernel(kind ? (const void *)resolve_kernel<true, true> : (const void *)resolve_kernel<false, true>,
-                                 dim3(4 * c->ncu), dim3(256), rargs, 0, c->stream);
+        size_t seg = 0;
+        long long used = 0;
+        for (int t0 = 0; t0 < n && le == hipSuccess;) {
+            if (t0) hipLaunchKernelGGL(empty_list, dim3(1), dim3(1), 0, c->stream, G[kind].cs.count, CAND_CAP, &b->count->emptied);
+            const int chunk = batch_chunk(b, *cut, kind, nt[kind] * halves, n - t0, seg, used);
+            G[kind].work = items + t0;
+            G[kind].item0 = t0;
+            G[kind].nitems = chunk;
+            void *args[] = {&G[kind]};
+            le = hipGetLastError();
+            if (le == hipSuccess) le = hipLaunchKernel(kfn[kind], dim3(chunk * halves), dim3(nt[kind]), args, 0, c->stream);
+            if (le == hipSuccess)
+                le = hipLaunchKernel(kind ? (const void *)resolve_kernel<true, true> : (const void *)resolve_kernel<false, true>,
+                                     dim3(4 * c->ncu), dim3(256), rargs, 0, c->stream);
+            t0 += chunk;
+        }
         if (le == hipSuccess)
             le = hipLaunchKernel(redo_batch_fn(b->work_sched, kind), dim3(2 * c->ncu), dim3(256), dargs, 0, c->stream);
     }
@@ -1883,15 +1928,15 @@ int batch_run(epi_batch *b, double *ms_out)
     HIPCHK(c, hipGraphLaunch(b->exec, c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     Counters n;
-    HIPCHK(c, hipMemcpyAsync(&n, b->nhits, sizeof(n), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(&n, b->count, sizeof(n), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     float ms = 0.0f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     b->last_ms = ms;
     b->last_nhits = (long long)n.nhits;
     b->last_screened = b->gscreened;
-    b->last_cand = n.candidates();
-    b->last_redone = n.redone();
+    b->last_cand = candidates(n);
+    b->last_redone = redone(n);
     b->fetched = false;
     if (ms_out) *ms_out = ms;
     return EPI_OK;
@@ -1951,7 +1996,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
             c->tl_sched = sc;
         }
     }
-    HIPCHK(c, hipMemsetAsync(c->nhits, 0, 4 * sizeof(unsigned long long), c->stream));  // and the screen's counters
+    HIPCHK(c, hipMemsetAsync(c->count, 0, sizeof(Counters), c->stream));
     DumpSink ds;
     memset(&ds, 0, sizeof(ds));
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -1966,23 +2011,23 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
         launches += c->last_launches;
         HIPCHK(c, hipEventRecord(c->ev1, c->stream));
         // the launched kernels read the device tile list that the next piece overwrites
-        HIPCHK(c, hipMemcpyAsync(&n, c->nhits, sizeof(n), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipMemcpyAsync(&n, c->count, sizeof(n), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        c->last_cand += n.candidates();
-        c->last_redone += n.redone();
-        if (n.redone()) {
+        c->last_cand += candidates(n);
+        c->last_redone += redone(n);
+        if (redone(n)) {
             // few scans have regions to redo: launched for every kind in every scan, N = 500, M = 2000 took 102.7 us, not 100.6
             if ((rc = launch_pairs<false>(c, p, sc, tl, ds, ctx_bufs(c), &cut, n.screen))) return rc;
             launches += c->last_launches;
             HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-            HIPCHK(c, hipMemcpyAsync(&n, c->nhits, sizeof(n), hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipMemcpyAsync(&n, c->count, sizeof(n), hipMemcpyDeviceToHost, c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));
         }
         if (done) break;
         tl = TileLists();
         done = build_tiles(c->d, be, p->form, sc, max_tiles, cur, tl);
         if ((rc = upload_tiles(c, tl))) return rc;
-        HIPCHK(c, hipMemsetAsync(c->scount, 0, 6 * sizeof(uint32_t), c->stream));
+        HIPCHK(c, hipMemsetAsync(c->count->screen, 0, sizeof(Counters) - offsetof(Counters, screen), c->stream));
         pairs += tl.pairs;
     }
     float ms = 0.0f;
@@ -2111,11 +2156,10 @@ int epi_open(int device, epi_ctx **out)
     }
     if (c->ncu <= 0) c->ncu = 1;
     for (int f = 0; f < 2; f++) c->sched[f] = default_schedule(f);
-    if (dalloc(c, c->nhits, 4) || dalloc(c, c->hits, (size_t)c->cap) || dalloc(c, c->cand, (size_t)CAND_CAP)) {
+    if (dalloc(c, c->count, 1) || dalloc(c, c->hits, (size_t)c->cap) || dalloc(c, c->cand, (size_t)CAND_CAP)) {
         epi_close(c);
         return EPI_ERR_NOMEM;
     }
-    c->scount = reinterpret_cast<uint32_t *>(c->nhits + 1);
     if (scratch_of(c, &c->scratch)) {
         epi_close(c);
         return EPI_ERR_HIP;
@@ -2131,7 +2175,7 @@ void epi_close(epi_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     free_dataset(c->d);
     dfree(c->hits);
-    dfree(c->nhits);
+    dfree(c->count);
     dfree(c->tiles);
     dfree(c->cand);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -2497,11 +2541,10 @@ int epi_batch_create(epi_ctx *c, epi_batch **out)
     int rc;
     if ((rc = dalloc(c, b->d_qpos, NKIND * NQ)) || (rc = dalloc(c, b->d_qbegin, NKIND * NQ)) ||
         (rc = dalloc(c, b->d_qend, NKIND * NQ)) ||
-        (rc = dalloc(c, b->nhits, 4)) || (rc = dalloc(c, b->hits, (size_t)b->cap))) {
+        (rc = dalloc(c, b->count, 1)) || (rc = dalloc(c, b->hits, (size_t)b->cap))) {
         epi_batch_destroy(b);
         return rc;
     }
-    b->scount = reinterpret_cast<uint32_t *>(b->nhits + 1);
     *out = b;
     return EPI_OK;
 }
@@ -2525,7 +2568,7 @@ void epi_batch_destroy(epi_batch *b)
     dfree(b->d_qbegin);
     dfree(b->d_qend);
     dfree(b->hits);
-    dfree(b->nhits);
+    dfree(b->count);
     delete b;
 }
 

@@ -43,13 +43,21 @@ struct ScreenBatchArgs {
     CandSink cs;
 };
 
-// Queue heads of every list ([NKIND][NQ]), the hit counter and the screen's two counters of every list.
-__global__ void batch_reset(int *qpos, const int *qbegin, unsigned long long *nhits, uint32_t *scount)
+// The hit counter and, behind it, the screen's: candidates and regions to redo of each tile kind, and the
+// candidates of lists that were emptied.
+struct Counters {
+    unsigned long long nhits;
+    uint32_t screen[2 * NKIND];
+    unsigned long long emptied;
+};
+
+// Queue heads of every list ([NKIND][NQ]) and the counters.
+__global__ void batch_reset(int *qpos, const int *qbegin, Counters *n)
 {
     const int t = threadIdx.x;
     if (t < NKIND * NQ) qpos[t] = qbegin[t];
-    if (t < 2 * NKIND) scount[t] = 0u;
-    if (t == 0) *nhits = 0ull;
+    if (t < 2 * NKIND) n->screen[t] = 0u;
+    if (t == 0) n->nhits = n->emptied = 0ull;
 }
 
 // Called by one thread: the next item for a workgroup whose home queue is

@@ -79,6 +79,7 @@ struct ScreenCut {
     float t1s, t2s;       // lowered thresholds
     int test, safe;
     int nd;               // digits of v; 0: the scan is not screened
+    float rate;           // predicted candidates per pair of unrelated SNPs
 };
 
 struct CandSink {
@@ -739,6 +740,13 @@ __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_gen_kernel(const 
     uint32_t region0;
     if (!scr_half<TA>(t % A.halves, A.halves, (uint32_t)(A.tile0 + t / A.halves), T.z, T.w, region0)) return;
     screen_gen_tile<TA, ND, NC>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, region0, wl, mg);
+}
+
+// After the candidates of a launch are resolved: the list is emptied for the next one.
+__global__ void empty_list(uint32_t *count, uint32_t cap, unsigned long long *total)
+{
+    *total += *count < cap ? *count : cap;
+    *count = 0u;
 }
 
 // --------------------------------------------------------------- redo ----

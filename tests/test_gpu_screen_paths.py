@@ -107,3 +107,29 @@ def test_not_screened_counts(sch):
     for form in ("mfma", "plain"):
         sch.scan(form=form, t1=3.0, t2=4.0)
         assert sch.last_screen() == {"digits": 0, "candidates": 0, "redone": 0}
+
+
+@pytest.mark.parametrize("nphen,gmiss", [(1, 0.0), (1, 0.01), (3, 0.0)])
+def test_many_candidates(scanner, buf, nphen, gmiss):
+    """More candidates than the list holds at a rate that admits the screen: the list is resolved in between, and no region
+    goes to the exact tiles."""
+    nid, nsnp = 600, 41000 if nphen == 1 else 24000
+    words = E.synth_genotypes(51, nid, nsnp, 0.1, 0.5, gmiss)
+    y = np.stack([phenotype("normal", nid, 52 + i) for i in range(nphen)])
+    kw = dict(test="f", t1=float(S.f_isf(1.3e-3, 8, nid - 9)), t2=10.5)
+    load(scanner, words, nid, y, [nsnp])
+    one = [scanner.scan(phen=r, **kw) for r in range(nphen)]
+    scr = scanner.last_screen()
+    if nphen > 1:
+        with E.Batch(scanner) as b:
+            b.add_phenotypes(b.add_dataset(words, nid), y)
+            for rep in range(2):
+                b.scan(**kw)
+                scr = dict(b.last_screen(), digits=1)
+                for r in range(nphen):
+                    g = b.hits(r)
+                    assert all(np.array_equal(g[k], one[r][k]) for k in ("hits", "F64", "F2_64", "block"))
+    print(f"candidates nphen={nphen} gmiss={gmiss} hits {[g['nhits'] for g in one]} {scr}", flush=True)
+    assert scr["digits"] and scr["candidates"] > (1 << 20)
+    assert scr["redone"] == 0
+    assert same_as_exact(scanner, buf, one[0], **kw) > 0

@@ -33,6 +33,21 @@ int main()
         CHECK(2 * (uint64_t)scr_piece(m) <= SCR_TILES);
     }
     CHECK(scr_piece((uint64_t)1 << 25) == (uint64_t)1 << 24);
+    // launches of the bound: whole XCD groups, half a list of predicted candidates, within the runtime's work-items, and
+    // no more pairs than the 32-bit counter counts
+    for (int TA : {32, 64})
+        for (int TB : {32, 64})
+            for (double rate : {0.0, 1e-12, 1e-7, 2.5e-4, 2e-3}) {
+                const int threads = 64 * scr_regions(TA, TB, TB == 32);
+                const uint64_t n = scr_chunk(rate, TA, TB, threads), pairs = n * TA * TB;
+                CHECK(n >= 256 && n % 256 == 0);
+                CHECK(n * threads <= (uint64_t)1 << 31);
+                CHECK(pairs < (uint64_t)1 << 32);
+                CHECK(pairs * rate <= 0.5 * CAND_CAP);
+                // not needlessly short: one more group would pass one of the bounds
+                const uint64_t m = n + 256;
+                CHECK(m * threads > (uint64_t)1 << 31 || m * TA * TB > (uint64_t)1 << 31 || m * TA * TB * rate > 0.5 * CAND_CAP);
+            }
     return bad;
 }
 """
