@@ -148,10 +148,11 @@ struct epi_ctx {
     DevHit *hits = nullptr;
     long long cap = 1ll << 22;
     long long last_nhits = 0;
-    // counters of the hits and of the screen; candidates; regions to redo (behind the tiles)
+    // counters of the hits and of the screen; candidates; blocks to redo and their masks (behind the tiles)
     Counters *count = nullptr;
     int4 *cand = nullptr;
     uint32_t *redo = nullptr;
+    size_t redo_blocks = 0;
     // tiles; the device list of the last scan is kept and reused while the
     // dataset, block range, form and schedule stay the same
     int4 *tiles = nullptr;
@@ -179,7 +180,7 @@ struct epi_batch {
     MfmaScan *d_mscan = nullptr;
     PlainScan *d_pscan = nullptr;
     ScreenCut *d_cut = nullptr;
-    uint32_t *redo = nullptr;    // behind the work items
+    uint32_t *redo = nullptr, *mask = nullptr;  // behind the work items
     int4 *d_work = nullptr;
     int *d_qpos = nullptr, *d_qbegin = nullptr, *d_qend = nullptr;  // [NKIND][NQ]: FAST, GENERAL, SPARSE items
     size_t work_cap = 0, scan_cap = 0;
@@ -1137,10 +1138,11 @@ int copy_tiles(epi_ctx *c, int4 *dst, const TileLists &tl)
 int upload_tiles(epi_ctx *c, const TileLists &tl)
 {
     c->tl_valid = false;
-    // behind the tiles, room for every region of the screen's tiles (at most four of 4 bytes per tile, eight
-    // per SPARSE tile)
-    const size_t nt = tl.count(), need = 2 * nt + tl.sp.size();
-    static_assert(sizeof(int4) == 64 / SCR_A * sizeof(uint32_t), "a tile's regions take the room of a tile");
+    // behind the tiles, room for the number and the mask of every block of the screen's tiles, of 64 or 32 rows
+    const size_t nt = tl.count();
+    const size_t blocks = scr_blocks(64, 64, false) * (tl.fast.size() + tl.gen.size()) + scr_blocks(64, 64, true) * tl.sp.size();
+    const size_t need = nt + (2 * blocks * sizeof(uint32_t) + sizeof(int4) - 1) / sizeof(int4);
+    static_assert(scr_blocks(64, 64, false) == scr_blocks(64, 32, true), "one count of blocks for FAST and GENERAL tiles");
     if (need > c->tiles_cap) {
         c->tiles_cap = 0;
         int rc = dalloc(c, c->tiles, need);
@@ -1148,6 +1150,8 @@ int upload_tiles(epi_ctx *c, const TileLists &tl)
         c->tiles_cap = need;
     }
     c->redo = reinterpret_cast<uint32_t *>(c->tiles + nt);
+    c->redo_blocks = blocks;
+    HIPCHK(c, hipMemsetAsync(c->redo + blocks, 0, blocks * sizeof(uint32_t), c->stream));  // the masks
     return copy_tiles(c, c->tiles, tl);
 }
 
@@ -1216,7 +1220,7 @@ struct ScanBufs {
 
 ScanBufs ctx_bufs(const epi_ctx *c)
 {
-    return {c->tiles, c->hits, &c->count->nhits, c->cap, {c->cand, c->count->screen, CAND_CAP, c->redo}, &c->count->emptied};
+    return {c->tiles, c->hits, &c->count->nhits, c->cap, {c->cand, c->count->screen, CAND_CAP, c->redo, c->redo + c->redo_blocks}, &c->count->emptied};
 }
 
 // Lanes per candidate of resolve_kernel for a cohort of Kl individuals (one 32-individual word each).
@@ -1330,17 +1334,17 @@ bool screen_fits(const Dataset &d)
 struct ScreenKind {
     const int4 *tiles;
     int n;
-    uint32_t *count;   // candidates and regions of this kind
-    uint32_t *redo;
+    uint32_t *count;   // candidates and blocks of this kind
+    uint32_t *redo, *mask;
     unsigned long long *emptied;
 };
 
-// Launches of the bound and the resolve kernel, a list of candidates at a time; or, once the host has their counters, of the redo of K's regions.
+// Launches of the bound and the resolve kernel, a list of candidates at a time; or, once the host has their counters, of the redo of K's blocks.
 template <bool GEN, int TA, int TB>
 int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind &K, bool redo)
 {
     if (redo) {
-        const RedoArgs D = {G.S, nullptr, hs, K.tiles, K.count, K.redo};
+        const RedoArgs D = {G.S, nullptr, hs, K.tiles, K.count, K.redo, K.mask};
         hipLaunchKernelGGL((redo_kernel<TA, TB, GEN, false>), dim3(2 * c->ncu), dim3(256), 0, c->stream, D);
         HIPCHK(c, hipGetLastError());
         c->last_launches++;
@@ -1348,6 +1352,7 @@ int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind
     }
     G.cs.count = K.count;
     G.cs.redo = K.redo;
+    G.cs.mask = K.mask;
     G.halves = GEN ? TB / 32 : 1;
     const ResolveArgs R = {G.S, nullptr, hs, G.cs.cand, K.count, G.cs.cap, resolve_lanes(G.S.Kl)};
     const int most = scr_chunk(G.cut.rate, TA, TB, scr_threads<TA>() * G.halves);
@@ -1399,7 +1404,7 @@ bool screened(const Dataset &d, const epi_scan_params *p, long long pairs, Scree
 }
 
 // Launch the pair kernels of one scan over the uploaded tile lists (fast tiles first).
-// counts: the screen's counters of an earlier call, whose regions are to be redone (nothing else is launched).
+// counts: the screen's counters of an earlier call, whose blocks are to be redone (nothing else is launched).
 template <bool DUMP>
 int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, const TileLists &tl,
                  const DumpSink &ds, const ScanBufs &B, const ScreenCut *cut = nullptr, const uint32_t *counts = nullptr)
@@ -1429,10 +1434,10 @@ int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, c
             G.S = A.S;
             G.cut = *cut;
             G.cs = B.cs;
-            uint32_t *redo = B.cs.redo;
-            const ScreenKind kf = {B.tiles, nf, B.cs.count, redo, B.emptied},
-                             ks = {B.tiles + nf, ns, B.cs.count + 2, redo + 4 * (size_t)nf, B.emptied},
-                             kg = {B.tiles + nf + ns, ng, B.cs.count + 4, redo + 4 * (size_t)nf + 8 * (size_t)ns, B.emptied};
+            const size_t of = scr_blocks(64, 64, false) * (size_t)nf, os = of + scr_blocks(64, 64, true) * (size_t)ns;
+            const ScreenKind kf = {B.tiles, nf, B.cs.count, B.cs.redo, B.cs.mask, B.emptied},
+                             ks = {B.tiles + nf, ns, B.cs.count + 2, B.cs.redo + of, B.cs.mask + of, B.emptied},
+                             kg = {B.tiles + nf + ns, ng, B.cs.count + 4, B.cs.redo + os, B.cs.mask + os, B.emptied};
             const bool again = counts != nullptr;
             const bool lf = sf && (!again || counts[1]), ls = ss && (!again || counts[3]), lg = sg && (!again || counts[5]);
             int rc = EPI_OK;
@@ -1553,6 +1558,8 @@ void emit_hits(const Dataset &d, const DevHit *h, const std::vector<int> &idx, e
 // so that the longest items do not end up in the tail. With 8 queues the list
 // is cut into NQ contiguous pieces of equal estimated cost, one per XCD;
 // with 1 queue every workgroup pulls from one shared queue.
+constexpr size_t batch_blocks(int kind) { return scr_blocks(64, kind == 1 ? 32 : 64, kind != 0); }
+
 int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
 {
     epi_ctx *c = b->ctx;
@@ -1607,6 +1614,7 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
             work.insert(work.end(), wk[kind][di].begin(), wk[kind][di].end());
             cost.insert(cost.end(), ct[kind][di].begin(), ct[kind][di].end());
         }
+        static_assert(SCR_TILES > INT32_MAX / 2, "the screen numbers the blocks of any list");
         if (work.size() > (size_t)INT32_MAX / 2) return fail(c, EPI_ERR_RANGE, "batch has too many tiles");
         const int n = (int)work.size();
         b->nkind[kind] = n - base;
@@ -1631,14 +1639,18 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     }
     b->nwork = (long long)work.size();
     int rc;
-    // behind the items, room for every region of the screen (at most four of 4 bytes per item, eight per SPARSE item)
-    const size_t room = 2 * work.size() + (size_t)b->nkind[2];
+    // behind the items, room for the number and the mask of every block of the screen's tiles, of 64 or 32 rows
+    size_t blocks = 0;
+    for (int kind = 0; kind < NKIND; kind++) blocks += batch_blocks(kind) * (size_t)b->nkind[kind];
+    const size_t room = work.size() + (2 * blocks * sizeof(uint32_t) + sizeof(int4) - 1) / sizeof(int4);
     if (room > b->work_cap) {
         b->work_cap = 0;
         if ((rc = dalloc(c, b->d_work, room))) return rc;
         b->work_cap = room;
     }
     b->redo = reinterpret_cast<uint32_t *>(b->d_work + work.size());
+    b->mask = b->redo + blocks;
+    HIPCHK(c, hipMemsetAsync(b->mask, 0, blocks * sizeof(uint32_t), c->stream));
     if (!work.empty())
         HIPCHK(c, hipMemcpyAsync(b->d_work, work.data(), work.size() * sizeof(int4), hipMemcpyHostToDevice,
                                  c->stream));
@@ -1812,7 +1824,6 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
 {
     epi_ctx *c = b->ctx;
     drop_graph(b);
-    if (b->nwork > (long long)SCR_TILES) cut = nullptr;
     if (cut) {
         HIPCHK(c, hipMemcpyAsync(b->d_cut, cut->data(), cut->size() * sizeof(ScreenCut), hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1825,13 +1836,14 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
     for (const Dataset *d : b->data) Kl = std::max(Kl, (d->nid + KC - 1) / KC * KC);
     ScreenBatchArgs G[NKIND];
     const int4 *work = b->d_work;
-    uint32_t *redo = b->redo;
+    uint32_t *redo = b->redo, *mask = b->mask;
     for (int kind = 0; kind < NKIND; kind++) {
         screen[kind] = cut && !(kind == 2 && b->work_sched.dense_missing == 2);  // SPARSE tiles that the schedule asks for
         nt[kind] = screen[kind] ? 4 * b->work_sched.fast_rows : batch_threads_of(p->form, b->work_sched, kind);
-        G[kind] = {b->d_mscan, b->d_cut, work, 0, 0, {c->cand, b->count->screen + 2 * kind, CAND_CAP, redo}};
+        G[kind] = {b->d_mscan, b->d_cut, work, 0, 0, {c->cand, b->count->screen + 2 * kind, CAND_CAP, redo, mask}};
         work += b->nkind[kind];
-        redo += (kind == 2 ? 8 : 4) * (size_t)b->nkind[kind];
+        redo += batch_blocks(kind) * (size_t)b->nkind[kind];
+        mask += batch_blocks(kind) * (size_t)b->nkind[kind];
         B[kind].mscan = b->d_mscan;
         B[kind].pscan = b->d_pscan;
         B[kind].work = b->d_work;
@@ -1860,7 +1872,7 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
         const int4 *items = G[kind].work;
         const int n = (int)b->nkind[kind], halves = kind == 2 ? 2 : 1;
         ResolveArgs R = {{}, b->d_mscan, B[kind].hs, c->cand, G[kind].cs.count, CAND_CAP, resolve_lanes(Kl)};
-        RedoArgs D = {{}, b->d_mscan, B[kind].hs, items, G[kind].cs.count, G[kind].cs.redo};
+        RedoArgs D = {{}, b->d_mscan, B[kind].hs, items, G[kind].cs.count, G[kind].cs.redo, G[kind].cs.mask};
         void *rargs[] = {&R}, *dargs[] = {&D};
         size_t seg = 0;
         long long used = 0;
@@ -1924,6 +1936,7 @@ int batch_prepare(epi_batch *b, const epi_scan_params *p)
 int batch_run(epi_batch *b, double *ms_out)
 {
     epi_ctx *c = b->ctx;
+    b->dirty = true;  // a run that fails may leave marked blocks: the list is then built again
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     HIPCHK(c, hipGraphLaunch(b->exec, c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
@@ -1932,6 +1945,7 @@ int batch_run(epi_batch *b, double *ms_out)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     float ms = 0.0f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
+    b->dirty = false;
     b->last_ms = ms;
     b->last_nhits = (long long)n.nhits;
     b->last_screened = b->gscreened;
@@ -1988,14 +2002,13 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
         tl = TileLists();
         done = build_tiles(c->d, be, p->form, sc, max_tiles, cur, tl);
         if ((rc = upload_tiles(c, tl))) return rc;
-        if (done) {
-            c->tl_valid = true;
-            c->tl_bb = bb;
-            c->tl_be = be;
-            c->tl_form = p->form;
-            c->tl_sched = sc;
-        }
+        c->tl_bb = bb;
+        c->tl_be = be;
+        c->tl_form = p->form;
+        c->tl_sched = sc;
     }
+    const bool whole = done;  // the list serves later scans
+    c->tl_valid = false;  // a scan that fails may leave marked blocks
     HIPCHK(c, hipMemsetAsync(c->count, 0, sizeof(Counters), c->stream));
     DumpSink ds;
     memset(&ds, 0, sizeof(ds));
@@ -2016,7 +2029,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
         c->last_cand += candidates(n);
         c->last_redone += redone(n);
         if (redone(n)) {
-            // few scans have regions to redo: launched for every kind in every scan, N = 500, M = 2000 took 102.7 us, not 100.6
+            // few scans have blocks to redo: launched for every kind in every scan, N = 500, M = 2000 took 102.7 us, not 100.6
             if ((rc = launch_pairs<false>(c, p, sc, tl, ds, ctx_bufs(c), &cut, n.screen))) return rc;
             launches += c->last_launches;
             HIPCHK(c, hipEventRecord(c->ev1, c->stream));
@@ -2032,6 +2045,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
     }
     float ms = 0.0f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
+    c->tl_valid = whole;
     c->last_ms = ms;
     c->last_pairs = pairs;
     c->last_launches = launches;

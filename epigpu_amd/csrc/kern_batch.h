@@ -43,7 +43,7 @@ struct ScreenBatchArgs {
     CandSink cs;
 };
 
-// The hit counter and, behind it, the screen's: candidates and regions to redo of each tile kind, and the
+// The hit counter and, behind it, the screen's: candidates and blocks to redo of each tile kind, and the
 // candidates of lists that were emptied.
 struct Counters {
     unsigned long long nhits;
@@ -135,7 +135,7 @@ __global__ __launch_bounds__((batch_threads<TA, KIND>()), (batch_waves_per_simd<
 template <int TA, int KIND, bool NC = false>
 __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_batch_kernel(const ScreenBatchArgs B)
 {
-    constexpr int HALVES = KIND == 2 ? 2 : 1, NW = scr_regions(TA, KIND == 1 ? 32 : 64, KIND != 0);
+    constexpr int HALVES = KIND == 2 ? 2 : 1, NBLK = scr_blocks(TA, KIND == 1 ? 32 : 64, KIND != 0);
     __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * sw_row<2>()];
     __shared__ float4 mg[KIND ? 2 * (TA + 32) : TA + 64];
     __shared__ float2 mg2[TA];
@@ -148,22 +148,25 @@ __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_batch_kernel(cons
     // (N = 4000, M = 20000 with 1 % missing calls: 9.1 against 7.2 ms a phenotype)
     const MfmaScan S = B.mscan[sc];
     const ScreenCut C = B.cut[sc];
-    uint32_t region0 = (uint32_t)(B.item0 + it) * NW;
+    uint32_t block0 = (uint32_t)(B.item0 + it) * NBLK;
     if (!C.nd) {
-        if (threadIdx.x == 0 && t % HALVES == 0) B.cs.redo[atomicAdd(B.cs.count + 1, 1u)] = SCR_WHOLE | region0;
+        if (threadIdx.x < NBLK && t % HALVES == 0) {
+            B.cs.mask[block0 + threadIdx.x] = 3u;
+            B.cs.redo[atomicAdd(B.cs.count + 1, 1u)] = block0 + threadIdx.x;
+        }
         return;
     }
     if constexpr (KIND == 0) {
         if (C.nd == 1)
-            screen_fast_tile<TA, 1>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg, mg2);
+            screen_fast_tile<TA, 1>(S, C, B.cs, a0, a1, b0, b1, block0, wl, mg, mg2);
         else
-            screen_fast_tile<TA, 2>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg, mg2);
+            screen_fast_tile<TA, 2>(S, C, B.cs, a0, a1, b0, b1, block0, wl, mg, mg2);
     } else {
-        if (!scr_half<TA>(t % HALVES, HALVES, (uint32_t)(B.item0 + it), b0, b1, region0)) return;
+        if (!scr_half<TA>(t % HALVES, HALVES, (uint32_t)(B.item0 + it), b0, b1, block0)) return;
         if (C.nd == 1)
-            screen_gen_tile<TA, 1, NC>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg);
+            screen_gen_tile<TA, 1, NC>(S, C, B.cs, a0, a1, b0, b1, block0, wl, mg);
         else
-            screen_gen_tile<TA, 2, NC>(S, C, B.cs, a0, a1, b0, b1, region0, wl, mg);
+            screen_gen_tile<TA, 2, NC>(S, C, B.cs, a0, a1, b0, b1, block0, wl, mg);
     }
 }
 

@@ -676,7 +676,7 @@ class Scanner:
         return {"fast": f.value, "sparse": sp.value, "general": g.value}
 
     def last_screen(self):
-        """What the screen did in the last scan: digits (0: not screened), candidates and redone regions."""
+        """What the screen did in the last scan: digits (0: not screened), candidates and redone blocks."""
         d, c, r = ctypes.c_int32(), ctypes.c_int64(), ctypes.c_int64()
         self._chk(self.L.epi_last_screen(self.ctx, ctypes.byref(d), ctypes.byref(c), ctypes.byref(r)),
                   "epi_last_screen")
@@ -779,7 +779,7 @@ class Batch:
                 "grid": grid.value, "nhits": n, "overflow": ovf}
 
     def last_screen(self):
-        """What the screen did in the last scan of the batch: screened scans, candidates and redone regions."""
+        """What the screen did in the last scan of the batch: screened scans, candidates and redone blocks."""
         s, c, r = ctypes.c_int32(), ctypes.c_int64(), ctypes.c_int64()
         self._chk(self.L.epi_batch_last_screen(self.b, ctypes.byref(s), ctypes.byref(c), ctypes.byref(r)),
                   "epi_batch_last_screen")

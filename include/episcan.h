@@ -182,7 +182,7 @@ int epi_set_hit_capacity(epi_ctx *ctx, int64_t cap);
  * pieces of about this many tiles (whole rows of super-tiles), with the
  * same hits; its epi_last_scan_stats time then includes the later pieces'
  * uploads. A screened scan (below) counts a tile twice: its list takes as much
- * room again for the regions that the exact tiles redo. No counterpart in the reference, which launches per chunk of
+ * room again for the blocks that the exact tiles redo. No counterpart in the reference, which launches per chunk of
  * -i SNPs (src/EpiOpenCL.c:1564-1607). 1 <= max_tiles <= 2^30 - 1. */
 int epi_set_max_tiles(epi_ctx *ctx, int64_t max_tiles);
 
@@ -258,7 +258,7 @@ int epi_last_tiles(epi_ctx *ctx, int64_t *fast, int64_t *sparse, int64_t *genera
 /* What the screen (see epi_schedule) did in the last epi_scan: the digits of
  * its coarse phenotype (1 or 2; 0: the scan was not screened), the pairs that
  * it kept one by one and that were then computed exactly (candidates), and the
- * regions of tiles that exact tiles redid. No counterpart in the reference; for
+ * blocks of at most 32 x 64 pairs that exact tiles redid. No counterpart in the reference; for
  * tests and measurement. */
 int epi_last_screen(epi_ctx *ctx, int32_t *digits, int64_t *candidates, int64_t *redone);
 
@@ -328,7 +328,7 @@ int epi_batch_stats(epi_batch *batch, double *kernel_ms, int64_t *pairs, int64_t
                     int32_t *captures, int32_t *grid);
 
 /* As epi_last_screen, for the last epi_batch_scan: how many of its scans were
- * screened, and the candidates and redone regions of all of them. */
+ * screened, and the candidates and redone blocks of all of them. */
 int epi_batch_last_screen(epi_batch *batch, int32_t *scans, int64_t *candidates, int64_t *redone);
 
 /* Schedule of the batch's scans of one form (defaults as epi_set_schedule,

@@ -133,3 +133,30 @@ def test_many_candidates(scanner, buf, nphen, gmiss):
     assert scr["digits"] and scr["candidates"] > (1 << 20)
     assert scr["redone"] == 0
     assert same_as_exact(scanner, buf, one[0], **kw) > 0
+
+
+def stratified(nid, nsnp, spread, seed):
+    """Two populations with allele frequencies that differ by `spread` SDs, and a phenotype that differs between them."""
+    rng = np.random.default_rng(seed)
+    pop = np.arange(nid) % 2
+    f = np.clip(rng.uniform(0.2, 0.5, nsnp)[:, None] + (rng.standard_normal(nsnp) * spread)[:, None] * pop, 0.02, 0.98)
+    codes = sum((rng.random((nsnp, nid), dtype=np.float32) < f).astype(np.int8) for _ in range(2))
+    return codes, (pop + rng.standard_normal(nid)).astype(np.float32)
+
+
+@pytest.mark.parametrize("gmiss", [0.0, 0.01])
+@pytest.mark.parametrize("nid", [1000, 2000])
+def test_dense_blocks(scanner, buf, nid, gmiss):
+    """Hits all over, where the screen expected none: the exact tiles redo blocks of 32 rows, each once."""
+    sizes = [2500, 433]
+    codes, y = stratified(nid, sum(sizes), 0.15, nid)
+    if gmiss:
+        codes[np.random.default_rng(1).random(codes.shape) < gmiss] = 3
+    load(scanner, S.pack(codes), nid, y, sizes)
+    kw = dict(test="i", t1=6.5, t2=10.5)
+    g = scanner.scan(**kw)
+    scr = scanner.last_screen()
+    blocks = tiles(sizes, 32, 32 if gmiss else 64)
+    print(f"dense nid={nid} gmiss={gmiss} hits {g['nhits']} of {g['pairs']} {scr} blocks {blocks}", flush=True)
+    assert scr["digits"] and blocks / 2 < scr["redone"] <= blocks
+    assert same_as_exact(scanner, buf, g, **kw) > 0.2 * g["pairs"]

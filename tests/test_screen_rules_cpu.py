@@ -15,15 +15,15 @@ static int bad = 0;
 
 int main()
 {
-    // a region's number leads back to its tile and stays below the bit of whole tiles, up to the longest list
+    // a block's number leads back to its tile, up to the longest list
     for (int TA : {32, 64})
         for (int kind = 0; kind < 3; kind++) {
-            const uint64_t n = scr_regions(TA, kind == 1 ? 32 : 64, kind != 0);
-            CHECK(n >= 2 && n <= 8);
+            const uint64_t n = scr_blocks(TA, kind == 1 ? 32 : 64, kind != 0);
+            CHECK(n >= 1 && n <= 4);
             for (uint64_t tile : {(uint64_t)0, (uint64_t)SCR_TILES / 2, (uint64_t)SCR_TILES - 1})
                 for (uint64_t k = 0; k < n; k++) {
                     const uint64_t r = tile * n + k;
-                    CHECK(r < SCR_WHOLE);
+                    CHECK(r < (uint64_t)1 << 32);
                     CHECK((uint32_t)r / n == tile && (uint32_t)r % n == k);
                 }
         }
@@ -38,7 +38,7 @@ int main()
     for (int TA : {32, 64})
         for (int TB : {32, 64})
             for (double rate : {0.0, 1e-12, 1e-7, 2.5e-4, 2e-3}) {
-                const int threads = 64 * scr_regions(TA, TB, TB == 32);
+                const int threads = 64 * TA / SCR_A * (TB / 32);
                 const uint64_t n = scr_chunk(rate, TA, TB, threads), pairs = n * TA * TB;
                 CHECK(n >= 256 && n % 256 == 0);
                 CHECK(n * threads <= (uint64_t)1 << 31);
