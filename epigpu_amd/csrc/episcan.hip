@@ -153,6 +153,7 @@ struct epi_ctx {
     int4 *cand = nullptr;
     uint32_t *redo = nullptr;
     size_t redo_blocks = 0;
+    bool masks_set = false;  // cleared since the list was built
     // tiles; the device list of the last scan is kept and reused while the
     // dataset, block range, form and schedule stay the same
     int4 *tiles = nullptr;
@@ -1151,7 +1152,7 @@ int upload_tiles(epi_ctx *c, const TileLists &tl)
     }
     c->redo = reinterpret_cast<uint32_t *>(c->tiles + nt);
     c->redo_blocks = blocks;
-    HIPCHK(c, hipMemsetAsync(c->redo + blocks, 0, blocks * sizeof(uint32_t), c->stream));  // the masks
+    c->masks_set = false;
     return copy_tiles(c, c->tiles, tl);
 }
 
@@ -1976,6 +1977,17 @@ int batch_fetch(epi_batch *b)
     return EPI_OK;
 }
 
+// Clears the counters (hits: that of the hits too) and, before the screen first runs over a tile list, the masks of its blocks.
+int reset_scan(epi_ctx *c, bool hits, bool screen)
+{
+    const size_t n = screen && !c->masks_set ? c->redo_blocks : 0;
+    hipLaunchKernelGGL(scan_reset, dim3((unsigned)std::min<size_t>(1 + n / 1024, 1024)), dim3(256), 0, c->stream, c->count,
+                       hits, c->redo + c->redo_blocks, n);
+    HIPCHK(c, hipGetLastError());
+    if (screen) c->masks_set = true;
+    return EPI_OK;
+}
+
 // One scan of the block range of p with schedule sc: tile list, upload,
 // pair kernels, hit count. Records the device time and counts in c. A tile
 // list of up to c->max_tiles tiles is built once and kept on the device; a
@@ -2009,7 +2021,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
     }
     const bool whole = done;  // the list serves later scans
     c->tl_valid = false;  // a scan that fails may leave marked blocks
-    HIPCHK(c, hipMemsetAsync(c->count, 0, sizeof(Counters), c->stream));
+    if ((rc = reset_scan(c, true, screen))) return rc;
     DumpSink ds;
     memset(&ds, 0, sizeof(ds));
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -2040,7 +2052,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
         tl = TileLists();
         done = build_tiles(c->d, be, p->form, sc, max_tiles, cur, tl);
         if ((rc = upload_tiles(c, tl))) return rc;
-        HIPCHK(c, hipMemsetAsync(c->count->screen, 0, sizeof(Counters) - offsetof(Counters, screen), c->stream));
+        if ((rc = reset_scan(c, false, screen))) return rc;
         pairs += tl.pairs;
     }
     float ms = 0.0f;

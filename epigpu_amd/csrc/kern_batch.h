@@ -51,6 +51,18 @@ struct Counters {
     unsigned long long emptied;
 };
 
+// The counters of a scan (of a later piece of it: without the hits), and the masks of the blocks of a new tile list (n words). One small launch (as two
+// hipMemsetAsync calls, a scan at N = 500, M = 2000, of 94 us, took 2.6 us more, and 45 more with a new list).
+__global__ __launch_bounds__(256) void scan_reset(Counters *c, bool hits, uint32_t *mask, size_t n)
+{
+    if (blockIdx.x == 0 && threadIdx.x < 2 * NKIND) c->screen[threadIdx.x] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        c->emptied = 0ull;
+        if (hits) c->nhits = 0ull;
+    }
+    for (size_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) mask[i] = 0u;
+}
+
 // Queue heads of every list ([NKIND][NQ]) and the counters.
 __global__ void batch_reset(int *qpos, const int *qbegin, Counters *n)
 {
