@@ -183,16 +183,18 @@ struct epi_batch {
     ScreenCut *d_cut = nullptr;
     uint32_t *redo = nullptr, *mask = nullptr;  // behind the work items
     int4 *d_work = nullptr;
-    int *d_qpos = nullptr, *d_qbegin = nullptr, *d_qend = nullptr;  // [NKIND][NQ]: FAST, GENERAL, SPARSE items
+    int *d_qpos = nullptr, *d_qbegin = nullptr, *d_qend = nullptr;  // [NLIST][NQ]
     size_t work_cap = 0, scan_cap = 0;
-    long long nkind[NKIND] = {0, 0, 0};  // work items of each tile kind (FAST first in d_work)
-    std::vector<std::pair<int, long long>> segs[NKIND];  // the datasets of a list, in its order, and their items
+    long long nlist[NLIST] = {};  // work items of each list (in this order in d_work)
+    std::vector<std::pair<int, long long>> segs[NKIND];  // the datasets of a screened list, in its order, and their items
     DevHit *hits = nullptr;
     Counters *count = nullptr;
     long long cap = 1ll << 22;
     // work list of the last build
     epi_schedule sched[2];  // per form
     epi_schedule work_sched = {};
+    std::vector<char> work_scr;  // the scans that are screened
+    int scr_rows = 0;            // tile height of their lists
     bool dirty = true;
     int work_form = -1;
     long long nwork = 0, pairs = 0;
@@ -1559,30 +1561,34 @@ void emit_hits(const Dataset &d, const DevHit *h, const std::vector<int> &idx, e
 // so that the longest items do not end up in the tail. With 8 queues the list
 // is cut into NQ contiguous pieces of equal estimated cost, one per XCD;
 // with 1 queue every workgroup pulls from one shared queue.
+// The scans of `scr` have lists of their own, with tiles of scr_rows.
 constexpr size_t batch_blocks(int kind) { return scr_blocks(64, kind == 1 ? 32 : 64, kind != 0); }
 
-int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
+int build_batch_work(epi_batch *b, int form, const epi_schedule &sched, const std::vector<char> &scr, int scr_rows)
 {
     epi_ctx *c = b->ctx;
     const int nd = (int)b->data.size();
-    std::vector<std::vector<int4>> wk[NKIND];
-    std::vector<std::vector<double>> ct[NKIND];
-    for (int kind = 0; kind < NKIND; kind++) {
-        wk[kind].resize(nd);
-        ct[kind].resize(nd);
+    std::vector<std::vector<int4>> wk[NLIST];
+    std::vector<std::vector<double>> ct[NLIST];
+    for (int l = 0; l < NLIST; l++) {
+        wk[l].resize(nd);
+        ct[l].resize(nd);
     }
     b->pairs = 0;
     // estimated cost per pair and individual, by kind
     const double unit[NKIND] = {form == EPI_FORM_MFMA ? 16.0 : 4.0, form == EPI_FORM_MFMA ? 40.0 : 10.0, 22.0};
-    for (int di = 0; di < nd; di++) {
+    for (int i = 0; i < 2 * nd; i++) {
+        const int di = i / 2, g = i % 2;
         const Dataset &d = *b->data[di];
         std::vector<int> sc;
         for (int s = 0; s < (int)b->scans.size(); s++)
-            if (b->scans[s].first == di) sc.push_back(s);
+            if (b->scans[s].first == di && !scr[s] == (g == 1)) sc.push_back(s);
         if (sc.empty()) continue;
         TileLists tl;
         TileCursor all;
-        build_tiles(d, 1 << 30, form, sched, SIZE_MAX, all, tl);
+        epi_schedule sg = sched;
+        if (!g) sg.fast_rows = scr_rows;
+        build_tiles(d, 1 << 30, form, sg, SIZE_MAX, all, tl);
         b->pairs += tl.pairs * (long long)sc.size();
         for (int kind = 0; kind < NKIND; kind++) {
             const std::vector<int4> &v = kind == 0 ? tl.fast : kind == 1 ? tl.gen : tl.sp;
@@ -1590,8 +1596,8 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
                 int ext = (t.y - t.x) | ((t.w - t.z) << 8) | (kind << 16);
                 double cst = (double)(t.y - t.x) * (t.w - t.z) * d.Kp * unit[kind] + 5e4;
                 for (int s : sc) {
-                    wk[kind][di].push_back(make_int4(t.x, t.z, ext, s));
-                    ct[kind][di].push_back(cst);
+                    wk[NKIND * g + kind][di].push_back(make_int4(t.x, t.z, ext, s));
+                    ct[NKIND * g + kind][di].push_back(cst);
                 }
             }
         }
@@ -1601,25 +1607,25 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     if (sched.order == 2)
         std::stable_sort(dorder.begin(), dorder.end(),
                          [&](int x, int y) { return b->data[x]->Kp > b->data[y]->Kp; });
-    // One list per tile kind (FAST items first in the work array), each run by its own persistent
+    // One list per tile kind, each run by its own
     // kernel so that a kernel holds the registers of one tile kind only; within a list the datasets
     // follow the schedule's order. Each list is cut into its own queues.
     std::vector<int4> work;
-    std::vector<int> qbegin(NKIND * NQ), qend(NKIND * NQ);
-    for (int kind = 0; kind < NKIND; kind++) {
+    std::vector<int> qbegin(NLIST * NQ), qend(NLIST * NQ);
+    for (int l = 0; l < NLIST; l++) {
         const int base = (int)work.size();
         std::vector<double> cost;
-        b->segs[kind].clear();
+        if (l < NKIND) b->segs[l].clear();
         for (int di : dorder) {
-            if (!wk[kind][di].empty()) b->segs[kind].push_back({di, (long long)wk[kind][di].size()});
-            work.insert(work.end(), wk[kind][di].begin(), wk[kind][di].end());
-            cost.insert(cost.end(), ct[kind][di].begin(), ct[kind][di].end());
+            if (l < NKIND && !wk[l][di].empty()) b->segs[l].push_back({di, (long long)wk[l][di].size()});
+            work.insert(work.end(), wk[l][di].begin(), wk[l][di].end());
+            cost.insert(cost.end(), ct[l][di].begin(), ct[l][di].end());
         }
         static_assert(SCR_TILES > INT32_MAX / 2, "the screen numbers the blocks of any list");
         if (work.size() > (size_t)INT32_MAX / 2) return fail(c, EPI_ERR_RANGE, "batch has too many tiles");
         const int n = (int)work.size();
-        b->nkind[kind] = n - base;
-        int *qb = qbegin.data() + kind * NQ, *qe = qend.data() + kind * NQ;
+        b->nlist[l] = n - base;
+        int *qb = qbegin.data() + l * NQ, *qe = qend.data() + l * NQ;
         for (int q = 0; q < NQ; q++) qb[q] = qe[q] = n;
         qb[0] = base;
         if (sched.queues == 1) {
@@ -1642,7 +1648,7 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     int rc;
     // behind the items, room for the number and the mask of every block of the screen's tiles, of 64 or 32 rows
     size_t blocks = 0;
-    for (int kind = 0; kind < NKIND; kind++) blocks += batch_blocks(kind) * (size_t)b->nkind[kind];
+    for (int kind = 0; kind < NKIND; kind++) blocks += batch_blocks(kind) * (size_t)b->nlist[kind];
     const size_t room = work.size() + (2 * blocks * sizeof(uint32_t) + sizeof(int4) - 1) / sizeof(int4);
     if (room > b->work_cap) {
         b->work_cap = 0;
@@ -1655,9 +1661,9 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     if (!work.empty())
         HIPCHK(c, hipMemcpyAsync(b->d_work, work.data(), work.size() * sizeof(int4), hipMemcpyHostToDevice,
                                  c->stream));
-    HIPCHK(c, hipMemcpyAsync(b->d_qbegin, qbegin.data(), NKIND * NQ * sizeof(int), hipMemcpyHostToDevice,
+    HIPCHK(c, hipMemcpyAsync(b->d_qbegin, qbegin.data(), NLIST * NQ * sizeof(int), hipMemcpyHostToDevice,
                              c->stream));
-    HIPCHK(c, hipMemcpyAsync(b->d_qend, qend.data(), NKIND * NQ * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(b->d_qend, qend.data(), NLIST * NQ * sizeof(int), hipMemcpyHostToDevice, c->stream));
     // scan descriptors
     size_t ns = b->scans.size();
     if (ns > b->scan_cap) {
@@ -1676,6 +1682,8 @@ int build_batch_work(epi_batch *b, int form, const epi_schedule &sched)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     b->work_form = form;
     b->work_sched = sched;
+    b->work_scr = scr;
+    b->scr_rows = scr_rows;
     b->dirty = false;
     return EPI_OK;
 }
@@ -1729,13 +1737,13 @@ const void *batch_kernel(int form, const epi_schedule &sc, int kind)
     return kind ? (const void *)plain_batch_kernel<256, 1> : (const void *)plain_batch_kernel<256, 0>;
 }
 
-// Whether a batch's tiles with missing calls contract those: one answer for the list, that of most of its work.
+// Whether a batch's screened tiles with missing calls contract those: one answer for the list, that of most of its work.
 bool batch_nocall(const epi_batch *b)
 {
     double large = 0.0, all = 0.0;
-    for (const auto &x : b->scans) {
-        const Dataset &d = *b->data[x.first];
-        if (!d.missum[d.nsnp]) continue;
+    for (size_t s = 0; s < b->scans.size(); s++) {
+        const Dataset &d = *b->data[b->scans[s].first];
+        if (!b->work_scr[s] || !d.missum[d.nsnp]) continue;
         const double w = (double)d.nsnp * d.nsnp * d.nid;
         all += w;
         if (scr_nocall((d.nid + KC - 1) / KC * KC)) large += w;
@@ -1766,22 +1774,27 @@ const void *redo_batch_fn(const epi_schedule &sc, int kind)
                      : (const void *)redo_kernel<32, 64, false, true>;
 }
 
-// The scans' cuts, and whether the batch goes through the screen: where it is long enough and at least half of
-// its scans are screened (the tiles of the others are redone whole, by exact tiles).
-bool batch_screen(const epi_batch *b, const epi_scan_params *p, std::vector<ScreenCut> &cut)
+// The scans' cuts and which of them go through the screen (scr): those that it would take by themselves, where
+// their work together is worth its launches. The others keep the exact tiles. (Screening the whole batch where half of its scans by
+// number allowed it, the rest redone after: a study of N = 1000, M = 3000 beside one of N = 4000, M = 20000 with an
+// outlier took 13.5 ms; the exact tiles alone, and this rule, 12.0.)
+bool batch_screen(const epi_batch *b, const epi_scan_params *p, std::vector<ScreenCut> &cut, std::vector<char> &scr)
 {
-    if (p->form != EPI_FORM_MFMA) return false;
-    cut.resize(b->scans.size());
-    size_t ok = 0;
+    const size_t n = b->scans.size();
+    cut.resize(n);
+    scr.assign(n, 0);
     double work = 0.0;
-    for (size_t s = 0; s < cut.size(); s++) {
+    for (size_t s = 0; s < n; s++) {
         const Dataset &d = *b->data[b->scans[s].first];
         const int nchr = (int)d.chrstart.size();
         memset(&cut[s], 0, sizeof(ScreenCut));
-        if (screen_fits(d) && screen_cut(d.ph[b->scans[s].second], p, cut[s])) ok++;  // cut.nd stays 0 otherwise
+        if (p->form != EPI_FORM_MFMA || !screen_fits(d) || !screen_cut(d.ph[b->scans[s].second], p, cut[s])) continue;
+        scr[s] = 1;
         work += (double)block_pairs(d, 0, nchr * (nchr + 1) / 2) * d.nid * (d.missum[d.nsnp] ? 2.5 : 1.0);
     }
-    return 2 * ok >= cut.size() && work >= SCR_MIN_WORK;
+    if (work >= SCR_MIN_WORK) return true;
+    scr.assign(n, 0);
+    return false;
 }
 
 // Items of the next launch of a list through the screen, of `left`: as many as scr_chunk allows at the mean rate of each
@@ -1789,7 +1802,7 @@ bool batch_screen(const epi_batch *b, const epi_scan_params *p, std::vector<Scre
 // list's segment and the items taken from it.
 int batch_chunk(const epi_batch *b, const std::vector<ScreenCut> &cut, int kind, int threads, int left, size_t &seg, long long &used)
 {
-    const int TA = b->work_sched.fast_rows, TB = kind == 1 ? 32 : 64;
+    const int TA = b->scr_rows, TB = kind == 1 ? 32 : 64;
     int n = 0;
     double full = 0.0;  // part of a launch taken
     while (seg < b->segs[kind].size() && n < left) {
@@ -1797,7 +1810,7 @@ int batch_chunk(const epi_batch *b, const std::vector<ScreenCut> &cut, int kind,
         double rate = 0.0;
         int ns = 0;
         for (size_t i = 0; i < b->scans.size(); i++)
-            if (b->scans[i].first == s.first) rate += cut[i].rate, ns++;
+            if (b->scans[i].first == s.first && b->work_scr[i]) rate += cut[i].rate, ns++;
         const double most = scr_chunk(rate / ns, TA, TB, threads);
         const long long fit = (long long)((1.0 - full) * most), take = std::min(s.second - used, fit);
         n += (int)take;
@@ -1817,10 +1830,10 @@ int batch_chunk(const epi_batch *b, const std::vector<ScreenCut> &cut, int kind,
     return up;
 }
 
-// Capture queue reset + the persistent scan kernels as one graph: one kernel
-// per tile kind that has items (GENERAL and SPARSE first under order 1), each with a grid
-// of its occupancy times the CU count, so that every workgroup is resident and
-// pulls work until its queues run dry.
+// Capture queue reset + the scan kernels as one graph: one kernel
+// per list that has items (GENERAL and SPARSE first under order 1). Those of the exact tiles are persistent, with a grid
+// of their occupancy times the CU count, so that every workgroup is resident and
+// pulls work until its queues run dry; the screen's take a workgroup per item, each followed by resolve and redo.
 int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<ScreenCut> *cut)
 {
     epi_ctx *c = b->ctx;
@@ -1829,70 +1842,84 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
         HIPCHK(c, hipMemcpyAsync(b->d_cut, cut->data(), cut->size() * sizeof(ScreenCut), hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
     }
-    BatchArgs B[NKIND];
-    const void *kfn[NKIND];
-    int grid[NKIND] = {0, 0, 0}, nt[NKIND];
-    bool screen[NKIND];
+    // The lists in the order of their launches: per kind the screened scans, then the others
+    struct List {
+        int kind, n, nt, grid;
+        bool screen;
+        const void *fn;
+        BatchArgs B;
+        ScreenBatchArgs G;
+    };
+    std::vector<List> lists;
     int Kl = 0;
-    for (const Dataset *d : b->data) Kl = std::max(Kl, (d->nid + KC - 1) / KC * KC);
-    ScreenBatchArgs G[NKIND];
+    for (size_t s = 0; s < b->scans.size(); s++)
+        if (b->work_scr[s]) Kl = std::max(Kl, (b->data[b->scans[s].first]->nid + KC - 1) / KC * KC);
     const int4 *work = b->d_work;
     uint32_t *redo = b->redo, *mask = b->mask;
-    for (int kind = 0; kind < NKIND; kind++) {
-        screen[kind] = cut && !(kind == 2 && b->work_sched.dense_missing == 2);  // SPARSE tiles that the schedule asks for
-        nt[kind] = screen[kind] ? 4 * b->work_sched.fast_rows : batch_threads_of(p->form, b->work_sched, kind);
-        G[kind] = {b->d_mscan, b->d_cut, work, 0, 0, {c->cand, b->count->screen + 2 * kind, CAND_CAP, redo, mask}};
-        work += b->nkind[kind];
-        redo += batch_blocks(kind) * (size_t)b->nkind[kind];
-        mask += batch_blocks(kind) * (size_t)b->nkind[kind];
-        B[kind].mscan = b->d_mscan;
-        B[kind].pscan = b->d_pscan;
-        B[kind].work = b->d_work;
-        B[kind].qpos = b->d_qpos + kind * NQ;
-        B[kind].qend = b->d_qend + kind * NQ;
-        B[kind].hs = make_sink(b->hits, &b->count->nhits, b->cap, p);
-        kfn[kind] = screen[kind] ? screen_batch_fn(b->work_sched, kind, batch_nocall(b)) : batch_kernel(p->form, b->work_sched, kind);
+    for (int l = 0; l < NLIST; l++) {
+        const int kind = l % NKIND, n = (int)b->nlist[l];
+        epi_schedule sg = b->work_sched;
+        if (l < NKIND) sg.fast_rows = b->scr_rows;
+        List L = {};
+        L.kind = kind;
+        L.n = n;
+        L.screen = l < NKIND && !(kind == 2 && sg.dense_missing == 2);  // SPARSE tiles that the schedule asks for
+        L.nt = L.screen ? 4 * sg.fast_rows : batch_threads_of(p->form, sg, kind);
+        L.G = {b->d_mscan, b->d_cut, work, 0, 0, {c->cand, b->count->screen + 2 * kind, CAND_CAP, redo, mask}};
+        L.B = {b->d_mscan, b->d_pscan, b->d_work, b->d_qpos + l * NQ, b->d_qend + l * NQ,
+               make_sink(b->hits, &b->count->nhits, b->cap, p)};
+        work += n;
+        if (l < NKIND) {
+            redo += batch_blocks(kind) * (size_t)n;
+            mask += batch_blocks(kind) * (size_t)n;
+        }
+        if (!n) continue;
+        L.fn = L.screen ? screen_batch_fn(sg, kind, batch_nocall(b)) : batch_kernel(p->form, sg, kind);
         int per_cu = 1;
-        HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn[kind], nt[kind], 0));
-        grid[kind] = std::max(1, per_cu) * c->ncu;
+        HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, L.fn, L.nt, 0));
+        L.grid = std::max(1, per_cu) * c->ncu;
+        lists.push_back(L);
     }
-    static const int korder[2][NKIND] = {{0, 2, 1}, {1, 2, 0}};
-    const int *ko = korder[b->work_sched.order == 1 ? 1 : 0];
+    // FAST, SPARSE, GENERAL; under order 1 GENERAL and SPARSE first
+    static const int place[2][NKIND] = {{0, 2, 1}, {2, 0, 1}};
+    const int *pl = place[b->work_sched.order == 1 ? 1 : 0];
+    std::stable_sort(lists.begin(), lists.end(), [&](const List &x, const List &y) { return pl[x.kind] < pl[y.kind]; });
+    epi_schedule scr_sched = b->work_sched;
+    scr_sched.fast_rows = b->scr_rows;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     hipLaunchKernelGGL(batch_reset, dim3(1), dim3(64), 0, c->stream, b->d_qpos, (const int *)b->d_qbegin, b->count);
     hipError_t le = hipGetLastError();
-    for (int t = 0; t < NKIND && le == hipSuccess; t++) {
-        const int kind = ko[t];
-        if (b->nkind[kind] == 0) continue;
-        if (!screen[kind]) {
-            void *args[] = {&B[kind]};
-            le = hipLaunchKernel(kfn[kind], dim3(grid[kind]), dim3(nt[kind]), args, 0, c->stream);
+    for (List &L : lists) {
+        if (le != hipSuccess) break;
+        if (!L.screen) {
+            void *args[] = {&L.B};
+            le = hipLaunchKernel(L.fn, dim3(L.grid), dim3(L.nt), args, 0, c->stream);
             continue;
         }
         // one workgroup per item, a list of candidates at a time
-        const int4 *items = G[kind].work;
-        const int n = (int)b->nkind[kind], halves = kind == 2 ? 2 : 1;
-        ResolveArgs R = {{}, b->d_mscan, B[kind].hs, c->cand, G[kind].cs.count, CAND_CAP, resolve_lanes(Kl)};
-        RedoArgs D = {{}, b->d_mscan, B[kind].hs, items, G[kind].cs.count, G[kind].cs.redo, G[kind].cs.mask};
+        const int4 *items = L.G.work;
+        const int halves = L.kind == 2 ? 2 : 1;
+        ResolveArgs R = {{}, b->d_mscan, L.B.hs, c->cand, L.G.cs.count, CAND_CAP, resolve_lanes(Kl)};
+        RedoArgs D = {{}, b->d_mscan, L.B.hs, items, L.G.cs.count, L.G.cs.redo, L.G.cs.mask};
         void *rargs[] = {&R}, *dargs[] = {&D};
         size_t seg = 0;
         long long used = 0;
-        for (int t0 = 0; t0 < n && le == hipSuccess;) {
-            if (t0) hipLaunchKernelGGL(empty_list, dim3(1), dim3(1), 0, c->stream, G[kind].cs.count, CAND_CAP, &b->count->emptied);
-            const int chunk = batch_chunk(b, *cut, kind, nt[kind] * halves, n - t0, seg, used);
-            G[kind].work = items + t0;
-            G[kind].item0 = t0;
-            G[kind].nitems = chunk;
-            void *args[] = {&G[kind]};
+        for (int t0 = 0; t0 < L.n && le == hipSuccess;) {
+            if (t0) hipLaunchKernelGGL(empty_list, dim3(1), dim3(1), 0, c->stream, L.G.cs.count, CAND_CAP, &b->count->emptied);
+            const int chunk = batch_chunk(b, *cut, L.kind, L.nt * halves, L.n - t0, seg, used);
+            L.G.work = items + t0;
+            L.G.item0 = t0;
+            L.G.nitems = chunk;
+            void *args[] = {&L.G};
             le = hipGetLastError();
-            if (le == hipSuccess) le = hipLaunchKernel(kfn[kind], dim3(chunk * halves), dim3(nt[kind]), args, 0, c->stream);
+            if (le == hipSuccess) le = hipLaunchKernel(L.fn, dim3(chunk * halves), dim3(L.nt), args, 0, c->stream);
             if (le == hipSuccess)
-                le = hipLaunchKernel(kind ? (const void *)resolve_kernel<true, true> : (const void *)resolve_kernel<false, true>,
+                le = hipLaunchKernel(L.kind ? (const void *)resolve_kernel<true, true> : (const void *)resolve_kernel<false, true>,
                                      dim3(4 * c->ncu), dim3(256), rargs, 0, c->stream);
             t0 += chunk;
         }
         if (le == hipSuccess)
-            le = hipLaunchKernel(redo_batch_fn(b->work_sched, kind), dim3(2 * c->ncu), dim3(256), dargs, 0, c->stream);
+            le = hipLaunchKernel(redo_batch_fn(scr_sched, L.kind), dim3(2 * c->ncu), dim3(256), dargs, 0, c->stream);
     }
     hipError_t ce = hipStreamEndCapture(c->stream, &b->graph);
     if (le != hipSuccess) return fail(c, EPI_ERR_HIP, "launch during capture: %s", hipGetErrorString(le));
@@ -1900,12 +1927,9 @@ int capture_batch(epi_batch *b, const epi_scan_params *p, const std::vector<Scre
     HIPCHK(c, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
     b->gkey = *p;
     b->gvalid = true;
-    b->gscreened = 0;
-    if (cut)
-        for (const ScreenCut &x : *cut) b->gscreened += x.nd != 0;
+    b->gscreened = (int)std::count(b->work_scr.begin(), b->work_scr.end(), 1);
     b->grid = 0;
-    for (int kind = 0; kind < NKIND; kind++)
-        if (b->nkind[kind]) b->grid = std::max(b->grid, grid[kind]);
+    for (const List &L : lists) b->grid = std::max(b->grid, L.grid);
     b->captures++;
     return EPI_OK;
 }
@@ -1918,15 +1942,17 @@ int batch_prepare(epi_batch *b, const epi_scan_params *p)
     if (p->form == EPI_FORM_MFMA)
         for (const auto &x : b->scans)
             if ((rc = check_mfma_phen(b->ctx, *b->data[x.first], x.second))) return rc;
-    epi_schedule sc = b->sched[p->form];
+    const epi_schedule &sc = b->sched[p->form];
     std::vector<ScreenCut> cut;
-    const bool screen = batch_screen(b, p, cut);
+    std::vector<char> scr;
+    const bool screen = batch_screen(b, p, cut, scr);
     int nid = 0;
-    for (const Dataset *d : b->data) nid = std::max(nid, d->nid);
-    if (screen) sc.fast_rows = screen_rows(nid);
-    if (b->dirty || b->work_form != p->form || !same_schedule(b->work_sched, sc)) {
+    for (size_t s = 0; s < scr.size(); s++)
+        if (scr[s]) nid = std::max(nid, b->data[b->scans[s].first]->nid);
+    const int rows = screen_rows(nid);
+    if (b->dirty || b->work_form != p->form || !same_schedule(b->work_sched, sc) || b->work_scr != scr || b->scr_rows != rows) {
         drop_graph(b);
-        if ((rc = build_batch_work(b, p->form, sc))) return rc;
+        if ((rc = build_batch_work(b, p->form, sc, scr, rows))) return rc;
     }
     if (!b->gvalid || !same_key(b->gkey, *p))
         if ((rc = capture_batch(b, p, screen ? &cut : nullptr))) return rc;
@@ -2565,8 +2591,8 @@ int epi_batch_create(epi_ctx *c, epi_batch **out)
     b->ctx = c;
     for (int f = 0; f < 2; f++) b->sched[f] = default_schedule(f);
     int rc;
-    if ((rc = dalloc(c, b->d_qpos, NKIND * NQ)) || (rc = dalloc(c, b->d_qbegin, NKIND * NQ)) ||
-        (rc = dalloc(c, b->d_qend, NKIND * NQ)) ||
+    if ((rc = dalloc(c, b->d_qpos, NLIST * NQ)) || (rc = dalloc(c, b->d_qbegin, NLIST * NQ)) ||
+        (rc = dalloc(c, b->d_qend, NLIST * NQ)) ||
         (rc = dalloc(c, b->count, 1)) || (rc = dalloc(c, b->hits, (size_t)b->cap))) {
         epi_batch_destroy(b);
         return rc;

@@ -1,8 +1,9 @@
 // Persistent batched scan: one launch walks the tiles of many scans (datasets
 // of uneven N and M, and several phenotypes per dataset).
 //
-// The host keeps one work list per tile kind (FAST, GENERAL, SPARSE), each run by its
-// own persistent kernel so that a kernel holds the registers of one tile kind
+// The host keeps one work list per tile kind (FAST, GENERAL, SPARSE) for the scans that go through the screen
+// and one for the others, each run by its
+// own kernel (persistent, but for the screen's) so that a kernel holds the registers of one tile kind
 // only. It orders the items of a list so that consecutive items share SNP data
 // (tile-major, phenotype-minor) and cuts the list into NQ contiguous queues of
 // equal estimated cost, one per XCD. A workgroup pulls items from the queue of
@@ -24,6 +25,7 @@ namespace epi {
 
 constexpr int NQ = 8;     // work queues, one per XCD
 constexpr int NKIND = 3;  // tile kinds: 0 FAST, 1 GENERAL, 2 SPARSE
+constexpr int NLIST = 2 * NKIND;  // work lists: the kinds of the screened scans, then of the others
 
 struct BatchArgs {
     const MfmaScan *mscan;   // [nscan]
@@ -63,11 +65,11 @@ __global__ __launch_bounds__(256) void scan_reset(Counters *c, bool hits, uint32
     for (size_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) mask[i] = 0u;
 }
 
-// Queue heads of every list ([NKIND][NQ]) and the counters.
+// Queue heads of every list ([NLIST][NQ]) and the counters.
 __global__ void batch_reset(int *qpos, const int *qbegin, Counters *n)
 {
     const int t = threadIdx.x;
-    if (t < NKIND * NQ) qpos[t] = qbegin[t];
+    if (t < NLIST * NQ) qpos[t] = qbegin[t];
     if (t < 2 * NKIND) n->screen[t] = 0u;
     if (t == 0) n->nhits = n->emptied = 0ull;
 }
@@ -142,7 +144,7 @@ __global__ __launch_bounds__((batch_threads<TA, KIND>()), (batch_waves_per_simd<
 
 // A list through the screen: one workgroup per item (two per SPARSE item), in the order of the list, with the XCD
 // mapping of single scans (a persistent grid that pulls from the queues measured 5 % more at N = 4000, M = 20000).
-// Tiles of scans that the screen does not take go to the redo list whole. NC (screen_gen_tile) is one for the list: both
+// NC (screen_gen_tile) is one for the list: both
 // variants in one kernel cost 1.5 % at N = 2504.
 template <int TA, int KIND, bool NC = false>
 __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_batch_kernel(const ScreenBatchArgs B)
@@ -161,13 +163,6 @@ __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_batch_kernel(cons
     const MfmaScan S = B.mscan[sc];
     const ScreenCut C = B.cut[sc];
     uint32_t block0 = (uint32_t)(B.item0 + it) * NBLK;
-    if (!C.nd) {
-        if (threadIdx.x < NBLK && t % HALVES == 0) {
-            B.cs.mask[block0 + threadIdx.x] = 3u;
-            B.cs.redo[atomicAdd(B.cs.count + 1, 1u)] = block0 + threadIdx.x;
-        }
-        return;
-    }
     if constexpr (KIND == 0) {
         if (C.nd == 1)
             screen_fast_tile<TA, 1>(S, C, B.cs, a0, a1, b0, b1, block0, wl, mg, mg2);

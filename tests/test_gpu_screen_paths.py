@@ -160,3 +160,29 @@ def test_dense_blocks(scanner, buf, nid, gmiss):
     print(f"dense nid={nid} gmiss={gmiss} hits {g['nhits']} of {g['pairs']} {scr} blocks {blocks}", flush=True)
     assert scr["digits"] and blocks / 2 < scr["redone"] <= blocks
     assert same_as_exact(scanner, buf, g, **kw) > 0.2 * g["pairs"]
+
+
+@pytest.mark.parametrize("gmiss,dense_missing", [(0.0, 0), (0.002, 0), (0.002, 2), (0.02, 0)])
+def test_batch_mixed(scanner, buf, gmiss, dense_missing):
+    """Scans that are not screened (an outlier) keep the exact kernels of their tiles, beside screened ones of the same and of
+    other datasets."""
+    data = [(1000, [1600], 0.0, [0]), (2500, [1900, 433], gmiss, [1, 0, 1])]
+    kw = dict(test="i", t1=5.0, t2=7.0)
+    with E.Batch(scanner) as b:
+        b.set_schedule("mfma", dense_missing=dense_missing)
+        made = []
+        for i, (nid, sizes, gm, outlier) in enumerate(data):
+            words = E.synth_genotypes(61 + i, nid, sum(sizes), 0.1, 0.5, gm)
+            y = np.stack([phenotype("normal", nid, 70 + i + 5 * r) for r in range(len(outlier))])
+            y[np.array(outlier) == 1, 11] = 1e4
+            y[0] += 8.0 / np.sqrt(nid) * (S.unpack(words[40:41], nid)[0] % 3)
+            d = b.add_dataset(words, nid, list(np.cumsum([0] + sizes[:-1])), sizes)
+            made += [(words, nid, sizes, yy, s) for yy, s in zip(y, b.add_phenotypes(d, y))]
+        for rep in range(3):
+            b.scan(**kw)
+            scr = b.last_screen()
+            print(f"mixed gmiss={gmiss} dense_missing={dense_missing} replay={rep} {b.stats()} {scr}", flush=True)
+            assert scr["scans"] == 2 and scr["redone"] == 0
+        for words, nid, sizes, y, s in made:
+            load(scanner, words, nid, y, sizes)
+            assert same_as_exact(scanner, buf, b.hits(s), **kw) > 0
