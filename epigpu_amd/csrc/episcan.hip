@@ -3,7 +3,7 @@
 // Device state of one dataset (a context holds one; a batch holds many):
 //   words   [nsnp][npack1] int32   genotypes as uploaded (layout A1), freed after the transcode
 //   mbits   [3][Kw][nsnp]  uint32  bitplanes of classes 0, 1 and call present (MFMA form)
-//   sbits   [3][nsnp][Kw]  uint32  the same by SNP (resolve kernel), or null
+//   sbits   [3][nsnp][Kw]  uint32  the same by SNP (resolve kernel), or null: given back where memory is short
 //   bits    [3][Kw][nsnp]  uint32  bitplanes of the two rarest classes and call present (plain form)
 //   cls     [nsnp]         int32   plain-form plane -> class map
 //   per phenotype r (wts, mp, yc, yw, vbits, ov and oidx in one allocation):
@@ -106,7 +106,7 @@ struct Dataset {
     int nid = 0, nsnp = 0, npack1 = 0, Kp = 0, Kw = 0;
     int32_t *words = nullptr;
     uint32_t *mbits = nullptr;
-    uint32_t *sbits = nullptr;  // behind mbits
+    uint32_t *sbits = nullptr;
     uint32_t *bits = nullptr;
     int32_t *dmiss = nullptr;
     int32_t *cls = nullptr;
@@ -144,11 +144,12 @@ struct epi_ctx {
     std::string err;
     char name[256] = {0};
     Dataset d;
+    std::vector<epi_batch *> batches;
     // hits
     DevHit *hits = nullptr;
     long long cap = 1ll << 22;
     long long last_nhits = 0;
-    // counters of the hits and of the screen; candidates; blocks to redo and their masks (behind the tiles)
+    // counters of the hits and of the screen; candidates; blocks to redo and their masks (behind the tiles, or null)
     Counters *count = nullptr;
     int4 *cand = nullptr;
     uint32_t *redo = nullptr;
@@ -246,14 +247,21 @@ void dfree(T *&p)
     p = nullptr;
 }
 
+bool give_back(epi_ctx *c);
+
 template <class T>
 int dalloc(epi_ctx *c, T *&p, size_t count)
 {
     dfree(p);
     if (count == 0) count = 1;
     hipError_t e = hipMalloc((void **)&p, count * sizeof(T));
+    if (e != hipSuccess && give_back(c)) {
+        (void)hipGetLastError();
+        e = hipMalloc((void **)&p, count * sizeof(T));
+    }
     if (e != hipSuccess) {
         p = nullptr;
+        (void)hipGetLastError();  // not to be found after a later launch
         return fail(c, EPI_ERR_NOMEM, "hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
     }
     return EPI_OK;
@@ -294,13 +302,32 @@ void free_dataset(Dataset &d)
 {
     dfree(d.words);
     dfree(d.mbits);
-    d.sbits = nullptr;
+    dfree(d.sbits);
     dfree(d.bits);
     dfree(d.dmiss);
     dfree(d.cls);
     drop_sparse(d);
     for (auto &p : d.ph) free_phen(p);
     d.ph.clear();
+}
+
+// The bits by SNP of every dataset of the context, which scans can do without, to an allocation that failed.
+// Whether there were any. The batches' descriptors point to them and are built again.
+bool give_back(epi_ctx *c)
+{
+    if (!c) return false;
+    bool any = c->d.sbits != nullptr;
+    for (epi_batch *b : c->batches)
+        for (Dataset *d : b->data) any |= d->sbits != nullptr;
+    if (!any) return false;
+    (void)hipStreamSynchronize(c->stream);
+    dfree(c->d.sbits);
+    for (epi_batch *b : c->batches)
+        for (Dataset *d : b->data) {
+            if (d->sbits) b->dirty = true;
+            dfree(d->sbits);
+        }
+    return true;
 }
 
 // ------------------------------------------------------ dataset preparation --
@@ -330,22 +357,19 @@ int ds_upload_genotypes(epi_ctx *c, Dataset &d, const int32_t *words, int nid, i
     d.Kw = d.Kp / 32;
     size_t nwords = (size_t)nsnp * d.npack1;
     int rc;
-    // Bits by SNP, where the screen can run and memory allows (scans without it take the exact tiles): the lanes of the resolve kernel, one word each,
-    // then read a SNP's words in a row (N = 3001, 67,000 hits: resolve 250 -> 156 us; N = 2000: 84 -> 42 us).
     const size_t planes = (size_t)3 * d.Kw * nsnp;
-    dfree(d.mbits);
-    d.sbits = nullptr;
-    if (planes_fit(d) && hipMalloc((void **)&d.mbits, 2 * planes * sizeof(uint32_t)) == hipSuccess) {
-        d.sbits = d.mbits + planes;
-    } else {
-        d.mbits = nullptr;
-        (void)hipGetLastError();
-        if ((rc = dalloc(c, d.mbits, planes))) return rc;
-    }
-    if ((rc = dalloc(c, d.words, nwords)) ||
-        (rc = dalloc(c, d.bits, (size_t)3 * d.Kw * nsnp)) || (rc = dalloc(c, d.dmiss, (size_t)4 * nsnp)) ||
+    dfree(d.sbits);
+    if ((rc = dalloc(c, d.mbits, planes)) || (rc = dalloc(c, d.words, nwords)) ||
+        (rc = dalloc(c, d.bits, planes)) || (rc = dalloc(c, d.dmiss, (size_t)4 * nsnp)) ||
         (rc = dalloc(c, d.cls, (size_t)nsnp)))
         return rc;
+    // Bits by SNP, where the screen can run and memory allows: the lanes of the resolve kernel, one word each,
+    // then read a SNP's words in a row (N = 3001, 67,000 hits: resolve 250 -> 156 us; N = 2000: 84 -> 42 us). Allocated last, and
+    // given back to whatever later finds no memory (give_back).
+    if (planes_fit(d) && hipMalloc((void **)&d.sbits, planes * sizeof(uint32_t)) != hipSuccess) {
+        d.sbits = nullptr;
+        (void)hipGetLastError();
+    }
     HIPCHK(c, hipMemcpyAsync(d.words, words, nwords * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
     int *cnt = d.dmiss + nsnp;  // class counts of the SNPs
     HIPCHK(c, hipMemsetAsync(cnt, 0, 3 * (size_t)nsnp * sizeof(int), c->stream));
@@ -1138,12 +1162,13 @@ int copy_tiles(epi_ctx *c, int4 *dst, const TileLists &tl)
     return EPI_OK;
 }
 
-int upload_tiles(epi_ctx *c, const TileLists &tl)
+int upload_tiles(epi_ctx *c, const TileLists &tl, bool screen)
 {
     c->tl_valid = false;
-    // behind the tiles, room for the number and the mask of every block of the screen's tiles, of 64 or 32 rows
+    // behind the tiles of a screened scan, room for the number and the mask of every block, of 64- or 32-row tiles
     const size_t nt = tl.count();
-    const size_t blocks = scr_blocks(64, 64, false) * (tl.fast.size() + tl.gen.size()) + scr_blocks(64, 64, true) * tl.sp.size();
+    size_t blocks = scr_blocks(64, 64, false) * (tl.fast.size() + tl.gen.size()) + scr_blocks(64, 64, true) * tl.sp.size();
+    if (!screen) blocks = 0;
     const size_t need = nt + (2 * blocks * sizeof(uint32_t) + sizeof(int4) - 1) / sizeof(int4);
     static_assert(scr_blocks(64, 64, false) == scr_blocks(64, 32, true), "one count of blocks for FAST and GENERAL tiles");
     if (need > c->tiles_cap) {
@@ -1152,7 +1177,7 @@ int upload_tiles(epi_ctx *c, const TileLists &tl)
         if (rc) return rc;
         c->tiles_cap = need;
     }
-    c->redo = reinterpret_cast<uint32_t *>(c->tiles + nt);
+    c->redo = screen ? reinterpret_cast<uint32_t *>(c->tiles + nt) : nullptr;
     c->redo_blocks = blocks;
     c->masks_set = false;
     return copy_tiles(c, c->tiles, tl);
@@ -1326,11 +1351,11 @@ bool screen_cut(const PhenDev &p, const epi_scan_params *q, ScreenCut &C)
     return true;
 }
 
-// The screen's 32-bit offsets reach two bitplanes (planes_fit; the resolve kernel's copy of them exists only then), and
+// The screen's 32-bit offsets reach two bitplanes (planes_fit), and
 // GENERAL tiles bound SST well up to an eighth of the calls missing.
 bool screen_fits(const Dataset &d)
 {
-    return d.sbits && d.missum[d.nsnp] <= (long long)d.nsnp * d.nid / 8;
+    return planes_fit(d) && d.missum[d.nsnp] <= (long long)d.nsnp * d.nid / 8;
 }
 
 // One kind of tile through the screen. tiles: the kind's list on the device.
@@ -2031,15 +2056,15 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
     if (screen) sc.fast_rows = screen_rows(c->d.nid);
     const size_t max_tiles = screen ? scr_piece(c->max_tiles) : c->max_tiles;
     TileLists &tl = c->tl;
-    const bool cached =
-        c->tl_valid && c->tl_bb == bb && c->tl_be == be && c->tl_form == p->form && same_schedule(c->tl_sched, sc);
+    const bool cached = c->tl_valid && c->tl_bb == bb && c->tl_be == be && c->tl_form == p->form &&
+                        same_schedule(c->tl_sched, sc) && (!screen || c->redo);
     TileCursor cur;
     cur.blk = bb;
     bool done = cached;
     if (!cached) {
         tl = TileLists();
         done = build_tiles(c->d, be, p->form, sc, max_tiles, cur, tl);
-        if ((rc = upload_tiles(c, tl))) return rc;
+        if ((rc = upload_tiles(c, tl, screen))) return rc;
         c->tl_bb = bb;
         c->tl_be = be;
         c->tl_form = p->form;
@@ -2077,7 +2102,7 @@ int run_scan(epi_ctx *c, const epi_scan_params *p, const epi_schedule &asked)
         if (done) break;
         tl = TileLists();
         done = build_tiles(c->d, be, p->form, sc, max_tiles, cur, tl);
-        if ((rc = upload_tiles(c, tl))) return rc;
+        if ((rc = upload_tiles(c, tl, screen))) return rc;
         if ((rc = reset_scan(c, false, screen))) return rc;
         pairs += tl.pairs;
     }
@@ -2529,7 +2554,7 @@ int epi_pair_dump(epi_ctx *c, const epi_scan_params *p, int32_t a0, int32_t a1, 
             emit_tile(d, x, x1, y, y1, gen_rows(p->form, sc), gen_cols(p->form, sc),
                       sp && grid(x, x1, TA) && grid(y, y1, 64), sc.dense_missing == 2, all);
         }
-    if ((rc = upload_tiles(c, all))) return rc;
+    if ((rc = upload_tiles(c, all, false))) return rc;
     long long np = (long long)(a1 - a0) * (b1 - b0);
     int32_t *dc = nullptr;
     double *dsum = nullptr, *dF = nullptr, *dF2 = nullptr;
@@ -2589,6 +2614,7 @@ int epi_batch_create(epi_ctx *c, epi_batch **out)
     HIPCHK(c, hipSetDevice(c->device));
     epi_batch *b = new epi_batch();
     b->ctx = c;
+    c->batches.push_back(b);
     for (int f = 0; f < 2; f++) b->sched[f] = default_schedule(f);
     int rc;
     if ((rc = dalloc(c, b->d_qpos, NLIST * NQ)) || (rc = dalloc(c, b->d_qbegin, NLIST * NQ)) ||
@@ -2605,6 +2631,7 @@ void epi_batch_destroy(epi_batch *b)
 {
     if (!b) return;
     epi_ctx *c = b->ctx;
+    c->batches.erase(std::remove(c->batches.begin(), c->batches.end(), b), c->batches.end());
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     drop_graph(b);

@@ -120,7 +120,7 @@ struct MfmaScan {                // one dataset x one phenotype
     const uint32_t *rbits;       // [3][Kw][nsnp] bitplanes: the two rarest classes of the SNP, call present
     const uint32_t *sw[2];       // [Kp / 32][sw_row] codes of the coarse phenotype, one and two digits
     const ScrMarg *sm;           // [nsnp]
-    const uint32_t *sbits;       // [3][nsnp][Kw] bits by SNP (resolve)
+    const uint32_t *sbits;       // [3][nsnp][Kw] bits by SNP (resolve), or null
 };
 
 // Class of outlier 16w+t at a SNP from its code word w (3: no call).

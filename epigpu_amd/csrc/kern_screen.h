@@ -872,7 +872,10 @@ __global__ __launch_bounds__(256) void resolve_kernel(const ResolveArgs A)
             const MfmaScan &S = BATCH ? A.scans[__shfl(mine.z, c)] : A.S;
             const bool on = c < m && a != b;
             const int Kw = S.Kp / 32, nw = on ? S.Kl / 32 : 0;
-            const size_t plane = (size_t)Kw * S.nsnp, oa = (size_t)a * Kw, ob = (size_t)b * Kw;
+            // bits by SNP, or the bitplanes where memory was short
+            const bool by = S.sbits != nullptr;
+            const uint32_t *bits = by ? S.sbits : S.bits;
+            const size_t plane = (size_t)Kw * S.nsnp, sw = by ? 1 : S.nsnp, oa = (size_t)a * (by ? Kw : 1), ob = (size_t)b * (by ? Kw : 1);
             int t[NV];
 #pragma unroll
             for (int i = 0; i < NV; i++) t[i] = 0;
@@ -882,8 +885,8 @@ __global__ __launch_bounds__(256) void resolve_kernel(const ResolveArgs A)
                     uint32_t ga[NG], hb[NG];
 #pragma unroll
                     for (int g = 0; g < NG; g++) {
-                        ga[g] = S.sbits[g * plane + oa + w];
-                        hb[g] = S.sbits[g * plane + ob + w];
+                        ga[g] = bits[g * plane + oa + w * sw];
+                        hb[g] = bits[g * plane + ob + w * sw];
                     }
 #pragma unroll
                     for (int g = 0; g < NG; g++)
