@@ -2031,9 +2031,10 @@ int batch_fetch(epi_batch *b)
 // Clears the counters (hits: that of the hits too) and, before the screen first runs over a tile list, the masks of its blocks.
 int reset_scan(epi_ctx *c, bool hits, bool screen)
 {
+    constexpr uint32_t words = sizeof(Counters) / sizeof(uint32_t), first = offsetof(Counters, screen) / sizeof(uint32_t);
     const size_t n = screen && !c->masks_set ? c->redo_blocks : 0;
-    hipLaunchKernelGGL(scan_reset, dim3((unsigned)std::min<size_t>(1 + n / 1024, 1024)), dim3(256), 0, c->stream, c->count,
-                       hits, c->redo + c->redo_blocks, n);
+    hipLaunchKernelGGL(clear_words, dim3((unsigned)(n / 256 + 1)), dim3(n ? 256 : 64), 0, c->stream,
+                       reinterpret_cast<uint32_t *>(c->count), hits ? 0u : first, words, c->redo + c->redo_blocks, n);
     HIPCHK(c, hipGetLastError());
     if (screen) c->masks_set = true;
     return EPI_OK;
