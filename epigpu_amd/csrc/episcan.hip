@@ -2352,10 +2352,10 @@ int epi_set_hit_capacity(epi_ctx *c, int64_t cap)
 {
     if (!c || cap < 1) return EPI_ERR_ARG;
     HIPCHK(c, hipSetDevice(c->device));
+    c->cap = c->last_nhits = 0;  // a failure leaves no buffer: scans then count their hits and report the overflow
     int rc = dalloc(c, c->hits, (size_t)cap);
     if (rc) return rc;
     c->cap = cap;
-    c->last_nhits = 0;
     return EPI_OK;
 }
 
@@ -2705,12 +2705,12 @@ int epi_batch_set_hit_capacity(epi_batch *b, int64_t cap)
     if (!b || cap < 1) return EPI_ERR_ARG;
     epi_ctx *c = b->ctx;
     HIPCHK(c, hipSetDevice(c->device));
+    drop_graph(b);  // it holds the old buffer
+    b->cap = b->last_nhits = 0;  // as epi_set_hit_capacity
+    b->fetched = false;
     int rc = dalloc(c, b->hits, (size_t)cap);
     if (rc) return rc;
     b->cap = cap;
-    b->last_nhits = 0;
-    b->fetched = false;
-    drop_graph(b);
     return EPI_OK;
 }
 

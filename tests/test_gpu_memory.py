@@ -99,3 +99,30 @@ def test_candidates_from_the_bitplanes(gmiss):
         assert s.last_screen()["digits"] and s.last_screen()["candidates"] > 0
         assert a["nhits"] == b["nhits"] > 0
         assert all(np.array_equal(a[k], b[k]) for k in ("hits", "F64", "F2_64", "block"))
+
+
+def test_failed_hit_capacity():
+    """A hit buffer that cannot be had: scans count their hits, store none and report the overflow; a later one serves again."""
+    nid, nsnp = 700, 1500
+    words = E.synth_genotypes(97, nid, nsnp, 0.1, 0.5, 0.0)
+    y = phenotype("normal", nid, 98)
+    kw = dict(test="f", t1=3.5, t2=10.5)
+    with E.Scanner(0) as s, E.Batch(s) as b:
+        s.set_genotypes(words, nid)
+        s.set_phenotypes(y)
+        b.add_phenotypes(b.add_dataset(words, nid), y)
+        want = s.scan(**kw)
+        b.scan(**kw)
+        assert b.hits(0)["nhits"] == want["nhits"] > 0
+        for x in (s, b):
+            with pytest.raises(E.EpiError):
+                x.set_hit_capacity(1 << 40)
+        g = s.scan(**kw)
+        assert g["nhits"] == want["nhits"] and g["overflow"] and len(g["hits"]) == 0
+        st = b.scan(**kw)
+        assert st["nhits"] == want["nhits"] and st["overflow"] and b.hits(0)["nhits"] == 0
+        for x in (s, b):
+            x.set_hit_capacity(1 << 20)
+        assert np.array_equal(s.scan(**kw)["hits"], want["hits"])
+        b.scan(**kw)
+        assert np.array_equal(b.hits(0)["hits"], want["hits"])
