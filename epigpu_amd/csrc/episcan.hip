@@ -2434,6 +2434,11 @@ int epi_autotune(epi_ctx *c, const epi_scan_params *p, int32_t dims, int32_t rep
     dims &= EPI_TUNE_ROWS | EPI_TUNE_SUPER | EPI_TUNE_MISSING;
     HIPCHK(c, hipSetDevice(c->device));
     if ((rc = ds_marginals(c, c->d))) return rc;
+    // a screened scan picks its tile height itself: the value for other scans is not to be had from its times
+    const int nchr = (int)c->d.chrstart.size(), nblk = nchr * (nchr + 1) / 2;
+    ScreenCut cut;
+    if (screened(c->d, p, block_pairs(c->d, std::max(0, p->blk_begin), p->blk_end <= 0 ? nblk : std::min(nblk, p->blk_end)), cut))
+        dims &= ~EPI_TUNE_ROWS;
     epi_schedule cur = c->sched[p->form];
     double tcur = 0.0;
     int n = 0;
@@ -2753,6 +2758,11 @@ int epi_batch_autotune(epi_batch *b, const epi_scan_params *p, int32_t dims, int
     if (dims == 0) dims = EPI_TUNE_ALL;
     HIPCHK(c, hipSetDevice(c->device));
     const int form = p->form;
+    // the tile height and the queues are those of scans that are not screened
+    std::vector<ScreenCut> cut;
+    std::vector<char> scr;
+    if (batch_screen(b, p, cut, scr) && std::count(scr.begin(), scr.end(), 1) == (long)scr.size())
+        dims &= ~(EPI_TUNE_ROWS | EPI_TUNE_QUEUES);
     epi_schedule cur = b->sched[form];
     double tcur = 0.0;
     int n = 0;

@@ -241,7 +241,8 @@ typedef struct epi_tune_entry {
  * warm-up, then `reps` timed times (median). The winner becomes the
  * context's schedule for p->form. `log` (optional) receives up to log_cap
  * measured candidates, *nlog the number measured. Hit buffers hold the last
- * candidate's hits. */
+ * candidate's hits. A scan that is screened (epi_schedule) leaves fast_rows as
+ * it is. */
 int epi_autotune(epi_ctx *ctx, const epi_scan_params *p, int32_t dims, int32_t reps,
                  epi_schedule *best, double *best_ms, epi_tune_entry *log, int32_t log_cap,
                  int32_t *nlog);
@@ -342,7 +343,8 @@ int epi_batch_get_schedule(epi_batch *batch, int32_t form, epi_schedule *s);
  * the whole batch as a captured graph: one warm-up replay, then the median
  * of `reps` timed replays. The winner becomes the batch's schedule for
  * p->form. `log` (optional) receives up to log_cap measured candidates,
- * *nlog the number measured. Hit buffers hold the last candidate's hits. */
+ * *nlog the number measured. Hit buffers hold the last candidate's hits. A
+ * batch whose scans are all screened leaves fast_rows and queues as they are. */
 int epi_batch_autotune(epi_batch *batch, const epi_scan_params *p, int32_t dims, int32_t reps,
                        epi_schedule *best, double *best_ms, epi_tune_entry *log,
                        int32_t log_cap, int32_t *nlog);

@@ -186,3 +186,29 @@ def test_batch_mixed(scanner, buf, gmiss, dense_missing):
         for words, nid, sizes, y, s in made:
             load(scanner, words, nid, y, sizes)
             assert same_as_exact(scanner, buf, b.hits(s), **kw) > 0
+
+
+def test_autotune_leaves_what_it_cannot_measure(sch):
+    """The tuner does not time values that a screened scan ignores, and keeps them as they were."""
+    nid, nsnp = 1000, 2000
+    words = E.synth_genotypes(111, nid, nsnp, 0.1, 0.5, 0.0)
+    y = phenotype("normal", nid, 112)
+    load(sch, words, nid, y, [nsnp])
+    for rows in (32, 64):
+        sch.set_schedule("mfma", fast_rows=rows, super_a=8, super_b=4)
+        r = sch.autotune(test="i")
+        assert sch.last_screen()["digits"]
+        assert {x["fast_rows"] for x in r["log"]} == {rows} and len(r["log"]) > 2
+        assert sch.schedule("mfma")["fast_rows"] == rows
+        # not screened: both heights are measured
+        assert {x["fast_rows"] for x in sch.autotune(test="f", t1=1.5)["log"]} == {32, 64}
+    with E.Batch(sch) as b:
+        d = b.add_dataset(words, nid)
+        b.add_phenotypes(d, y)
+        for queues in (8, 1):
+            b.set_schedule("mfma", fast_rows=64, queues=queues)
+            r = b.autotune(test="i")
+            assert b.last_screen()["scans"] == 1
+            assert {(x["fast_rows"], x["queues"]) for x in r["log"]} == {(64, queues)} and len(r["log"]) > 2
+        r = b.autotune(test="f", t1=1.5)
+        assert {x["queues"] for x in r["log"]} == {1, 8} and {x["fast_rows"] for x in r["log"]} == {32, 64}
