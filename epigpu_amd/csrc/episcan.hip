@@ -2611,6 +2611,66 @@ int epi_pair_dump(epi_ctx *c, const epi_scan_params *p, int32_t a0, int32_t a1, 
     return hrc;
 }
 
+int epi_screen_dump(epi_ctx *c, const epi_scan_params *p, int32_t digits, int32_t a0, int32_t a1, int32_t b0, int32_t b1,
+                    int32_t *v, float *counts, float *sums)
+{
+    if (!c) return EPI_ERR_ARG;
+    int rc = check_params(c, p);
+    if (rc) return rc;
+    if (p->form != EPI_FORM_MFMA || digits < 1 || digits > 2 || !counts || !sums)
+        return fail(c, EPI_ERR_ARG, "the MFMA form, one or two digits, and both outputs");
+    const Dataset &d = c->d;
+    if (a0 < 0 || b0 < 0 || a1 > d.nsnp || b1 > d.nsnp || a1 <= a0 || b1 <= b0)
+        return fail(c, EPI_ERR_ARG, "dump rectangle out of range");
+    const PhenDev &ph = d.ph[p->phen];
+    if (!planes_fit(d) || !(ph.scr[digits - 1].delta > 0.0))
+        return fail(c, EPI_ERR_RANGE, "the screen does not take this dataset or phenotype");
+    HIPCHK(c, hipSetDevice(c->device));
+    if ((rc = ds_marginals(c, c->d))) return rc;
+    const int TA = screen_rows(d.nid);
+    TileLists all;
+    for (int x = a0; x < a1; x += TA)
+        for (int y = b0; y < b1; y += TILE_B) emit_tile(d, x, std::min(a1, x + TA), y, std::min(b1, y + TILE_B), TA, 32, false, false, all);
+    if (all.count() >= 1u << 23) return fail(c, EPI_ERR_ARG, "dump rectangle too large");  // one launch of 256-thread tiles
+    if ((rc = upload_tiles(c, all, false))) return rc;
+    const size_t n = (size_t)(a1 - a0) * (b1 - b0) * 9;
+    float *out = nullptr;
+    if ((rc = dalloc(c, out, 2 * n))) return rc;
+    ScreenArgs A;
+    memset(&A, 0, sizeof(A));
+    A.S = mfma_scan(d, p->phen, p->phen);
+    A.cut.N = (float)(ph.nV / 64.0);
+    A.cut.vs = (float)(ph.scr[digits - 1].vsum / 64.0);
+    const ScreenDump D = {out, out + n, a0, b0, b1 - b0};
+    const bool nocall = TA == 64 && scr_nocall(A.S.Kl);
+    hipError_t he = hipMemsetAsync(out, 0xFF, 2 * n * sizeof(float), c->stream);  // NaN
+    auto launch = [&](auto kernel, const int4 *tiles, size_t nt) {
+        if (he != hipSuccess || !nt) return;
+        A.tiles = tiles;
+        A.ntiles = (int)nt;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nt), dim3(4 * TA), 0, c->stream, A, D);
+        he = hipGetLastError();
+    };
+    const size_t nf = all.fast.size(), ng = all.gen.size();
+    if (TA == 64) {
+        launch(digits == 1 ? screen_fast_dump<64, 1> : screen_fast_dump<64, 2>, c->tiles, nf);
+        if (nocall) launch(digits == 1 ? screen_gen_dump<64, 1, true> : screen_gen_dump<64, 2, true>, c->tiles + nf, ng);
+        else launch(digits == 1 ? screen_gen_dump<64, 1, false> : screen_gen_dump<64, 2, false>, c->tiles + nf, ng);
+    } else {
+        launch(digits == 1 ? screen_fast_dump<32, 1> : screen_fast_dump<32, 2>, c->tiles, nf);
+        launch(digits == 1 ? screen_gen_dump<32, 1, false> : screen_gen_dump<32, 2, false>, c->tiles + nf, ng);
+    }
+    std::vector<MissPhen> mp(v ? d.nid : 0);
+    if (he == hipSuccess) he = hipMemcpyAsync(counts, out, n * sizeof(float), hipMemcpyDeviceToHost, c->stream);
+    if (he == hipSuccess) he = hipMemcpyAsync(sums, out + n, n * sizeof(float), hipMemcpyDeviceToHost, c->stream);
+    if (he == hipSuccess && v) he = hipMemcpyAsync(mp.data(), ph.mp, mp.size() * sizeof(MissPhen), hipMemcpyDeviceToHost, c->stream);
+    if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
+    dfree(out);
+    if (he != hipSuccess) return fail(c, EPI_ERR_HIP, "screen dump: %s", hipGetErrorString(he));
+    for (size_t k = 0; k < mp.size(); k++) v[k] = mp[k].sv[digits - 1];
+    return EPI_OK;
+}
+
 // ------------------------------------------------------------------ batch --
 
 int epi_batch_create(epi_ctx *c, epi_batch **out)

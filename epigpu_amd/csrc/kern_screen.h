@@ -90,6 +90,12 @@ struct CandSink {
     uint32_t *mask;           // per block, 0 between scans: bit w: the rows SCR_A w on of the block are to be redone
 };
 
+// The sums of the screen for every pair of a rectangle, a > b, instead of its decisions (epi_screen_dump).
+struct ScreenDump {
+    float *n, *s;             // [pair][9] counts and sums of v, both / 64, in genotype order
+    int a0, b0, nb;
+};
+
 struct ScreenArgs {
     MfmaScan S;
     ScreenCut cut;
@@ -213,6 +219,18 @@ __device__ __forceinline__ bool screen_bound(const float n[9], const float s[9],
     return ri * ri * d2 > 4.0f * C.t2s * ssw;
 }
 
+__device__ __forceinline__ void screen_dump(const ScreenDump &D, const MfmaScan &S, int a, int b, const float n[9], const float s[9])
+{
+    const size_t p = (size_t)(a - D.a0) * D.nb + (b - D.b0);
+    const int ca = S.marg[a].cls, cb = S.marg[b].cls;
+#pragma unroll
+    for (int c = 0; c < 9; c++) {
+        const int o = 3 * ((ca >> (2 * (c / 3))) & 3) + ((cb >> (2 * (c % 3))) & 3);
+        D.n[9 * p + o] = n[c];
+        D.s[9 * p + o] = s[c];
+    }
+}
+
 // n rows of weights from global memory into LDS, four loads in flight per thread.
 template <int NT, int ROW>
 __device__ __forceinline__ void scr_stage(uint32_t *wl, const uint32_t *src, int n, int tid)
@@ -277,10 +295,10 @@ __device__ __forceinline__ void scr_append(const CandSink &cs, uint32_t bits, ui
 // (one dword per operand and 64 individuals, coalesced along SNPs) and expands
 // them in registers: no operand passes through LDS, and the waves run
 // without barriers. LDS holds the phenotype's codes, which all waves share.
-template <int TA, int ND>
+template <int TA, int ND, bool DUMP = false>
 __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const ScreenCut &C, const CandSink &cs, int a0,
                                                  int a1, int b0, int b1, uint32_t block0, uint32_t *wl,
-                                                 float4 *mg, float2 *mg2)
+                                                 float4 *mg, float2 *mg2, const ScreenDump &D = {})
 {
     constexpr int NT = scr_threads<TA>(), ROW = sw_row<ND>();
     const uint32_t *sw = S.sw[ND - 1];
@@ -422,6 +440,11 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const Screen
         };
         fill(n, av[2 * bg], av[2 * bg + 1], ma.x, ma.y, ma2.x, mb[bg].x, mb[bg].y);
         fill(s, al[2 * bg], al[2 * bg + 1], ma.z, ma.w, ma2.y, mb[bg].z, mb[bg].w);
+        if constexpr (DUMP) {
+            const int a = aw + 4 * j + 2 * hf + p, b = b0 + 32 * bg + m;
+            if (a < a1 && b < b1 && a > b) screen_dump(D, S, a, b, n, s);
+            return;
+        }
         float u = 0.0f;
 #pragma unroll
         for (int c = 0; c < 9; c++) u = __builtin_fmaf(s[c] * s[c], rcp_above(n[c]), u);
@@ -435,6 +458,7 @@ __device__ __forceinline__ void screen_fast_tile(const MfmaScan &S, const Screen
         }
         __builtin_amdgcn_sched_barrier(0);
     });
+    if constexpr (DUMP) return;
     scr_append<16>(cs, bits, block0, wid, S.tag, [&](int k, int &a, int &b) {
         a = aw + 4 * (k >> 2) + 2 * hf + (k >> 1 & 1);
         b = b0 + 32 * (k & 1) + m;
@@ -477,9 +501,10 @@ __device__ __forceinline__ v4f scr_mfma16x32(const v8i &a, const v8i &b, const v
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 2, 0, 0x84848484, 0, 0x7f7f7f7f);
 }
 
-template <int TA, int ND, bool NC>
+template <int TA, int ND, bool NC, bool DUMP = false>
 __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenCut &C, const CandSink &cs, int a0, int a1,
-                                                int b0, int b1, uint32_t block0, uint32_t *wl, float4 *mg)
+                                                int b0, int b1, uint32_t block0, uint32_t *wl, float4 *mg,
+                                                const ScreenDump &D = {})
 {
     constexpr int TB = 32, NT = scr_threads<TA>(), ROW = sw_row<ND>();
     const uint32_t *sw = S.sw[ND - 1];
@@ -696,6 +721,11 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
                 tc += s[c];
             }
         }
+        if constexpr (DUMP) {
+            const int a = aw + 4 * kq + i, b = bw + 16 * bg + m;
+            if (a < a1 && b < b1 && a > b) screen_dump(D, S, a, b, n, s);
+            return;
+        }
         tc = __builtin_fmaf(C.c0, nc, tc);
         const float zlow = ma2.z + mb2[bg].z - C.zall;
         float u = 0.0f;
@@ -714,6 +744,7 @@ __device__ __forceinline__ void screen_gen_tile(const MfmaScan &S, const ScreenC
         }
         __builtin_amdgcn_sched_barrier(0);
     });
+    if constexpr (DUMP) return;
     scr_append<8>(cs, bits, block0, wid, S.tag, [&](int k, int &a, int &b) {
         a = aw + 4 * kq + (k >> 1);
         b = bw + 16 * (k & 1) + m;
@@ -744,6 +775,26 @@ __global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_gen_kernel(const 
     uint32_t block0;
     if (!scr_half<TA>(t % A.halves, A.halves, (uint32_t)(A.tile0 + t / A.halves), T.z, T.w, block0)) return;
     screen_gen_tile<TA, ND, NC>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, block0, wl, mg);
+}
+
+// The tiles above without decisions.
+template <int TA, int ND>
+__global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_fast_dump(const ScreenArgs A, const ScreenDump D)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_LDS_ROWS * sw_row<ND>()];
+    __shared__ float4 mg[TA + 64];
+    __shared__ float2 mg2[TA];
+    const int4 T = A.tiles[blockIdx.x];
+    screen_fast_tile<TA, ND, true>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, 0, wl, mg, mg2, D);
+}
+
+template <int TA, int ND, bool NC>
+__global__ __launch_bounds__(scr_threads<TA>(), 2) void screen_gen_dump(const ScreenArgs A, const ScreenDump D)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t wl[SCR_GEN_ROWS * sw_row<ND>()];
+    __shared__ float4 mg[2 * (TA + 32)];
+    const int4 T = A.tiles[blockIdx.x];
+    screen_gen_tile<TA, ND, NC, true>(A.S, A.cut, A.cs, T.x, T.y, T.z, T.w, 0, wl, mg, D);
 }
 
 // After the candidates of a launch are resolved: the list is emptied for the next one.

@@ -159,6 +159,7 @@ def _declare(name, L):
             "epi_last_screen": (ctypes.c_int, [vp, _p(i32), _p(i64), _p(i64)]),
             "epi_batch_last_screen": (ctypes.c_int, [vp, _p(i32), _p(i64), _p(i64)]),
             "epi_pair_dump": (ctypes.c_int, [vp, _p(ScanParams), i32, i32, i32, i32, vp, vp, vp, vp]),
+            "epi_screen_dump": (ctypes.c_int, [vp, _p(ScanParams), i32, i32, i32, i32, i32, vp, vp, vp]),
             "epi_batch_create": (ctypes.c_int, [vp, _p(vp)]),
             "epi_batch_destroy": (None, [vp]),
             "epi_batch_add_dataset": (ctypes.c_int, [vp, vp, i32, i32, vp, vp, i32, _p(i32)]),
@@ -702,6 +703,16 @@ class Scanner:
         self._chk(self.L.epi_pair_dump(self.ctx, ctypes.byref(p), a0, a1, b0, b1, _ptr(counts), _ptr(sums),
                                        _ptr(F), _ptr(F2)), "epi_pair_dump")
         return counts, sums, F, F2
+
+    def screen_dump(self, digits, a0, a1, b0, b1, phen=0):
+        """Coarse phenotype v and, per pair, the screen's counts and sums of v (both / 64; NaN where a <= b)."""
+        p = self.params("f", "mfma", 6.5, 10.5, phen)
+        v = np.zeros(self.nid, dtype=np.int32)
+        counts = np.empty((a1 - a0, b1 - b0, 9), dtype=np.float32)
+        sums = np.empty((a1 - a0, b1 - b0, 9), dtype=np.float32)
+        self._chk(self.L.epi_screen_dump(self.ctx, ctypes.byref(p), digits, a0, a1, b0, b1, _ptr(v), _ptr(counts),
+                                         _ptr(sums)), "epi_screen_dump")
+        return v, counts, sums
 
 
 class Batch:

@@ -273,6 +273,16 @@ int epi_pair_dump(epi_ctx *ctx, const epi_scan_params *p, int32_t a0, int32_t a1
                   int32_t b0, int32_t b1, int32_t *counts, double *sums, double *F,
                   double *F2);
 
+/* Debug entry for the screen (see epi_schedule), through the kernels of screened
+ * scans: for every pair of the rectangle, a > b, the nine counts and the sums of
+ * the coarse phenotype of one or two digits that the bound is taken from, both
+ * divided by 64, indexed as in epi_pair_dump (other entries NaN). v (optional,
+ * [nid]) receives the coarse phenotype, integers, 0 where missing. All are
+ * exact: the sums stay below 2^24 units. EPI_ERR_RANGE where the screen takes
+ * no scan of this phenotype. No counterpart in the reference. */
+int epi_screen_dump(epi_ctx *ctx, const epi_scan_params *p, int32_t digits, int32_t a0, int32_t a1,
+                    int32_t b0, int32_t b1, int32_t *v, float *counts, float *sums);
+
 /* ---------------------------------------------------------------- batch ---
  * Many scans in one persistent launch: datasets of different nid and nsnp,
  * each with one or more phenotypes (a scan is one (dataset, phenotype)
