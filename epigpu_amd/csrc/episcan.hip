@@ -48,8 +48,8 @@ using namespace epi;
 namespace {
 
 constexpr int KPAD = 256;
-// The transcode grid has one row of workgroups per 32 individuals, and a grid
-// row index stays below 65536: at most 8191 K-pads of individuals.
+// The grid of tbits_kernel has one row of workgroups per 32 individuals, and a
+// grid row index stays below 65536: at most 8191 K-pads of individuals.
 constexpr int MAX_NID = 65535 / (KPAD / 32) * KPAD;
 constexpr long long QMAX = 8355711;     // largest |q| with three balanced int8 limbs
 constexpr long long ZMAX = 2139062143;  // largest |z| with four balanced int8 limbs
@@ -583,8 +583,9 @@ void encode_screen(const std::vector<int> &P, int Kp, int nd, PhenEnc &e)
 // Phenotype prep (src/EpiOpenCL.c:1364-1376 computes mY and SSY over all nid
 // and the kernel drops -9 values, :135-147; here the missing values are
 // dropped up front). Centre, outliers and fixed-point scale of the MFMA
-// form, the plain form's scaled FP32 values, presence bits.
-int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, int r, PhenEnc &e)
+// form, the plain form's scaled FP32 values, presence bits, the coarse phenotypes of the screen; without `arrays` only
+// what epi_phen_encoding reports.
+int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, int r, bool arrays, PhenEnc &e)
 {
     auto missing = [&](float v) { return v != v || (!nine_value && v == -9.0f); };
     std::vector<int> P;
@@ -659,13 +660,12 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
     // phenotypes far from unit scale neither overflow nor underflow FP32 (F is scale-free)
     int ye = 0;
     if (maxall > 0.0) std::frexp(maxall, &ye);
+    p.fbits = f;
+    p.ybits = ye;
+    p.centre = centre;
+    p.nV = nv;
     const int Kw = Kp / 32;
-    e.w.assign((size_t)(NWP + 3 + NWC) * Kp, 0);
     e.qv.assign(Kp, 0);
-    e.yc.assign(Kp, 0.0f);
-    e.yw.assign((size_t)2 * Kp, 0.0f);
-    e.vb.assign(Kw, 0u);
-    e.mp.assign(Kp, MissPhen{});
     long long qmax2 = 0;
     for (int k : P) {
         const long long q = out[k] ? 0 : std::llround(std::ldexp((double)y[k] - centre, f));
@@ -676,6 +676,13 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
     // q^2 limbs: the smallest shift that fits four limbs (15 when |q| reaches QMAX)
     int zb = 0;
     while (std::llround(std::ldexp((double)qmax2, -zb)) > ZMAX) zb++;
+    p.zbits = zb;
+    if (!arrays) return EPI_OK;
+    e.w.assign((size_t)(NWP + 3 + NWC) * Kp, 0);
+    e.yc.assign(Kp, 0.0f);
+    e.yw.assign((size_t)2 * Kp, 0.0f);
+    e.vb.assign(Kw, 0u);
+    e.mp.assign(Kp, MissPhen{});
     long long qsum = 0;
     double sq = 0.0, ys = 0.0, y2 = 0.0;
     for (int k : P) {
@@ -719,11 +726,6 @@ int encode_phen(epi_ctx *c, const float *y, int nid, int Kp, bool nine_value, in
         p.ouSum += u;
         p.ouSq += u * u;
     }
-    p.fbits = f;
-    p.zbits = zb;
-    p.ybits = ye;
-    p.centre = centre;
-    p.nV = nv;
     p.qV = qsum;
     p.sqV = sq;
     p.ysV = ys;
@@ -744,7 +746,7 @@ int ds_set_phenotypes(epi_ctx *c, Dataset &d, const float *phen, int nphen, int 
     const int Kp = (nid + KPAD - 1) / KPAD * KPAD, Kw = Kp / 32;
     std::vector<PhenEnc> enc(nphen);
     for (int r = 0; r < nphen; r++) {
-        int rc = encode_phen(c, phen + (size_t)r * nid, nid, Kp, nine_value, r, enc[r]);
+        int rc = encode_phen(c, phen + (size_t)r * nid, nid, Kp, nine_value, r, true, enc[r]);
         if (rc) return rc;
     }
     std::vector<PhenDev> ph(nphen);
@@ -2310,7 +2312,7 @@ int epi_phen_encoding(const float *phen, int32_t nid, int32_t flags, epi_phen_in
     if (!phen || !info || nid < 2 || nid > MAX_NID || (flags & ~EPI_PHEN_NINE_IS_VALUE)) return EPI_ERR_ARG;
     PhenEnc e;
     const int Kp = (nid + KPAD - 1) / KPAD * KPAD;
-    const int rc = encode_phen(nullptr, phen, nid, Kp, (flags & EPI_PHEN_NINE_IS_VALUE) != 0, 0, e);
+    const int rc = encode_phen(nullptr, phen, nid, Kp, (flags & EPI_PHEN_NINE_IS_VALUE) != 0, 0, false, e);
     if (rc) return rc;
     memset(info, 0, sizeof(*info));
     info->present = e.p.nV;
