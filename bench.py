@@ -70,29 +70,30 @@ def cpu_baseline(wl, seconds, threads):
 
 
 # HBM bytes per scan (screen and resolve kernels), from the committed rocprofv3 summary of the same workload
-# (FETCH_SIZE + WRITE_SIZE, each scaled by its factor on a copy of known size). A screened scan picks its own tile
-# height; it was profiled with 16 x 2 super-tiles, and other shapes differ only in L2 reuse.
-PROFILED = {("c3", "mfma", 64): ("profiles/screen_kernels_c3_c2.md", "TRAFFIC_BYTES_PER_LAUNCH"),
-            ("c3", "mfma", 32): ("profiles/screen_kernels_c3_c2.md", "TRAFFIC_BYTES_PER_LAUNCH")}
+# (FETCH_SIZE + WRITE_SIZE, each scaled by its factor on a copy of known size). Screened scans only, which pick their own
+# tile height; profiled with 16 x 2 super-tiles, and other shapes differ only in L2 reuse.
+PROFILED = {("c3", "mfma"): ("profiles/screen_kernels_c3_c2.md", "TRAFFIC_BYTES_PER_LAUNCH")}
 
 
-def profiled_traffic(workload, form, sched):
-    path, key = PROFILED.get((workload, form, sched["fast_rows"]), (None, None))
-    if not path or not os.path.exists(os.path.join(ROOT, path)):
-        return None
+def profiled_traffic(workload, form, digits):
+    """(bytes, source) of a scan, or (None, None)."""
+    path, key = PROFILED.get((workload, form), (None, None))
+    if not digits or not path or not os.path.exists(os.path.join(ROOT, path)):
+        return None, None
     for line in open(os.path.join(ROOT, path)):
         f = line.split()
         if len(f) == 2 and f[0] == key:
-            return float(f[1])
-    return None
+            return float(f[1]), path
+    return None, None
 
 
 FP32_PEAK_TFLOPS = 157.3  # MI355X vector FP32
 FP6_PEAK_TOPS = 10066.0  # MI355X dense FP6
 
 
-def roofline(form, wl, kernel_ms, traffic=None, source=None):
-    """MFMA form: 36 N logical INT8 ops per pair (9 cells x N x (count + sum) MACs) against the dense INT8 peak.
+def roofline(form, wl, kernel_ms, digits=0, traffic=None, source=None):
+    """MFMA form: 36 N logical INT8 ops per pair (9 cells x N x (count + sum) MACs) against the dense INT8 peak, and what
+    the scan executed: with `digits` of the screen's coarse phenotype on 6-bit operands, without (0) the exact tiles.
     Plain form: 18 N logical FP32 flops per pair (9 cells x N sum FMAs) against the vector FP32 peak."""
     if form == "mfma":
         ops, peak, bound, note = (36.0 * wl.nid * wl.pairs, INT8_PEAK_TOPS, "mfma",
@@ -106,12 +107,13 @@ def roofline(form, wl, kernel_ms, traffic=None, source=None):
     out = {"bound": bound, "achieved": achieved, "peak": peak, "unit": "TFLOP/s", "frac": achieved / peak,
            "traffic": traffic, "traffic_source": source, "ops_per_pair": ops / wl.pairs, "note": note}
     if form == "mfma":
-        # what the screen executes with a two-digit coarse phenotype: 4 cells (GENERAL tiles 9) x (count + 2 digits)
-        exe = 2.0 * wl.nid * 3 * (4 if wl.gmiss == 0 else 9)
+        # screen: 4 cells (GENERAL tiles 9) x (count + digits); exact tiles: 4 cells x (count + 3 limbs), GENERAL ones 40
+        # MACs. The exact tables of the screen's candidates are not counted.
+        exe = 2.0 * wl.nid * ((1 + digits) * (4 if wl.gmiss == 0 else 9) if digits else 16 if wl.gmiss == 0 else 40)
         out["executed_ops_per_pair"] = exe
         out["executed_achieved"] = exe * wl.pairs / (kernel_ms * 1e-3) / 1e12
-        out["executed_peak"] = FP6_PEAK_TOPS
-        out["executed_frac"] = out["executed_achieved"] / FP6_PEAK_TOPS
+        out["executed_peak"] = FP6_PEAK_TOPS if digits else INT8_PEAK_TOPS
+        out["executed_frac"] = out["executed_achieved"] / out["executed_peak"]
     if form != "mfma":
         # what the plain kernel executes: FAST tiles (no missing call) 4 cell FMAs per individual, GENERAL
         # tiles 9 cell FMAs and one of y^2; a workload with missing calls has them in every tile
@@ -163,6 +165,22 @@ def accuracy(s, wl, form, phen=0):
     return out
 
 
+def timed_hits(wl, r, phen=0, most=4096):
+    """The hits that the timed scan reported (up to `most` of them) against the FP64 oracle."""
+    import oracle as O
+    h = r["hits"][:most]
+    if not len(h):
+        return {"hits_checked": 0}
+    snps, inv = np.unique(np.concatenate([h["snp1"], h["snp2"]]), return_inverse=True)
+    ref = O.pairs(O.unpack(wl.words[snps], wl.nid), wl.y[phen], inv.reshape(2, -1).T.astype(np.int32))
+    rel = lambda x, y: float((np.abs(x - y) / np.maximum(np.abs(y), 1.0)).max())
+    out = {"hits_checked": len(h), "f_relerr_max": rel(r["F64"][:most], ref["F"]),
+           "df_exact": bool((h["df1"] == ref["df1"]).all() and (h["df2"] == ref["df2"]).all())}
+    if wl.test == "i":
+        out["f2_relerr_max"] = rel(r["F2_64"][:most], ref["F2"])
+    return out
+
+
 def stress_hit_sets(E, s, wl, p=1e-4):
     """The whole workload scanned by both kernel forms at thresholds for p < 1e-4 (F^-1(1-p; 8 and 4, N-9)),
     where the null alone gives about p * pairs hits per test: the two forms are independent implementations
@@ -205,8 +223,10 @@ def run_c2(E, s, steps=3):
             if i:
                 kms.append(r["kernel_ms"])
         km = float(np.mean(kms))
+        scr = s.last_screen()
         out[form] = {"kernel_ms": km, "pairs_per_s": wl.pairs / (km * 1e-3), "hits": r["nhits"],
-                     "schedule": s.schedule(form), "roofline": roofline(form, wl, km), "check": accuracy(s, wl, form)}
+                     "schedule": s.schedule(form), "screen": scr, "roofline": roofline(form, wl, km, scr["digits"]),
+                     "check": dict(accuracy(s, wl, form), timed=timed_hits(wl, r))}
         log(f"[bench c2] {form}: {km:.1f} ms kernel, {out[form]['pairs_per_s']:.3e} pairs/s")
     out["mfma_over_plain"] = out["plain"]["kernel_ms"] / out["mfma"]["kernel_ms"]
     out["stress_hit_sets"] = stress_hit_sets(E, s, wl)
@@ -253,7 +273,7 @@ def run_batch(E, s, steps, warmup, tune=True, plain=True, check=True, sched=None
         log(f"[bench c4] step {i}: {st['kernel_ms']:.1f} ms kernel, {st['nhits']} hits")
     elapsed = time.perf_counter() - t0
     out.update(value=bw.pairs * steps / elapsed, unit="pair-tests/s", ms_per_step=elapsed * 1e3 / steps,
-               kernel_ms_per_step=float(np.mean(kms)), schedule=b.schedule("mfma"), grid=st["grid"],
+               kernel_ms_per_step=float(np.mean(kms)), schedule=b.schedule("mfma"), screen=b.last_screen(), grid=st["grid"],
                captures=st["captures"], hits=st["nhits"])
     if check:
         # two scans of the batch against single scans of the same data
@@ -313,7 +333,7 @@ def run_multi(E, s, steps, warmup, nsnp=0, check=True, sched=None):
                        f"(N(0,1), Gamma(2,1), t(5), Bernoulli(0.2)), genotype missing {wl.gmiss}, test {wl.test}",
            "pair_tests_per_step": tests, "value": tests * steps / elapsed, "unit": "pair-tests/s",
            "ms_per_step": elapsed * 1e3 / steps, "kernel_ms_per_step": kernel_ms, "prep_ms": prep_s * 1e3,
-           "items": st["tiles"], "grid": st["grid"], "schedule": b.schedule("mfma"),
+           "items": st["tiles"], "grid": st["grid"], "schedule": b.schedule("mfma"), "screen": b.last_screen(),
            "hits_per_phenotype": [b.hit_count(sc)[0] for sc in scans]}
     logical = 36.0 * wl.nid * tests
     out["roofline"] = {"bound": "mfma", "achieved": logical / (kernel_ms * 1e-3) / 1e12, "peak": INT8_PEAK_TOPS,
@@ -327,6 +347,12 @@ def run_multi(E, s, steps, warmup, nsnp=0, check=True, sched=None):
         log(f"[bench c5] oracle check {out['check']}")
     b.close()
     return out
+
+
+def dtype(form, screened):
+    """int8: 24-bit fixed point in 8-bit limbs, INT32 sums, FP64 statistics, for every value reported; fp6: a screened scan first
+    bounds every pair's statistics, on 6-bit operands with FP32 sums that are exact integers."""
+    return "fp32" if form != "mfma" else "fp6+int8" if screened else "int8"
 
 
 def main():
@@ -391,7 +417,8 @@ def main():
         s.close()
         out = {"metric": METRIC, "value": r["value"], "unit": "pair-tests/s", "n_gpus": 1, "steps": args.steps,
                "warmup": args.warmup, "ms_per_step": r["ms_per_step"], "higher_is_better": True, "scaling": "weak",
-               "vs_baseline": None, "dtype": "int8", "data": "synthetic (seeded generator, see epigpu_amd/workloads.py)",
+               "vs_baseline": None, "dtype": dtype("mfma", r["screen"]["scans"]),
+               "data": "synthetic (seeded generator, see epigpu_amd/workloads.py)",
                "config": {"workload": r.pop("workload"), "form": "mfma"}, "detail": r}
         print(json.dumps(out), flush=True)
         return
@@ -449,22 +476,21 @@ def main():
         found = sum((int(a), int(b)) in hs for a, b, _, _ in wl.planted_pairs)
 
     kernel_ms = float(np.mean(kms))
-    tiles = s.last_tiles()
-    traffic = profiled_traffic(wl.name, args.form, s.schedule(args.form))
+    tiles, scr = s.last_tiles(), s.last_screen()
+    traffic, source = profiled_traffic(wl.name, args.form, scr["digits"])
     out = {
         "metric": METRIC, "value": value, "unit": "pair-tests/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": elapsed * 1e3 / args.steps, "higher_is_better": True,
-        "scaling": "weak", "vs_baseline": None, "dtype": "int8" if args.form == "mfma" else "fp32",
+        "scaling": "weak", "vs_baseline": None, "dtype": dtype(args.form, scr["digits"]),
         "data": "synthetic (seeded generator, see epigpu_amd/workloads.py)",
         "config": {"workload": f"{wl.name}: N={wl.nid}, M={wl.nsnp} ({len(wl.chr_sizes)} chr), "
                                f"{wl.pairs} pairs, test {wl.test}, t1={wl.t1:g}, t2={wl.t2:g}, "
                                f"MAF U{wl.maf}, genotype missing {wl.gmiss}",
                    "form": args.form, "pairs_per_step": wl.pairs},
         "kernel_ms_per_step": kernel_ms,
-        "roofline": roofline(args.form, wl, kernel_ms, traffic,
-                             PROFILED.get((wl.name, args.form, s.schedule(args.form)["fast_rows"]), (None,))[0]),
+        "roofline": roofline(args.form, wl, kernel_ms, scr["digits"], traffic, source),
         "hits": int(r["nhits"]), "planted_found": found,
-        "prep_ms": prep_s * 1e3, "tiles": tiles,
+        "prep_ms": prep_s * 1e3, "tiles": tiles, "screen": scr,
     }
     if not args.no_plain and args.form == "mfma":
         r2 = step("plain")
@@ -477,12 +503,15 @@ def main():
         out["plain_same_hits"] = bool(same)
         log(f"[bench] plain form: {r2['kernel_ms']:.1f} ms kernel; mfma/plain = {out['mfma_over_plain']:.2f}x")
     if not args.no_check:
-        out["check"] = accuracy(s, wl, args.form)
+        out["check"] = dict(accuracy(s, wl, args.form), timed=timed_hits(wl, r))
         log(f"[bench] oracle check: {out['check']}")
         if not args.no_plain and args.form == "mfma":
             out["stress_hit_sets"] = stress_hit_sets(E, s, wl)
             log(f"[bench] stress hit sets: {out['stress_hit_sets']}")
+    # the schedule of scans that are not screened; a screened one takes 64-row tiles from 2000 individuals on, 32 below
     out["config"]["schedule"] = s.schedule(args.form)
+    if scr["digits"]:
+        out["config"]["schedule"]["fast_rows"] = 64 if wl.nid >= 2000 else 32
     if tuned:
         out["autotune"] = tuned
     if not args.no_batch:
