@@ -301,11 +301,10 @@ void drop_phenotypes(Dataset &d)
 void free_dataset(Dataset &d)
 {
     dfree(d.words);
-    dfree(d.mbits);
+    dfree(d.mbits);  // with the arrays behind it
+    d.bits = nullptr;
+    d.dmiss = d.cls = nullptr;
     dfree(d.sbits);
-    dfree(d.bits);
-    dfree(d.dmiss);
-    dfree(d.cls);
     drop_sparse(d);
     for (auto &p : d.ph) free_phen(p);
     d.ph.clear();
@@ -357,15 +356,17 @@ int ds_upload_genotypes(epi_ctx *c, Dataset &d, const int32_t *words, int nid, i
     d.Kw = d.Kp / 32;
     size_t nwords = (size_t)nsnp * d.npack1;
     int rc;
-    const size_t planes = (size_t)3 * d.Kw * nsnp;
-    dfree(d.sbits);
-    if ((rc = dalloc(c, d.mbits, planes)) || (rc = dalloc(c, d.words, nwords)) ||
-        (rc = dalloc(c, d.bits, planes)) || (rc = dalloc(c, d.dmiss, (size_t)4 * nsnp)) ||
-        (rc = dalloc(c, d.cls, (size_t)nsnp)))
-        return rc;
+    // one allocation for what the dataset keeps: bitplanes, bits, dmiss, cls, each on a 256-byte boundary
+    const size_t planes = (size_t)3 * d.Kw * nsnp, room = (planes + 63) / 64 * 64, per = ((size_t)4 * nsnp + 63) / 64 * 64;
+    if ((rc = dalloc(c, d.mbits, 2 * room + per + nsnp)) || (rc = dalloc(c, d.words, nwords))) return rc;
+    d.bits = d.mbits + room;
+    d.dmiss = reinterpret_cast<int32_t *>(d.bits + room);
+    d.cls = d.dmiss + per;
     // Bits by SNP, where the screen can run and memory allows: the lanes of the resolve kernel, one word each,
     // then read a SNP's words in a row (N = 3001, 67,000 hits: resolve 250 -> 156 us; N = 2000: 84 -> 42 us). Allocated last, and
-    // given back to whatever later finds no memory (give_back).
+    // given back to whatever finds no memory (give_back). The old ones are freed here and not first, so that the new ones find their
+    // place: loading another dataset of N = 4000, M = 20000 takes 1.01 and not 1.25 ms.
+    dfree(d.sbits);
     if (planes_fit(d) && hipMalloc((void **)&d.sbits, planes * sizeof(uint32_t)) != hipSuccess) {
         d.sbits = nullptr;
         (void)hipGetLastError();
@@ -1420,8 +1421,8 @@ int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind
 }
 
 // Tile height of a screened scan. The K loop of a small cohort's tile is short, and workgroups of two waves overlap
-// their starts and ends better (kernel time of 64 rows over 32: N = 500 to 1500 1.03 without missing calls and 1.01
-// with 1 %, N = 2000 1.02 and 0.98, N = 3000 0.99 and 0.95, N = 20000 0.99 and 0.97); the list of 64-row tiles is half as
+// their starts and ends better (kernel time of 64 rows over 32: N = 500 to 1500 1.02 to 1.04 without missing calls and
+// 1.01 to 1.03 with 1 or 2 %, N = 2000 1.02 and 0.98, N = 3000 0.99 and 0.95, N = 20000 0.99 and 0.97); the list of 64-row tiles is half as
 // long, which a first scan pays for on the host.
 int screen_rows(int nid) { return nid >= 2000 ? 64 : 32; }
 

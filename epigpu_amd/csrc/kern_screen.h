@@ -7,6 +7,9 @@
 // and resolve_kernel computes the candidates' tables exactly, as integers, and
 // decides them in FP64 with the same code as the exact tiles. The hits and
 // their values are those of the exact tiles.
+// What decides which pairs are dropped has fewer bits than a table: 6-bit digits, FP32 sums and an
+// FP32 decision. The bound below pays for the digits, every sum is an exact integer (screen_dump shows them), and the thresholds'
+// margin covers the decision.
 //
 // Coarse phenotype: v = D0, or v = 32 D1 + D0, with digits representable in FP6 (E2M3:
 // in units of 1/8 the integers 0..16, then steps of 2 to 30 and of 4 to 60),
@@ -21,9 +24,9 @@
 // about 1.8 GHz in the scans).
 //
 // What bounds it: the matrix cores and their power. At N = 8000, M = 50000 without missing calls a scan's
-// kernels take 35 ms (exact 64 x 64 tiles: 92-97 ms): 2.4e14 operations at 6.9 POP/s, against the 8.0 POP/s that
+// kernels take 34.5 ms (exact 64 x 64 tiles: 92-97 ms): 2.4e14 operations at 7.0 POP/s, against the 8.0 POP/s that
 // a register-only loop of this MFMA with five VALU instructions beside each sustains (9.1 without any,
-// 4.8 for v_mfma_i32_32x32x32_i8); the matrix cores are busy 84 % of the cycles, at 1.8 GHz.
+// 4.8 for v_mfma_i32_32x32x32_i8); the matrix cores are busy 81 % of the cycles, at 1.8 GHz.
 //
 // Bound: over a pair's complete cases let P y be the projection of a phenotype
 // onto the cell-constant vectors less the mean, so SSB(y) = |P y|^2. Then
@@ -58,7 +61,8 @@ constexpr int scr_threads() { return 64 * TA / SCR_A; }  // a workgroup takes a 
 constexpr int SCR_REDO = 8;   // candidates per pair slot of a wave (64 pairs) above which the exact tile redoes its pairs
 
 // Per SNP and phenotype: counts and sums of v (one and two digits) of the two rarest classes and
-// the commonest one (present phenotypes), divided by 64 as the kernels' accumulators are, and the sum of z over all calls.
+// the commonest one (present phenotypes; the fourth sum is padding), divided by 64 as the kernels' accumulators are, and
+// the sum of z over all calls.
 struct ScrMarg {
     float n[3], zs;
     float s[2][4];

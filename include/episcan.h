@@ -197,12 +197,13 @@ int epi_set_max_tiles(epi_ctx *ctx, int64_t max_tiles);
  * max(8, nid / 16) calls; dense_missing 0 makes it SPARSE when its SNPs
  * also miss at most 1/150 of their calls on average. The plain form's GENERAL
  * tiles are 16 x 64.
- * MFMA scans and batches of more than a few hundred million pairs times
- * individuals, at thresholds that few pairs pass, are screened: their tiles,
- * whose height follows nid and not fast_rows, first bound every pair's statistics, and
- * only the pairs that could pass are computed exactly, with the same hits and
- * values. fast_rows and queues then have no effect, and SPARSE tiles are kept
- * only where dense_missing is 2. */
+ * MFMA scans of more than a few hundred million pairs times individuals, at
+ * thresholds that few pairs pass, are screened (in a batch, each scan by
+ * itself, where those together have as many): their tiles, whose height follows nid
+ * and not fast_rows, first bound every pair's statistics, and only the pairs
+ * that could pass are computed exactly, with the same hits and values.
+ * fast_rows and queues then have no effect, and SPARSE tiles are screened as two
+ * GENERAL ones, except where dense_missing is 2. */
 typedef struct epi_schedule {
     int32_t fast_rows;  /* MFMA form: 64 or 32; plain form: 32 or 16 */
     int32_t super_a;    /* tiles are issued in super-tiles of super_a x super_b */

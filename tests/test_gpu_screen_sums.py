@@ -53,3 +53,23 @@ def test_sums_are_exact(scanner, nid, gmiss, kind):
         assert np.array_equal(64.0 * n[below], want_n[below])
         assert np.array_equal(64.0 * s[below], want_s[below])
         assert np.isnan(n[~below]).all() and np.isnan(s[~below]).all()
+
+
+def test_sums_of_a_large_cohort(scanner):
+    """300,000 individuals: one digit alone is coarse enough for its sums to stay exact."""
+    nid, nsnp = 300000, 40
+    words = E.synth_genotypes(7, nid, nsnp, 0.1, 0.5, 0.02)
+    codes = S.unpack(words, nid)
+    for kind in ("normal", "casecontrol"):
+        y = phenotype(kind, nid, 8)
+        scanner.set_genotypes(words, nid)
+        scanner.set_phenotypes(y)
+        v, n, s = scanner.screen_dump(1, 0, nsnp, 0, nsnp)
+        assert 0 < np.abs(v).sum() < 1 << 24
+        want_n, want_s = expected(codes, v.astype(np.float64), np.ones(nid, bool), np.arange(nsnp), np.arange(nsnp))
+        below = np.tril(np.ones((nsnp, nsnp), bool), -1)
+        print(f"sums nid={nid} {kind} largest {np.abs(want_s).max()}", flush=True)
+        assert np.array_equal(64.0 * n[below], want_n[below]) and np.array_equal(64.0 * s[below], want_s[below])
+        if kind == "normal":
+            with pytest.raises(E.EpiError):
+                scanner.screen_dump(2, 0, nsnp, 0, nsnp)
