@@ -6,7 +6,7 @@
 // every pair whose true statistics could pass the thresholds (candidates),
 // and resolve_kernel computes the candidates' tables exactly, as integers, and
 // decides them in FP64 with the same code as the exact tiles. The hits and
-// their values are those of the exact tiles.
+// their values are those of exact tiles of the same height.
 // What decides which pairs are dropped has fewer bits than a table: 6-bit digits, FP32 sums and an
 // FP32 decision. The bound below pays for the digits, every sum is an exact integer (screen_dump shows them), and the thresholds'
 // margin covers the decision.
