@@ -1372,11 +1372,11 @@ struct ScreenKind {
 
 // Launches of the bound and the resolve kernel, a list of candidates at a time; or, once the host has their counters, of the redo of K's blocks.
 template <bool GEN, int TA, int TB>
-int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind &K, bool redo)
+int launch_screen(epi_ctx *c, ScreenArgs &G, const HitSink &hs, const ScreenKind &K, uint32_t redo)
 {
     if (redo) {
         const RedoArgs D = {G.S, nullptr, hs, K.tiles, K.count, K.redo, K.mask};
-        hipLaunchKernelGGL((redo_kernel<TA, TB, GEN, false>), dim3(2 * c->ncu), dim3(256), 0, c->stream, D);
+        hipLaunchKernelGGL((redo_kernel<TA, TB, GEN, false>), dim3(std::min(redo, 1u << 22)), dim3(256), 0, c->stream, D);
         HIPCHK(c, hipGetLastError());
         c->last_launches++;
         return EPI_OK;
@@ -1471,15 +1471,16 @@ int launch_pairs(epi_ctx *c, const epi_scan_params *p, const epi_schedule &sc, c
                              kg = {B.tiles + nf + ns, ng, B.cs.count + 4, B.cs.redo + os, B.cs.mask + os, B.emptied};
             const bool again = counts != nullptr;
             const bool lf = sf && (!again || counts[1]), ls = ss && (!again || counts[3]), lg = sg && (!again || counts[5]);
+            const uint32_t rf = again ? counts[1] : 0u, rs = again ? counts[3] : 0u, rg = again ? counts[5] : 0u;
             int rc = EPI_OK;
             if (sc.fast_rows == 64) {
-                if (lf) rc = launch_screen<false, 64, 64>(c, G, hs, kf, again);
-                if (ls && !rc) rc = launch_screen<true, 64, 64>(c, G, hs, ks, again);
-                if (lg && !rc) rc = launch_screen<true, 64, 32>(c, G, hs, kg, again);
+                if (lf) rc = launch_screen<false, 64, 64>(c, G, hs, kf, rf);
+                if (ls && !rc) rc = launch_screen<true, 64, 64>(c, G, hs, ks, rs);
+                if (lg && !rc) rc = launch_screen<true, 64, 32>(c, G, hs, kg, rg);
             } else {
-                if (lf) rc = launch_screen<false, 32, 64>(c, G, hs, kf, again);
-                if (ls && !rc) rc = launch_screen<true, 32, 64>(c, G, hs, ks, again);
-                if (lg && !rc) rc = launch_screen<true, 32, 32>(c, G, hs, kg, again);
+                if (lf) rc = launch_screen<false, 32, 64>(c, G, hs, kf, rf);
+                if (ls && !rc) rc = launch_screen<true, 32, 64>(c, G, hs, ks, rs);
+                if (lg && !rc) rc = launch_screen<true, 32, 32>(c, G, hs, kg, rg);
             }
             if (rc || again) return rc;
         }

@@ -810,9 +810,9 @@ __global__ void empty_list(uint32_t *count, uint32_t cap, unsigned long long *to
 
 // --------------------------------------------------------------- redo ----
 // Blocks that the screen handed back, through the exact tiles of 32 rows (16, where only one of the two waves asked for
-// it): a persistent grid over the device's count of them. (One exact tile per wave, half of its rows unused,
-// N = 3000, M = 30000 with 1.5 % of the pairs hits: 44.3 ms, now 33.3.) Each marked block is in the list once;
-// its mask is left at 0 for the next scan.
+// it): a workgroup per block where the host knows their number (single scans), otherwise a persistent grid. (One exact
+// tile per wave, half of its rows unused, N = 3000, M = 30000 with 1.5 % of the pairs hits: 44.3 ms; a persistent grid over
+// blocks 33.3, now 32.6.) Each marked block is in the list once; its mask is left at 0 for the next scan.
 struct RedoArgs {
     MfmaScan S;               // single scans
     const MfmaScan *scans;    // batches: by scan id
@@ -832,7 +832,7 @@ __global__ __launch_bounds__(256, 2) void redo_kernel(const RedoArgs A)
     const uint32_t n = A.count[1];
     const DumpSink nodump = {};
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-        const uint32_t r = __builtin_amdgcn_readfirstlane(A.redo[i]), half = __builtin_amdgcn_readfirstlane(A.mask[r]);
+        const uint32_t r = __builtin_amdgcn_readfirstlane(A.redo[gridDim.x == n ? xcd_tile(i, n) : i]), half = __builtin_amdgcn_readfirstlane(A.mask[r]);
         __syncthreads();  // the mask is read, and the previous tile is done with LDS
         if (threadIdx.x == 0) A.mask[r] = 0u;
         int4 T = A.tiles[r / NBLK];
